@@ -12,8 +12,8 @@
 //
 // The next block's K / V are fetched into registers behind the score products and stored to the other LDS
 // buffer after the value products: one barrier per block.  A wave fetches keys of ONE 16-key group, which
-// lie in one page (pages of 16 tokens or more), so its page is a scalar and every lane offset a loop
-// constant; the sequence's page list sits in LDS.  O and l are rescaled on blocks that raise some column's
+// lie in one page (pages of 16 tokens or more), so its page and the group's place in the page are scalars and
+// every lane offset a loop constant; the sequence's page list sits in LDS.  O and l are rescaled on blocks that raise some column's
 // maximum.  (Letting the maximum lag by up to 2^8 saves ~3 % but then the largest weight is not exactly 1
 // and its rounding counts: error against 64 bits 3.2e-3 instead of 3.0e-3.)
 //
@@ -128,27 +128,27 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
 
   // staging: wave w moves keys of group sg = w / WPG; its part of the group's chunks starts at `sub`
   const int sg = w / WPG, sub = (w % WPG) * 64 + lane;
-  const int koff_page = (16 * sg) & (bs - 1);
   int k_src[KU], k_dst[KU], v_src[VU], v_dst[VU];
 #pragma unroll
   for (int u = 0; u < KU; ++u) {
     const int i = sub + u * 64 * WPG, key = i / (DK / 8), c8 = i % (DK / 8);
-    k_src[u] = (koff_page + key) * DK + c8 * 8;
+    k_src[u] = key * DK + c8 * 8;
     k_dst[u] = (16 * sg + key) * KS + c8 * 8;
   }
 #pragma unroll
   for (int u = 0; u < VU; ++u) {
     const int i = sub + u * 64 * WPG, ch = i >> 1;
-    v_src[u] = ch * bs + koff_page + 8 * (i & 1);
+    v_src[u] = ch * bs + 8 * (i & 1);
     v_dst[u] = ch * kVS + 16 * sg + 8 * (i & 1);
   }
   const int last_page = npages - 1;
   u32x4 kr[NMAP][KU], vr[VU];
   auto load_block = [&](int k0) {
     // keys at or past kend read a clamped page or stale slots: their scores are masked and their V zeroed
-    const int pg = __builtin_amdgcn_readfirstlane(lds_bt[min((k0 + 16 * sg) >> a.bs_shift, last_page)]);
-    const __bf16* kb = k_cache + (static_cast<int64_t>(pg) * G + NMAP * g) * bs * DK;
-    const __bf16* vb = v_cache + (static_cast<int64_t>(pg) * GV + gv) * DV * bs;
+    const int key = k0 + 16 * sg, at = key & (bs - 1);   // (a page may hold several blocks)
+    const int pg = __builtin_amdgcn_readfirstlane(lds_bt[min(key >> a.bs_shift, last_page)]);
+    const __bf16* kb = k_cache + ((static_cast<int64_t>(pg) * G + NMAP * g) * bs + at) * DK;
+    const __bf16* vb = v_cache + (static_cast<int64_t>(pg) * GV + gv) * DV * bs + at;
 #pragma unroll
     for (int e = 0; e < NMAP; ++e)
 #pragma unroll

@@ -1042,14 +1042,14 @@ def test_flash_attention_edges(H, G, d, dv, window, keep, bs):
 
 @pytest.mark.parametrize("H,G", [(4, 4), (8, 2), (24, 8)])
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 4), (64, 70)])
-def test_flash_two_maps_edges(H, G, window, keep):
+def test_flash_two_maps_edges(H, G, window, keep, bs=16):
     torch.manual_seed(H + window)
     lens, starts = [64, 65, 1, 130, 17], [0, 63, 0, 62, 255]
-    md = ragged(lens, starts, list(range(5)), width=32)
+    md = ragged(lens, starts, list(range(5)), bs=bs, width=32)
     T, nb, d, dv = int(md["seq_qstart"][-1]), md["num_pages"], 64, 128
     q = torch.randn(T, 2 * H, d).to(torch.bfloat16)
     gate = torch.randn(T, H * dv).to(torch.bfloat16)
-    k, v = torch.randn(nb, 2 * G, 16, d).to(torch.bfloat16), torch.randn(nb, G, dv, 16).to(torch.bfloat16)
+    k, v = torch.randn(nb, 2 * G, bs, d).to(torch.bfloat16), torch.randn(nb, G, dv, bs).to(torch.bfloat16)
 
     def run(m, *t):
         q, k, v, gate = t
@@ -1062,6 +1062,15 @@ def test_flash_two_maps_edges(H, G, window, keep):
     # the join divides by the root mean square of a1 - lam a2, which amplifies the maps' rounding by at
     # most |a| / rms(a1 - lam a2): a few units of 2^-8 of values up to 4
     assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
+
+
+@pytest.mark.parametrize("bs", [64, 128, 512])
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 70)])
+def test_flash_attention_wide_pages(window, keep, bs):
+    """Pages of one, two and more key blocks, every width pair: the later blocks of a page."""
+    for H, G, d, dv in ((4, 4, 64, 64), (6, 2, 128, 128), (5, 1, 256, 192)):
+        test_flash_attention_edges(H, G, d, dv, window, keep, bs)
+    test_flash_two_maps_edges(4, 2, window, keep, bs)
 
 
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
