@@ -192,9 +192,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
 
   // ---- global -> register staging of one K/V block --------------------------------------
   // Wave w stages keys 16 w .. 16 w + 15 of the block for BOTH tensors: with BS >= 16 those
-  // keys sit in one page, so the page lookup is wave-uniform (one LDS read + readfirstlane,
-  // a scalar base) and every lane offset is a loop constant - the per-lane 64-bit address
-  // arithmetic of 8 independent lookups was ~70 VALU per block and wave.
+  // keys sit in one page, so the page lookup and the keys' place in the page are wave-uniform
+  // (one LDS read + readfirstlane, a scalar base) and every lane offset is a loop constant - the
+  // per-lane 64-bit address arithmetic of 8 independent lookups was ~70 VALU per block and wave.
   //   K: lane l, chunk u -> key row 16 w + 4 u + (l >> 4), dims 8 (l & 15): each
   //      instruction reads 4 contiguous 256 B rows (1 KiB);
   //   V: lane l, chunk u -> d-row 32 u + (l >> 1), keys 16 w + 8 (l & 1) .. + 7: each
@@ -208,9 +208,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
   constexpr bool kBoth = NW == 4;
   const bool stage_k = kBoth || wid < 4;
   const bool stage_v = kBoth || wid >= 4;
-  const int w_keyoff = (16 * sg) & (BS - 1);                // group's first key in its page
-  const int k_lane = (lane >> 4) * kD + 8 * (lane & 15) + w_keyoff * kD;
-  const int v_lane = (lane >> 1) * BS + 8 * (lane & 1) + w_keyoff;
+  const int k_lane = (lane >> 4) * kD + 8 * (lane & 15);
+  const int v_lane = (lane >> 1) * BS + 8 * (lane & 1);
   const int k_lds = (16 * sg + (lane >> 4)) * kKStride + 8 * (lane & 15);
   const int v_lds = (lane >> 1) * kVStride + 16 * sg + 4 * (lane & 1);  // permuted: see kVStride
   // LDS only (the launcher rejects bt_stride > kBtLds): a select between the LDS copy and the
@@ -222,11 +221,12 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
   // (no invariant on the cache contents is needed).
   u32x4 kr[kBoth ? kChunks : 1], vr[kChunks];  // NW = 8: one register set (vr) per wave
   auto load_block = [&](int kb) {
-    const int pi = min((kb * kKB + 16 * sg) >> p.bs_shift, last_page);
+    const int key = kb * kKB + 16 * sg, at = key & (BS - 1);   // (a page may hold several blocks)
+    const int pi = min(key >> p.bs_shift, last_page);
     const int pg = __builtin_amdgcn_readfirstlane(lds_bt[pi]);
     const uint64_t off = static_cast<uint64_t>(static_cast<uint32_t>(pg * p.n_kv_heads + hk)) << pshift;
-    const uint16_t* kb_ = p.k_cache + off;
-    const uint16_t* vb_ = p.v_cache + off;
+    const uint16_t* kb_ = p.k_cache + off + at * kD;
+    const uint16_t* vb_ = p.v_cache + off + at;
     if constexpr (kBoth) {
 #pragma unroll
       for (int u = 0; u < kChunks; ++u)

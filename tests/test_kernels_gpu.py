@@ -202,6 +202,18 @@ def test_flash_prefill_8_waves_bit_identical(dtype, hq, hkv):
     close(outs[8], exp, 1.5e-2, 2e-2)
 
 
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("bs", [64, 128, 512])
+def test_flash_prefill_wide_pages(waves, bs):
+    """Pages of one, two and more key blocks: the later blocks of a page."""
+    try:
+        ops.set_flash_waves(waves)
+        for hq, hkv in ((32, 8), (24, 8)):
+            test_attention_prefill("flash", torch.bfloat16, hq, hkv, bs)
+    finally:
+        ops.set_flash_waves(int(os.environ.get("ATTA_FLASH_WAVES", "4")))
+
+
 @pytest.mark.parametrize("hq,hkv", [(32, 8), (64, 8), (24, 8)])
 def test_flash_prefill_long_chunked(hq, hkv):
     """2.6k-token prompt (the fan-out synthesis size) plus a chunk after a 3k cached prefix
