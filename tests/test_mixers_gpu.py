@@ -1219,6 +1219,43 @@ def test_chunked_scans_keep_earlier_tokens(bad):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_chunked_scans_pass_non_finite_inputs(dt, bad):
+    """One non-finite entry in any input of a recurrence: finite results and states exactly where the token-by-token
+    reference has them, rows before it and other sequences untouched."""
+    torch.manual_seed(1)
+    H, d, dv, hit, col = 2, 64, 64, 41, 5       # token 41: third chunk of the first portion
+    md = ragged([170, 140], [0, 0], [0, 1], width=64)
+    T, g, z, zz = 310, cuda(md), torch.zeros(H), torch.zeros(H * d)
+    at = (md["positions"], md["seq_qstart"], md["seq_slot"])
+    at_g = (g["positions"], g["seq_qstart"], g["seq_slot"])
+    q, k, v, wide = (torch.randn(T, H * d).to(dt) for _ in range(4))
+    one, two = torch.randn(T, H).to(dt), torch.randn(T, H).to(dt)
+    tab, pw = torch.zeros(T, 0), mx.retention_powers([0.9, 0.99], "cpu")
+    for name, inputs, rest, last in (
+            ("gated_delta_rule", (torch.cat([q, k, v], 1), one, two), (z, z), (H, H, d, dv)),
+            ("gated_delta_rule", (torch.cat([q, k, v], 1), one, wide), (z, zz), (H, H, d, dv)),
+            ("forget_gate_scan", (q, wide, v), (zz, zz), (H, d, dv)),
+            ("state_space_scan", (v, k, q, one), (z, z, z), (H, H, d, dv)),
+            ("retention", (q, k, v), (pw, tab), (H, d, dv))):
+        def run(mod, inputs, at, dev):
+            r = rest if mod is mx or name != "retention" else (pw[:, 1], tab)
+            st = torch.zeros(2, H, d, dv, device=dev)
+            o = getattr(mod, name)(*(t.to(dev) for t in (*inputs, *r)), st, *at, *last)
+            return o.cpu(), st.cpu()
+
+        fine = run(mx, inputs, at_g, "cuda")[0]
+        for i, t in enumerate(inputs):
+            for c in sorted({min(col, t.shape[1] - 1), t.shape[1] // 2, t.shape[1] - 1}):
+                broken = [x.clone() for x in inputs]
+                broken[i][hit, c] = bad
+                got, want = run(mx, broken, at_g, "cuda"), run(mref, broken, at, "cpu")
+                assert torch.equal(got[0][:hit], fine[:hit]) and torch.equal(got[0][170:], fine[170:]), (name, i, c)
+                for a, b in zip(got, want):
+                    assert torch.equal(torch.isfinite(a), torch.isfinite(b)), (name, i, c)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("lens", [[1] * 9, [1, 4, 1, 3, 1, 2, 1, 1, 1], [1, 40, 1, 1, 17, 1, 5, 1, 1]])
 @pytest.mark.parametrize("d,dv", [(128, 128), (64, 72), (60, 10), (1, 64), (129, 68), (256, 100), (200, 7)])
 def test_step_scans(dt, lens, d, dv):
