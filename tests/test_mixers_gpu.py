@@ -1255,6 +1255,51 @@ def test_chunked_scans_pass_non_finite_inputs(dt, bad):
                     assert torch.equal(torch.isfinite(a), torch.isfinite(b)), (name, i, c)
 
 
+def portions_and_rows(call, n, S):
+    """``call(rows, at, state)`` for S portions of n tokens at once (chunks) and row by row (decode form): the rows'
+    results and states of both; a portion's rows lie together."""
+    whole = cuda(ragged([n] * S, [3] * S, list(range(S)), width=64))
+    one = cuda(ragged([1] * S, [3] * S, list(range(S)), width=64))
+    got = call(torch.arange(S * n, device="cuda"), (whole["positions"], whole["seq_qstart"], whole["seq_slot"]))
+    rows = torch.arange(S, device="cuda") * n
+    outs, st = torch.empty_like(got[0]), None
+    for t in range(n):
+        o, st = call(rows + t, (one["positions"] + t, one["seq_qstart"], one["seq_slot"]), st)
+        outs[rows + t] = o
+    return got, (outs, st)
+
+
+def rms_error(x, want):
+    return float((((x.double() - want) / want) ** 2).mean().sqrt()) * 2.0 ** 24
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+def test_chunked_forget_gate_rounds_like_rows(dt):
+    """Decays and queries alone (one channel of one head sees a state of ones): errors against 64 bits at the level of
+    the decode form's.  Same roundings per token, 2^16 samples of them: 5 % is ten times what the statistics leave."""
+    torch.manual_seed(3)
+    H, d, dv, S, n = 32, 64, 4, 64, 20
+    f, q = (torch.randn(S * n, H * d, device="cuda") - 2).to(dt), torch.zeros(S * n, H, d, device="cuda").to(dt)
+    q[:, :, 5] = (3 * torch.randn(S * n, H, device="cuda")).to(dt)
+    v, zero = torch.zeros(S * n, H * dv, device="cuda").to(dt), torch.zeros(H * d, device="cuda")
+
+    def run(f):
+        def call(rows, at, st=None):
+            st = torch.ones(S, H, d, dv, device="cuda") if st is None else st
+            o = mx.forget_gate_scan(q.flatten(1)[rows], f[rows], v[rows], zero, zero, st, *at, H, d, dv)
+            return o[..., 0], st
+        return portions_and_rows(call, n, S)
+
+    want = torch.nn.functional.silu(q[:, :, 5].double())
+    chunk, row = run(torch.full_like(f, 80.0))      # decays of 1: the queries' error
+    assert rms_error(chunk[0], want) <= 1.05 * rms_error(row[0], want)
+    chunk, row = run(f)
+    prod = torch.sigmoid(f.double()).view(S, n, H, d).cumprod(1)
+    for a, b, w in ((chunk[0], row[0], want * prod[..., 5].reshape(S * n, H)),
+                    (chunk[1][..., 0], row[1][..., 0], prod[:, -1])):
+        assert rms_error(a, w) <= 1.05 * rms_error(b, w)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("lens", [[1] * 9, [1, 4, 1, 3, 1, 2, 1, 1, 1], [1, 40, 1, 1, 17, 1, 5, 1, 1]])
 @pytest.mark.parametrize("d,dv", [(128, 128), (64, 72), (60, 10), (1, 64), (129, 68), (256, 100), (200, 7)])
