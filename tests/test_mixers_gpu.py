@@ -1301,6 +1301,46 @@ def test_chunked_forget_gate_rounds_like_rows(dt):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("rate", [1.0, 5.0, 16.0])
+@pytest.mark.parametrize("x", [-17.0, -9.0, -3.0, 1.0])
+def test_chunked_delta_decay_rounds_like_rows(dt, rate, x):
+    """A state that only decays (beta 0), fast and slow channels, one decay per channel: its error against 64 bits at
+    the level of the decode form's (15 %: the products of the decays are taken in another order, by which the fp32
+    forms, with equal decays, differ by 7 %); and after 1024 equal tokens at most 2 roundings of 2^-24 each - the
+    decay's (the exponential is good to one) and the product's - off."""
+    torch.manual_seed(4)
+    H, d, dv, S, n = 16, 64, 4, 64, 12
+    a_log = torch.log(torch.full((H,), rate, device="cuda"))
+    used = torch.exp(a_log.double())[:, None]
+    bias = x + torch.rand(H * d, device="cuda")
+
+    def scan(dec, rows, at, st):
+        T = rows.numel()
+        qkv = torch.ones(T, 2 * H * d + H * dv, device="cuda").to(dt)
+        beta = torch.full((T, H), -200.0, device="cuda").to(dt)
+        o = mx.gated_delta_rule(qkv, beta, dec[rows], a_log, bias, st, *at, H, H, d, dv)
+        return o, st
+
+    dec = torch.randn(S * n, H * d, device="cuda").to(dt)
+    log = -used * torch.nn.functional.softplus(dec.double() + bias.double(), threshold=60).view(S, n, H, d).sum(1)
+    seen = log > -60
+    (_, chunk), (_, row) = portions_and_rows(
+        lambda rows, at, st=None: scan(dec, rows, at, torch.ones(S, H, d, dv, device="cuda") if st is None else st),
+        n, S)
+    if seen.any():
+        want = torch.exp(log)[seen]
+        assert rms_error(chunk[..., 0][seen], want) <= 1.15 * rms_error(row[..., 0][seen], want)
+    md = cuda(ragged([1024], [5], [0], width=80))
+    at = (md["positions"], md["seq_qstart"], md["seq_slot"])
+    _, st = scan(torch.zeros(1024, H * d, device="cuda").to(dt), torch.arange(1024, device="cuda"), at,
+                 torch.ones(1, H, d, dv, device="cuda"))
+    log = -used * torch.nn.functional.softplus(bias.double(), threshold=60).view(H, d) * 1024
+    slow = log > -16     # (per token: an exponent whose own rounding is below the decay's)
+    err = (st[0, ..., 0].double() / torch.exp(log) - 1).abs()[slow]
+    assert err.numel() == 0 or float(err.max()) <= 1024 * 2.0 ** -23
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("lens", [[1] * 9, [1, 4, 1, 3, 1, 2, 1, 1, 1], [1, 40, 1, 1, 17, 1, 5, 1, 1]])
 @pytest.mark.parametrize("d,dv", [(128, 128), (64, 72), (60, 10), (1, 64), (129, 68), (256, 100), (200, 7)])
 def test_step_scans(dt, lens, d, dv):
