@@ -1300,6 +1300,70 @@ def test_chunked_forget_gate_rounds_like_rows(dt):
         assert rms_error(a, w) <= 1.05 * rms_error(b, w)
 
 
+@pytest.mark.parametrize("name", ["delta", "delta per channel", "forget gate", "state space", "retention"])
+def test_chunked_results_round_like_rows(name):
+    """32-bit inputs, portions of 60 tokens: results as close to 64 bits as the decode form's (sums of 128 terms per
+    token there, of 128 and 16 here).  2^18 results leave the errors within 1 %; 5 % more for the delta rule's
+    triangular system, whose roundings decode rows do not have."""
+    torch.manual_seed(6)
+    H, d, S, n = 4, 128, 8, 60
+    q, k, v, wide = (torch.randn(S * n, H * d, device="cuda") for _ in range(4))
+    one, two = torch.randn(S * n, H, device="cuda") - 2, torch.randn(S * n, H, device="cuda")
+    z, zz, lower = torch.zeros(H, device="cuda"), torch.zeros(H * d, device="cuda"), 0.9 * torch.rand(H * d).cuda()
+    decays = [0.9, 0.97, 0.99, 0.999]
+    tab, pw = torch.zeros(S * n, 0, device="cuda"), mx.retention_powers(decays, "cuda")
+    start = torch.randn(S, H, d, d, device="cuda")
+
+    def call(rows, at, st=None):
+        st = start.clone() if st is None else st
+        x = [t[rows] for t in (q, k, v, wide, one, two)]
+        if name == "forget gate":
+            o = mx.forget_gate_scan(x[0], x[3], x[2], zz, lower, st, *at, H, d, d)
+        elif name == "state space":
+            o = mx.state_space_scan(x[2], x[1], x[0], x[4], z, z, z, st, *at, H, H, d, d)
+        elif name == "retention":
+            o = mx.retention(x[0], x[1], x[2], pw, tab[rows], st, *at, H, d, d)
+        else:
+            wide_form = name == "delta per channel"
+            o = mx.gated_delta_rule(torch.cat(x[:3], 1), x[5], x[3] if wide_form else x[4], z, zz if wide_form else z,
+                                    st, *at, H, H, d, d)
+        return o, st
+
+    chunk, row = portions_and_rows(call, n, S)
+    # the recurrence in 64 bits: S = a S + k u^T
+    a, kk, qq, vv = (t.double().view(S, n, H, d) for t in (torch.sigmoid(wide.double()), k, q, v))
+    beta = None
+    sp = torch.nn.functional.softplus
+    if name == "forget gate":
+        lo = lower.double().view(H, d)
+        a = lo + (1 - lo) * a
+        kk, qq = 1 - a, torch.nn.functional.silu(qq)
+    elif name == "state space":
+        dt = sp(one.double()).view(S, n, H, 1)
+        a, kk = torch.exp(-dt).expand(S, n, H, d), kk * dt
+    elif name == "retention":
+        a, kk = torch.tensor(decays, dtype=torch.float64, device="cuda").view(H, 1).expand(S, n, H, d), kk * d ** -0.5
+    else:
+        wide_form = name == "delta per channel"
+        a = torch.exp(-sp((wide if wide_form else one).double().view(S, n, H, -1))).expand(S, n, H, d)
+        qq, kk = (t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6) for t in (qq, kk))
+        qq = qq * d ** -0.5
+        beta = torch.sigmoid(two.double()).view(S, n, H, 1)
+    st, want = start.double(), []
+    for t in range(n):
+        st = st * a[:, t, :, :, None]
+        u = vv[:, t] if beta is None else beta[:, t] * (vv[:, t] - (st * kk[:, t, :, :, None]).sum(2))
+        st = st + kk[:, t, :, :, None] * u[:, :, None]
+        want.append((st * qq[:, t, :, :, None]).sum(2))
+    want = torch.stack(want, 1).reshape(S * n, H, d)
+
+    def error(got, w):
+        return float((got.double() - w).norm() / w.norm())
+
+    assert error(chunk[0], want) <= 1.055 * error(row[0], want)
+    assert error(chunk[1], st) <= 1.055 * error(row[1], st)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("rate", [1.0, 5.0, 16.0])
 @pytest.mark.parametrize("x", [-17.0, -9.0, -3.0, 1.0])
