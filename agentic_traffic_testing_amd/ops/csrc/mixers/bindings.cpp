@@ -369,7 +369,7 @@ void diff_combine(at::Tensor out, const at::Tensor& a, const c10::optional<at::T
 // scratch of the chunked recurrences, where the batch takes them
 c10::optional<at::Tensor> scan_records(const at::Tensor& like, int64_t T, int64_t S, int64_t H, int64_t dk,
                                        int64_t dv, int mode) {
-  if (!mixk::scan_use_chunks(T, S, static_cast<int>(dk))) return c10::nullopt;
+  if (mixk::scan_route(T, S, H, dk, dv, mode) != mixk::kScanChunks) return c10::nullopt;
   return at::empty({mixk::scan_scratch_floats(T, S, H, dk, dv, mode)}, like.options().dtype(at::kFloat));
 }
 

@@ -7,7 +7,6 @@ namespace mixk {
 
 constexpr int kScanChunk = 16;         // tokens per chunk
 constexpr int kPowers = 65;            // retention: powers 0 ... 64 of a head's decay
-constexpr int kScanMinRows = 5;        // shorter portions run token by token
 constexpr int kWalkCols = 64;          // value columns of a workgroup of the walk
 enum ScanMode { kModeRetention = 0, kModeForget = 1, kModeStateSpace = 2, kModeDelta = 3,
                 kModeDeltaChannel = 4 };
@@ -30,6 +29,7 @@ struct ChunkArgs {
   const int* seq_slot;
   int64_t q_stride, k_stride, v_stride, dec_stride, beta_stride;
   int S, H, G, dk, dv, n_freq, n_slots;   // n_slots: chunk slots (scan_chunk_slots)
+  int min_rows;           // shorter portions of a chunked batch run token by token (kScanMinRows)
   float* seg;             // scratch: states at the ends of segments and the decays over them (scan_segments)
   int seg_chunks, seg_states;
   float kscale;
@@ -70,17 +70,41 @@ inline int64_t scan_scratch_floats(int64_t T, int64_t S, int64_t H, int64_t dk, 
   return scan_chunk_slots(T, S) * H * scan_record_floats(mode) +
          scan_segments(T, H, dv, mode).states * scan_segment_floats(H, dk, dv);
 }
-// whether the chunked form pays for a batch of T rows in S portions
-inline bool scan_use_chunks(int64_t T, int64_t S, int dk) { return dk <= 128 && T > 3 * S && T >= 2 * kScanMinRows; }
-// portions (not decode rows) with keys wider than the chunk kernel's
-inline bool scan_wide_portions(int64_t T, int64_t S, int dk) { return dk > 128 && T > 3 * S; }
 
+// Which kernels take a batch.  The host knows its T rows and S portions; if every portion has a row, the longest has at
+// most T - S + 1.  All at 32 heads of 128, bf16, us; "R + N" R decode rows beside a portion of N, "S x N" S portions.
+// - Rows (step_scan.h) cost the state's traffic and then 1 us per token of the longest portion, 2 us with a delta rule.
+// - Chunks cost 15 us (28 with per-channel decays) besides the state's traffic, then 2 us per 16 tokens, and 0.2 - 0.3 us
+//   per decode row for the empty workgroups of the walk and rows that share the scores' launch: they pay from 7 - 28 rows
+//   on, a sixth of a row later per portion.  Rows / chunks: delta rule 15 + 8 27 / 27, 15 + 32 75 / 29, 63 + 32 106 / 65;
+//   per channel 15 + 16 42 / 40, 63 + 32 105 / 79; forget gate 15 + 24 37 / 41, 15 + 32 45 / 41; state space 7 + 16
+//   26 / 16; retention 15 + 16 28 / 25, 127 + 256 437 / 175.
+// - Tokens (delta_rule.hip, linear_scan.hip) load a round of tokens ahead, 0.3 - 0.7 us per token, but with slower state
+//   accesses: for short portions whose workgroups find room at once.  Rows / chunks / tokens: forget gate 1 x 33
+//   36 / 33 / 21, 4 x 16 22 / 30 / 20; per channel 1 x 12 27 / 28 / 18, 2 x 16 35 / 28 / 20; state space 1 x 9
+//   14 / 12 / 9, 2 x 16 22 / 13 / 11.  A long portion among decode rows must not be taken for many short ones, hence
+//   the bounds on T - S.  Keys wider than a chunk's: for anything but a few rows per portion.
+// In a chunked batch, portions below kScanMinRows run token by token: a chunk that is not full costs as much as one that
+// is, and with portions in many heads the row kernel's tokens overlap: 16 x 8, rows / chunks: forget gate 24 / 67, per
+// channel 36 / 67, retention 21 / 46.
+enum ScanRoute { kScanRows, kScanChunks, kScanTokens };
+constexpr int kScanMinRows[] = {12, 28, 9, 7, 12};   // by ScanMode
+inline ScanRoute scan_route(int64_t T, int64_t S, int64_t H, int64_t dk, int64_t dv, int mode) {
+  const int64_t longest = T - S + 1;
+  if (dk > 128) return mode != kModeRetention && T > 3 * S ? kScanTokens : kScanRows;
+  if (S * H * ((dv + 31) / 32) <= 512) {
+    if (mode == kModeForget && (T > 3 * S || longest >= 12) && T < 96 * S && T - S < 256) return kScanTokens;
+    if (mode == kModeStateSpace && longest >= 5 && T < 24 * S && T - S < 31) return kScanTokens;
+    if (mode == kModeDeltaChannel && longest >= 6 && T < 32 * S && T - S < 48) return kScanTokens;
+  }
+  return longest >= kScanMinRows[mode] + S / 6 ? kScanChunks : kScanRows;
+}
 // A batch with scratch (a.rec, a.n_slots, a.seg): portions of kScanMinRows rows or more in chunks, the others token by
 // token (dk <= 128).
 int launch_chunk_scan(const ChunkArgs& a, int mode, int dtype, hipStream_t st);
 // Portions of up to max_rows rows, token by token (dk <= 256).
 int launch_step_scan(const ChunkArgs& a, int mode, int max_rows, int dtype, hipStream_t st);
-// A batch: long portions in chunks where there is scratch for them, the others token by token.
+// A batch on the route kScanChunks (with scratch for it) or kScanRows.
 inline int launch_scan_batch(ChunkArgs a, int mode, int64_t T, int dtype, hipStream_t st) {
   // (the chunk kernels address the 16 rows of a chunk with 32 bits)
   const int64_t strides[] = {a.q_stride, a.k_stride, a.v_stride, a.dec_stride, static_cast<int64_t>(a.H) * a.dv};
@@ -88,6 +112,7 @@ inline int launch_scan_batch(ChunkArgs a, int mode, int64_t T, int dtype, hipStr
     if (x >= 1ll << 26) a.rec = nullptr;
   if (a.rec == nullptr) return launch_step_scan(a, mode, 1 << 30, dtype, st);
   a.n_slots = static_cast<int>(scan_chunk_slots(T, a.S));
+  a.min_rows = kScanMinRows[mode];
   const ScanSegments g = scan_segments(T, a.H, a.dv, mode);
   a.seg = a.rec + static_cast<int64_t>(a.n_slots) * a.H * scan_record_floats(mode);
   a.seg_chunks = static_cast<int>(g.chunks);

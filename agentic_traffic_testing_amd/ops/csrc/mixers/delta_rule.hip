@@ -1,6 +1,6 @@
-// Gated delta rule over ragged batches of portions, state carried per sequence in fp32.  Keys up to 128 wide
-// and decode rows run the kernels of chunk_scan.hip and step_scan.hip; the kernel here takes portions whose
-// keys are wider than a chunk's.
+// Gated delta rule over ragged batches of portions, state carried per sequence in fp32.  Most batches run the
+// kernels of chunk_scan.hip and step_scan.hip; the kernel here takes portions whose keys are wider than a chunk's, and
+// short ones with per-channel decays (scan_route).
 //
 // Per head, with S [dim, vdim] the state, per token:
 //     S = diag(g) S            (g: one decay per head, or one per key channel)
@@ -208,17 +208,21 @@ int launch_dp(float* out, const void* qkv, const void* beta, int64_t beta_stride
               const float* dt_bias, float* state, const int* positions, const int* seq_qstart,
               const int* seq_slot, int S, int H, int G, int dim, int vdim, hipStream_t st) {
   const dim3 grid(S, H, (vdim + 63) / 64);
-  if (per_channel)
+  if (per_channel) {
     hipLaunchKernelGGL((gated_delta_rule_kernel<T, DP, true>), grid, dim3(64 * lanes_per_column(DP)), 0, st, out,
                        static_cast<const T*>(qkv), static_cast<const T*>(beta), beta_stride,
                        static_cast<const T*>(decay), decay_stride, a_log, dt_bias, state,
                        positions, seq_qstart, seq_slot, H, G, dim, vdim);
-  else
+    return static_cast<int>(hipGetLastError());
+  }
+  if constexpr (DP > 128) {
     hipLaunchKernelGGL((gated_delta_rule_kernel<T, DP, false>), grid, dim3(64 * lanes_per_column(DP)), 0, st, out,
                        static_cast<const T*>(qkv), static_cast<const T*>(beta), beta_stride,
                        static_cast<const T*>(decay), decay_stride, a_log, dt_bias, state,
                        positions, seq_qstart, seq_slot, H, G, dim, vdim);
-  return static_cast<int>(hipGetLastError());
+    return static_cast<int>(hipGetLastError());
+  }
+  return -1;   // (scan_route)
 }
 
 template <typename T>
@@ -230,6 +234,10 @@ int launch_t(float* out, const void* qkv, const void* beta, int64_t beta_stride,
   if (dim <= N)                                                                                 \
     return launch_dp<T, N>(out, qkv, beta, beta_stride, decay, decay_stride, per_channel, a_log, \
                            dt_bias, state, positions, seq_qstart, seq_slot, S, H, G, dim, vdim, st)
+  MIXK_DP(32);
+  MIXK_DP(64);
+  MIXK_DP(96);
+  MIXK_DP(128);
   MIXK_DP(192);
   MIXK_DP(256);
 #undef MIXK_DP
@@ -259,8 +267,8 @@ extern "C" int mixk_gated_delta_rule(float* out, const void* qkv, const void* be
   a.positions = positions; a.seq_qstart = seq_qstart; a.seq_slot = seq_slot;
   a.q_stride = a.k_stride = a.v_stride = C; a.dec_stride = decay_stride; a.beta_stride = beta_stride;
   a.S = S; a.H = H; a.G = G; a.dk = dim; a.dv = vdim;
-  if (!scan_wide_portions(T, S, dim))
-    return launch_scan_batch(a, per_channel ? kModeDeltaChannel : kModeDelta, T, dtype, st);
+  const int mode = per_channel ? kModeDeltaChannel : kModeDelta;
+  if (scan_route(T, S, H, dim, vdim, mode) != kScanTokens) return launch_scan_batch(a, mode, T, dtype, st);
   int rc = 0;
   MIXK_DISPATCH(dtype, rc = launch_t<T>(out, qkv, beta, beta_stride, decay, decay_stride,
                                         per_channel, a_log, dt_bias, state, positions, seq_qstart,

@@ -1,6 +1,6 @@
-// Gated linear recurrence over ragged batches of portions, state carried per sequence in fp32.  Keys up to 128
-// wide and decode rows run the kernels of chunk_scan.hip and step_scan.hip; the kernel here takes portions
-// whose keys are wider than a chunk's, and short ones of the forget-gate form (scan_short_portions).
+// Gated linear recurrence over ragged batches of portions, state carried per sequence in fp32.  Most batches run the
+// kernels of chunk_scan.hip and step_scan.hip; the kernel here takes portions whose keys are wider than a chunk's,
+// and short ones (scan_route).
 //
 // Per head, with S [dk, dv] the state, per token:
 //     S[i, :] = a[i] S[i, :] + k[i] v[:]        o[:] = sum_i q[i] S[i, :]  (+ skip * v[:])
@@ -196,15 +196,6 @@ gated_linear_scan_kernel(ScanArgs a) {
   }
 }
 
-// Short portions of the forget-gate form whose workgroups (32 columns) find room at once: the chunks' scores take 14 us
-// before the walk starts, whatever the length, a token here 0.3 us.  One portion of 40 rows in 8 heads: 17 us, in
-// chunks 29; 4 of ~35 in 32 heads 25 and 32; 2 of ~55 23 and 32; 2 of ~120 43 and 43.  The batch tells only the
-// number of rows and portions: the mean must be below 96, and a single long one among them not take too long.
-// (State-space form: 19 and 17 at 40 rows.)
-bool scan_short_portions(int64_t T, int64_t S, int64_t H, int dk, int dv) {
-  return dk <= 128 && T > 3 * S && T < 96 * S && T - S < 256 && S * H * ((dv + kScanCols - 1) / kScanCols) <= 512;
-}
-
 template <typename T, int MODE>
 int launch_scan(const ScanArgs& a, int S, hipStream_t st) {
   const dim3 grid(S, a.H, (a.dv + kScanCols - 1) / kScanCols);
@@ -217,10 +208,8 @@ int launch_scan(const ScanArgs& a, int S, hipStream_t st) {
   // fewer than ~3 four-wave workgroups per SIMD-quad of the chip: 16 lanes per column
   const int64_t groups = static_cast<int64_t>(grid.x) * grid.y * grid.z;
   if (groups < 768) {
-    if constexpr (MODE == 0) {   // (short portions of the forget-gate form)
-      MIXK_SCAN(16, 4)
-      MIXK_SCAN(16, 8)
-    }
+    MIXK_SCAN(16, 4)
+    MIXK_SCAN(16, 8)
     MIXK_SCAN(16, 16)
   }
   MIXK_SCAN(8, 24)
@@ -246,13 +235,14 @@ extern "C" int mixk_gated_linear_scan(float* out, float* state, const void* q, i
   if (S <= 0) return 0;
   if (dk <= 0 || dv <= 0 || H <= 0) return -1;
   if (mode == 1 && (G <= 0 || H % G != 0)) return -1;
-  if (!scan_wide_portions(T, S, dk) && !(mode == 0 && scan_short_portions(T, S, H, dk, dv))) {
+  const int scan_mode = mode == 0 ? kModeForget : kModeStateSpace;
+  if (scan_route(T, S, H, dk, dv, scan_mode) != kScanTokens) {
     ChunkArgs c{};
     c.out = out; c.state = state; c.q = q; c.k = k; c.v = v; c.dec = dt; c.p0 = p0; c.p1 = p1; c.p2 = p2;
     c.rec = rec; c.positions = positions; c.seq_qstart = seq_qstart; c.seq_slot = seq_slot;
     c.q_stride = q_stride; c.k_stride = k_stride; c.v_stride = v_stride; c.dec_stride = dt_stride;
     c.S = S; c.H = H; c.G = mode == 1 ? G : H; c.dk = dk; c.dv = dv;
-    return launch_scan_batch(c, mode == 0 ? kModeForget : kModeStateSpace, T, dtype, st);
+    return launch_scan_batch(c, scan_mode, T, dtype, st);
   }
   ScanArgs a{out, state, q, k, v, dt, p0, p1, p2, positions, seq_qstart, seq_slot,
              q_stride, k_stride, v_stride, dt_stride, H, mode == 1 ? G : H, dk, dv};

@@ -1276,10 +1276,10 @@ def rms_error(x, want):
 @pytest.mark.parametrize("dt", DTYPES)
 def test_chunked_forget_gate_rounds_like_rows(dt):
     """Decays and queries alone (one channel of one head sees a state of ones): errors against 64 bits at the level of
-    the decode form's.  Same roundings per token, 2^16 samples of them: 5 % is ten times what the statistics leave."""
+    the decode form's.  Same roundings per token, 7000 samples of them: 5 % is six times what the statistics leave."""
     torch.manual_seed(3)
-    H, d, dv, S, n = 32, 64, 4, 64, 20
-    f, q = (torch.randn(S * n, H * d, device="cuda") - 2).to(dt), torch.zeros(S * n, H, d, device="cuda").to(dt)
+    H, d, dv, S, n = 8, 64, 4, 31, 30
+    f, q = (torch.randn(S * n, H * d, device="cuda") - 1).to(dt), torch.zeros(S * n, H, d, device="cuda").to(dt)
     q[:, :, 5] = (3 * torch.randn(S * n, H, device="cuda")).to(dt)
     v, zero = torch.zeros(S * n, H * dv, device="cuda").to(dt), torch.zeros(H * d, device="cuda")
 
@@ -1365,6 +1365,44 @@ def test_chunked_results_round_like_rows(name):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("live", [8, 40, 130])
+@pytest.mark.parametrize("name", ["delta", "delta per channel", "forget gate", "state space", "retention"])
+def test_portion_beside_decode_rows(dt, live, name):
+    """A portion takes the same route, bit for bit, alone and behind any number of decode rows (up to and past the
+    number whose rows get a launch of their own); the rows too."""
+    torch.manual_seed(live)
+    H, d, n = 32, 128, 100
+    T = live + n
+    q, k, v, wide = (torch.randn(T, H * d).to(dt).cuda() for _ in range(4))
+    one, two = torch.randn(T, H).to(dt).cuda(), torch.randn(T, H).to(dt).cuda()
+    z, zz = torch.zeros(H).cuda(), torch.zeros(H * d).cuda()
+    pw = mx.retention_powers([1 - 2.0 ** (-3 - h % 7) for h in range(H)], "cuda")
+    start = torch.randn(live + 1, H, d, d, device="cuda")
+
+    def run(a, b, lens, slots):
+        md = cuda(ragged(lens, [7] * len(lens), slots, width=64))
+        at, st = (md["positions"], md["seq_qstart"], md["seq_slot"]), start.clone()
+        x = [t[a:b] for t in (q, k, v, wide, one, two)]
+        if name == "forget gate":
+            o = mx.forget_gate_scan(x[0], x[3], x[2], zz, zz, st, *at, H, d, d)
+        elif name == "state space":
+            o = mx.state_space_scan(x[2], x[1], x[0], x[4], z, z, z, st, *at, H, H, d, d)
+        elif name == "retention":
+            o = mx.retention(x[0], x[1], x[2], pw, torch.zeros(b - a, 0).cuda(), st, *at, H, d, d, len(lens) - 1)
+        else:
+            form = name == "delta per channel"
+            o = mx.gated_delta_rule(torch.cat(x[:3], 1), x[5], x[3] if form else x[4], z, zz if form else z, st, *at, H,
+                                    H, d, d)
+        return o, st
+
+    both, st = run(0, T, [1] * live + [n], list(range(live + 1)))
+    alone, st_a = run(live, T, [n], [live])
+    rows, st_r = run(0, live, [1] * live, list(range(live)))
+    assert torch.equal(both[live:], alone) and torch.equal(st[live], st_a[live])
+    assert torch.equal(both[:live], rows) and torch.equal(st[:live], st_r[:live])
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("rate", [1.0, 5.0, 16.0])
 @pytest.mark.parametrize("x", [-17.0, -9.0, -3.0, 1.0])
 def test_chunked_delta_decay_rounds_like_rows(dt, rate, x):
@@ -1373,7 +1411,7 @@ def test_chunked_delta_decay_rounds_like_rows(dt, rate, x):
     forms, with equal decays, differ by 7 %); and after 1024 equal tokens at most 2 roundings of 2^-24 each - the
     decay's (the exponential is good to one) and the product's - off."""
     torch.manual_seed(4)
-    H, d, dv, S, n = 16, 64, 4, 64, 12
+    H, d, dv, S, n = 16, 64, 4, 40, 16
     a_log = torch.log(torch.full((H,), rate, device="cuda"))
     used = torch.exp(a_log.double())[:, None]
     bias = x + torch.rand(H * d, device="cuda")
