@@ -99,6 +99,14 @@ inline ScanRoute scan_route(int64_t T, int64_t S, int64_t H, int64_t dk, int64_t
   }
   return longest >= kScanMinRows[mode] + S / 6 ? kScanChunks : kScanRows;
 }
+// A grid of gx workgroups for each of n portions: a grid's y and z end at 65535, portions do not.
+constexpr int kGridY = 65535;
+inline dim3 scan_grid(int64_t gx, int64_t n) {
+  return dim3(static_cast<unsigned>(gx), static_cast<unsigned>(n < kGridY ? n : kGridY),
+              static_cast<unsigned>((n + kGridY - 1) / kGridY));
+}
+__device__ __forceinline__ int scan_grid_portion() { return static_cast<int>(blockIdx.z) * kGridY + static_cast<int>(blockIdx.y); }
+
 // A batch with scratch (a.rec, a.n_slots, a.seg): portions of kScanMinRows rows or more in chunks, the others token by
 // token (dk <= 128).
 int launch_chunk_scan(const ChunkArgs& a, int mode, int dtype, hipStream_t st);

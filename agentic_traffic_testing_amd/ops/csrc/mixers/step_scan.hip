@@ -8,12 +8,13 @@ template <typename T, int MODE, int R, bool V4>
 __global__ void __launch_bounds__(256)
 scan_step_kernel(ChunkArgs a, int max_rows) {
   __shared__ StepLds<MODE, R> lds;
-  scan_step<T, MODE, R, V4>(a, max_rows, blockIdx.x, blockIdx.y, lds);
+  const int s = scan_grid_portion();
+  if (s < a.S) scan_step<T, MODE, R, V4>(a, max_rows, blockIdx.x, s, lds);
 }
 
 template <typename T, int MODE, int R>
 int launch(const ChunkArgs& a, int max_rows, hipStream_t st) {
-  const dim3 grid(a.H * ((a.dv + kCols - 1) / kCols), a.S);
+  const dim3 grid = scan_grid(static_cast<int64_t>(a.H) * ((a.dv + kCols - 1) / kCols), a.S);
   if (scan_step_v4(a))
     hipLaunchKernelGGL((scan_step_kernel<T, MODE, R, true>), grid, dim3(256), 0, st, a, max_rows);
   else

@@ -1402,6 +1402,41 @@ def test_portion_beside_decode_rows(dt, live, name):
     assert torch.equal(both[:live], rows) and torch.equal(st[:live], st_r[:live])
 
 
+@pytest.mark.parametrize("n", [1, 20])
+def test_scans_of_many_portions(n):
+    """More portions than a grid's y extent: decode rows, and portions in chunks; a few of them against a batch of their
+    own."""
+    torch.manual_seed(n)
+    S, H, d, dv = 65535 + 40, 1, 16, 8
+    T, pick = S * n, torch.cat([torch.arange(9), torch.arange(65530, S)])
+    few = len(pick)
+    rows = (pick[:, None] * n + torch.arange(n)).flatten()
+    x, one = torch.randn(T, 2 * d + dv).cuda(), torch.randn(T, 1).cuda()
+    wide, z, zz, tab = torch.randn(T, d).cuda(), torch.zeros(1).cuda(), torch.zeros(d).cuda(), torch.zeros(T, 0).cuda()
+    pw, start = mx.retention_powers([0.9], "cuda"), torch.randn(S, H, d, dv).cuda()
+    i32 = lambda t: t.to(torch.int32).cuda()  # noqa: E731
+
+    def run(name, r, count, st):
+        at = (i32(torch.arange(1, n + 1).repeat(count)), i32(torch.arange(count + 1) * n), i32(torch.arange(count)))
+        x_, one_, wide_ = (t if r is None else t[r.cuda()] for t in (x, one, wide))
+        q, k, v = (x_[:, a:b] for a, b in ((0, d), (d, 2 * d), (2 * d, 2 * d + dv)))
+        if name == "delta":
+            o = mx.gated_delta_rule(x_.contiguous(), one_, one_, z, z, st, *at, 1, 1, d, dv)
+        elif name == "forget":
+            o = mx.forget_gate_scan(q, wide_, v, zz, zz, st, *at, 1, d, dv)
+        else:
+            o = mx.retention(q, k, v, pw, tab[:count * n], st, *at, 1, d, dv)
+        return o, st
+
+    for name in ("delta", "forget", "retention"):
+        got, st = run(name, None, S, start.clone())
+        want, st_w = run(name, rows, few, start[pick.cuda()].clone())
+        assert torch.isfinite(want).all()
+        # (a batch of few may take another kernel)
+        assert torch.allclose(got[rows.cuda()], want, rtol=1e-4, atol=1e-4)
+        assert torch.allclose(st[pick.cuda()], st_w, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("rate", [1.0, 5.0, 16.0])
 @pytest.mark.parametrize("x", [-17.0, -9.0, -3.0, 1.0])
