@@ -94,7 +94,8 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
   const int pos_first = ctx + wcol / rep, pos_last = ctx + max(w_last, 0) / rep;
   const int kend = min(kvlen, ctx + (min(cols_total, col0 + COLS) - 1) / rep + 1);
   // key blocks: the kept keys in front of the window, then from the window's start (block-aligned)
-  const int kbeg = window_start(ctx + col0 / rep, a.window) & ~(kBlock - 1);
+  const int klow = window_start(ctx + col0 / rep, a.window);   // no column sees keys in [keep, klow)
+  const int kbeg = klow & ~(kBlock - 1);
   const int kkeep = min(a.keep, kbeg);
   const int nk = (kkeep + kBlock - 1) / kBlock;
   const int nb = nk + (kend - kbeg + kBlock - 1) / kBlock;
@@ -144,7 +145,8 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
   const int last_page = npages - 1;
   u32x4 kr[NMAP][KU], vr[VU];
   auto load_block = [&](int k0) {
-    // keys at or past kend read a clamped page or stale slots: their scores are masked and their V zeroed
+    // keys at or past kend read a clamped page or stale slots, keys in front of the window whatever is there: their
+    // scores are masked and their V zeroed (0 x NaN)
     const int key = k0 + 16 * sg, at = key & (bs - 1);   // (a page may hold several blocks)
     const int pg = __builtin_amdgcn_readfirstlane(lds_bt[min(key >> a.bs_shift, last_page)]);
     const __bf16* kb = k_cache + ((static_cast<int64_t>(pg) * G + NMAP * g) * bs + at) * DK;
@@ -164,12 +166,13 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
       for (int u = 0; u < KU; ++u)
         *reinterpret_cast<u32x4*>(&lds_k[buf][e][k_dst[u]]) = kr[e][u];
     const int key = k0 + 16 * sg + 8 * (lane & 1);
-    if (key + 8 > kend) {
+    if (key + 8 > kend || (WIN && key < klow && key + 8 > a.keep)) {
+      auto seen = [&](int t) { return t < kend && (!WIN || t >= klow || t < a.keep); };
 #pragma unroll
       for (int u = 0; u < VU; ++u)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          vr[u][j] &= (key + 2 * j < kend ? 0x0000ffffu : 0u) | (key + 2 * j + 1 < kend ? 0xffff0000u : 0u);
+          vr[u][j] &= (seen(key + 2 * j) ? 0x0000ffffu : 0u) | (seen(key + 2 * j + 1) ? 0xffff0000u : 0u);
     }
 #pragma unroll
     for (int u = 0; u < VU; ++u) *reinterpret_cast<u32x4*>(&lds_v[buf][v_dst[u]]) = vr[u];

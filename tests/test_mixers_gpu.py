@@ -1073,6 +1073,37 @@ def test_flash_attention_wide_pages(window, keep, bs):
     test_flash_two_maps_edges(4, 2, window, keep, bs)
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(4, 4, 64, 64), (8, 2, 128, 128), (5, 1, 256, 192), (8, 4, 64, 128)])
+@pytest.mark.parametrize("window,keep", [(100, 0), (100, 40), (37, 3), (64, 64)])
+def test_flash_window_without_expired_keys(H, G, d, dv, window, keep):
+    """NaN in the pages of keys that no token of the portion sees, up to the last one in front of the window (other
+    tokens of a workgroup still see some that a later one does not)."""
+    torch.manual_seed(window)
+    n = 4 if dv == 192 else 12                  # tokens of one workgroup
+    starts = [300, 159, 224]
+    md = ragged([n] * 3, starts, [0, 1, 2], width=32)
+    nb, T, pair = md["num_pages"], 3 * n, (d, dv) == (64, 128)
+    q = torch.randn(T, H, d).to(torch.bfloat16)
+    k, v = torch.randn(nb, G, 16, d).to(torch.bfloat16), torch.randn(nb, G // 2 if pair else G, dv, 16).to(torch.bfloat16)
+    gone = v.clone()
+    for i, s0 in enumerate(starts):
+        for p in range(keep, s0 - window + 1):
+            gone[md["block_tables"][i, p // 16], :, :, p % 16] = float("nan")
+    gate = torch.randn(T, H // 2 * dv).to(torch.bfloat16)
+
+    def run(m, to, v):
+        if pair:
+            return mx.differential_attention(to(q), to(k), to(v), m["block_tables"], m["seq_kvlen"], m["seq_qstart"],
+                                             m["tile_seq"], m["tile_qoff"], d ** -0.5, 0.4, 0.3, 1e-5, to(gate), 0, 0,
+                                             window, keep)
+        return mx.sink_attention(to(q), to(k), to(v), m["block_tables"], m["seq_kvlen"], m["seq_qstart"], m["tile_seq"],
+                                 m["tile_qoff"], d ** -0.5, True, window=window, keep_first=keep)
+
+    want, got = run(md, lambda t: t, v), run(cuda(md), lambda t: t.cuda(), gone)
+    # as the edges' tests
+    assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
