@@ -364,8 +364,6 @@ void diff_combine(at::Tensor out, const at::Tensor& a, const c10::optional<at::T
         "diff_combine");
 }
 
-// q, k [T, H dk], v [T, H dv] (row-strided), powers fp32 [H, n] (decay^0 ... decay^(n-1)), cos_sin
-// [rows, 2 n_freq]; sequences [0, num_decode) have one row each.
 // scratch of the chunked recurrences, where the batch takes them
 c10::optional<at::Tensor> scan_records(const at::Tensor& like, int64_t T, int64_t S, int64_t H, int64_t dk,
                                        int64_t dv, int mode) {
@@ -373,11 +371,12 @@ c10::optional<at::Tensor> scan_records(const at::Tensor& like, int64_t T, int64_
   return at::empty({mixk::scan_scratch_floats(T, S, H, dk, dv, mode)}, like.options().dtype(at::kFloat));
 }
 
+// q, k [T, H dk], v [T, H dv] (row-strided), powers fp32 [H, n] (decay^0 ... decay^(n-1)), cos_sin
+// [rows, 2 n_freq].
 void retention(at::Tensor out, at::Tensor state, const at::Tensor& q, const at::Tensor& k,
                const at::Tensor& v, const at::Tensor& powers, const at::Tensor& cos_sin,
                const at::Tensor& positions, const at::Tensor& seq_qstart,
-               const at::Tensor& seq_slot, int64_t H, int64_t dk, int64_t dv,
-               int64_t num_decode) {
+               const at::Tensor& seq_slot, int64_t H, int64_t dk, int64_t dv) {
   rows2d(v, v, "v");
   rows2d(q, v, "q");
   rows2d(k, v, "k");
@@ -392,8 +391,7 @@ void retention(at::Tensor out, at::Tensor state, const at::Tensor& q, const at::
                   out.numel() == T * H * dv && state.dim() == 4 && state.size(1) == H &&
                   state.size(2) == dk && state.size(3) == dv && powers.dim() == 2 &&
                   powers.size(0) == H && powers.size(1) == 65 && cos_sin.dim() == 2 &&
-                  cos_sin.size(0) >= T && cos_sin.size(1) % 2 == 0 && cos_sin.size(1) <= dk &&
-                  num_decode >= 0 && num_decode <= S,
+                  cos_sin.size(0) >= T && cos_sin.size(1) % 2 == 0 && cos_sin.size(1) <= dk,
               "retention: shapes");
   const at::DeviceGuard g(v.device());
   const auto rec = scan_records(v, T, S, H, dk, dv, mixk::kModeRetention);
@@ -998,20 +996,6 @@ void post_norm(const c10::optional<at::Tensor>& h, at::Tensor x, double alpha, c
         "post_norm");
 }
 
-void proj_inv_rms(at::Tensor out, const at::Tensor& qx, const at::Tensor& kx, double eps) {
-  f32c(out, "out");
-  rows2d(qx, qx, "q");
-  rows2d(kx, qx, "k");
-  TORCH_CHECK(out.numel() == 2 * qx.size(0) && kx.size(0) == qx.size(0) && qx.size(1) > 0 &&
-                  kx.size(1) > 0,
-              "proj_inv_rms: out [T, 2], q [T, nq], k [T, nk]");
-  const at::DeviceGuard g(qx.device());
-  rc_ok(mixk_proj_inv_rms(out.data_ptr<float>(), qx.data_ptr(), qx.stride(0), qx.size(1),
-                          kx.data_ptr(), kx.stride(0), kx.size(1), qx.size(0),
-                          static_cast<float>(eps), code(qx), cur_stream()),
-        "proj_inv_rms");
-}
-
 void scale_softcap(at::Tensor out, const at::Tensor& logits, double scale, double cap) {
   f32c(out, "out");
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && out.sizes() == logits.sizes() &&
@@ -1053,7 +1037,7 @@ TORCH_LIBRARY(atta_mix, m) {
         "int kv_heads) -> ()");
   m.def("retention(Tensor(a!) out, Tensor(b!) state, Tensor q, Tensor k, Tensor v, Tensor powers, "
         "Tensor cos_sin, Tensor positions, Tensor seq_qstart, Tensor seq_slot, int H, int dk, "
-        "int dv, int num_decode) -> ()");
+        "int dv) -> ()");
   m.def("sigmoid_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, "
         "Tensor block_tables, Tensor seq_kvlen, Tensor seq_qstart, Tensor tile_seq, "
         "Tensor tile_qoff, float scale, float cap, Tensor bias, Tensor talk, int num_decode, "
@@ -1097,7 +1081,6 @@ TORCH_LIBRARY(atta_mix, m) {
         "Tensor? post_scale, float eps, bool layer) -> ()");
   m.def("post_norm(Tensor(a!)? h, Tensor(b!) x, float alpha, Tensor a, float sa, Tensor? b, "
         "float sb, Tensor w, float eps) -> ()");
-  m.def("proj_inv_rms(Tensor(a!) out, Tensor qx, Tensor kx, float eps) -> ()");
   m.def("scale_softcap(Tensor(a!) out, Tensor logits, float scale, float cap) -> ()");
 }
 
@@ -1136,6 +1119,5 @@ TORCH_LIBRARY_IMPL(atta_mix, CUDA, m) {
   m.impl("moe_combine", &moe_combine);
   m.impl("norm_add_norm", &norm_add_norm);
   m.impl("post_norm", &post_norm);
-  m.impl("proj_inv_rms", &proj_inv_rms);
   m.impl("scale_softcap", &scale_softcap);
 }

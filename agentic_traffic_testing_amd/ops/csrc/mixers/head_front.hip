@@ -71,13 +71,6 @@ __device__ __forceinline__ float lane_group_sum(float v, int L) {
 }
 
 // Workgroup (rb, y) of the V part: rows [2 HR rb, 2 HR (rb + 1)) in two halves; item = (head, half), L lanes each.
-// an LDS-only barrier: loads from memory stay in flight
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // NORM: every row's head divided by its root mean square over vdim, times v_weight.
 template <typename T, int HR, bool NORM>
 __device__ __forceinline__ void v_part(const FrontArgs& a, int rb, int y, int lsh) {

@@ -89,6 +89,13 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// Workgroup barrier that orders LDS only: loads and stores to memory stay in flight (__syncthreads() waits for them).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Index of the sequence whose portion holds `row` (seq_qstart ascending, S >= 1), or -1 for a
 // row past the last portion.
 __device__ __forceinline__ int seq_of_row(const int* __restrict__ seq_qstart, int S, int row) {

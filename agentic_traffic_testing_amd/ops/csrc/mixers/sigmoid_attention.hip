@@ -114,8 +114,8 @@ __device__ __forceinline__ sg_bf16x8 keep_keys(sg_bf16x8 v, int t8, int kend) {
     if (t8 + j >= kend) v[j] = static_cast<__bf16>(0.f);
   return v;
 }
-// Workgroup barrier that orders LDS only: global loads in flight stay in flight.
-__device__ __forceinline__ void lds_barrier() {
+// As lds_barrier, and nothing is scheduled across it.
+__device__ __forceinline__ void sg_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
@@ -335,7 +335,7 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
     };
     if (ONE && wave_on) load_v(0);
     pv = page_at(nk + 8 * c);
-    lds_barrier();
+    sg_barrier();
     const int rb = fresh(r);
     // B: the wave mixes the pairs of tokens 2 w and 2 w + 1
 #pragma unroll
@@ -361,7 +361,7 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
         }
       }
     }
-    lds_barrier();
+    sg_barrier();
     if (wave_on) {   // C
       const bool tail = nk > kend;
       const int rc = fresh(r);

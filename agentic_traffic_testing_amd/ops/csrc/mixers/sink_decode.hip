@@ -28,13 +28,6 @@ constexpr int kPStride = kPartTokens + 8;
 static_assert(kPartTokens == kWaves * kTile, "a wave per tile");
 constexpr float kLog2e = 1.44269504088896341f;
 
-// an LDS-only barrier: the V loads stay in flight over it
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // dim = 16 ND, vdim = 32 NV
 template <int ND, int NV>
 __global__ void __launch_bounds__(256, ND > 8 ? 1 : 2)

@@ -21,12 +21,6 @@ namespace ss {
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int kCols = 64;
 
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // R: rows per thread (dk <= 16 R <= 256); V4: 16-byte state accesses (dv % 4 == 0, aligned state)
 template <int MODE, int R>
 struct StepLds {

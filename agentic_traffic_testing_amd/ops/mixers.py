@@ -485,7 +485,7 @@ def state_space_scan(x, B, C, dt, dt_bias, a_log, skip, state, positions, seq_qs
 
 
 
-RETENTION_CHUNK = 64      # tokens per chunk of the matrix-core prefill kernel
+RETENTION_CHUNK = 64      # the longest chunk a table of powers serves (the kernels' chunks have 16 tokens)
 
 
 def retention_powers(decay, device) -> torch.Tensor:
@@ -502,13 +502,16 @@ def retention(q, k, v, powers, cos_sin, state, positions, seq_qstart, seq_slot, 
     rotate-half positions (table ``cos_sin`` [T, 2 n], n <= dim / 2) on q and k and k times
     dim^-0.5, all in fp32.  q, k [T, heads * dim], v [T, heads * vdim] (row-strided); ``powers``:
     ``retention_powers``; state fp32 [slots, heads, dim, vdim] advanced in place; returns fp32
-    [T, heads, vdim].  Sequences [0, num_decode) have one row each."""
+    [T, heads, vdim].  Sequences [0, num_decode) have one row each (the kernels find that out from
+    seq_qstart)."""
     if not v.is_cuda:
         return mref.retention(q, k, v, powers[:, 1], cos_sin, state, positions, seq_qstart, seq_slot,
                               heads, dim, vdim)
+    if not 0 <= num_decode <= seq_slot.numel():
+        raise RuntimeError(f"retention: num_decode {num_decode} of {seq_slot.numel()} sequences")
     out = torch.empty(v.shape[0], heads, vdim, dtype=torch.float32, device=v.device)
     _native().retention(out, state, q, k, v, powers, cos_sin, positions, seq_qstart, seq_slot, heads,
-                        dim, vdim, int(num_decode))
+                        dim, vdim)
     return out
 
 
