@@ -99,13 +99,12 @@ inline ScanRoute scan_route(int64_t T, int64_t S, int64_t H, int64_t dk, int64_t
   }
   return longest >= kScanMinRows[mode] + S / 6 ? kScanChunks : kScanRows;
 }
-// A grid of gx workgroups for each of n portions: a grid's y and z end at 65535, portions do not.
-constexpr int kGridY = 65535;
-inline dim3 scan_grid(int64_t gx, int64_t n) {
-  return dim3(static_cast<unsigned>(gx), static_cast<unsigned>(n < kGridY ? n : kGridY),
-              static_cast<unsigned>((n + kGridY - 1) / kGridY));
+// gx workgroups for each of n portions: launch(grid, first portion).  A grid's y ends at 65535, portions do not.
+template <typename F>
+inline void scan_grids(unsigned gx, int64_t n, F launch) {
+  for (int64_t y = 0; y < n; y += 65535)
+    launch(dim3(gx, static_cast<unsigned>(n - y < 65535 ? n - y : 65535)), static_cast<int>(y));
 }
-__device__ __forceinline__ int scan_grid_portion() { return static_cast<int>(blockIdx.z) * kGridY + static_cast<int>(blockIdx.y); }
 
 // A batch with scratch (a.rec, a.n_slots, a.seg): portions of kScanMinRows rows or more in chunks, the others token by
 // token (dk <= 128).

@@ -6,19 +6,20 @@ namespace ss {
 
 template <typename T, int MODE, int R, bool V4>
 __global__ void __launch_bounds__(256)
-scan_step_kernel(ChunkArgs a, int max_rows) {
+scan_step_kernel(ChunkArgs a, int max_rows, int portion0) {
   __shared__ StepLds<MODE, R> lds;
-  const int s = scan_grid_portion();
-  if (s < a.S) scan_step<T, MODE, R, V4>(a, max_rows, blockIdx.x, s, lds);
+  scan_step<T, MODE, R, V4>(a, max_rows, blockIdx.x, portion0 + blockIdx.y, lds);
 }
 
 template <typename T, int MODE, int R>
 int launch(const ChunkArgs& a, int max_rows, hipStream_t st) {
-  const dim3 grid = scan_grid(static_cast<int64_t>(a.H) * ((a.dv + kCols - 1) / kCols), a.S);
-  if (scan_step_v4(a))
-    hipLaunchKernelGGL((scan_step_kernel<T, MODE, R, true>), grid, dim3(256), 0, st, a, max_rows);
-  else
-    hipLaunchKernelGGL((scan_step_kernel<T, MODE, R, false>), grid, dim3(256), 0, st, a, max_rows);
+  const bool v4 = scan_step_v4(a);
+  scan_grids(a.H * ((a.dv + kCols - 1) / kCols), a.S, [&](dim3 grid, int first) {
+    if (v4)
+      hipLaunchKernelGGL((scan_step_kernel<T, MODE, R, true>), grid, dim3(256), 0, st, a, max_rows, first);
+    else
+      hipLaunchKernelGGL((scan_step_kernel<T, MODE, R, false>), grid, dim3(256), 0, st, a, max_rows, first);
+  });
   return static_cast<int>(hipGetLastError());
 }
 
