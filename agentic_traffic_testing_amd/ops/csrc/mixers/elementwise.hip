@@ -342,7 +342,7 @@ __global__ void group_rms_norm_kernel(T* __restrict__ out, const float* __restri
 
 // The same for narrow groups (gs % 8 == 0, gs <= 8 LPR, aligned rows): LPR lanes of 8 values per (row, group), all of
 // a group's loads at once and the gated values kept for the scaling.  Bound: memory; 7470 rows of 32 groups of 128,
-// no gate: two bytes and two passes per lane 81 -> 27 us.
+// no gate: two bytes and two passes per lane 82 -> 27 us.
 template <typename T, int LPR>
 __global__ void __launch_bounds__(256)
 group_rms_norm_lanes_kernel(T* __restrict__ out, const float* __restrict__ y, const T* __restrict__ gate,

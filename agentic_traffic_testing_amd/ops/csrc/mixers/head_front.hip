@@ -13,8 +13,8 @@
 // row, so portions that start anywhere in the batch are stored 16 bytes at a time.
 //
 // Bound: memory traffic.  Measured, before (element-wise, two or three launches) -> now, with the time of a copy of
-// the same bytes: 7580 rows, 32 + 8 + 8 heads of 128: 125 -> 46 us (38); latent, 7580 rows x 32 heads of 192 + 64:
-// 138 -> 82 (51); norm over the projection, 1908 rows of 24 + 8 + 8 heads: 35 -> 17.
+// the same bytes: 7580 rows, 32 + 8 + 8 heads of 128: 120 -> 44 us (38); latent, 7580 rows x 32 heads of 192 + 64:
+// 137 -> 76 (51); norm over the projection, 1908 rows of 24 + 8 + 8 heads: 33 -> 16.
 #include <initializer_list>
 
 #include "head_front.h"
@@ -347,7 +347,7 @@ bool launch_head_front(const FrontArgs& args, bool whole, int dtype, hipStream_t
   if (whole && !wide) return false;
   const int threads = wide ? max(256, hf::ceil_div(lanes, 64) * 64) : 256;
   // Four rows per thread once a quarter of the threads fills the chip (256 CUs x 2048 lanes): 7580 rows of 40 heads of
-  // 128 take 60 us with one row per thread, 50 with two, 46 with four; latent 106, 92, 82.
+  // 128 take 30 % more time with one row per thread, 9 % with two; latent 30 % and 12 %.
   const int rows = static_cast<int64_t>(a.T) * lanes >= hf::kManyRows * 256 * 2048 && vh == 8 ? hf::kManyRows : 1;
   const int uy = wide ? 1 : hf::ceil_div(lanes, threads);
   const int64_t qk = static_cast<int64_t>(hf::ceil_div(a.T, rows)) * uy;

@@ -68,8 +68,8 @@ __global__ void short_conv_silu_kernel(T* __restrict__ out, const T* __restrict_
 // before the first sequence and portion S + 1 for those after the last one (zeros, as for padding sequences).
 //
 // Bound: one read and one write of the rows, and the SiLU's arithmetic.  Measured, before (8 rows per workgroup, every
-// tap loaded again, a second launch for the tails) -> now: 7580 rows of 6144 channels in bf16 129 -> 57 us (copy: 38);
-// 1023 rows of 8192 in fp32 89 -> 27 (14); 16 decode rows 13 -> 5.
+// tap loaded again, a second launch for the tails) -> now: 7580 rows of 6144 channels in bf16 125 -> 53 us (copy: 38);
+// 1023 rows of 8192 in fp32 87 -> 26 (14); 16 decode rows 13 -> 5.
 constexpr int kConvRows = 16;
 
 template <typename T, int TAPS>

@@ -24,8 +24,8 @@
 // units; two waves per SIMD overlap them only in part (matrix cores 37 % busy, vector units 45 %, LDS port
 // 34 %, at 1.8 GHz).  Wave priority from the score products to the end of the value products lets the other
 // wave fall behind and fill gaps instead of running the same phase in step: 7580 rows of 32 + 8 heads of 128
-// 189 -> 180 us, latent 306 -> 299, two maps 75.6 -> 75.2.  (Taking block b + 1's scores beside block b's weights in
-// the same wave: 170, 634 and 85 - registers.)
+// 5 %, latent 2 %, two maps 1 %.  (Taking block b + 1's scores beside block b's weights in the same wave: 128 wide 6 %
+// less, latent 2.1 times, two maps 1.1 times the time - registers.)
 #include "sink_attention.h"
 
 namespace mixk {
@@ -364,10 +364,12 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
 // two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two)
 // and contexts past the LDS page list run sink_attention.hip's kernel.  Measured at 4 prompts of ~1850
 // tokens (us, old kernel -> this one; variants at the same shapes):
-//   128 / 128, 32 heads over 8:  475 -> 187 (8 waves per workgroup: +1 %; 64 columns per wave: +30 %)
-//   256 / 192, 32 heads over 1: 1058 -> 298 (4 waves 447: one wave per SIMD hides no latency)
-//   two maps 64 / 128, 8 over 2, 5 x 1165 tokens, window 1024: 129 -> 75 (both maps in each of 4 waves
-//     110: few workgroups there, so a wave's own chain counts; 2 waves per SIMD 82, 4 spill: 154)
+//   128 / 128, 32 heads over 8:  463 -> 167 (8 waves per workgroup: +1 %; 64 columns per wave: +30 %)
+//   256 / 192, 32 heads over 1: 1059 -> 267 (4 waves +50 %: one wave per SIMD hides no latency)
+//   two maps 64 / 128, 8 over 2, 5 x 1165 tokens, window 1024: 125 -> 71 (both maps in each of 4 waves
+//     +45 %: few workgroups there, so a wave's own chain counts; 2 waves per SIMD +10 %, 4 spill)
+// The workgroups of the 256 / 192 form hold 8 tokens (the old kernel's 4): so far ahead a NaN value reaches back (a weight
+// of 0 times NaN), as it did there.
 bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void* v_cache,
                        const AttnArgs& a, int num_tiles, hipStream_t st) {
   if (a.block_size < 16 || a.bt_width > sf::kPages || !(a.scale > 0.f)) return false;

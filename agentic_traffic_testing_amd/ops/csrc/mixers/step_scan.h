@@ -9,7 +9,7 @@
 //
 // Bound: the state is read and written once, 128 KB per (sequence, head) of 128 x 128.  Its loads are issued first
 // and nothing waits for them until the token's operands are in LDS (an LDS-only barrier; __syncthreads() would
-// wait).  Measured at 16 sequences, 32 heads, delta rule: 48 -> 12.5 us (half of the 134 MB from the last-level cache);
+// wait).  Measured at 16 sequences, 32 heads, delta rule: 46 -> 12.3 us (half of the 134 MB from the last-level cache);
 // 8 sequences: forget gate 13.5 -> 6.9, state space (128 heads of 128 x 64) 23 -> 10.8.
 #pragma once
 
