@@ -44,6 +44,8 @@ KERNEL_SO = OPS / "_atta_kernels.so"
 RUNTIME_DIR = PKG / "runtime"
 RUNTIME_CSRC = RUNTIME_DIR / "csrc"
 
+# hipcc only: keep fp32 arithmetic on the scalar-per-lane VALU forms (some packed fp32 forms have given wrong results)
+NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 ARCH = os.environ.get("ATTA_OFFLOAD_ARCH", "gfx950")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = shutil.which("hipcc") or os.path.join(ROCM, "bin", "hipcc")
@@ -135,9 +137,9 @@ def _build_kernels(force: bool, jobs: int, verbose: bool) -> Path:
     objs = []
     for src in sorted(CSRC.glob("*.hip")):
         obj = BUILD / (src.stem + ".o")
-        cmd = [HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
-               "-munsafe-fp-atomics", "-Wno-unused-result", "-I", str(CSRC),
-               "-c", str(src), "-o", str(obj)]
+        cmd = [HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", *NO_PACKED_FP32,
+               "-munsafe-fp-atomics", "-Wno-unused-result", "-Wno-unknown-warning-option",
+               "-I", str(CSRC), "-c", str(src), "-o", str(obj)]
         objs.append(obj)
         jobs_.append((cmd, obj, _sha([*cmd, src.read_bytes(), *hdr_digest])))
     inc, libdirs = _torch_paths()
@@ -182,8 +184,6 @@ def _build_kernels(force: bool, jobs: int, verbose: bool) -> Path:
 # ---- sequence-mixer kernel library (csrc/mixers -> _atta_mixers.so) -----------------------
 MIX_CSRC = CSRC / "mixers"
 MIXER_SO = OPS / "_atta_mixers.so"
-# hipcc only: keep fp32 arithmetic on the scalar-per-lane VALU forms
-NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
 def mixer_sources() -> list[Path]:

@@ -338,7 +338,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
       // defer-max (guide §5.5 T13): the running max m_run moves only when some column's max
       // grew by more than kRescale (log2 units), so P = 2^(s - m_run) stays <= 2^kRescale;
       // O and l are rescaled only then - with the max nearly settled after the first block,
-      // the 32 packed multiplies of the rescale were paid on most blocks.  O, l and P of a
+      // the multiplies of the rescale were paid on most blocks.  O, l and P of a
       // block always use the same m_run, so the result is exact up to rounding.
       const float m_cand = fmaxf(m_run, tmax * p.scale_log2);
       const bool grow = m_cand > m_run + kRescale;  // m_run == -inf: any finite m_cand
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
         m_run = m_new;
       }
       const float m_use = (m_run == kNegInf) ? 0.f : m_run;
-      // exponent arguments and the row sum on packed f32 pairs (v_pk_fma_f32 / v_pk_add_f32)
+      // exponent arguments and the row sum in two chains
       typedef float f32x2_t __attribute__((ext_vector_type(2)));
       const f32x2_t sc2 = {p.scale_log2, p.scale_log2};
       const f32x2_t nm2 = {-m_use, -m_use};

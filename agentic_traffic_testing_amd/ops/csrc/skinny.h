@@ -25,8 +25,8 @@ struct MfmaK32<__bf16> {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
   // sum of squares of the 8 activations (fused RMSNorm): bf16 -> f32 is a shift / mask,
-  // the squares go through packed FMAs (v_pk_fma_f32, two per instruction).  (v_dot2c_f32_bf16
-  // was measured 1.6 % high on this use - rounds its products - and is not used.)
+  // the squares are summed in two chains.  (v_dot2c_f32_bf16 was measured 1.6 % high on this
+  // use - rounds its products - and is not used.)
   __device__ static __forceinline__ float sq8(frag8 a, float s) {
     const u32x4 w = __builtin_bit_cast(u32x4, a);
     f32x2_t acc = {0.f, 0.f};

@@ -1,5 +1,7 @@
 """The in-tree native libraries build for gfx950 and load on a CPU-only host (catches
 undefined symbols / missing registrations before a GPU box ever sees them)."""
+import types
+
 import torch
 
 from agentic_traffic_testing_amd.ops import build
@@ -100,3 +102,24 @@ def test_build_lock_serialises_processes(tmp_path):
     ps = [subprocess.Popen([sys.executable, "-c", code]) for _ in range(2)]
     assert all(p.wait(timeout=60) == 0 for p in ps)
     assert log.read_text().split() == ["in", "out", "in", "out"]
+
+
+def test_hip_units_are_compiled_without_packed_fp32(tmp_path, monkeypatch):
+    """Every HIP translation unit of both libraries: some packed fp32 instruction forms have given wrong results."""
+    commands = []
+
+    def run(cmd):
+        commands.append(cmd)
+        return types.SimpleNamespace(stdout="", stderr="", returncode=0)
+
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "BUILD", tmp_path)
+    monkeypatch.setattr(build, "KERNEL_SO", tmp_path / "kernels.so")
+    monkeypatch.setattr(build, "MIXER_SO", tmp_path / "mixers.so")
+    build._build_kernels(True, 1, False)
+    build._build_mixers(True, 1, False)
+    units = [c for c in commands if any(str(x).endswith(".hip") for x in c)]
+    assert len(units) == sum(len(list(d.glob("*.hip"))) for d in (build.CSRC, build.MIX_CSRC))
+    for c in units:
+        at = c.index("-packed-fp32-ops")
+        assert c[at - 3:at] == ["-Xclang", "-target-feature", "-Xclang"]
