@@ -1064,6 +1064,34 @@ def test_flash_two_maps_edges(H, G, window, keep, bs=16):
     assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(4, 4, 64, 64), (8, 4, 64, 128), (8, 2, 128, 128), (40, 1, 256, 192)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (300, 0), (200, 70)])
+def test_decode_largest_weights_exact(H, G, d, dv, window, keep):
+    """One key in 32 has a weight: the largest weight of every tile is 1 before its 16-bit rounding, whatever the other
+    tiles hold (fp32 results; exponents below 2^5 rounded to 2^-20, a few of them per result)."""
+    torch.manual_seed(H + window)
+    starts = [0, 31, 96, 330, 700]
+    S = len(starts)
+    md = ragged([1] * S, starts, list(range(S)), width=64)
+    nb = md["num_pages"]
+    q = torch.zeros(S, H, d).to(torch.bfloat16)
+    q[..., 0] = 1.0
+    k = torch.zeros(nb, G, 16, d).to(torch.bfloat16)
+    v = torch.randn(nb, G, dv, 16).to(torch.bfloat16)
+    for i, s0 in enumerate(starts):
+        for p in range(s0 + 1):
+            k[md["block_tables"][i, p // 16], :, p % 16, 0] = -100.0
+        for p in range(0, s0 + 1, 32):   # (one of the tile's keys that are there)
+            p += int(torch.randint(min(32, s0 + 1 - p), ()))
+            k[md["block_tables"][i, p // 16], :, p % 16, 0] = 4 * torch.randn(G)
+    want = mref.sink_attention(q.double(), k.double(), v.double(), md["block_tables"], md["seq_kvlen"], md["seq_qstart"],
+                               1.0, False, None, window, None, keep, torch.float64)
+    g, none = cuda(md), torch.zeros(0, dtype=torch.int32, device="cuda")
+    got = mx.sink_attention(q.cuda(), k.cuda(), v.cuda(), g["block_tables"], g["seq_kvlen"], g["seq_qstart"], none, none,
+                            1.0, False, S, 701, window=window, keep_first=keep, out_dtype=torch.float32)
+    assert float((got.cpu().double() - want).norm() / want.norm()) < 2.0 ** -17
+
+
 @pytest.mark.parametrize("bs", [64, 128, 512])
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 70)])
 def test_flash_attention_wide_pages(window, keep, bs):
