@@ -42,6 +42,12 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 constexpr int kBlock = 64;               // keys per block (two 32-key score tiles)
 constexpr int kVS = kBlock + 8;          // V^T row in LDS: 144 B, 16-byte reads free of bank conflicts
 constexpr int kPages = 2048;             // page-table entries in LDS
+// Pair form: in the first blocks each of the two tiles has its own maximum.  Largest weights are rounded to exactly 1;
+// with a maximum per 64 keys there are fewer of them than per 32, half of the difference from the first block, 90 %
+// from four.  Error against 64 bits, prompts of 600 (1e-3): one per block 2.345, the first four split 2.328 (the kernel
+// before, 32 keys: 2.332); 5 x 1165 tokens, window 1024: 82.2 -> 83.3 us, with all blocks split 85.3.  (One map: sums of
+// the rounded weights make up for more than that: 2.928 against 2.935.)
+constexpr int kSplitBlocks = 4;
 constexpr float kLog2e = 1.44269504088896341f;
 
 __device__ __forceinline__ float xor32(float v, int idx4) {
@@ -115,10 +121,10 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
   const __bf16* qp = q + row * a.q_stride + static_cast<int64_t>(head) * DK + 8 * h;
 #pragma unroll
   for (int st = 0; st < ND; ++st) qf[st] = *reinterpret_cast<const bf16x8*>(qp + 16 * st);
-  float m = kNegBig, l = 0.f;
+  float m = kNegBig, l = 0.f;   // l: of the lane's keys
   if (a.sink) {   // the sink is the state the online softmax starts from (log2 units)
     m = a.sink_val != nullptr ? a.sink_val[head] * kLog2e : 0.f;
-    l = 1.f;
+    l = h == 0 ? 1.f : 0.f;
   }
   f32x16 O[NV];
 #pragma unroll
@@ -219,30 +225,41 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
             if (o >= hi || (WIN && o < lo && o >= kp)) S[t][i] = -INFINITY;
           }
       }
-      float tmax = S[0][0];
+      // maxima of the block: one, or in the pair form's first blocks one per tile (kSplitBlocks)
+      constexpr int MT = NMAP, TPM = 2 / MT;
+      float tmax[MT], mt[MT], psum[MT];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int e = 0; e < MT; ++e) {
+        tmax[e] = S[e * TPM][0];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, S[t][i]);
-      tmax = fmaxf(tmax, xor32(tmax, x32)) * scale2;
-      const bool grow = tmax > m;   // (scale > 0; all keys masked: -inf, never)
-      if (__any(grow)) {
-        const float mn = grow ? tmax : m;
-        const float alpha = __builtin_amdgcn_exp2f(m - mn);
+        for (int t = e * TPM; t < (e + 1) * TPM; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) tmax[e] = fmaxf(tmax[e], S[t][i]);
+      }
+#pragma unroll
+      for (int e = 0; e < MT; ++e) tmax[e] = fmaxf(tmax[e], xor32(tmax[e], x32)) * scale2;
+      if (MT > 1 && b >= kSplitBlocks) tmax[0] = fmaxf(tmax[0], tmax[MT - 1]);
+      auto rescale = [&](float alpha) {
         l *= alpha;
 #pragma unroll
         for (int vt = 0; vt < NV; ++vt)
 #pragma unroll
           for (int i = 0; i < 16; ++i) O[vt][i] *= alpha;
-        m = mn;
-      }
+      };
+      bool grow = tmax[0] > m;   // (scale > 0; all keys masked: -inf, never)
+      mt[0] = grow ? tmax[0] : m;
+      if (__any(grow)) rescale(__builtin_amdgcn_exp2f(m - mt[0]));
+      grow = MT > 1 && tmax[MT - 1] > mt[0];
+      mt[MT - 1] = grow ? tmax[MT - 1] : mt[0];
+      m = mt[MT - 1];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          S[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i], scale2, -m));
+          S[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i], scale2, -mt[t / TPM]));
       bf16x8 pf[4];
-      float psum = 0.f;   // of the weights as the value products take them, rounded
+#pragma unroll
+      for (int e = 0; e < MT; ++e) psum[e] = 0.f;   // of the weights as the value products take them, rounded
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         u32x4 wv;
@@ -254,16 +271,20 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
         pf[ks] = __builtin_bit_cast(bf16x8, wv);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          psum += __builtin_bit_cast(float, wv[j] << 16) + __builtin_bit_cast(float, wv[j] & 0xffff0000u);
+          psum[(ks >> 1) / TPM] += __builtin_bit_cast(float, wv[j] << 16) + __builtin_bit_cast(float, wv[j] & 0xffff0000u);
       }
-      l += psum + xor32(psum, x32);
 #pragma unroll
-      for (int vt = 0; vt < NV; ++vt)
+      for (int e = 0; e < MT; ++e) {
+        if (e > 0 && __any(grow)) rescale(__builtin_amdgcn_exp2f(mt[0] - m));
+        l += psum[e];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const bf16x8 vf = *reinterpret_cast<const bf16x8*>(&lds_v[buf][(32 * vt + r) * kVS + 16 * ks + 8 * h]);
-          O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[ks], O[vt], 0, 0, 0);
-        }
+        for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+          for (int ks = 2 * e * TPM; ks < 2 * (e + 1) * TPM; ++ks) {
+            const bf16x8 vf = *reinterpret_cast<const bf16x8*>(&lds_v[buf][(32 * vt + r) * kVS + 16 * ks + 8 * h]);
+            O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[ks], O[vt], 0, 0, 0);
+          }
+      }
       __builtin_amdgcn_s_setprio(0);
     }
     if (more) {
@@ -273,6 +294,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
     __syncthreads();
   }
 
+  l += xor32(l, x32);
   if constexpr (NMAP == 2) {
     // the second map's waves hand lam / l * O to the first map's through LDS (the K / V buffers are free)
     static_assert(sizeof(lds_k) + sizeof(lds_v) >= CW * 64 * 16 * NV * sizeof(float), "room for the second map");

@@ -1092,6 +1092,38 @@ def test_decode_largest_weights_exact(H, G, d, dv, window, keep):
     assert float((got.cpu().double() - want).norm() / want.norm()) < 2.0 ** -17
 
 
+def test_two_maps_largest_weights_exact():
+    """One key of the first 32 and a larger one of the next have a weight (first map; the second counts nothing).  Both
+    are 1 before their 16-bit rounding, so their ratio, from 64 channels each, is off only by what the results' rounding
+    leaves: 2^-9 / sqrt(3) / sqrt(64) on either side, together 2.0e-4; a rounded weight is off by 2^-9 / sqrt(6) = 8e-4."""
+    torch.manual_seed(9)
+    S, H, G, d, dv = 20, 8, 2, 64, 128
+    md = ragged([2] * S, [64] * S, list(range(S)), width=8)
+    nb = md["num_pages"]
+    q = torch.zeros(2 * S, 2 * H, d)
+    q[..., 0] = 1 + torch.arange(2 * H) % (H // G) / 8
+    k, v = torch.zeros(nb, 2 * G, 16, d), torch.zeros(nb, G, dv, 16)
+    k[..., 0] = -100.0
+    big = (1 + torch.rand(dv)).to(torch.bfloat16).float()
+    peak = torch.randn(S, 2, G).to(torch.bfloat16).float()
+    peak[:, 1] = (peak[:, 0] + 2 * torch.rand(S, G)).to(torch.bfloat16).float()
+    for i in range(S):
+        for t in range(2):
+            p = 32 * t + int(torch.randint(32, ()))
+            page = md["block_tables"][i, p // 16]
+            k[page, 0::2, p % 16, 0] = peak[i, t]
+            v[page, :, 64 * t:64 * t + 64, p % 16] = big[64 * t:64 * t + 64]
+    g = cuda(md)
+    q, k, v = (t.to(torch.bfloat16).cuda() for t in (q, k, v))
+    got = mx.differential_attention(q, k, v, g["block_tables"], g["seq_kvlen"], g["seq_qstart"], g["tile_seq"],
+                                    g["tile_qoff"], 1.0, 0.0, 0.0, 1e-5)
+    r = (got.cpu().double().view(S, 2, G, H // G, 2, 64) / big.double().view(2, 64)).mean(-1)
+    scale = 1 + torch.arange(H // G).double() / 8
+    want = torch.exp((peak[:, 0] - peak[:, 1]).double()[:, None, :, None] * scale)
+    err = r[..., 0] / r[..., 1] / want - 1
+    assert float(err.pow(2).mean().sqrt()) < 4e-4
+
+
 @pytest.mark.parametrize("bs", [64, 128, 512])
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 70)])
 def test_flash_attention_wide_pages(window, keep, bs):
