@@ -485,7 +485,7 @@ def state_space_scan(x, B, C, dt, dt_bias, a_log, skip, state, positions, seq_qs
 
 
 
-RETENTION_CHUNK = 64      # the longest chunk a table of powers serves (the kernels' chunks have 16 tokens)
+RETENTION_CHUNK = 64      # powers in a table (the kernels' chunks have 16 tokens; the last power corrects the 16th's rounding)
 
 
 def retention_powers(decay, device) -> torch.Tensor:

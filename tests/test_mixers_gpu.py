@@ -1817,6 +1817,32 @@ def test_group_norm_widths(dt, gs, full):
         assert torch.allclose(got, want, rtol=2.0 ** (-7 if dt == torch.bfloat16 else -18), atol=1e-6)
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n,S,H", [(8000, 1, 8), (1999, 16, 16)])
+def test_retention_slow_decays(dt, n, S, H):
+    """States of heads that remember thousands of tokens, in segments and without, whose decay over a chunk of 16 tokens
+    is rounded by nearly half a place: the chunks' roundings do not add up.  Against 64 bits with the decay that the
+    table's last power says: per chunk five roundings of the state (the decay, four products), each 2^-24 / sqrt(3) at
+    most (rms), and 2^-24 for the product of the decays."""
+    torch.manual_seed(8)
+    d = 64
+    g = 1 - 2e-4 * (1 + torch.arange(1000, dtype=torch.float64) / 1000)
+    off = (g ** 16).float().double() / g ** 16 - 1
+    pw = mx.retention_powers(g[off.abs() > 0.45 * 2.0 ** -24][:H].tolist(), "cuda")
+    q, k, v = (torch.randn(S * n, H * d, device="cuda").to(dt) for _ in range(3))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    st = torch.zeros(S, H, d, d, device="cuda")
+    mx.retention(q, k, v, pw, torch.zeros(S * n, 0, device="cuda"), st, i32(list(range(n)) * S),
+                 i32([n * s for s in range(S + 1)]), i32(list(range(S))), H, d, d)
+    age = torch.arange(n - 1, -1, -1, dtype=torch.float64, device="cuda") / 64
+    bound = 2.0 ** -24 * (1 + (5 * n / 16 / 3) ** 0.5)
+    for h in range(H):
+        w = pw[h, 64].double() ** age
+        kk, vv = (x.view(S, n, H, d)[0, :, h].double() for x in (k, v))
+        want = (kk * w[:, None]).t().contiguous() @ vv * d ** -0.5
+        assert float((st[0, h].double() - want).norm() / want.norm()) < bound, h
+
+
 def chunks_per_segment(T, H, dv):
     """The length that the kernels aim at for a batch of T rows (chunk_scan.h, scan_segments)."""
     n, cols = T // 16, -(-dv // 64)
