@@ -13,8 +13,8 @@
 // row, so portions that start anywhere in the batch are stored 16 bytes at a time.
 //
 // Bound: memory traffic.  Measured, before (element-wise, two or three launches) -> now, with the time of a copy of
-// the same bytes: 7580 rows, 32 + 8 + 8 heads of 128: 120 -> 44 us (38); latent, 7580 rows x 32 heads of 192 + 64:
-// 137 -> 76 (51); norm over the projection, 1908 rows of 24 + 8 + 8 heads: 33 -> 16.
+// the same bytes: 7580 rows, 32 + 8 + 8 heads of 128: 119 -> 43 us (38); latent, 7580 rows x 32 heads of 192 + 64:
+// 137 -> 77 (51); norm over the projection, 1908 rows of 24 + 8 + 8 heads: 33 -> 16.
 #include <initializer_list>
 
 #include "head_front.h"

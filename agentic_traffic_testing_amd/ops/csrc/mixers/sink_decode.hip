@@ -14,7 +14,7 @@
 // Bound: latency of one chain (row, context length -> block table -> keys -> weights -> store) for short contexts,
 // the pages' bytes for long ones.  Measured, tiles staged in LDS one after the other -> now: 8 rows,
 // contexts of 1500, 32 + 8 heads of 128: 15.4 -> 10.8 us (32 rows of 2000: 38 us, 6.9 TB/s with the last-level cache's
-// help); latent, 16 rows of 2000: 26 -> 12.5; two maps 21 -> 10.
+// help); latent, 16 rows of 2000: 26 -> 12.1; two maps 21 -> 10.
 //
 // Join: four waves per (row, head) take every fourth partition, with the first four of them loaded before their
 // weights are known: 6.2 -> 3.7 us, latent 10.7 -> 4.4, two maps 7.1 -> 5.7.

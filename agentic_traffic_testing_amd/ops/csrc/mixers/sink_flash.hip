@@ -386,9 +386,9 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
 // two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two)
 // and contexts past the LDS page list run sink_attention.hip's kernel.  Measured at 4 prompts of ~1850
 // tokens (us, old kernel -> this one; variants at the same shapes):
-//   128 / 128, 32 heads over 8:  463 -> 167 (8 waves per workgroup: +1 %; 64 columns per wave: +30 %)
-//   256 / 192, 32 heads over 1: 1059 -> 267 (4 waves +50 %: one wave per SIMD hides no latency)
-//   two maps 64 / 128, 8 over 2, 5 x 1165 tokens, window 1024: 125 -> 71 (both maps in each of 4 waves
+//   128 / 128, 32 heads over 8:  463 -> 159 (8 waves per workgroup: +1 %; 64 columns per wave: +30 %)
+//   256 / 192, 32 heads over 1: 1052 -> 261 (4 waves +50 %: one wave per SIMD hides no latency)
+//   two maps 64 / 128, 8 over 2, 5 x 1165 tokens, window 1024: 126 -> 72 (both maps in each of 4 waves
 //     +45 %: few workgroups there, so a wave's own chain counts; 2 waves per SIMD +10 %, 4 spill)
 // The workgroups of the 256 / 192 form hold 8 tokens (the old kernel's 4): so far ahead a NaN value reaches back (a weight
 // of 0 times NaN), as it did there.
