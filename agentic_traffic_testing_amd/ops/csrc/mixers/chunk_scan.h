@@ -7,9 +7,12 @@ namespace mixk {
 
 constexpr int kScanChunk = 16;         // tokens per chunk
 constexpr int kPowers = 65;            // retention: powers 0 ... 64 of a head's decay
-constexpr int kWalkCols = 64;          // value columns of a workgroup of the walk
 enum ScanMode { kModeRetention = 0, kModeForget = 1, kModeStateSpace = 2, kModeDelta = 3,
                 kModeDeltaChannel = 4 };
+constexpr int kWalkCols = 64;          // value columns of four of the walk's waves
+// the walk's waves that prepare operands for keys of up to dk channels
+constexpr int operand_waves(int mode, int dk) { return mode >= kModeDelta ? dk / 16 : 4; }
+constexpr int kWalkThreads = 64 * 12;
 
 struct ChunkArgs {
   float* out;             // [T, H, dv]
@@ -33,6 +36,8 @@ struct ChunkArgs {
   float* seg;             // scratch: states at the ends of segments and the decays over them (scan_segments)
   int seg_chunks, seg_states;
   float kscale;
+  int64_t T;              // rows in all
+  int walk_heads;         // heads per workgroup of the walk (walk_shape)
 };
 
 // Chunk c of sequence s has the slot seq_qstart[s] / 16 + s + c: disjoint runs, known on the device only.
@@ -45,6 +50,24 @@ constexpr int scan_record_floats(int mode) { return mode >= kModeDelta ? 576 : 3
 // into segments that run side by side, in two passes (chunk_scan.hip).  `chunks`: a segment's length with which the
 // batch makes about 256 workgroups (one per CU: the registers allow no second one), at least 10 and a 16th of the batch
 // (a segment's start is put together from all segments before it).
+// A workgroup of the walk: eight waves of 16 columns of S beside four that prepare the operands, once for 128 columns or
+// for two heads of 64 whose keys are the same: the operands' vector work is half of the walk's at 64 columns.  Where such
+// workgroups do not fill the chip, not even with segments of 10 chunks, four waves and 64 columns; so the delta rule,
+// whose portions are not cut, with eight waves for its operands.
+inline bool walk_wide(int64_t T, int64_t S, int64_t H, int64_t dv, int mode) {
+  const int64_t units = H * ((dv + kWalkCols - 1) / kWalkCols);
+  return mode < kModeDelta && (S * units >= 512 || T / kScanChunk * units >= 5120);
+}
+struct WalkShape {
+  int waves, heads, cols;   // waves with products; heads per workgroup; columns per workgroup and head
+};
+inline WalkShape walk_shape(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dv, int mode) {
+  if (walk_wide(T, S, H, dv, mode)) {
+    if (dv > kWalkCols) return {8, 1, 2 * kWalkCols};
+    if (mode == kModeStateSpace && H / G % 2 == 0) return {8, 2, kWalkCols};
+  }
+  return {4, 1, kWalkCols};
+}
 struct ScanSegments {
   int64_t chunks, states;   // states: an upper bound of the cut portions' segments, 0: no portion can be cut
 };
@@ -54,9 +77,10 @@ __host__ __device__ inline int scan_segment_chunks(int n, int chunks) {
   const int P = (4 * n + chunks) / (4 * chunks);
   return P < 2 ? (n > 0 ? n : 1) : (n + P - 1) / P;
 }
-inline ScanSegments scan_segments(int64_t T, int64_t H, int64_t dv, int mode) {
+inline ScanSegments scan_segments(int64_t T, int64_t S, int64_t H, int64_t dv, int mode) {
   const int64_t n = T / kScanChunk, cols = (dv + kWalkCols - 1) / kWalkCols;
-  int64_t chunks = (n * H * cols + 255) / 256;
+  const int64_t all = walk_wide(T, S, H, dv, mode) ? 512 : 256;
+  int64_t chunks = (n * H * cols + all - 1) / all;
   if (chunks < 10) chunks = 10;
   if (chunks < (n + 15) / 16) chunks = (n + 15) / 16;
   // cut portions have n >= 1.75 `chunks` and at most n / chunks + 1 / 4 segments; their chunks are the rows' 16ths,
@@ -68,7 +92,7 @@ constexpr int64_t scan_segment_floats(int64_t H, int64_t dk, int64_t dv) { retur
 // floats of scratch: the records, then the segments
 inline int64_t scan_scratch_floats(int64_t T, int64_t S, int64_t H, int64_t dk, int64_t dv, int mode) {
   return scan_chunk_slots(T, S) * H * scan_record_floats(mode) +
-         scan_segments(T, H, dv, mode).states * scan_segment_floats(H, dk, dv);
+         scan_segments(T, S, H, dv, mode).states * scan_segment_floats(H, dk, dv);
 }
 
 // Which kernels take a batch.  The host knows its T rows and S portions; if every portion has a row, the longest has at
@@ -118,9 +142,10 @@ inline int launch_scan_batch(ChunkArgs a, int mode, int64_t T, int dtype, hipStr
   for (const int64_t x : strides)
     if (x >= 1ll << 26) a.rec = nullptr;
   if (a.rec == nullptr) return launch_step_scan(a, mode, 1 << 30, dtype, st);
+  a.T = T;
   a.n_slots = static_cast<int>(scan_chunk_slots(T, a.S));
   a.min_rows = kScanMinRows[mode];
-  const ScanSegments g = scan_segments(T, a.H, a.dv, mode);
+  const ScanSegments g = scan_segments(T, a.S, a.H, a.dv, mode);
   a.seg = a.rec + static_cast<int64_t>(a.n_slots) * a.H * scan_record_floats(mode);
   a.seg_chunks = static_cast<int>(g.chunks);
   a.seg_states = static_cast<int>(g.states);

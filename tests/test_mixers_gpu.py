@@ -1969,3 +1969,32 @@ def test_segments_in_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager[i][0]) and torch.equal(st, eager[i][1])
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,G,d,dv", [(16, 8, 128, 64), (16, 4, 64, 40), (15, 5, 128, 64), (8, 8, 128, 128),
+                                      (8, 4, 100, 70), (6, 6, 64, 129)])
+def test_scans_of_many_portions(dt, H, G, d, dv):
+    """Batches that fill the chip (walk_wide): 128 columns per workgroup, or two heads of 64 with the same keys, portions
+    of odd and even numbers of chunks, full and not, fresh and continued."""
+    torch.manual_seed(H + d + dv)
+    S = 512 // (H * -(-dv // 64)) + 3
+    lens = [(16, 33, 47, 64, 30, 80)[i % 6] for i in range(S)]
+    md = ragged(lens, [9 * (i % 2) for i in range(S)], list(range(S))[::-1], width=64)
+    T, g = sum(lens), cuda(md)
+    at, at_g = (tuple(m[k] for k in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    q, f, k = (torch.randn(T, H * d).to(dt) for _ in range(3))
+    B, C, v = torch.randn(T, G * d).to(dt), torch.randn(T, G * d).to(dt), torch.randn(T, H * dv).to(dt)
+    dts, z, skip = torch.randn(T, H).to(dt), torch.zeros(H), torch.randn(H)
+    bias, lower, tab = torch.randn(H * d), 0.9 * torch.rand(H * d), torch.zeros(T, 0)
+    pw = mx.retention_powers([1.0 - 2.0 ** (-3 - h % 6) for h in range(H)], "cpu")
+    for name, args, last in (("forget_gate_scan", (q, f, v, bias, lower), (H, d, dv)),
+                             ("state_space_scan", (v, B, C, dts, z, z, skip), (H, G, d, dv)),
+                             ("retention", (q, k, v, pw, tab), (H, d, dv))):
+        st = torch.randn(S, H, d, dv)
+        st_g = st.clone().cuda()
+        got = getattr(mx, name)(*(a.cuda() for a in args), st_g, *at_g, *last)
+        if name == "retention":
+            args = (q, k, v, pw[:, 1], tab)
+        want = getattr(mref, name)(*args, st, *at, *last)
+        chunk_compare(got, want, st_g, st, torch.ones(T, dtype=torch.bool))
