@@ -215,11 +215,13 @@ __global__ void __launch_bounds__(256)
 gated_rms_norm_vec_kernel(T* __restrict__ out, const float* __restrict__ o,
                           const T* __restrict__ gate, int64_t gate_stride, const T* __restrict__ w,
                           int64_t items, int H, int dv, float eps, int act) {
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * (256 / LPR) + threadIdx.x / LPR;
+  // (below 2^31, and divided as such: a 64-bit division is a third of the kernel)
+  const unsigned at = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  const int64_t item = at;
   const int i = (threadIdx.x % LPR) * 8;
   const bool on = item < items && i < dv;
-  const int64_t t = on ? item / H : 0;
-  const int h = static_cast<int>(on ? item % H : 0);
+  const int64_t t = on ? at / static_cast<unsigned>(H) : 0;
+  const int h = static_cast<int>(on ? at % static_cast<unsigned>(H) : 0);
   float v[8], gv[8];
   float ss = 0.f;
   if (on) {
@@ -233,7 +235,7 @@ gated_rms_norm_vec_kernel(T* __restrict__ out, const float* __restrict__ o,
   if (!on) return;
   const float inv = 1.0f / sqrtf(ss / static_cast<float>(dv) + eps);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] *= inv * (act == 1 ? sigmoidf_(gv[e]) : siluf_(gv[e]));
+  for (int e = 0; e < 8; ++e) v[e] *= inv * (act == 1 ? gate_sigmoid<T>(gv[e]) : gate_silu<T>(gv[e]));
   if (w != nullptr) {
     float wv[8];
     ld8(w + i, wv);
@@ -348,11 +350,12 @@ __global__ void __launch_bounds__(256)
 group_rms_norm_lanes_kernel(T* __restrict__ out, const float* __restrict__ y, const T* __restrict__ gate,
                             int64_t gate_stride, const T* __restrict__ w, int64_t items, int n_groups, int gs,
                             float eps, int w_full) {
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * (256 / LPR) + threadIdx.x / LPR;
+  const unsigned at = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;   // (below 2^31)
+  const int64_t item = at;
   const int i = (threadIdx.x % LPR) * 8;
   const bool on = item < items && i < gs;
-  const int64_t t = on ? item / n_groups : 0;
-  const int g = static_cast<int>(on ? item - t * n_groups : 0);
+  const int64_t t = on ? at / static_cast<unsigned>(n_groups) : 0;
+  const int g = static_cast<int>(on ? at % static_cast<unsigned>(n_groups) : 0);
   float u[8], wv[8], ss = 0.f;
   if (on) {
     ld8(y + item * gs + i, u);
@@ -361,7 +364,7 @@ group_rms_norm_lanes_kernel(T* __restrict__ out, const float* __restrict__ y, co
       float gv[8];
       ld8(gate + t * gate_stride + static_cast<int64_t>(g) * gs + i, gv);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) u[e] *= siluf_(gv[e]);
+      for (int e = 0; e < 8; ++e) u[e] *= gate_silu<T>(gv[e]);
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss += u[e] * u[e];
@@ -397,7 +400,7 @@ __global__ void group_rms_norm_vec_kernel(T* __restrict__ out, const float* __re
         float gv[8];
         ld8(gr + i, gv);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) u[c][e] *= siluf_(gv[e]);
+        for (int e = 0; e < 8; ++e) u[c][e] *= gate_silu<T>(gv[e]);
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += u[c][e] * u[c][e];
@@ -548,7 +551,7 @@ extern "C" int mixk_gated_rms_norm(void* out, const float* o, const void* gate,
   if (T_ <= 0) return 0;
   const uintptr_t mask = dtype == 2 ? 31 : 15;
   const int64_t items = static_cast<int64_t>(T_) * H;
-  const bool vec = dv % 8 == 0 && dv <= 512 && gate_stride % 8 == 0 &&
+  const bool vec = dv % 8 == 0 && dv <= 512 && gate_stride % 8 == 0 && items < (1ll << 31) &&
                    ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(gate) |
                      reinterpret_cast<uintptr_t>(w)) & mask) == 0 &&
                    (reinterpret_cast<uintptr_t>(o) & 31) == 0;

@@ -58,32 +58,40 @@ __global__ void short_conv_silu_kernel(T* __restrict__ out, const T* __restrict_
   stf(o, siluf_(acc));
 }
 
-// Sixteen bytes at a time, the state's update included: a workgroup takes up to kConvRows rows of one portion, a
-// thread 8 channels of them, with the last TAPS - 1 inputs in registers as it walks down the rows, 8 rows of loads
-// ahead.  Only a portion's first workgroup reads its state slot (kConvRows >= TAPS - 1), so the same threads write
+// Sixteen bytes at a time, the state's update included: a workgroup takes up to ROWS rows of one portion, a
+// thread 8 channels of them, with the last TAPS - 1 inputs in registers as it walks down the rows, up to 8 rows of loads
+// ahead.  Only a portion's first workgroup reads its state slot (ROWS >= TAPS - 1), so the same threads write
 // the new tail: no second launch, no order between workgroups.
 //
 // Workgroup -> portion without a host plan: with `at(k)` the first row of portion k, portion k owns the workgroups
-// from at(k) / kConvRows + k on; there are at least ceil(n / kConvRows) of them.  Portion 0 stands for the rows
+// from at(k) / ROWS + k on; there are at least ceil(n / ROWS) of them.  Portion 0 stands for the rows
 // before the first sequence and portion S + 1 for those after the last one (zeros, as for padding sequences).
 //
-// Bound: one read and one write of the rows, and the SiLU's arithmetic.  Measured, before (8 rows per workgroup, every
-// tap loaded again, a second launch for the tails) -> now: 7580 rows of 6144 channels in bf16 125 -> 53 us (copy: 38);
-// 1023 rows of 8192 in fp32 87 -> 26 (14); 16 decode rows 13 -> 5.
+// Bound: one read and one write of the rows; the SiLU's arithmetic (library functions: 35 of 45 instructions per result,
+// 52 us in the first line).  Measured, before (8 rows per workgroup, every tap loaded again, a second launch for the
+// tails) -> now: 7580 rows of 6144 channels in bf16 125 -> 43 us (copy: 38); 1023 rows of 8448 in fp32 87 -> 20 (14);
+// 16 decode rows 13 -> 5.
+//
+// A thread takes its rows one after the other, about 0.5 us each, so batches that do not fill the chip have workgroups of
+// 4 rows (8 where a tail is longer).  16 rows / 4 rows, us, 6144 channels in bf16: 64 rows 9.4 / 7.1, 1024 10.9 / 9.0, 2048
+// 17.2 / 14.0, 4096 (768 workgroups of 16) 23.1 / 24.0, 8000 40.0 / 42.0; 8448 in fp32: 64 13.0 / 7.3, 2048 35.6 / 33.7,
+// 4096 61.6 / 60.8, 6000 92 / 104.
 constexpr int kConvRows = 16;
+constexpr int kConvFew = 768;   // workgroups
 
-template <typename T, int TAPS>
+template <typename T, int TAPS, int ROWS>
 __global__ void __launch_bounds__(256)
 short_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, int64_t x_stride, const T* __restrict__ w,
                        const T* __restrict__ bias, T* __restrict__ conv_state, const int* __restrict__ positions,
                        const int* __restrict__ seq_qstart, const int* __restrict__ seq_slot, int T_, int S, int C) {
-  constexpr int KEEP = TAPS - 1, NH = KEEP > 0 ? KEEP : 1;
+  constexpr int KEEP = TAPS - 1, NH = KEEP > 0 ? KEEP : 1, AHEAD = ROWS < 8 ? ROWS : 8;
+  static_assert(KEEP <= AHEAD, "only a portion's first workgroup reads the state");
   const int b = blockIdx.x, lane = threadIdx.x & 63;
   // the last portion whose first workgroup is not after b (every wave looks, 64 portions at a time)
   int k = -1, first = 0;
   for (int k0 = 0; k0 <= S + 1; k0 += kWave) {
     const int i = k0 + lane, at = i == 0 || i > S + 1 ? 0 : seq_qstart[i - 1];
-    const uint64_t m = __ballot(i <= S + 1 && at / kConvRows + i <= b);
+    const uint64_t m = __ballot(i <= S + 1 && at / ROWS + i <= b);
     if (m == 0) break;
     const int top = 63 - __builtin_clzll(m);
     k = k0 + top;
@@ -91,12 +99,12 @@ short_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, int64_t x_s
     if (m != ~0ull) break;
   }
   const int end = k <= S ? seq_qstart[k] : T_;
-  const int n = end - first, j0 = (b - (first / kConvRows + k)) * kConvRows;   // row of the portion
+  const int n = end - first, j0 = (b - (first / ROWS + k)) * ROWS;   // row of the portion
   if (j0 >= n) return;
   const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
   if (c >= C) return;
   const int slot = k >= 1 && k <= S ? seq_slot[k - 1] : -1;
-  const int rows = min(kConvRows, n - j0), r0 = first + j0;
+  const int rows = min(ROWS, n - j0), r0 = first + j0;
   T* o = out + static_cast<int64_t>(r0) * C + c;
   if (slot < 0) {
     const float zero[8] = {};
@@ -106,9 +114,9 @@ short_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, int64_t x_s
   const T* xr = x + r0 * x_stride + c;
   const int pos = positions[r0];
   T* tail = conv_state + static_cast<int64_t>(slot) * KEEP * C + c;
-  float xv[8][8], hist[NH][8], wv[TAPS * 8], bv[8];   // hist[u]: the input KEEP - u tokens before the row
+  float xv[AHEAD][8], hist[NH][8], wv[TAPS * 8], bv[8];   // hist[u]: the input KEEP - u tokens before the row
 #pragma unroll
-  for (int j = 0; j < 8; ++j) ld8(xr + min(j, rows - 1) * x_stride, xv[j]);
+  for (int j = 0; j < AHEAD; ++j) ld8(xr + min(j, rows - 1) * x_stride, xv[j]);
 #pragma unroll
   for (int u = 0; u < KEEP; ++u) ld8(j0 == 0 ? tail + static_cast<int64_t>(u) * C : xr + (u - KEEP) * x_stride, hist[u]);
 #pragma unroll
@@ -136,9 +144,9 @@ short_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, int64_t x_s
       st8(tail + static_cast<int64_t>(u) * C, nv[u]);
     }
   }
-  for (int j = 0; j < rows; j += 8) {
+  for (int j = 0; j < rows; j += AHEAD) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < AHEAD; ++i) {
       if (j + i >= rows) break;
       float acc[8];
 #pragma unroll
@@ -150,16 +158,16 @@ short_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, int64_t x_s
         for (int e = 0; e < 8; ++e) acc[e] += wv[e * TAPS + t] * (t + i < KEEP ? hist[(t + i) % NH][e] : xv[t + i - KEEP < 0 ? 0 : t + i - KEEP][e]);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = siluf_(acc[e]);
+      for (int e = 0; e < 8; ++e) acc[e] = gate_silu<T>(acc[e]);
       st8(o + static_cast<int64_t>(j + i) * C, acc);
     }
-    if (j + 8 >= rows) break;
+    if (ROWS <= AHEAD || j + AHEAD >= rows) break;
 #pragma unroll
     for (int u = 0; u < KEEP; ++u)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) hist[u][e] = xv[8 - KEEP + u][e];
+      for (int e = 0; e < 8; ++e) hist[u][e] = xv[AHEAD - KEEP + u][e];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ld8(xr + min(j + 8 + i, rows - 1) * x_stride, xv[i]);
+    for (int i = 0; i < AHEAD; ++i) ld8(xr + min(j + AHEAD + i, rows - 1) * x_stride, xv[i]);
   }
 }
 
@@ -167,11 +175,17 @@ template <typename T>
 int launch_conv_rows(T* out, const T* x, int64_t x_stride, const T* w, const T* bias, T* conv_state,
                      const int* positions, const int* seq_qstart, const int* seq_slot, int T_, int S, int C, int taps,
                      hipStream_t st) {
-  const dim3 grid(T_ / kConvRows + S + 2, (C / 8 + 255) / 256);
+  const unsigned cols = (C / 8 + 255) / 256;
+  const bool few = (static_cast<int64_t>(T_) / kConvRows + S) * cols < kConvFew;
+  const dim3 grid(T_ / (few ? (taps <= 5 ? 4 : 8) : kConvRows) + S + 2, cols);
 #define MIXK_TAPS(N)                                                                                                \
   case N:                                                                                                           \
-    hipLaunchKernelGGL((short_conv_rows_kernel<T, N>), grid, dim3(256), 0, st, out, x, x_stride, w, bias, conv_state, \
-                       positions, seq_qstart, seq_slot, T_, S, C);                                                  \
+    if (few)                                                                                                        \
+      hipLaunchKernelGGL((short_conv_rows_kernel<T, N, (N <= 5 ? 4 : 8)>), grid, dim3(256), 0, st, out, x, x_stride, \
+                         w, bias, conv_state, positions, seq_qstart, seq_slot, T_, S, C);                           \
+    else                                                                                                            \
+      hipLaunchKernelGGL((short_conv_rows_kernel<T, N, kConvRows>), grid, dim3(256), 0, st, out, x, x_stride, w,    \
+                         bias, conv_state, positions, seq_qstart, seq_slot, T_, S, C);                              \
     break;
   switch (taps) {
     MIXK_TAPS(1) MIXK_TAPS(2) MIXK_TAPS(3) MIXK_TAPS(4) MIXK_TAPS(5) MIXK_TAPS(6) MIXK_TAPS(7) MIXK_TAPS(8)

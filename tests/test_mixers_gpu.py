@@ -1998,3 +1998,25 @@ def test_scans_of_many_portions(dt, H, G, d, dv):
             args = (q, k, v, pw[:, 1], tab)
         want = getattr(mref, name)(*args, st, *at, *last)
         chunk_compare(got, want, st_g, st, torch.ones(T, dtype=torch.bool))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("taps", [2, 4, 8])
+def test_short_conv_rows_of_full_chip(dt, taps):
+    """Enough channels for 16 rows per workgroup: portions around that and shorter than the taps, fresh and continued."""
+    torch.manual_seed(taps)
+    lens, starts = [1, 15, 16, 17, 33, 2, 3, 64, 5, 1], [0, 0, 1, 2, 0, 1, 0, 9, 3, 1]
+    S = len(lens)
+    md = ragged(lens, starts, [S - 1 - i for i in range(S)], width=64)
+    g, T, C = cuda(md), sum(lens), 2048 * 41 + 8
+    x, w, st = torch.randn(T, C).to(dt), torch.randn(C, taps).to(dt), torch.randn(S, taps - 1, C).to(dt)
+    for i, p in enumerate(starts):
+        if p:                                   # as the earlier portion left it: nothing before position 0
+            st[int(md["seq_slot"][i]), :max(0, taps - 1 - p)] = 0
+    stg = st.cuda()
+    want = mref.short_conv_silu(x, w, st, md["positions"], md["seq_qstart"], md["seq_slot"])
+    got = mx.short_conv_silu(x.cuda(), w.cuda(), stg, g["positions"], g["seq_qstart"], g["seq_slot"])
+    assert torch.equal(stg.cpu(), st)
+    # up to 8 products in fp32, then one rounding to the storage type
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
+    assert torch.allclose(got.cpu().float(), want.float(), rtol=2 * eps, atol=2 * eps)
