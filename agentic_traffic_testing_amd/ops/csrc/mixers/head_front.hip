@@ -13,9 +13,13 @@
 // row, so portions that start anywhere in the batch are stored 16 bytes at a time.
 //
 // Bound: memory traffic.  Measured, before (element-wise, two or three launches) -> now, with the time of a copy of
-// the same bytes: 7580 rows, 32 + 8 + 8 heads of 128: 119 -> 43 us (38); latent, 7580 rows x 32 heads of 192 + 64:
-// 137 -> 77 (51); norm over the projection, 1908 rows of 24 + 8 + 8 heads: 33 -> 16.
+// the same bytes: 7580 rows, 32 + 8 + 8 heads of 128: 119 -> 38.5 us (38); latent, 7580 rows x 32 heads of 192 + 64:
+// 137 -> 57.6 (51), 1300 rows x 8 heads 9.7; norm over the projection, 1908 rows of 24 + 8 + 8 heads: 33 -> 13.9.
+// V workgroups come first in the grid: their chain (slots, rows, norm, transposed stores: 11 us) is the longest (the last
+// lines 63.7, 13.5 and 13.9 us; at the grid's end 68.7, 16.8 and 16.4).  Sums over a group's lanes are taken of all rows
+// of a thread at once (one after the other: 41.2, 63.7, 13.5 us in the first three).
 #include <initializer_list>
+#include <type_traits>
 
 #include "head_front.h"
 
@@ -65,9 +69,12 @@ __device__ __forceinline__ void rotate(float* y, const Table& t, int lane0, int 
   }
 }
 
-__device__ __forceinline__ float lane_group_sum(float v, int L) {
-  for (int o = L >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+// sums over the lanes of a group, of several rows at once: an exchange's latency is paid once per step
+template <int N>
+__device__ __forceinline__ void lane_group_sums(float (&v)[N], int L) {
+  for (int o = L >> 1; o > 0; o >>= 1)
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] += __shfl_xor(v[r], o, kWave);
 }
 
 // Workgroup (rb, y) of the V part: rows [2 HR rb, 2 HR (rb + 1)) in two halves; item = (head, half), L lanes each.
@@ -115,19 +122,25 @@ __device__ __forceinline__ void v_part(const FrontArgs& a, int rb, int y, int ls
   const int heads = (mask_lds[0] >> (HR * half)) & ((1 << HR) - 1);
   const int single = (mask_lds[1] >> (HR * half)) & ((1 << HR) - 1);
   T* cache = static_cast<T*>(a.v_cache) + (static_cast<int64_t>(g) * a.vdim + ch) * bs;
-  auto norm = [&](int rows) {
+  auto norm = [&](auto rows) {
+    constexpr int R = decltype(rows)::value;
+    float ss[R];
 #pragma unroll
-    for (int j = 0; j < rows; ++j) {
-      float ss = 0.f;
+    for (int j = 0; j < R; ++j) {
+      ss[j] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ss += v[j][e] * v[j][e];
-      ss = lane_group_sum(on ? ss : 0.f, L);
-      const float inv = 1.0f / sqrtf(ss / static_cast<float>(a.vdim) + a.eps);
+      for (int e = 0; e < 8; ++e) ss[j] += v[j][e] * v[j][e];
+      ss[j] = on ? ss[j] : 0.f;
+    }
+    lane_group_sums(ss, L);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const float inv = 1.0f / sqrtf(ss[j] / static_cast<float>(a.vdim) + a.eps);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[j][e] = v[j][e] * inv * w[e];
     }
   };
-  if (NORM) norm(HR);
+  if (NORM) norm(std::integral_constant<int, HR>{});
 #pragma unroll
   for (int j = 0; j < HR; ++j) {
     if (!on || !(single >> j & 1)) continue;
@@ -139,7 +152,7 @@ __device__ __forceinline__ void v_part(const FrontArgs& a, int rb, int y, int ls
   const int j0 = __builtin_ctz(heads);
   if (HR < 8 || j0 != 0) {
     load(r0 + HR * half + j0, 8);
-    if (NORM) norm(8);
+    if (NORM) norm(std::integral_constant<int, 8>{});
   }
   if (!on) return;
   T* dst = cache + at_lds[HR * half + j0];
@@ -154,11 +167,10 @@ __device__ __forceinline__ void v_part(const FrontArgs& a, int rb, int y, int ls
 
 template <typename T, int ROWS, int VH, bool WHOLE>
 __global__ void __launch_bounds__(WHOLE ? 1024 : 256)
-head_front_kernel(FrontArgs a, int qk_blocks, int uy, int lsh, int vy, int vlsh) {
+head_front_kernel(FrontArgs a, int v_blocks, int uy, int lsh, int vy, int vlsh) {
   __shared__ float sums[WHOLE ? ROWS : 1][2][16];
-  const int bid = blockIdx.x;
-  if (bid >= qk_blocks) {   // uniform over the workgroup
-    const int vb = bid - qk_blocks;
+  const int vb = blockIdx.x, bid = vb - v_blocks;
+  if (bid < 0) {   // uniform over the workgroup
     if (a.v_norm)
       v_part<T, VH, true>(a, vb / vy, vb % vy, vlsh);
     else
@@ -199,15 +211,22 @@ head_front_kernel(FrontArgs a, int qk_blocks, int uy, int lsh, int vy, int vlsh)
     ss[r] = on ? ss[r] : 0.f;
   }
   if (WHOLE) {
+    float both[2 * ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-      const float sq = wave_sum(is_q ? ss[r] : 0.f), sk = wave_sum(is_q ? 0.f : ss[r]);
-      if ((tid & 63) == 0) {
-        sums[WHOLE ? r : 0][0][tid >> 6] = sq;
-        sums[WHOLE ? r : 0][1][tid >> 6] = sk;
-      }
+      both[2 * r] = is_q ? ss[r] : 0.f;
+      both[2 * r + 1] = is_q ? 0.f : ss[r];
     }
+    lane_group_sums(both, kWave);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+      if ((tid & 63) == 0) {
+        sums[WHOLE ? r : 0][0][tid >> 6] = both[2 * r];
+        sums[WHOLE ? r : 0][1][tid >> 6] = both[2 * r + 1];
+      }
     lds_barrier();
+  } else if (!a.plain && !whole) {
+    lane_group_sums(ss, L);
   }
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
@@ -223,7 +242,7 @@ head_front_kernel(FrontArgs a, int qk_blocks, int uy, int lsh, int vy, int vlsh)
     } else if (whole) {
       inv = a.row_inv[2 * static_cast<int64_t>(t) + (is_q ? 0 : 1)];
     } else {
-      inv = 1.0f / sqrtf(lane_group_sum(ss[r], L) / static_cast<float>(a.dim) + a.eps);
+      inv = 1.0f / sqrtf(ss[r] / static_cast<float>(a.dim) + a.eps);
     }
     // (the temperature is a common factor of the head, so it commutes with the rotation)
     if (is_q && a.temp_coef != 0.f)
@@ -243,10 +262,9 @@ head_front_kernel(FrontArgs a, int qk_blocks, int uy, int lsh, int vy, int vlsh)
 // Latent form: item = query head (copy of q_lat | rotated channels of qx) or, last, the row's key.
 template <typename T, int ROWS, int VH>
 __global__ void __launch_bounds__(256)
-latent_front_kernel(FrontArgs a, int qk_blocks, int uy, int lsh, int vy, int vlsh) {
-  const int bid = blockIdx.x;
-  if (bid >= qk_blocks) {
-    const int vb = bid - qk_blocks;
+latent_front_kernel(FrontArgs a, int v_blocks, int uy, int lsh, int vy, int vlsh) {
+  const int vb = blockIdx.x, bid = vb - v_blocks;
+  if (bid < 0) {
     v_part<T, VH, true>(a, vb / vy, vb % vy, vlsh);
     return;
   }
@@ -278,27 +296,36 @@ latent_front_kernel(FrontArgs a, int qk_blocks, int uy, int lsh, int vy, int vls
 #pragma unroll
   for (int e = 0; e < 8; ++e) w[e] = 1.f;
   if (!is_q && a.kx != nullptr && ch < rank) ld8(static_cast<const T*>(a.k_norm) + ch, w);
-  if (a.n_freq > 0)
+  if (a.n_freq > 0 && cr >= 0)   // (the lanes that copy would load twice what they copy)
 #pragma unroll
     for (int r = 0; r < ROWS; ++r)
-      tab[r] = load_table(a.cos_sin + static_cast<int64_t>(min(t0 + r, a.T - 1)) * 2 * a.n_freq, max(cr, 0), a.n_freq,
-                          a.half);
+      tab[r] = load_table(a.cos_sin + static_cast<int64_t>(min(t0 + r, a.T - 1)) * 2 * a.n_freq, cr, a.n_freq, a.half);
   int slot[ROWS];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) slot[r] = a.slots[min(t0 + r, a.T - 1)];
   const int lane0 = ((tid & 63) & ~(L - 1)) + rc;
+  if (__any(on && !is_q)) {   // (most waves hold queries only)
+    float ss[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      ss[r] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss[r] += x[r][e] * x[r][e];
+      ss[r] = on && ch < rank ? ss[r] : 0.f;
+    }
+    lane_group_sums(ss, L);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const float inv = 1.0f / sqrtf(ss[r] / static_cast<float>(rank) + a.eps);
+      if (!is_q && cr < 0)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[r][e] = x[r][e] * inv * w[e];
+    }
+  }
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
     const int t = t0 + r;
     if (t >= a.T) break;
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += x[r][e] * x[r][e];
-    ss = lane_group_sum(on && ch < rank ? ss : 0.f, L);
-    const float inv = 1.0f / sqrtf(ss / static_cast<float>(rank) + a.eps);
-    if (!is_q && cr < 0)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[r][e] = x[r][e] * inv * w[e];
     if (a.n_freq > 0) rotate(x[r], tab[r], lane0, cr, a.n_freq, a.half);
     if (!on || (!is_q && slot[r] < 0)) continue;
     T* dst = is_q ? static_cast<T*>(a.q_out) + (static_cast<int64_t>(t) * a.H + item) * kd
@@ -357,7 +384,7 @@ bool launch_head_front(const FrontArgs& args, bool whole, int dtype, hipStream_t
   if (wide) a.row_inv = nullptr;
 #define MIXK_FRONT(R, V, W)                                                                                      \
   MIXK_DISPATCH(dtype, hipLaunchKernelGGL((hf::head_front_kernel<T, R, V, W>), dim3(static_cast<unsigned>(grid)), \
-                                          dim3(threads), 0, st, a, static_cast<int>(qk), uy, lsh, vy, vlsh))
+                                          dim3(threads), 0, st, a, static_cast<int>(grid - qk), uy, lsh, vy, vlsh))
   if (wide) {
     if (rows == hf::kManyRows) MIXK_FRONT(hf::kManyRows, 8, true);
     else if (vh == 8) MIXK_FRONT(1, 8, true);
@@ -386,7 +413,7 @@ bool launch_latent_front(const FrontArgs& a, int dtype, hipStream_t st) {
   if (grid > 0x7fffffff) return false;
 #define MIXK_FRONT(R, V)                                                                                        \
   MIXK_DISPATCH(dtype, hipLaunchKernelGGL((hf::latent_front_kernel<T, R, V>), dim3(static_cast<unsigned>(grid)), \
-                                          dim3(256), 0, st, a, static_cast<int>(qk), uy, lsh, vy, vlsh))
+                                          dim3(256), 0, st, a, static_cast<int>(grid - qk), uy, lsh, vy, vlsh))
   if (rows == hf::kManyRows) MIXK_FRONT(hf::kManyRows, 8);
   else if (vh == 8) MIXK_FRONT(1, 8);
   else MIXK_FRONT(1, 1);
