@@ -77,7 +77,7 @@ def _native():
 ATTN_TILE_TOKENS = 64     # query tokens per prefill attention tile (the block manager tiles by it)
 DECODE_PART_TOKENS = 128  # keys per decode-attention partition
 SIGMOID_PART_TOKENS = 64  # ... of the sigmoid attention
-SIGMOID_MAX_SPLIT = int(os.environ.get("ATTA_MIX_SIGMOID_SPLIT", "4"))  # key shares of a tile
+SIGMOID_MAX_SPLIT = int(os.environ.get("ATTA_MIX_SIGMOID_SPLIT", "6"))  # key shares of a tile
 ATTENTION_MFMA = os.environ.get("ATTA_MIX_ATTENTION_MFMA", "1") != "0"
 ACT_SILU, ACT_SIGMOID, ACT_GELU_TANH = 0, 1, 2
 _SCORE_CODES = {"sigmoid": 0, "softmax": 1, "logit": 2}
@@ -307,10 +307,17 @@ def sigmoid_attention(q, k_cache, v_cache, block_tables, seq_kvlen, seq_qstart, 
         parts = max(1, -(-int(max_decode_kv) // SIGMOID_PART_TOKENS))
         part = torch.empty(num_decode, q.shape[1], parts, v_cache.shape[2], dtype=torch.float32,
                            device=q.device)
-    # few query tiles: the key range is cut over `split` workgroups per tile so the launch fills the
-    # chip; the fp32 partial rows are added by a second kernel
+    # Few query tiles: the key range is cut over `split` workgroups per tile so the launch fills the
+    # chip once (by registers and LDS a CU holds one workgroup, of up to 16 heads two, of up to 8
+    # three); the fp32 partial rows are added by a second kernel.  Half a round more than that does
+    # not pay, except for a nearly full chip where the longest rows are half of the work: hence the
+    # rounding.  us by shares, 1 / 2 / 3 / 4 / 6: 24 heads, 44 workgroups 106 / 69 / 57 / 51 / 45,
+    # 84 110 / 71 / 61 / 67 / 74, 124 110 / 76 / 87 / 87 / 106, 244 111 / 131 / 141 / 151; 32 heads,
+    # 88 253 / 149 / 115 / 126 / 128, 188 (one prompt) 516 / 295 / 356 / 321, 240 187 / 207; 8 heads,
+    # 40 61 / 40 / 31 / 28 / 25, 216 94 / 79 / 73 / 76, 416 138 / 115.
     split_out, tiles = None, 4 * tile_seq.shape[0]
-    split = min(SIGMOID_MAX_SPLIT, 512 // tiles) if tiles else 1
+    room = 256 * (3 if q.shape[1] <= 8 else 2 if q.shape[1] <= 16 else 1)
+    split = max(1, min(SIGMOID_MAX_SPLIT, int(room / tiles + 0.64))) if tiles else 1
     if split > 1 and q.dtype == torch.bfloat16 and ATTENTION_MFMA:
         split_out = torch.empty(split, q.shape[0], q.shape[1], v_cache.shape[2],
                                 dtype=torch.float32, device=q.device)
