@@ -2020,3 +2020,34 @@ def test_short_conv_rows_of_full_chip(dt, taps):
     # up to 8 products in fp32, then one rounding to the storage type
     eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
     assert torch.allclose(got.cpu().float(), want.float(), rtol=2 * eps, atol=2 * eps)
+
+
+@pytest.mark.parametrize("lens", [[45, 64, 30], [33, 31, 48]])
+@pytest.mark.parametrize("d", [72, 128])
+@pytest.mark.parametrize("bad", [None, float("nan"), float("inf")])
+def test_scores_of_bf16_rows(lens, d, bad):
+    """Scores straight from the rows (keys of 72 - 128 channels in bf16): chunks that are full and not; a non-finite entry
+    in the last token of a chunk that is not full, whose rows stand in for the missing ones, stays where the reference
+    has it."""
+    torch.manual_seed(d)
+    H, G, dv, T = 4, 2, 64, sum(lens)
+    md = ragged(lens, [0, 7, 0], [1, 0, 2], width=32)
+    g = cuda(md)
+    at, at_g = (tuple(m[k] for k in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    dt, z, one = torch.bfloat16, torch.zeros(H), torch.randn(T, H).to(torch.bfloat16)
+    beta, hit = torch.randn(T, H).to(dt), lens[0] - 1
+    for name, widths in (("gated_delta_rule", (G * d, G * d, H * dv)), ("state_space_scan", (H * dv, G * d, G * d))):
+        for which in range(3):
+            x = [torch.randn(T, w).to(dt) for w in widths]
+            if bad is not None:
+                x[which][hit, 3] = bad
+            args = (torch.cat(x, 1), beta, one, z, z) if name == "gated_delta_rule" else (*x, one, z, z, z)
+            st = torch.randn(3, H, d, dv)
+            st_g = st.clone().cuda()
+            got = getattr(mx, name)(*(a.cuda() for a in args), st_g, *at_g, H, G, d, dv)
+            want = getattr(mref, name)(*args, st, *at, H, G, d, dv)
+            for a, b in ((got.cpu(), want), (st_g.cpu(), st)):
+                assert torch.equal(torch.isfinite(a), torch.isfinite(b)), (name, which)
+                a, b = a[torch.isfinite(b)], b[torch.isfinite(b)]
+                # as chunk_compare
+                assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()), (name, which)
