@@ -38,6 +38,7 @@ struct ChunkArgs {
   float kscale;
   int64_t T;              // rows in all
   int walk_heads;         // heads per workgroup of the walk (walk_shape)
+  int walk_portions;      // portions of the walk's grid: at most so many of the S have min_rows rows
 };
 
 // Chunk c of sequence s has the slot seq_qstart[s] / 16 + s + c: disjoint runs, known on the device only.
@@ -57,10 +58,14 @@ constexpr int scan_record_floats(int mode) {
 // A workgroup of the walk: eight waves of 16 columns of S beside four that prepare the operands, once for 128 columns or
 // for two heads of 64 whose keys are the same: the operands' vector work is half of the walk's at 64 columns.  Where such
 // workgroups do not fill the chip, not even with segments of 10 chunks, four waves and 64 columns; so the delta rule,
-// whose portions are not cut, with eight waves for its operands.
+// whose portions are not cut, with eight waves for its operands.  Many portions count from 6 chunks per CU on: few rows in
+// many portions are decode rows and one prompt, which is done sooner in more workgroups (state space, 32 heads, us with
+// four / eight waves: 63 rows + 128 64 / 69, 127 + 256 123 / 132, 31 + 300 74 / 80, but 64 x 12 132 / 93, 127 + 600
+// 192 / 170 and, on the wrong side of the line, 20 + 8 x 40 50 / 40).
 inline bool walk_wide(int64_t T, int64_t S, int64_t H, int64_t dv, int mode) {
   const int64_t units = H * ((dv + kWalkCols - 1) / kWalkCols);
-  return mode < kModeDelta && (S * units >= 512 || T / kScanChunk * units >= 5120);
+  const int64_t chunks = T / kScanChunk * units;
+  return mode < kModeDelta && ((S * units >= 512 && chunks >= 1536) || chunks >= 5120);
 }
 struct WalkShape {
   int waves, heads, cols;   // waves with products; heads per workgroup; columns per workgroup and head
@@ -102,11 +107,10 @@ inline int64_t scan_scratch_floats(int64_t T, int64_t S, int64_t H, int64_t dk, 
 // Which kernels take a batch.  The host knows its T rows and S portions; if every portion has a row, the longest has at
 // most T - S + 1.  All at 32 heads of 128, bf16, us; "R + N" R decode rows beside a portion of N, "S x N" S portions.
 // - Rows (step_scan.h) cost the state's traffic and then 1 us per token of the longest portion, 2 us with a delta rule.
-// - Chunks cost 15 us (28 with per-channel decays) besides the state's traffic, then 2 us per 16 tokens, and 0.2 - 0.3 us
-//   per decode row for the empty workgroups of the walk and rows that share the scores' launch: they pay from 7 - 28 rows
-//   on, a sixth of a row later per portion.  Rows / chunks: delta rule 15 + 8 27 / 27, 15 + 32 75 / 29, 63 + 32 106 / 65;
-//   per channel 15 + 16 42 / 40, 63 + 32 105 / 79; forget gate 15 + 24 37 / 41, 15 + 32 45 / 41; state space 7 + 16
-//   26 / 16; retention 15 + 16 28 / 25, 127 + 256 437 / 175.
+// - Chunks cost 15 us (25 with per-channel decays) besides the state's traffic, then 1.7 us per 16 tokens: they pay from
+//   7 - 28 rows on, a sixth of a row later per portion (decode rows share the scores' launch).  Rows / chunks: delta rule
+//   15 + 8 25 / 27, 15 + 32 75 / 26, 63 + 32 106 / 60; per channel 15 + 16 42 / 33, 63 + 32 105 / 68; forget gate
+//   15 + 24 33 / 37, 15 + 32 45 / 31; state space 7 + 16 26 / 14; retention 15 + 16 28 / 22, 127 + 256 437 / 129.
 // - Tokens (delta_rule.hip, linear_scan.hip) load a round of tokens ahead, 0.3 - 0.7 us per token, but with slower state
 //   accesses: for short portions whose workgroups find room at once.  Rows / chunks / tokens: forget gate 1 x 33
 //   36 / 33 / 21, 4 x 16 22 / 30 / 20; per channel 1 x 12 27 / 28 / 18, 2 x 16 35 / 28 / 20; state space 1 x 9

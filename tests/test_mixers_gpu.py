@@ -2051,3 +2051,34 @@ def test_scores_of_bf16_rows(lens, d, bad):
                 a, b = a[torch.isfinite(b)], b[torch.isfinite(b)]
                 # as chunk_compare
                 assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()), (name, which)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,lens", [(16, [1] * 70 + [64] + [3] * 60 + [33, 1]), (3, [1] * 70 + [700] + [2] * 64 + [30]),
+                                    (2, [5] * 63 + [28, 0, 1, 45] + [1] * 70)])
+def test_scans_of_few_portions_among_rows(dt, H, lens):
+    """More portions than could have rows for chunks: those that do are searched for, 64 at a time, also where long ones
+    are cut; slots of nobody among both."""
+    torch.manual_seed(H)
+    d, dv, S, T = 64, 64, len(lens), sum(lens)
+    assert T // 7 < S or max(lens) == 700
+    slots = [-1 if i in (3, 66, S - 1) else i for i in range(S)]
+    md = ragged(lens, [4 * (i % 2) for i in range(S)], slots, width=64)
+    live = torch.tensor([s >= 0 for n, s in zip(lens, slots) for _ in range(n)])
+    g = cuda(md)
+    at, at_g = (tuple(m[k] for k in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    q, f, k, v = (torch.randn(T, H * d).to(dt) for _ in range(4))
+    dts, z, skip, bias = torch.randn(T, H).to(dt), torch.zeros(H), torch.randn(H), torch.randn(H * d)
+    lower, tab, pw = 0.9 * torch.rand(H * d), torch.zeros(T, 0), mx.retention_powers([0.9] * H, "cpu")
+    for name, args, last in (("forget_gate_scan", (q, f, v, bias, lower), (H, d, dv)),
+                             ("state_space_scan", (v, k, q, dts, z, z, skip), (H, H, d, dv)),
+                             ("gated_delta_rule", (torch.cat([q, k, v], 1), dts, dts, z, z), (H, H, d, dv)),
+                             ("gated_delta_rule", (torch.cat([q, k, v], 1), dts, f, z, bias), (H, H, d, dv)),
+                             ("retention", (q, k, v, pw, tab), (H, d, dv))):
+        st = torch.randn(S, H, d, dv)
+        st_g = st.clone().cuda()
+        got = getattr(mx, name)(*(a.cuda() for a in args), st_g, *at_g, *last)
+        if name == "retention":
+            args = (q, k, v, pw[:, 1], tab)
+        want = getattr(mref, name)(*args, st, *at, *last)
+        chunk_compare(got, want, st_g, st, live)
