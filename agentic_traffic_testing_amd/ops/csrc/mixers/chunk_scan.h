@@ -53,11 +53,13 @@ constexpr int scan_record_floats(int mode) {
 }
 // A long portion in few heads leaves most of the chip idle: with one number or one per channel as the decay it is cut
 // into segments that run side by side, in two passes (chunk_scan.hip).  `chunks`: a segment's length with which the
-// batch makes about 256 workgroups (one per CU: the registers allow no second one), at least 10 and a 16th of the batch
-// (a segment's start is put together from all segments before it).
+// batch makes about 256 workgroups (one per CU: the registers allow no second one), at least 7 and a 16th of the batch
+// (a segment's start is put together from all segments before it; us with at least 10 / 7, 8 heads: 350 rows forget gate
+// 55 / 46, state space 42 / 35, retention 49 / 40, 600 rows 53 / 48, 40 / 36, 46 / 41).  Up to 19 chunks no cut pays
+// (find_segment).
 // A workgroup of the walk: eight waves of 16 columns of S beside four that prepare the operands, once for 128 columns or
 // for two heads of 64 whose keys are the same: the operands' vector work is half of the walk's at 64 columns.  Where such
-// workgroups do not fill the chip, not even with segments of 10 chunks, four waves and 64 columns; so the delta rule,
+// workgroups do not fill the chip, not even with segments of 10 chunks each, four waves and 64 columns; so the delta rule,
 // whose portions are not cut, with eight waves for its operands.  Many portions count from 6 chunks per CU on: few rows in
 // many portions are decode rows and one prompt, which is done sooner in more workgroups (state space, 32 heads, us with
 // four / eight waves: 63 rows + 128 64 / 69, 127 + 256 123 / 132, 31 + 300 74 / 80, but 64 x 12 132 / 93, 127 + 600
@@ -90,11 +92,11 @@ inline ScanSegments scan_segments(int64_t T, int64_t S, int64_t H, int64_t dv, i
   const int64_t n = T / kScanChunk, cols = (dv + kWalkCols - 1) / kWalkCols;
   const int64_t all = walk_wide(T, S, H, dv, mode) ? 512 : 256;
   int64_t chunks = (n * H * cols + all - 1) / all;
-  if (chunks < 10) chunks = 10;
+  if (chunks < 7) chunks = 7;
   if (chunks < (n + 15) / 16) chunks = (n + 15) / 16;
   // cut portions have n >= 1.75 `chunks` and at most n / chunks + 1 / 4 segments; their chunks are the rows' 16ths,
   // each rounded up once: at most 8 / 7 x 18 / 17 x (T / 16 + 1) / chunks in all
-  if (mode >= kModeDelta || 4 * (n + 1) < 7 * chunks) return {0, 0};
+  if (mode >= kModeDelta || n + 1 < 20 || 4 * (n + 1) < 7 * chunks) return {0, 0};
   return {chunks, 5 * (n + 1) / (4 * chunks) + 2};
 }
 constexpr int64_t scan_segment_floats(int64_t H, int64_t dk, int64_t dv) { return H * (dk * dv + 128); }
