@@ -1974,7 +1974,7 @@ def test_segments_in_a_graph():
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("H,G,d,dv", [(16, 8, 128, 64), (16, 4, 64, 40), (15, 5, 128, 64), (8, 8, 128, 128),
                                       (8, 4, 100, 70), (6, 6, 64, 129)])
-def test_scans_of_many_portions(dt, H, G, d, dv):
+def test_scans_of_full_chip(dt, H, G, d, dv):
     """Batches that fill the chip (walk_wide): 128 columns per workgroup, or two heads of 64 with the same keys, portions
     of odd and even numbers of chunks, full and not, fresh and continued."""
     torch.manual_seed(H + d + dv)
