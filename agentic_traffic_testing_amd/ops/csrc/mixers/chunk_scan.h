@@ -44,9 +44,9 @@ struct ChunkArgs {
 // Chunk c of sequence s has the slot seq_qstart[s] / 16 + s + c: disjoint runs, known on the device only.
 inline int64_t scan_chunk_slots(int64_t T, int64_t S) { return T / kScanChunk + S; }
 // record: A [16][16], then the 16-entry scales of q, of k against the state and of k into the state, the
-// decay over the chunk (x 16), then with a delta rule T [16][16], and with one per channel the decays [16][64 or 128] of the
+// decay over the chunk (x 16, but for the mark of keys without bf16 parts), then with a delta rule T [16][16], and with one per channel the decays [16][64 or 128] of the
 // chunk, 1 for a token or channel that is not there
-constexpr int kRecQ = 256, kRecK = 272, kRecKt = 288, kRecEnd = 304, kRecT = 320, kRecDecay = 576;
+constexpr int kRecQ = 256, kRecK = 272, kRecKt = 288, kRecEnd = 304, kRecNoParts = 305, kRecT = 320, kRecDecay = 576;
 constexpr bool scan_keeps_decays(int mode) { return mode == kModeForget || mode == kModeDeltaChannel; }
 constexpr int scan_record_floats(int mode) {
   return scan_keeps_decays(mode) ? 576 + kScanChunk * 128 : mode >= kModeDelta ? 576 : 320;

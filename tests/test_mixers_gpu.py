@@ -2082,3 +2082,52 @@ def test_scans_of_few_portions_among_rows(dt, H, lens):
             args = (q, k, v, pw[:, 1], tab)
         want = getattr(mref, name)(*args, st, *at, *last)
         chunk_compare(got, want, st_g, st, live)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("lens", [[45, 64, 30], [700, 20]])
+@pytest.mark.parametrize("G,d,dv", [(2, 128, 64), (1, 64, 72), (2, 100, 20)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38])
+def test_scans_with_values_without_parts(dt, lens, G, d, dv, value):
+    """An infinity, NaN or a number above those of bf16 in one entry of q, k, v or the state: what is infinite, NaN and
+    finite in the state and in the outputs from the next chunk on is what the reference has, infinities' signs included.
+    Decays that do not reach 0 over a segment (700 rows: 0 x infinity where the segments are put together)."""
+    H, T, hit = 2, sum(lens), 26                # token 26 of the first portion: the second chunk's, outputs from 32 on
+    md = ragged(lens, [3] * len(lens), list(range(len(lens)))[::-1], width=64)
+    g = cuda(md)
+    at, at_g = (tuple(m[key] for key in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    z, tab, pw = torch.zeros(H), torch.zeros(T, 0), mx.retention_powers([0.97, 0.9], "cpu")
+    later = torch.tensor([i >= 32 for i in range(T)])
+    for name in ("forget_gate_scan", "state_space_scan", "retention", "gated_delta_rule"):
+        for which in ("q", "k", "v", "state"):
+            if value == 3.4e38 and which != "state":   # (results around the largest number: by the order of a sum)
+                continue
+            torch.manual_seed(d + dv)
+            groups = G if name in ("state_space_scan", "gated_delta_rule") else H
+            x = {"q": torch.randn(T, groups * d).to(dt), "k": torch.randn(T, groups * d).to(dt),
+                 "v": torch.randn(T, H * dv).to(dt)}
+            one, st = torch.randn(T, H).to(dt), torch.randn(len(lens), H, d, dv)
+            if which == "state":
+                st[len(lens) - 1, 0, 3, 5] = value
+            else:
+                x[which][hit, 3] = value
+            args, last = {
+                "forget_gate_scan": ((x["q"], x["k"], x["v"], torch.randn(H * d), 0.97 + 0.03 * torch.rand(H * d)),
+                                     (H, d, dv)),
+                "state_space_scan": ((x["v"], x["k"], x["q"], one, z, z - 4, z), (H, groups, d, dv)),
+                "retention": ((x["q"], x["k"], x["v"], pw, tab), (H, d, dv)),
+                "gated_delta_rule": ((torch.cat([x["q"], x["k"], x["v"]], 1), one, one, z, z), (H, groups, d, dv)),
+            }[name]
+            st_g = st.clone().cuda()
+            got = getattr(mx, name)(*(a.cuda() for a in args), st_g, *at_g, *last)
+            if name == "retention":
+                args = (*args[:3], pw[:, 1], tab)
+            want = getattr(mref, name)(*args, st, *at, *last)
+            for a, b in ((got.cpu()[later].flatten(), want[later].flatten()), (st_g.cpu().flatten(), st.flatten())):
+                kinds = [(torch.isnan(y), y == float("inf"), y == float("-inf")) for y in (a, b)]
+                assert all(torch.equal(p, q) for p, q in zip(*kinds)), (name, which)
+                fin = torch.isfinite(b)
+                a, b = a[fin].double(), b[fin].double()
+                # as chunk_compare; of what the state began with the reference rounds the product with a decay per token
+                bound = max(1e-5, max(lens) * 2.0 ** -24)
+                assert float((a - b).abs().max()) <= bound * float(b.abs().max()), (name, which)
