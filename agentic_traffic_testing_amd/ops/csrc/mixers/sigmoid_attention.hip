@@ -23,8 +23,8 @@
 //   barrier interval, so a tile costs two barriers (which order LDS only: the V fragments of the
 //   tile are in flight during B, the first K fragments of the next one late in C).  The LDS images
 //   are XOR-swizzled (sg_place) to spread the accesses of every phase over the banks.
-//   A launch with few query tiles is split over the keys: every share writes fp32 partial rows, a
-//   join kernel adds them.
+//   A launch with few query tiles is split over the keys (sg_shares): every share writes fp32 partial
+//   rows, a join kernel adds them.
 // * matrix-core decode kernel (bf16, dim % 8 == 0, dim <= 256, vdim % 16 == 0, H <= 64): one
 //   workgroup per (sequence, 64-key partition), columns = the query heads of a KV head; the mix
 //   runs on the VALU in fp32; the partition's sums go to `part`, a combine kernel adds them.
@@ -65,8 +65,41 @@ struct SigArgs {
   int bt_width, H, G, dim, vdim, block_size, bs_shift, max_parts, rows;
   float scale, cap;
   float* split_out;     // prefill split over the keys: fp32 partial rows [split, T, H, vdim]
-  int split, total_rows;
+  int split, total_rows;   // split: most shares
+  int room;                // query tiles that take as long together as one alone
 };
+
+// Key shares of a launch's query tiles.  The host knows how many tiles there are and not how many keys they have; where
+// the shares do not all run at once, the better number is a question of these: at 24 heads a second share takes 3300 rows
+// of one prompt from 461 to 260 us, and 50 prompts of 64 rows, whose partial rows are written and read for nothing, from 26
+// to 57.  Of up to `split` shares the kernels take the cheapest by the time of the longest piece or of all pieces, half of
+// it more for uneven ones, and what a partial row costs, about that of 18 keys.  The workgroups of the others end at once.
+__device__ __forceinline__ int sg_shares(const SigArgs& a, int num_tiles) {
+  if (a.split == 1 || num_tiles * (kSgTile / kSgTok) * a.split <= 256 + 12) return a.split;   // (all at once)
+  const int lane = threadIdx.x & 63;
+  int work = 0, most = 0, rows = 0;   // keys / 32 of all workgroups, of one; every wave adds up the list, 64 entries at a time
+  for (int i = lane; i < num_tiles; i += kWave) {
+    const int s = a.tile_seq[i], qo = a.tile_qoff[i], n = a.seq_qstart[s + 1] - a.seq_qstart[s];
+    const int here = max(0, min(kSgTile, n - qo)), keys = max(0, a.seq_kvlen[s] - n + qo) / kSgKeys + 1;
+    work += (here + kSgTok - 1) / kSgTok * keys;
+    most = max(most, keys + 1);
+    rows += here;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    work += __shfl_xor(work, o, kWave);
+    most = max(most, __shfl_xor(most, o, kWave));
+    rows += __shfl_xor(rows, o, kWave);
+  }
+  int best = 1;
+  float least = INFINITY;
+  for (int s = 1; s <= a.split; ++s) {
+    const float time = fmaxf(static_cast<float>(most) * a.room / s, 1.5f * work) + (s > 1 ? 0.55f * s * rows : 0.f);
+    best = time < least ? s : best;
+    least = fminf(least, time);
+  }
+  return best;
+}
 
 // Weight of one key on the fast transcendental units.  With a cap: t = tanh(y) as
 // 1 - 2 / (1 + exp(2 y)); everything in log2 units with the constants folded by the caller:
@@ -158,7 +191,10 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
   const int pos0 = kvlen - n + qo;          // position of the first query token
   const int kend = pos0 + ntok;             // keys [0, kend) are visible to somebody
   // this workgroup's share of the key tiles
-  const int ntiles = (kend + kSgKeys - 1) / kSgKeys, per = (ntiles + a.split - 1) / a.split;
+  const int ntiles = (kend + kSgKeys - 1) / kSgKeys;
+  const int shares = __builtin_amdgcn_readfirstlane(sg_shares(a, gridDim.x / (kSgTile / kSgTok)));
+  if (static_cast<int>(blockIdx.y) >= shares) return;
+  const int per = (ntiles + shares - 1) / shares;
   const int kfirst = static_cast<int>(blockIdx.y) * per * kSgKeys;
   const int kstop = min(kend, kfirst + per * kSgKeys);
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, c = lane >> 4;
@@ -413,7 +449,7 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
   for (int hh = 0; hh < HW; ++hh) {
     const int h = h0 + hh;
     if (h < H) {
-      if (a.split > 1) {
+      if (shares > 1) {
         const int64_t row = static_cast<int64_t>(blockIdx.y) * a.total_rows + row0 + qo + r;
         float* o = a.split_out + (row * H + h) * vdim + 4 * c;
 #pragma unroll
@@ -440,11 +476,13 @@ __global__ void sigmoid_attention_join_kernel(__bf16* __restrict__ out, SigArgs 
   const int s = a.tile_seq[blockIdx.x], qo = a.tile_qoff[blockIdx.x] + blockIdx.y;
   const int row0 = a.seq_qstart[s], n = a.seq_qstart[s + 1] - row0;
   if (qo >= n || a.seq_kvlen[s] <= 0) return;
+  const int shares = sg_shares(a, gridDim.x);
+  if (shares == 1) return;
   const int width = a.H * a.vdim;   // a multiple of 16
   const int64_t base = static_cast<int64_t>(row0 + qo) * width;
   for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int z = 0; z < a.split; ++z) {
+    for (int z = 0; z < shares; ++z) {
       float p[8];
       ld8(a.split_out + static_cast<int64_t>(z) * a.total_rows * width + base + i, p);
 #pragma unroll
@@ -817,7 +855,8 @@ extern "C" int mixk_sigmoid_attention(void* out, const void* q, const void* k_ca
   while ((1 << bs_shift) < block_size) ++bs_shift;
   const SigArgs a{block_tables, seq_kvlen, seq_qstart, tile_seq, tile_qoff, part, bias, talk,
                   bt_width, H, G, dim, vdim, block_size, bs_shift, max_parts, 0, scale, cap,
-                  split_out, split_out != nullptr ? split : 1, total_rows};
+                  split_out, split_out != nullptr ? split : 1, total_rows,
+                  H <= 8 ? 640 : H <= 16 ? 320 : 256};   // (a CU holds 3, 2, 1 workgroups)
   const bool pages_ok = block_size >= 8 && (block_size & (block_size - 1)) == 0;
   const bool base_ok = use_mfma && dtype == 0 && pages_ok && dim % 8 == 0 && vdim % 16 == 0;
   int rc = 0, rows_tiles = num_tiles, rows_decode = num_decode;

@@ -307,17 +307,17 @@ def sigmoid_attention(q, k_cache, v_cache, block_tables, seq_kvlen, seq_qstart, 
         parts = max(1, -(-int(max_decode_kv) // SIGMOID_PART_TOKENS))
         part = torch.empty(num_decode, q.shape[1], parts, v_cache.shape[2], dtype=torch.float32,
                            device=q.device)
-    # Few query tiles: the key range is cut over `split` workgroups per tile so the launch fills the
-    # chip once (by registers and LDS a CU holds one workgroup, of up to 16 heads two, of up to 8
-    # three); the fp32 partial rows are added by a second kernel.  Half a round more than that does
-    # not pay, except for a nearly full chip where the longest rows are half of the work: hence the
-    # rounding.  us by shares, 1 / 2 / 3 / 4 / 6: 24 heads, 44 workgroups 106 / 69 / 57 / 51 / 45,
-    # 84 110 / 71 / 61 / 67 / 74, 124 110 / 76 / 87 / 87 / 106, 244 111 / 131 / 141 / 151; 32 heads,
-    # 88 253 / 149 / 115 / 126 / 128, 188 (one prompt) 516 / 295 / 356 / 321, 240 187 / 207; 8 heads,
-    # 40 61 / 40 / 31 / 28 / 25, 216 94 / 79 / 73 / 76, 416 138 / 115.
+    # Few query tiles: the key range is cut over up to `split` workgroups per tile so the launch fills
+    # the chip once (by registers and LDS a CU holds one workgroup, of up to 16 heads two, of up to 8
+    # three); the fp32 partial rows are added by a second kernel.  The kernels take fewer where the
+    # tiles' lengths, which are on the device, say so (sg_shares), so a nearly full chip has room for
+    # two.  us by shares, 1 / 2 / 3 / 4 / 6: 24 heads, 44 workgroups 105 / 69 / 57 / 50 / 45, 88
+    # 205 / 120 / 92 / 99 / 99, 132 (3 prompts) 110 / 77 / 93 / 93 / 113; one prompt in 188 419 / 238,
+    # 208 461 / 259, 252 556 / 349, 4 prompts in 256 151 / 185, 12 in 240 58 / 86.
     split_out, tiles = None, 4 * tile_seq.shape[0]
     room = 256 * (3 if q.shape[1] <= 8 else 2 if q.shape[1] <= 16 else 1)
-    split = max(1, min(SIGMOID_MAX_SPLIT, int(room / tiles + 0.64))) if tiles else 1
+    split = max(2 if tiles <= room else 1, int(room / tiles + 0.64)) if tiles else 1
+    split = max(1, min(SIGMOID_MAX_SPLIT, split))
     if split > 1 and q.dtype == torch.bfloat16 and ATTENTION_MFMA:
         split_out = torch.empty(split, q.shape[0], q.shape[1], v_cache.shape[2],
                                 dtype=torch.float32, device=q.device)

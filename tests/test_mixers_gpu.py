@@ -2131,3 +2131,29 @@ def test_scans_with_values_without_parts(dt, lens, G, d, dv, value):
                 # as chunk_compare; of what the state began with the reference rounds the product with a decay per token
                 bound = max(1e-5, max(lens) * 2.0 ** -24)
                 assert float((a - b).abs().max()) <= bound * float(b.abs().max()), (name, which)
+
+
+@pytest.mark.parametrize("H,lens,starts,shares", [(18, [3200], [0], 2), (18, [64] * 50, [0] * 50, 1), (18, [300] * 12, [0] * 12, 1),
+                                                  (18, [3100] + [64] * 14, [0] * 15, 2), (18, [64] * 50, [2500] * 50, 1),
+                                                  (10, [3200], [40], 2), (6, [1, 3150, 17], [70, 9, 0], 3)])
+def test_sigmoid_shares_by_lengths(H, lens, starts, shares):
+    """Beside a nearly full chip the device takes the number of key shares by the tiles' keys: a long prompt is cut, short
+    ones are not, whose further shares' rows stay untouched."""
+    torch.manual_seed(H)
+    dim, vdim, S = 32, 16, len(lens)
+    md = ragged(lens, starts, list(range(S)), width=-(-max(a + b for a, b in zip(lens, starts)) // 16))
+    g, T = cuda(md), sum(lens)
+    q = torch.randn(T, H, dim).to(torch.bfloat16).cuda()
+    kc, vc = (x.cuda() for x in ragged_pages(md, 2, dim, vdim, 16, torch.bfloat16))
+    bias, talk = (torch.randn(H) - 6.0).cuda(), (torch.eye(H) + 0.2 * torch.randn(H, H)).to(torch.bfloat16).float().cuda()
+    at = (kc, vc, g["block_tables"], g["seq_kvlen"], g["seq_qstart"])
+    want = mref.sigmoid_attention(q, *at, 0.2, 0.0, bias, talk).float()
+    out, part = torch.empty(T, H, vdim, dtype=torch.bfloat16, device="cuda"), torch.full((3, T, H, vdim), float("nan")).cuda()
+    mx._native().sigmoid_attention(out, q, *at, g["tile_seq"], g["tile_qoff"], 0.2, 0.0, bias, talk, 0, 1, None, True, part)
+    written = [bool(torch.isfinite(p).all()) for p in part]
+    assert written == ([z < shares for z in range(3)] if shares > 1 else [False] * 3)
+    assert shares == 3 or not torch.isfinite(part[shares if shares > 1 else 0:]).any()
+    got = mx.sigmoid_attention(q, *at, g["tile_seq"], g["tile_qoff"], 0.2, 0.0, bias, talk)
+    for x in (out, got):   # as test_sigmoid_attention
+        err = (x.float() - want).abs() / (want.abs() + want.pow(2).mean().sqrt())
+        assert float(err.max()) < 4e-2 and float(err.mean()) < 4e-3
