@@ -2157,3 +2157,38 @@ def test_sigmoid_shares_by_lengths(H, lens, starts, shares):
     for x in (out, got):   # as test_sigmoid_attention
         err = (x.float() - want).abs() / (want.abs() + want.pow(2).mean().sqrt())
         assert float(err.max()) < 4e-2 and float(err.mean()) < 4e-3
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,d,dv,skip,pad", [(2, 64, 64, 1, 1), (2, 64, 65, 0, 0), (3, 128, 33, 0, 0), (2, 128, 128, 0, 1), (4, 72, 1, 0, 0),
+                                             (2, 20, 7, 3, 0)])
+@pytest.mark.parametrize("lens", [[47, 33, 1, 64], [640, 30], [17] * 90])
+def test_scans_of_unaligned_values(dt, H, d, dv, skip, pad, lens):
+    """Aligned rows of q and k beside rows of v that are not (odd widths, strides and starts): values column by column, in
+    portions, segments and batches that fill the chip."""
+    torch.manual_seed(H * d + dv)
+    if len(lens) == 90:
+        H *= 12
+    S, T = len(lens), sum(lens)
+    md = ragged(lens, [3 * (i % 2) for i in range(S)], list(range(S))[::-1], width=64)
+    g = cuda(md)
+    at, at_g = (tuple(m[key] for key in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    q, f, k = (torch.randn(T, H * d).to(dt) for _ in range(3))
+    wide = torch.randn(T, skip + H * dv + pad).to(dt)
+    v, v_g = wide[:, skip:skip + H * dv], wide.cuda()[:, skip:skip + H * dv]
+    dts, z, bias, lower = torch.randn(T, H).to(dt), torch.zeros(H), torch.randn(H * d), 0.9 * torch.rand(H * d)
+    pw, n = mx.retention_powers([0.97] * H, "cpu"), d // 8 * 4
+    tab = torch.randn(T, 2 * n)
+    for name, args, last in (("forget_gate_scan", (q, f, v, bias, lower), (H, d, dv)),
+                             ("state_space_scan", (v, k, q, dts, z, z, z), (H, H, d, dv)),
+                             ("retention", (q, k, v, pw, tab), (H, d, dv))):
+        st = torch.randn(S, H, d, dv)
+        st_g = st.clone().cuda()
+        got = getattr(mx, name)(*(v_g if a is v else a.cuda() for a in args), st_g, *at_g, *last)
+        if name == "retention":
+            args = (q, k, v, pw[:, 1], tab)
+        want = getattr(mref, name)(*args, st, *at, *last)
+        # as chunk_compare; what remains of 640 tokens adds the roundings of as many
+        bound = max(1e-5, max(lens) * 2.0 ** -24)
+        for a, b in ((got.cpu(), want), (st_g.cpu(), st)):
+            assert float((a - b).abs().max()) <= bound * float(b.abs().max()), name
