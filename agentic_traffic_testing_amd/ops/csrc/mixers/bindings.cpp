@@ -365,10 +365,22 @@ void diff_combine(at::Tensor out, const at::Tensor& a, const c10::optional<at::T
 }
 
 // scratch of the chunked recurrences, where the batch takes them
-c10::optional<at::Tensor> scan_records(const at::Tensor& like, int64_t T, int64_t S, int64_t H, int64_t dk,
+c10::optional<at::Tensor> scan_records(const at::Tensor& like, int64_t T, int64_t S, int64_t H, int64_t G, int64_t dk,
                                        int64_t dv, int mode) {
   if (mixk::scan_route(T, S, H, dk, dv, mode) != mixk::kScanChunks) return c10::nullopt;
-  return at::empty({mixk::scan_scratch_floats(T, S, H, dk, dv, mode)}, like.options().dtype(at::kFloat));
+  return at::empty({mixk::scan_scratch_floats(T, S, H, G, dk, dv, mode)}, like.options().dtype(at::kFloat));
+}
+
+// What a batch of a recurrence (ScanMode) runs as: the route (ScanRoute); in chunks the walk's product waves, heads and
+// columns per workgroup, the chunks per segment that it aims at, the scratch's segment states (0: not cut), floats of scratch.
+std::vector<int64_t> scan_plan(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dk, int64_t dv, int64_t mode) {
+  TORCH_CHECK(T >= 0 && S > 0 && H > 0 && G > 0 && dk > 0 && dk <= 256 && dv > 0 && mode >= 0 && mode <= mixk::kModeDeltaChannel,
+              "scan_plan: sizes");
+  const int m = static_cast<int>(mode);
+  const mixk::WalkShape w = mixk::walk_shape(T, S, H, G, dv, m);
+  const mixk::ScanSegments g = mixk::scan_segments(T, S, H, G, dk, dv, m);
+  return {mixk::scan_route(T, S, H, dk, dv, m), w.waves, w.heads, w.cols, g.chunks, g.states,
+          mixk::scan_scratch_floats(T, S, H, G, dk, dv, m)};
 }
 
 // q, k [T, H dk], v [T, H dv] (row-strided), powers fp32 [H, n] (decay^0 ... decay^(n-1)), cos_sin
@@ -394,7 +406,7 @@ void retention(at::Tensor out, at::Tensor state, const at::Tensor& q, const at::
                   cos_sin.size(0) >= T && cos_sin.size(1) % 2 == 0 && cos_sin.size(1) <= dk,
               "retention: shapes");
   const at::DeviceGuard g(v.device());
-  const auto rec = scan_records(v, T, S, H, dk, dv, mixk::kModeRetention);
+  const auto rec = scan_records(v, T, S, H, H, dk, dv, mixk::kModeRetention);
   rc_ok(mixk_retention(out.data_ptr<float>(), state.data_ptr<float>(), q.data_ptr(), q.stride(0),
                        k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                        powers.data_ptr<float>(), powers.size(1), cos_sin.data_ptr<float>(),
@@ -519,7 +531,7 @@ void gated_delta_rule(at::Tensor out, const at::Tensor& qkv, const at::Tensor& b
               "gated_delta_rule: shapes");
   const at::DeviceGuard g(qkv.device());
   const int64_t S = seq_slot.numel();
-  const auto rec = scan_records(qkv, T, S, H, dim, vdim,
+  const auto rec = scan_records(qkv, T, S, H, G, dim, vdim,
                                 per_channel ? mixk::kModeDeltaChannel : mixk::kModeDelta);
   rc_ok(mixk_gated_delta_rule(out.data_ptr<float>(), qkv.data_ptr(), beta.data_ptr(),
                               beta.stride(0), decay.data_ptr(), decay.stride(0), per_channel,
@@ -710,7 +722,8 @@ void gated_linear_scan(at::Tensor out, at::Tensor state, const at::Tensor& q, co
   }
   const at::DeviceGuard g(v.device());
   const int64_t S = seq_slot.numel();
-  const auto rec = scan_records(v, T, S, H, dk, dv, mode == 0 ? mixk::kModeForget : mixk::kModeStateSpace);
+  const auto rec = scan_records(v, T, S, H, mode == 0 ? H : G, dk, dv,
+                                mode == 0 ? mixk::kModeForget : mixk::kModeStateSpace);
   rc_ok(mixk_gated_linear_scan(out.data_ptr<float>(), state.data_ptr<float>(), q.data_ptr(),
                                q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                                dt_ptr, dt_stride, p0.data_ptr<float>(), p1.data_ptr<float>(),
@@ -1011,6 +1024,7 @@ void scale_softcap(at::Tensor out, const at::Tensor& logits, double scale, doubl
 }  // namespace
 
 TORCH_LIBRARY(atta_mix, m) {
+  m.def("scan_plan(int T, int S, int H, int G, int dk, int dv, int mode) -> int[]", &scan_plan);
   m.def("embed_pair(Tensor(a!) out, Tensor table, Tensor pair_table, Tensor ids, Tensor positions, "
         "Tensor seq_qstart, Tensor seq_slot, Tensor(b!) prev_token, int mul_prev, int mul_cur, "
         "int buckets) -> ()");

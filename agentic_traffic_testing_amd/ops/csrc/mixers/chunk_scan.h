@@ -55,25 +55,30 @@ constexpr int scan_record_floats(int mode) {
 // into segments that run side by side, in two passes (chunk_scan.hip).  `chunks`: a segment's length with which the
 // batch makes about 256 workgroups (one per CU: the registers allow no second one), at least 7 and a 16th of the batch
 // (a segment's start is put together from all segments before it; us with at least 10 / 7, 8 heads: 350 rows forget gate
-// 55 / 46, state space 42 / 35, retention 49 / 40, 600 rows 53 / 48, 40 / 36, 46 / 41).  Up to 19 chunks no cut pays
-// (find_segment).
+// 55 / 46, state space 42 / 35, retention 49 / 40, 600 rows 53 / 48, 40 / 36, 46 / 41).  A batch of less than 20 chunks is
+// not cut.
 // A workgroup of the walk: eight waves of 16 columns of S beside four that prepare the operands, once for 128 columns or
-// for two heads of 64 whose keys are the same: the operands' vector work is half of the walk's at 64 columns.  Where such
-// workgroups do not fill the chip, not even with segments of 10 chunks each, four waves and 64 columns; so the delta rule,
-// whose portions are not cut, with eight waves for its operands.  Many portions count from 6 chunks per CU on: few rows in
-// many portions are decode rows and one prompt, which is done sooner in more workgroups (state space, 32 heads, us with
-// four / eight waves: 63 rows + 128 64 / 69, 127 + 256 123 / 132, 31 + 300 74 / 80, but 64 x 12 132 / 93, 127 + 600
-// 192 / 170 and, on the wrong side of the line, 20 + 8 x 40 50 / 40).
-inline bool walk_wide(int64_t T, int64_t S, int64_t H, int64_t dv, int mode) {
-  const int64_t units = H * ((dv + kWalkCols - 1) / kWalkCols);
-  const int64_t chunks = T / kScanChunk * units;
-  return mode < kModeDelta && ((S * units >= 512 && chunks >= 1536) || chunks >= 5120);
-}
+// for two heads of 64 whose keys are the same (the operands' vector work is half of the walk's at 64 columns), or four waves
+// and 64 columns; so the delta rule, whose portions are not cut, with eight waves for its operands.  256 workgroups run at
+// once.  In `units` of a head's 64 columns, S portions make S x units of them:
+// - From 512 on eight waves, if there are 6 chunks per CU: few rows in many portions are decode rows and one prompt, which is
+//   done sooner in more workgroups (state space, 32 heads, us with four / eight waves: 63 rows + 128 64 / 69, 127 + 256
+//   123 / 132, 31 + 300 74 / 80, but 64 x 12 132 / 93, 127 + 600 192 / 170, 8 x 512 127 / 91 and, on the wrong side of the
+//   line, 20 + 8 x 40 50 / 40); from 257 on if there are as many as for long portions.
+// - 192 - 256 fill the chip with four waves, and uncut: a portion in half the workgroups would have to be cut to fill it
+//   (32 heads, four waves uncut / eight cut: retention 4 x 350 55 / 72, 4 x 1000 135 / 159, 4 x 2000 283 / 297, forget gate
+//   4 x 700 126 / 135, state space 4 x 1000 121 / 130, 8 heads 16 x 512 68 / 86).
+// - Fewer: long portions are cut, with eight waves where a 16th of the batch per segment is enough to fill the chip (32
+//   heads, one prompt of 2048, four / eight waves: retention 120 / 98, state space 102 / 84; 8 heads, 4 x 2000: retention
+//   120 / 143, one of 8192 138 / 156).
 struct WalkShape {
   int waves, heads, cols;   // waves with products; heads per workgroup; columns per workgroup and head
 };
+inline int64_t walk_units(int64_t H, int64_t dv) { return H * ((dv + kWalkCols - 1) / kWalkCols); }
 inline WalkShape walk_shape(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dv, int mode) {
-  if (walk_wide(T, S, H, dv, mode)) {
+  const int64_t units = walk_units(H, dv), chunks = T / kScanChunk * units, busy = S * units;
+  const bool wide = busy >= 512 && chunks >= 1536 ? true : chunks >= 5120 && (busy > 256 || (busy < 192 && units >= 32));
+  if (mode < kModeDelta && wide) {
     if (dv > kWalkCols) return {8, 1, 2 * kWalkCols};
     if (mode == kModeStateSpace && H / G % 2 == 0) return {8, 2, kWalkCols};
   }
@@ -88,22 +93,30 @@ __host__ __device__ inline int scan_segment_chunks(int n, int chunks) {
   const int P = (4 * n + chunks) / (4 * chunks);
   return P < 2 ? (n > 0 ? n : 1) : (n + P - 1) / P;
 }
-inline ScanSegments scan_segments(int64_t T, int64_t S, int64_t H, int64_t dv, int mode) {
-  const int64_t n = T / kScanChunk, cols = (dv + kWalkCols - 1) / kWalkCols;
-  const int64_t all = walk_wide(T, S, H, dv, mode) ? 512 : 256;
-  int64_t chunks = (n * H * cols + all - 1) / all;
+inline ScanSegments scan_segments(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dk, int64_t dv, int mode) {
+  const int64_t n = T / kScanChunk, units = walk_units(H, dv);
+  // As many units as run at once, or twice as many for a long prompt in workgroups of 64 columns where these fill the chip
+  // better so (units that do not divide 256: 96 heads of 64, one prompt of 2048, twice / once: retention 196 / 217, forget
+  // gate 240 / 264, state space 157 / 180 us) or fit on a CU twice (the forget gate's with keys of up to 64: 64 heads of
+  // 64, one prompt of 2048 86 / 95, 2 x 1000 84 / 93; retention, that do not, 107 / 95).
+  const int64_t busy = S * units;
+  const bool wide = walk_shape(T, S, H, G, dv, mode).waves == 8;
+  const bool fits = 512 / units * 10 > 256 / units * 24 || (mode == kModeForget && dk <= 64);
+  const int64_t all = wide || (fits && n * units >= 5120 && (busy < 192 || busy > 256)) ? 512 : 256;
+  int64_t chunks = (n * units + all - 1) / all;
   if (chunks < 7) chunks = 7;
   if (chunks < (n + 15) / 16) chunks = (n + 15) / 16;
-  // cut portions have n >= 1.75 `chunks` and at most n / chunks + 1 / 4 segments; their chunks are the rows' 16ths,
-  // each rounded up once: at most 8 / 7 x 18 / 17 x (T / 16 + 1) / chunks in all
+  // (one prompt of 300 rows or less gains nothing: 8 heads, forget gate 51 / 51; find_segment cuts by the lengths)
   if (mode >= kModeDelta || n + 1 < 20 || 4 * (n + 1) < 7 * chunks) return {0, 0};
+  // Cut portions have m >= 1.75 `chunks` of them, so at least 13, and at most m / chunks + 1 / 4 <= 8 / 7 m / chunks
+  // segments; m is the rows' 16ths rounded up, at most 13 / 12.06 of them: 8 / 7 x 13 / 12.06 < 5 / 4.
   return {chunks, 5 * (n + 1) / (4 * chunks) + 2};
 }
 constexpr int64_t scan_segment_floats(int64_t H, int64_t dk, int64_t dv) { return H * (dk * dv + 128); }
 // floats of scratch: the records, then the segments
-inline int64_t scan_scratch_floats(int64_t T, int64_t S, int64_t H, int64_t dk, int64_t dv, int mode) {
+inline int64_t scan_scratch_floats(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dk, int64_t dv, int mode) {
   return scan_chunk_slots(T, S) * H * scan_record_floats(mode) +
-         scan_segments(T, S, H, dv, mode).states * scan_segment_floats(H, dk, dv);
+         scan_segments(T, S, H, G, dk, dv, mode).states * scan_segment_floats(H, dk, dv);
 }
 
 // Which kernels take a batch.  The host knows its T rows and S portions; if every portion has a row, the longest has at
@@ -155,7 +168,7 @@ inline int launch_scan_batch(ChunkArgs a, int mode, int64_t T, int dtype, hipStr
   a.T = T;
   a.n_slots = static_cast<int>(scan_chunk_slots(T, a.S));
   a.min_rows = kScanMinRows[mode];
-  const ScanSegments g = scan_segments(T, a.S, a.H, a.dv, mode);
+  const ScanSegments g = scan_segments(T, a.S, a.H, a.G, a.dk, a.dv, mode);
   a.seg = a.rec + static_cast<int64_t>(a.n_slots) * a.H * scan_record_floats(mode);
   a.seg_chunks = static_cast<int>(g.chunks);
   a.seg_states = static_cast<int>(g.states);
