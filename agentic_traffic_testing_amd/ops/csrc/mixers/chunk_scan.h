@@ -44,12 +44,15 @@ struct ChunkArgs {
 // Chunk c of sequence s has the slot seq_qstart[s] / 16 + s + c: disjoint runs, known on the device only.
 inline int64_t scan_chunk_slots(int64_t T, int64_t S) { return T / kScanChunk + S; }
 // record: A [16][16], then the 16-entry scales of q, of k against the state and of k into the state, the
-// decay over the chunk (x 16, but for the mark of keys without bf16 parts), then with a delta rule T [16][16], and with one per channel the decays [16][64 or 128] of the
-// chunk, 1 for a token or channel that is not there
-constexpr int kRecQ = 256, kRecK = 272, kRecKt = 288, kRecEnd = 304, kRecNoParts = 305, kRecT = 320, kRecDecay = 576;
+// decay over the chunk (x 16, but for the mark of keys without bf16 parts), then with a delta rule T [16][16], then with a
+// decay per channel the decays [16][64 or 128] of the chunk, 1 for a token or channel that is not there: 5.4 or 9.5 KB per
+// chunk and head (8192 tokens, 32 heads of 128: forget gate 155 MB, per-channel delta rule 172, the others 21 and 38)
+constexpr int kRecQ = 256, kRecK = 272, kRecKt = 288, kRecEnd = 304, kRecNoParts = 305, kRecT = 320;
+constexpr int scan_rec_decay(int mode) { return mode >= kModeDelta ? 576 : 320; }
+constexpr int scan_decay_width(int dk) { return dk <= 64 ? 64 : 128; }
 constexpr bool scan_keeps_decays(int mode) { return mode == kModeForget || mode == kModeDeltaChannel; }
-constexpr int scan_record_floats(int mode) {
-  return scan_keeps_decays(mode) ? 576 + kScanChunk * 128 : mode >= kModeDelta ? 576 : 320;
+constexpr int scan_record_floats(int mode, int dk) {
+  return scan_rec_decay(mode) + (scan_keeps_decays(mode) ? kScanChunk * scan_decay_width(dk) : 0);
 }
 // A long portion in few heads leaves most of the chip idle: with one number or one per channel as the decay it is cut
 // into segments that run side by side, in two passes (chunk_scan.hip).  `chunks`: a segment's length with which the
@@ -115,7 +118,7 @@ inline ScanSegments scan_segments(int64_t T, int64_t S, int64_t H, int64_t G, in
 constexpr int64_t scan_segment_floats(int64_t H, int64_t dk, int64_t dv) { return H * (dk * dv + 128); }
 // floats of scratch: the records, then the segments
 inline int64_t scan_scratch_floats(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dk, int64_t dv, int mode) {
-  return scan_chunk_slots(T, S) * H * scan_record_floats(mode) +
+  return scan_chunk_slots(T, S) * H * scan_record_floats(mode, static_cast<int>(dk)) +
          scan_segments(T, S, H, G, dk, dv, mode).states * scan_segment_floats(H, dk, dv);
 }
 
@@ -169,7 +172,7 @@ inline int launch_scan_batch(ChunkArgs a, int mode, int64_t T, int dtype, hipStr
   a.n_slots = static_cast<int>(scan_chunk_slots(T, a.S));
   a.min_rows = kScanMinRows[mode];
   const ScanSegments g = scan_segments(T, a.S, a.H, a.G, a.dk, a.dv, mode);
-  a.seg = a.rec + static_cast<int64_t>(a.n_slots) * a.H * scan_record_floats(mode);
+  a.seg = a.rec + static_cast<int64_t>(a.n_slots) * a.H * scan_record_floats(mode, a.dk);
   a.seg_chunks = static_cast<int>(g.chunks);
   a.seg_states = static_cast<int>(g.states);
   return launch_chunk_scan(a, mode, dtype, st);

@@ -2192,3 +2192,25 @@ def test_scans_of_unaligned_values(dt, H, d, dv, skip, pad, lens):
         bound = max(1e-5, max(lens) * 2.0 ** -24)
         for a, b in ((got.cpu(), want), (st_g.cpu(), st)):
             assert float((a - b).abs().max()) <= bound * float(b.abs().max()), name
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("d,dv", [(13, 33), (30, 64), (61, 40), (67, 20)])
+@pytest.mark.parametrize("lens", [[47, 33, 1, 64], [500, 30]])
+def test_kept_decays_of_unaligned_keys(dt, d, dv, lens):
+    """Keys that are loaded element by element, narrower and wider than the decays' 64 columns in a chunk's record."""
+    torch.manual_seed(d)
+    H, S, T = 3, len(lens), sum(lens)
+    md = ragged(lens, [3 * (i % 2) for i in range(S)], list(range(S))[::-1], width=64)
+    g = cuda(md)
+    at, at_g = (tuple(m[key] for key in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    q, f, k = (torch.randn(T, H * d).to(dt) for _ in range(3))
+    v, beta, z = torch.randn(T, H * dv).to(dt), torch.randn(T, H).to(dt), torch.zeros(H)
+    bias, lower = torch.randn(H * d), 0.9 * torch.rand(H * d)
+    for name, args, last in (("forget_gate_scan", (q, f, v, bias, lower), (H, d, dv)),
+                             ("gated_delta_rule", (torch.cat([q, k, v], 1), beta, f, z, bias), (H, H, d, dv))):
+        st = torch.randn(S, H, d, dv)
+        st_g = st.clone().cuda()
+        got = getattr(mx, name)(*(a.cuda() for a in args), st_g, *at_g, *last)
+        want = getattr(mref, name)(*args, st, *at, *last)
+        chunk_compare(got, want, st_g, st, torch.ones(T, dtype=torch.bool))

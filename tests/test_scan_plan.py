@@ -66,3 +66,13 @@ def test_shapes_of_the_walk(plan, H, G, dv, T, S, shape):
     for mode in (DELTA, DELTA_CHANNEL):
         q = plan(T, S, H, G, 128, dv, mode)
         assert (q["waves"], q["states"]) == (4, 0)
+
+
+@pytest.mark.parametrize("mode,dk,floats", [(RETENTION, 64, 320), (STATE_SPACE, 128, 320), (DELTA, 64, 576), (FORGET, 13, 320 + 16 * 64),
+                                            (FORGET, 64, 320 + 16 * 64), (FORGET, 72, 320 + 16 * 128),
+                                            (DELTA_CHANNEL, 64, 576 + 16 * 64), (DELTA_CHANNEL, 128, 576 + 16 * 128)])
+def test_scratch_per_chunk(plan, mode, dk, floats):
+    """A chunk's record holds the decays that the recurrence keeps, at the width of its keys, and nothing for others."""
+    H, dv, T, S = 4, 64, 800, 3
+    p = plan(T, S, H, H, dk, dv, mode)
+    assert p["floats"] == (T // 16 + S) * H * floats + p["states"] * H * (dk * dv + 128)
