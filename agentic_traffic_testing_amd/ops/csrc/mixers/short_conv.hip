@@ -76,10 +76,10 @@ __global__ void short_conv_silu_kernel(T* __restrict__ out, const T* __restrict_
 // 4 rows (8 where a tail is longer).  16 rows / 4 rows, us, 6144 channels in bf16: 64 rows 9.4 / 7.1, 1024 10.9 / 9.0, 2048
 // 17.2 / 14.0, 4096 (768 workgroups of 16) 23.1 / 24.0, 8000 40.0 / 42.0; 8448 in fp32: 64 13.0 / 7.3, 2048 35.6 / 33.7,
 // 4096 61.6 / 60.8, 6000 92 / 104.
-// In 32 bits, from 512 workgroups on (two per CU) now one and now the other is faster, and 16 rows are kept: 2048 channels,
-// 8192 rows 29.8 / 31.4, 12000 38.9 / 43.4; 4096 channels, 4096 rows 29.7 / 32.7, 16 x 256 35.5 / 32.4.
+// In 32 bits, from 480 workgroups on (two per CU) now one and now the other is faster, and 16 rows are kept: 2048 channels,
+// 4 x 2000 rows 28.1 / 30.9, 8192 29.8 / 31.4, 12000 38.9 / 43.4; 4096 channels, 4096 rows 29.7 / 32.7, 16 x 256 35.5 / 32.4.
 constexpr int kConvRows = 16;
-constexpr int conv_few(size_t item) { return item == 4 ? 512 : 768; }   // workgroups
+constexpr int conv_few(size_t item) { return item == 4 ? 480 : 768; }   // workgroups
 
 template <typename T, int TAPS, int ROWS>
 __global__ void __launch_bounds__(256)

@@ -1843,10 +1843,13 @@ def test_retention_slow_decays(dt, n, S, H):
         assert float((st[0, h].double() - want).norm() / want.norm()) < bound, h
 
 
-def chunks_per_segment(T, H, dv):
-    """The length that the kernels aim at for a batch of T rows (chunk_scan.h, scan_segments)."""
-    n, cols = T // 16, -(-dv // 64)
-    return max(10, -(-n * H * cols // 256), -(-n // 16))
+SCAN_MODES = {"retention": 0, "forget_gate_scan": 1, "state_space_scan": 2}
+
+
+def scan_plan(name, lens, H, G, d, dv):
+    """What the kernels make of a batch (scan_plan): chunks per segment and so on."""
+    p = mx._native().scan_plan(sum(lens), len(lens), H, G, d, dv, SCAN_MODES[name])
+    return dict(zip(("route", "waves", "heads", "cols", "chunks", "states", "floats"), p))
 
 
 def segments_of(n, c):
@@ -1856,20 +1859,20 @@ def segments_of(n, c):
     return -(-n // size), size
 
 
-def segment_lens(H, dv, edge):
+def segment_lens(H, d, dv, edge):
     """Portions on both sides of the length from which one is cut, and of 2 and 5 full segments give or take a row."""
-    for c in range(10, 100):
+    for c in range(7, 100):
         first = -(-7 * c // 4)
-        lens = [16 * (first - 1), 16 * (first - 1) + 1, 16 * 5 * c + edge, 3, 16 * 2 * c + edge, 2, 40]
-        if chunks_per_segment(66 + sum(lens), H, dv) == c:
+        lens = [1] * 66 + [16 * (first - 1), 16 * (first - 1) + 1, 16 * 5 * c + edge, 3, 16 * 2 * c + edge, 2, 40]
+        if all(scan_plan(name, lens, H, H, d, dv)["chunks"] == c for name in SCAN_MODES):
             break
-    n = [-(-x // 16) for x in lens]
+    n = [-(-x // 16) for x in lens[66:]]
     parts = [segments_of(x, c) for x in n]
     assert [p for p, _ in parts] == [1, 2, 5, 1, 2, 1, 1] and parts[2][1] == c + (edge > 0)
     # the batch is cut at all: the rule of the kernels' find_segment
     uncut = max(x for x, (p, _) in zip(n, parts) if p == 1)
     assert 39 * max(n) > 39 * uncut + 63 * max(k for p, k in parts if p > 1) + 120
-    return [1] * 66 + lens
+    return lens
 
 
 @pytest.mark.parametrize("dt", DTYPES)
@@ -1882,9 +1885,12 @@ def test_scans_in_segments(dt, H, d, dv, slow, edge):
     segments (slow) and that forget within one."""
     torch.manual_seed(d + dv)
     if H == 40:
-        lens = [1, 3, 9, 1500 + edge, 17, 1]      # 80 workgroups per portion: segments of 30 chunks
+        lens = [1, 3, 9, 1500 + edge, 17, 1]      # 40 workgroups of 128 columns per portion: segments of 15 chunks
+        for name in SCAN_MODES:
+            p = scan_plan(name, lens, H, H, d, dv)
+            assert (p["waves"], p["cols"], p["chunks"]) == (8, 128, 15)
     else:
-        lens = segment_lens(H, dv, edge)
+        lens = segment_lens(H, d, dv, edge)
     S = len(lens)
     starts = [0 if i % 3 == 0 else 5 for i in range(S)]
     slots = [S - 1 - i for i in range(S)]
@@ -1975,11 +1981,17 @@ def test_segments_in_a_graph():
 @pytest.mark.parametrize("H,G,d,dv", [(16, 8, 128, 64), (16, 4, 64, 40), (15, 5, 128, 64), (8, 8, 128, 128),
                                       (8, 4, 100, 70), (6, 6, 64, 129)])
 def test_scans_of_full_chip(dt, H, G, d, dv):
-    """Batches that fill the chip (walk_wide): 128 columns per workgroup, or two heads of 64 with the same keys, portions
+    """Batches that fill the chip (walk_shape): 128 columns per workgroup, or two heads of 64 with the same keys, portions
     of odd and even numbers of chunks, full and not, fresh and continued."""
     torch.manual_seed(H + d + dv)
-    S = 512 // (H * -(-dv // 64)) + 3
+    S = 768 // (H * -(-dv // 64)) + 3
     lens = [(16, 33, 47, 64, 30, 80)[i % 6] for i in range(S)]
+    # (with a fifth less they still would)
+    wide = {name: dv > 64 or (name == "state_space_scan" and H // G % 2 == 0) for name in SCAN_MODES}
+    for name in SCAN_MODES:
+        p = scan_plan(name, lens[:S - S // 5], H, G, d, dv)
+        shape = (4, 1, 64) if not wide[name] else (8, 1, 128) if dv > 64 else (8, 2, 64)
+        assert (p["waves"], p["heads"], p["cols"]) == shape, name
     md = ragged(lens, [9 * (i % 2) for i in range(S)], list(range(S))[::-1], width=64)
     T, g = sum(lens), cuda(md)
     at, at_g = (tuple(m[k] for k in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
@@ -2214,3 +2226,27 @@ def test_kept_decays_of_unaligned_keys(dt, d, dv, lens):
         got = getattr(mx, name)(*(a.cuda() for a in args), st_g, *at_g, *last)
         want = getattr(mref, name)(*args, st, *at, *last)
         chunk_compare(got, want, st_g, st, torch.ones(T, dtype=torch.bool))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,G,dv,lens", [(96, 8, 64, [1023]), (96, 24, 40, [1, 950, 33, 1]), (64, 8, 64, [1100, 260])])
+def test_two_heads_in_segments(dt, H, G, dv, lens):
+    """State-space prompts whose segments walk two heads with the same keys each: the states, their copy and the decays of
+    both, fresh and continued."""
+    torch.manual_seed(H + dv)
+    d, S, T = 128, len(lens), sum(lens)
+    p = scan_plan("state_space_scan", lens, H, G, d, dv)
+    assert (p["waves"], p["heads"]) == (8, 2) and segments_of(-(-max(lens) // 16), p["chunks"])[0] > 1 and p["states"] > 0
+    md = ragged(lens, [5 * (i % 2) for i in range(S)], list(range(S))[::-1], width=80)
+    g = cuda(md)
+    at, at_g = (tuple(m[key] for key in ("positions", "seq_qstart", "seq_slot")) for m in (md, g))
+    B, C, v = torch.randn(T, G * d).to(dt), torch.randn(T, G * d).to(dt), torch.randn(T, H * dv).to(dt)
+    dts, z, a_log, skip = torch.randn(T, H).to(dt), torch.zeros(H), torch.linspace(-8.0, 1.0, H), torch.randn(H)
+    st = torch.randn(S, H, d, dv)
+    st_g = st.clone().cuda()
+    args = (v, B, C, dts, z, a_log, skip)
+    got = mx.state_space_scan(*(a.cuda() for a in args), st_g, *at_g, H, G, d, dv)
+    want = mref.state_space_scan(*args, st, *at, H, G, d, dv)
+    # as test_scans_in_segments
+    for a, b in ((got.cpu(), want), (st_g.cpu(), st)):
+        assert float((a - b).abs().max()) <= 2e-5 * float(b.abs().max())
