@@ -311,9 +311,11 @@ def sigmoid_attention(q, k_cache, v_cache, block_tables, seq_kvlen, seq_qstart, 
     # the chip once (by registers and LDS a CU holds one workgroup, of up to 16 heads two, of up to 8
     # three); the fp32 partial rows are added by a second kernel.  The kernels take fewer where the
     # tiles' lengths, which are on the device, say so (sg_shares), so a nearly full chip has room for
-    # two.  us by shares, 1 / 2 / 3 / 4 / 6: 24 heads, 44 workgroups 105 / 69 / 57 / 50 / 45, 88
-    # 205 / 120 / 92 / 99 / 99, 132 (3 prompts) 110 / 77 / 93 / 93 / 113; one prompt in 188 419 / 238,
-    # 208 461 / 259, 252 556 / 349, 4 prompts in 256 151 / 185, 12 in 240 58 / 86.
+    # two.  A third and more are rounded up from 0.36 on: the chip then is a little more than full, and
+    # the longest pieces are shorter.  us by shares, 1 / 2 / 3 / 4 / 6: 24 heads, 44 workgroups
+    # 105 / 69 / 57 / 50 / 45, 76 177 / 107 / 82 / 71 / 88, 108 244 / 142 / 108 / 126 / 125, 132 (3
+    # prompts) 110 / 77 / 93 / 93 / 113; one prompt in 188 419 / 238, 208 461 / 259, 252 556 / 349, 4
+    # prompts in 256 151 / 185, 12 in 240 58 / 86.
     split_out, tiles = None, 4 * tile_seq.shape[0]
     room = 256 * (3 if q.shape[1] <= 8 else 2 if q.shape[1] <= 16 else 1)
     split = max(2 if tiles <= room else 1, int(room / tiles + 0.64)) if tiles else 1
