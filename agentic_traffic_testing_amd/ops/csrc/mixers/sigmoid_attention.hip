@@ -91,12 +91,14 @@ __device__ __forceinline__ int sg_shares(const SigArgs& a, int num_tiles) {
     most = max(most, __shfl_xor(most, o, kWave));
     rows += __shfl_xor(rows, o, kWave);
   }
+  // (in whole numbers: both kernels must come to the same.  They stay below 2^32: up to 768 workgroups of up to 2^22 keys)
   int best = 1;
-  float least = INFINITY;
-  for (int s = 1; s <= a.split; ++s) {
-    const float time = fmaxf(static_cast<float>(most) * a.room / s, 1.5f * work) + (s > 1 ? 0.55f * s * rows : 0.f);
-    best = time < least ? s : best;
-    least = fminf(least, time);
+  unsigned least = ~0u;
+  const unsigned longest = 20u * min(most, 1 << 17) * a.room, all = 30u * min(work, 1 << 27);
+  for (unsigned s = 1; s <= static_cast<unsigned>(a.split); ++s) {
+    const unsigned time = max(longest / s, all) + (s > 1 ? 11u * s * min(rows, 1 << 14) : 0u);
+    best = time < least ? static_cast<int>(s) : best;
+    least = min(time, least);
   }
   return best;
 }
