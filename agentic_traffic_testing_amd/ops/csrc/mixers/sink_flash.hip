@@ -1,31 +1,40 @@
 // Prefill of the paged softmax attention on the matrix cores (bf16, gfx950): flash form of the kernel in
 // sink_attention.hip, same masks, sink, gates and pair epilogue (see there for what they mean).
 //
-// A workgroup = NW waves x 32 columns, a column = (query token, query head of the KV head's group); it walks
-// 64-key blocks:
+// A piece of work = up to NW x 32 columns of one 64-token tile, a column = (query token, query head of the KV head's
+// group); its workgroup walks blocks of 32 KT keys:
 //   S^T[32 keys x 32 cols] = K . Q^T    (mfma 32x32x16, A = K rows from LDS, B = Q in registers)
 //   O^T[vdim x 32 cols]   += V^T . P^T  (A = V^T rows from LDS, B = P^T from the S^T registers)
 // A lane holds one column of S^T, so the softmax statistics are lane-local plus one exchange with
 // lane ^ 32.  K rows are read in the order that swaps bits 2 and 3 of the row: the eight probabilities a
 // lane half then holds per 16-key step belong to eight neighbouring keys, so a V^T fragment is one plain
-// 16-byte read.
+// 16-byte read.  O and l are rescaled by every block's maximum.  (Letting the maximum lag by up to 2^8 saves time but then
+// the largest weight is not exactly 1 and its rounding counts: error against 64 bits 3.2e-3 instead of 3.0e-3.)
 //
-// The next block's K / V are fetched into registers behind the score products and stored to the other LDS
-// buffer after the value products: one barrier per block.  A wave fetches keys of ONE 16-key group, which
-// lie in one page (pages of 16 tokens or more), so its page and the group's place in the page are scalars and
-// every lane offset a loop constant; the sequence's page list sits in LDS.  O and l are rescaled on blocks that raise some column's
-// maximum.  (Letting the maximum lag by up to 2^8 saves ~3 % but then the largest weight is not exactly 1
-// and its rounding counts: error against 64 bits 3.2e-3 instead of 3.0e-3.)
+// Pipeline: step i takes the scores of block i, the weights of block i - 1 and the value products of block i - 2, so that
+// matrix and vector work of one step do not depend on each other, and `quick` deals them out by hand: a product (32 cycles
+// of the matrix core), then as many vector instructions as fit behind it.  Left to the compiler the two ran one after the
+// other, also across the two waves of a SIMD (5000 cycles per block and pair of waves; 3350 now, 2300 of them products).  Steps
+// with masks, at the window's edges and at both ends go part by part.  K of block i + 1 and V of block i - 1 travel straight
+// from memory to LDS in the meantime: no registers, one wait and one barrier per step.  A wave moves keys of ONE 16-key
+// group, which lie in one page (pages of 16 tokens or more), so its page and the group's place in it are scalars.
+//
+// Work: the hardware hands workgroups to the shader engines strictly in turn, a free place in one waits for its turn, and a
+// workgroup's start (page list, queries, first keys: a chain of loads) costs 3 - 4 us; both together left CUs idle a fifth
+// of the time.  So large batches run one workgroup of eight waves per CU that takes several pieces: sorted by length and
+// dealt back and forth (their sums come out equal within 3 %), the next piece's page list, queries and first keys on their way
+// behind the present one's last steps.  Batches whose pieces of 128 columns number up to six per CU run one piece per
+// workgroup of four waves, two workgroups per CU (the rule, with both sides measured, at launch_sink_flash).
 //
 // Pair form: a workgroup's first four waves carry the first map, the other four the second one, over the
-// same columns and one V block; the second map's result goes to the first's waves through LDS at the end.
+// same columns and one V block; at the end each wave finishes half of the channels.
 //
-// Bound (128 wide): per block and wave 1024 cycles of matrix products and ~1000 of softmax on the vector
-// units; two waves per SIMD overlap them only in part (matrix cores 37 % busy, vector units 45 %, LDS port
-// 34 %, at 1.8 GHz).  Wave priority from the score products to the end of the value products lets the other
-// wave fall behind and fill gaps instead of running the same phase in step: 7580 rows of 32 + 8 heads of 128
-// 5 %, latent 2 %, two maps 1 %.  (Taking block b + 1's scores beside block b's weights in the same wave: 128 wide 6 %
-// less, latent 2.1 times, two maps 1.1 times the time - registers.)
+// Bound (128 wide): matrix cores 60 - 70 % and vector units 60 % busy inside the steps, at 2.0 - 2.1 GHz: with both busy the
+// clock gives way (the kernel before, half as busy: 2.2 GHz; products alone: 1.85 GHz).  4 prompts of ~1.9k tokens, us, before ->
+// now: 32 + 8 heads of 128 159 -> 138, latent 257 -> 221, two maps (8 heads, 5 x 1165, window 1024) 72 -> 50.
+#include <algorithm>
+#include <type_traits>
+
 #include "sink_attention.h"
 
 namespace mixk {
@@ -37,371 +46,774 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+typedef __attribute__((address_space(3))) void* lds_ptr;
 
-constexpr int kBlock = 64;               // keys per block (two 32-key score tiles)
-constexpr int kVS = kBlock + 8;          // V^T row in LDS: 144 B, 16-byte reads free of bank conflicts
 constexpr int kPages = 2048;             // page-table entries in LDS
+constexpr int kSortTiles = 1024;         // tiles that a workgroup puts in order
+constexpr int kPieces = 64;              // pieces of work per workgroup in LDS
 // Pair form: in the first blocks each of the two tiles has its own maximum.  Largest weights are rounded to exactly 1;
 // with a maximum per 64 keys there are fewer of them than per 32, half of the difference from the first block, 90 %
-// from four.  Error against 64 bits, prompts of 600 (1e-3): one per block 2.345, the first four split 2.328 (the kernel
-// before, 32 keys: 2.332); 5 x 1165 tokens, window 1024: 82.2 -> 83.3 us, with all blocks split 85.3.  (One map: sums of
-// the rounded weights make up for more than that: 2.928 against 2.935.)
+// from four.  Error against 64 bits, prompts of 600 (1e-3): one per block 2.345, the first four split 2.328.  (One map:
+// sums of the rounded weights make up for more than that.)
 constexpr int kSplitBlocks = 4;
 constexpr float kLog2e = 1.44269504088896341f;
+#define SF_INLINE __attribute__((always_inline))
 
 __device__ __forceinline__ float xor32(float v, int idx4) {
   return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(idx4, __builtin_bit_cast(int, v)));
 }
+// larger value of the lane's and lane ^ 32's (the builtin's two results are taken for one where both operands are the
+// same value)
+__device__ __forceinline__ float both(float v) {
+  float a = v, b = v;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+#endif
+  return fmaxf(a, b);
+}
+// 16 (send4: 4) bytes per lane from base + offset to 64 lanes' LDS from `to` on, without registers; there after
+// wait_sent().  (After the builtin the compiler makes every read of LDS wait for all transfers.)
+__device__ __forceinline__ void send16(const void* base, uint32_t offset, void* to) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(at) : "m0", "memory");
+#endif
+}
+__device__ __forceinline__ void send4(const void* base, uint32_t offset, void* to) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "s"(at) : "m0", "memory");
+#endif
+}
+__device__ __forceinline__ void wait_sent() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+}
+// the value, computed anew from here on (what follows from it is not kept in registers from one piece of work to the next)
+__device__ __forceinline__ int fresh(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v));
+#endif
+  return v;
+}
+// the value is there at this point of the program
+template <typename X>
+__device__ __forceinline__ void hold(const X& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" ::"v"(x));
+#endif
+}
 
-// DK = 16 ND (q / k width), DV = 32 NV (value width).
-template <int ND, int NV, int NMAP, int NW, int WPS, bool WIN>
-__global__ void __launch_bounds__(NW * 64, WPS)
-sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q,
-                  const __bf16* __restrict__ k_cache, const __bf16* __restrict__ v_cache, AttnArgs a,
-                  int num_tiles, int chunks) {
-  constexpr int DK = 16 * ND, DV = 32 * NV, CW = NW / NMAP, COLS = CW * 32;
-  constexpr int KS = DK + 8;
-  constexpr int WPG = NW / 4;                       // waves per 16-key group
-  constexpr int KU = 16 * (DK / 8) / (64 * WPG);    // 16-byte chunks of K per lane, map and block
-  constexpr int VU = 2 * DV / (64 * WPG);           // ... of V
-  static_assert(NMAP == 1 || NW == 8, "pair form: four waves per map");
-  static_assert(KU * 64 * WPG == 2 * DK && VU * 64 * WPG == 2 * DV, "staging covers a block");
-  typedef __bf16 KBuf[2][NMAP][kBlock * KS];
-  typedef __bf16 VBuf[2][DV * kVS];
-  __shared__ __attribute__((aligned(16))) char lds[sizeof(KBuf) + sizeof(VBuf)];
-  KBuf& lds_k = *reinterpret_cast<KBuf*>(lds);
-  VBuf& lds_v = *reinterpret_cast<VBuf*>(lds + sizeof(KBuf));
-  __shared__ int lds_bt[kPages];
+// DK = 16 ND (q / k width), DV = 32 NV (value width), blocks of 32 KT keys.
+template <int ND, int NV, int NMAP, int NW, int KT, bool WIN>
+__global__ void __launch_bounds__(NW * 64, 2)
+sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __bf16* __restrict__ k_cache,
+                  const __bf16* __restrict__ v_cache, AttnArgs a, int num_tiles, int chunks, int workers) {
+  constexpr int DK = 16 * ND, DV = 32 * NV, CW = NW / NMAP, COLS = CW * 32, BLK = 32 * KT;
+  constexpr bool MANY = NW == 8;                    // a workgroup takes several pieces of work in turn
+  constexpr int GR = 2 * KT, WPG = NW / GR;         // 16-key groups of a block, waves per group
+  constexpr int CK = DK / 8;                        // 16-byte chunks of a K row
+  constexpr int KN = CK / 4, KU = (KN + WPG - 1) / WPG;   // transfers (64 chunks) of K per group and map; per wave
+  constexpr int VN = NV, VU = (VN + WPG - 1) / WPG;
+  constexpr int RB = CK < 16 ? 16 / CK : 1;         // K rows per 256 bytes
+  constexpr int KB = NMAP * BLK * DK, VB = DV * BLK;   // elements of a buffer
+  constexpr int MT = NMAP, TPM = KT / MT;           // maxima per block, tiles per maximum
+  static_assert(NMAP == 1 || (NW == 8 && KT == 2), "pair form: four waves per map");
+  __shared__ __attribute__((aligned(1024))) __bf16 lds_k[2 * KB], lds_v[2 * VB];
+  __shared__ __attribute__((aligned(1024))) char lds_x[MANY ? (NMAP == 2 ? 65536 : 32768) : 16];
+  __shared__ float lds_ss[NMAP == 2 ? NW : 1][32];
+  __shared__ int lds_bt[MANY ? 2 : 1][kPages];
+  __shared__ int lds_piece[MANY ? kPieces : 1][8];
   const int H = a.H, G = a.G, bs = a.block_size;
   const int rep = H / G, GO = G / NMAP, GV = G / a.v_share;
   // KV head fastest: workgroups are dealt round-robin to the eight XCDs, so with eight KV heads a head's
-  // K / V stay in one L2.  Tiles are listed in token order: the longest go first.
+  // K / V stay in one L2.
   const int bid = static_cast<int>(blockIdx.x);
   const int g = bid % GO;                           // K head (pair form: V head, K heads 2 g and 2 g + 1)
-  const int rest = bid / GO;
-  const int chunk = chunks - 1 - rest % chunks;
-  const int tile = num_tiles - 1 - rest / chunks;
+  const int worker = bid / GO;
   const int gv = NMAP == 2 ? g : g / a.v_share;
-  const int s = a.tile_seq[tile], qo = a.tile_qoff[tile];
-  const int row0 = a.seq_qstart[s], n = a.seq_qstart[s + 1] - row0, kvlen = a.seq_kvlen[s];
-  if (n <= 0 || kvlen <= 0 || qo >= n) return;
-  const int cols_total = min(kTileTokens, n - qo) * rep;
-  const int col0 = chunk * COLS;
-  if (col0 >= cols_total) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5, x32 = (lane ^ 32) << 2;
-  const int ctx = kvlen - n + qo;                   // position of the tile's first token
   const int mp = NMAP == 2 ? w / CW : 0;            // the wave's map
-  const int wcol = col0 + (w % CW) * 32;       // the wave's first column
-  const bool wave_on = wcol < cols_total;
-  const int w_last = min(cols_total, wcol + 32) - 1;
-  const int pos_first = ctx + wcol / rep, pos_last = ctx + max(w_last, 0) / rep;
-  const int kend = min(kvlen, ctx + (min(cols_total, col0 + COLS) - 1) / rep + 1);
-  // key blocks: the kept keys in front of the window, then from the window's start (block-aligned)
-  const int klow = window_start(ctx + col0 / rep, a.window);   // no column sees keys in [keep, klow)
-  const int kbeg = klow & ~(kBlock - 1);
-  const int kkeep = min(a.keep, kbeg);
-  const int nk = (kkeep + kBlock - 1) / kBlock;
-  const int nb = nk + (kend - kbeg + kBlock - 1) / kBlock;
-  auto block_key = [&](int b) { return b < nk ? b * kBlock : kbeg + (b - nk) * kBlock; };
+  const float scale2 = a.scale * kLog2e;
+  const uint32_t per = 0xffffffffu / rep + 1;       // (columns x rep < 2^32; rep 1: 0)
+  auto token_of = [&](int c) SF_INLINE { return rep == 1 ? c : static_cast<int>(__umulhi(static_cast<uint32_t>(c), per)); };
 
-  const int* btg = a.block_tables + static_cast<int64_t>(s) * a.bt_width;
-  const int npages = min((kend + bs - 1) >> a.bs_shift, kPages);   // (the launcher bounds the table)
-  for (int i = tid; i < npages; i += NW * 64) lds_bt[i] = btg[i];
-
-  const int col = wcol + r;
-  const bool valid = col < cols_total;
-  const int tok = valid ? col / rep : 0, head = (NMAP * g + mp) * rep + (valid ? col % rep : 0);
-  const int64_t row = row0 + qo + tok;
-  const int qpos = valid ? ctx + tok : -1;          // no key is visible to a column that is not there
-  const int qlow = window_start(qpos, a.window);
-  bf16x8 qf[ND];
-  const __bf16* qp = q + row * a.q_stride + static_cast<int64_t>(head) * DK + 8 * h;
-#pragma unroll
-  for (int st = 0; st < ND; ++st) qf[st] = *reinterpret_cast<const bf16x8*>(qp + 16 * st);
-  float m = kNegBig, l = 0.f;   // l: of the lane's keys
-  if (a.sink) {   // the sink is the state the online softmax starts from (log2 units)
-    m = a.sink_val != nullptr ? a.sink_val[head] * kLog2e : 0.f;
-    l = h == 0 ? 1.f : 0.f;
-  }
-  f32x16 O[NV];
-#pragma unroll
-  for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) O[vt][i] = 0.f;
-  __syncthreads();
-
-  // staging: wave w moves keys of group sg = w / WPG; its part of the group's chunks starts at `sub`
-  const int sg = w / WPG, sub = (w % WPG) * 64 + lane;
-  int k_src[KU], k_dst[KU], v_src[VU], v_dst[VU];
+  // ---- transfers: wave w moves keys of group w % GR, all in one page.  K rows lie in LDS as they are, V as
+  // [group][channel][16 keys]; the 16-byte chunks of a K row and the halves of a V row change places so that the
+  // fragments' reads have no bank conflicts
+  const int sg = w % GR, part = w / GR;
+  uint32_t k_src[KU], v_src[VU];   // bytes
 #pragma unroll
   for (int u = 0; u < KU; ++u) {
-    const int i = sub + u * 64 * WPG, key = i / (DK / 8), c8 = i % (DK / 8);
-    k_src[u] = key * DK + c8 * 8;
-    k_dst[u] = (16 * sg + key) * KS + c8 * 8;
+    const int row = (u * WPG + part) * (64 / CK) + lane / CK;   // of the group
+    k_src[u] = 2u * (row * DK + ((lane % CK) ^ ((row / RB) & (CK - 1) & 15)) * 8);
   }
+  const int v_half = 8 * ((lane ^ (lane >> 4)) & 1);
 #pragma unroll
-  for (int u = 0; u < VU; ++u) {
-    const int i = sub + u * 64 * WPG, ch = i >> 1;
-    v_src[u] = ch * bs + 8 * (i & 1);
-    v_dst[u] = ch * kVS + 16 * sg + 8 * (i & 1);
+  for (int u = 0; u < VU; ++u) v_src[u] = 2u * ((32 * (u * WPG + part) + (lane >> 1)) * bs + v_half);
+  const int k_lds = 16 * sg * DK + part * 512, v_lds = sg * DV * 16 + part * 512;
+  const __bf16* k_base = k_cache + static_cast<int64_t>(NMAP * g) * bs * DK;
+  const __bf16* v_base = v_cache + static_cast<int64_t>(gv) * DV * bs;
+  const uint32_t k_page = G * bs * DK, v_page = GV * DV * bs;
+  auto k_at = [&](int pg, int k0) SF_INLINE {
+    return k_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * k_page + ((k0 + 16 * sg) & (bs - 1)) * DK;
+  };
+  auto v_at = [&](int pg, int k0) SF_INLINE {
+    return v_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * v_page + ((k0 + 16 * sg) & (bs - 1));
+  };
+  auto send_k = [&](const __bf16* kb, __bf16* to, int u) SF_INLINE {
+    if (KU * WPG == KN || (u % KU) * WPG + part < KN)
+      send16(kb + (u / KU) * bs * DK, k_src[u % KU], to + (u / KU) * BLK * DK + k_lds + (u % KU) * WPG * 512);
+  };
+  auto send_v = [&](const __bf16* vb, __bf16* to, int u) SF_INLINE {
+    if (VU * WPG == VN || u * WPG + part < VN) send16(vb, v_src[u], to + v_lds + u * WPG * 512);
+  };
+  // ---- fragments.  A row of the score products: key with bits 2 and 3 swapped
+  const int krow = (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);
+  const int kfrag = mp * BLK * DK + krow * DK, vfrag = r * 16 + 8 * (h ^ ((r >> 3) & 1));
+  constexpr int KO = ND < 8 ? ND : 8;
+  int kofs[KO];
+#pragma unroll
+  for (int st = 0; st < KO; ++st) kofs[st] = kfrag + ((2 * st + h) ^ ((krow / RB) & (CK - 1) & 15)) * 8;
+  auto kf = [&](const __bf16* b, int t, int st) SF_INLINE {
+    return *reinterpret_cast<const bf16x8*>(b + 32 * t * DK + kofs[st % 8] + st / 8 * 128);
+  };
+  auto vf = [&](const __bf16* b, int vt, int ks) SF_INLINE {
+    return *reinterpret_cast<const bf16x8*>(b + vfrag + ks * DV * 16 + vt * 512);
+  };
+
+  // ---- the workgroup's pieces of work, `mine` of them
+  const int pieces = num_tiles * chunks;
+  // every other round the other way about: long pieces come together with short ones
+  auto rank_of = [&](int k) { return k * workers + ((k & 1) ? workers - 1 - worker : worker); };
+  int mine = pieces / workers;
+  if (rank_of(mine) < pieces) ++mine;
+  struct Piece {
+    int s, qo, col0, row0, n, kvlen;
+  };
+  auto cols_of = [&](const Piece& p) SF_INLINE { return min(kTileTokens, p.n - p.qo) * rep; };
+  auto kend_of = [&](const Piece& p) SF_INLINE {
+    return p.kvlen - p.n + p.qo + (min(cols_of(p), p.col0 + COLS) - 1) / rep + 1;
+  };
+  auto fetch = [&](int item) SF_INLINE {
+    Piece p;
+    const int tile = item / chunks;
+    p.s = a.tile_seq[tile], p.qo = a.tile_qoff[tile], p.col0 = item % chunks * COLS;
+    p.row0 = a.seq_qstart[p.s], p.n = a.seq_qstart[p.s + 1] - p.row0, p.kvlen = a.seq_kvlen[p.s];
+    // nothing to do: an empty sequence, a chunk past a short tile's columns
+    if (p.n <= 0 || p.kvlen <= 0 || p.qo >= p.n || p.col0 >= min(kTileTokens, p.n - p.qo) * rep) p.n = 0;
+    return p;
+  };
+  if constexpr (MANY) {
+    // Long ones first: a piece's rank among the tiles' numbers of blocks, found by bisection of the keys (blocks, then
+    // place in the list: no two are alike), which every wave holds for itself
+    constexpr int KR = kSortTiles / 64;
+    if (pieces > workers && num_tiles <= kSortTiles) {
+      unsigned int key[KR];
+      Piece own[KR];
+      const int most = (a.bt_width << a.bs_shift) / BLK + 2;
+#pragma unroll
+      for (int i = 0; i < KR; ++i) {
+        key[i] = 0;
+        own[i] = Piece{};
+        if (64 * i >= num_tiles) continue;
+        const int t = min(lane + 64 * i, num_tiles - 1);
+        own[i] = fetch(t * chunks);
+        const int first = window_start(own[i].kvlen - own[i].n + own[i].qo, a.window);
+        if (lane + 64 * i < num_tiles)
+          key[i] = static_cast<unsigned int>(min(max((own[i].kvlen - own[i].n + min(own[i].n, own[i].qo + kTileTokens) - first) / BLK, 0) + 1, most)) << 10 | (kSortTiles - 1 - t);
+      }
+      for (int k = w; k < mine; k += NW) {
+        const int rk = rank_of(k), want = rk / chunks, col0 = (chunks - 1 - rk % chunks) * COLS;
+        unsigned int v = 0;   // the largest value that more than `want` keys reach: that rank's key
+        for (int bit = 31 - __builtin_clz(most << 10 | (kSortTiles - 1)); bit >= 0; --bit) {
+          const unsigned int c = v | 1u << bit;
+          int n = 0;
+#pragma unroll
+          for (int i = 0; i < KR; ++i) {
+            if (64 * i >= num_tiles) break;
+            n += __builtin_popcountll(__ballot(key[i] >= c));
+          }
+          if (n > want) v = c;
+        }
+#pragma unroll
+        for (int i = 0; i < KR; ++i)
+          if (key[i] == v) {
+            const Piece& p = own[i];
+            int* e = lds_piece[k];
+            e[0] = p.s, e[1] = p.qo, e[2] = col0, e[3] = p.row0, e[4] = col0 < cols_of(p) ? p.n : 0, e[5] = p.kvlen;
+          }
+      }
+    } else {
+      for (int k = w; k < mine; k += NW) {
+        const Piece p = fetch(pieces - 1 - rank_of(k));
+        int* e = lds_piece[k];
+        if (lane == 0) e[0] = p.s, e[1] = p.qo, e[2] = p.col0, e[3] = p.row0, e[4] = p.n, e[5] = p.kvlen;
+      }
+    }
+    __syncthreads();
   }
-  const int last_page = npages - 1;
-  u32x4 kr[NMAP][KU], vr[VU];
-  auto load_block = [&](int k0) {
+  // the next piece with work, from number k on
+  auto next_piece = [&](int& k, Piece& p) SF_INLINE {
+    if constexpr (!MANY) {
+      if (k > 0) return false;
+      p = fetch(pieces - 1 - worker);
+      return p.n > 0;
+    } else {
+      // (each workgroup begins at another of its pieces: queries and results of all of them do not come at once)
+      for (; k < mine; ++k) {
+        const int* e = lds_piece[(k + worker) % mine];
+        p.n = __builtin_amdgcn_readfirstlane(e[4]);
+        if (p.n == 0) continue;
+        p.s = __builtin_amdgcn_readfirstlane(e[0]), p.qo = __builtin_amdgcn_readfirstlane(e[1]);
+        p.col0 = __builtin_amdgcn_readfirstlane(e[2]), p.row0 = __builtin_amdgcn_readfirstlane(e[3]);
+        p.kvlen = __builtin_amdgcn_readfirstlane(e[5]);
+        return true;
+      }
+      return false;
+    }
+  };
+  // ---- what a piece needs before its first step
+  auto pages_of = [&](const Piece& p) SF_INLINE { return min((kend_of(p) + bs - 1) >> a.bs_shift, kPages); };   // (the launcher bounds the table)
+  // key blocks: the kept keys in front of the window, then from the window's start (block-aligned)
+  auto klow_of = [&](const Piece& p) SF_INLINE { return window_start(p.kvlen - p.n + p.qo + p.col0 / rep, a.window); };
+  auto first_key = [&](const Piece& p) SF_INLINE { return min(a.keep, klow_of(p) & ~(BLK - 1)) > 0 ? 0 : klow_of(p) & ~(BLK - 1); };
+  auto send_pages = [&](const Piece& p, int* bt) SF_INLINE {
+    const int* btg = a.block_tables + static_cast<int64_t>(p.s) * a.bt_width;
+    const int npages = pages_of(p);
+    for (int i = w * 64; i < npages; i += NW * 64)
+      if (i + lane < npages) send4(btg, 4u * (i + lane), bt + i);
+  };
+  auto send_block_k = [&](const int* bt, int last_page, int k0, __bf16* to) SF_INLINE {
+    const __bf16* kb = k_at(__builtin_amdgcn_readfirstlane(bt[min((k0 + 16 * sg) >> a.bs_shift, last_page)]), k0);
+#pragma unroll
+    for (int u = 0; u < NMAP * KU; ++u) send_k(kb, to, u);
+  };
+  bf16x8 qf[ND];
+  auto load_q = [&](const Piece& p) SF_INLINE {
+    const int ln = fresh(lane), col = p.col0 + (w % CW) * 32 + (ln & 31);
+    const bool valid = col < cols_of(p);
+    const int tok = valid ? token_of(col) : 0, head = (NMAP * g + mp) * rep + (valid ? col - tok * rep : 0);
+    const __bf16* qp = q + (p.row0 + p.qo + tok) * a.q_stride + static_cast<int64_t>(head) * DK + 8 * (ln >> 5);
+#pragma unroll
+    for (int st = 0; st < ND; ++st) qf[st] = *reinterpret_cast<const bf16x8*>(qp + 16 * st);
+  };
+
+  int pn = 0;
+  Piece now, nxt;
+  if (!next_piece(pn, now)) return;
+  // (queries are there before a loop, which would wait for its transfers with them)
+  auto hold_q = [&]() SF_INLINE {
+#pragma unroll
+    for (int st = 0; st < ND; ++st) hold(qf[st]);
+  };
+  send_pages(now, lds_bt[0]);
+  load_q(now);
+  hold_q();
+  wait_sent();
+  __syncthreads();
+  send_block_k(lds_bt[0], pages_of(now) - 1, first_key(now), lds_k);
+  wait_sent();
+  __syncthreads();
+
+  for (int turn = 0;; ++turn) {
+    ++pn;
+    nxt = now;   // (after the last one its queries are read once more, for nothing)
+    const bool more = next_piece(pn, nxt);
+    const int* const bt = lds_bt[MANY ? turn & 1 : 0];
+    const int qo = now.qo, row0 = now.row0, kvlen = now.kvlen, col0 = now.col0;
+    const int cols_total = cols_of(now);
+    const int ctx = kvlen - now.n + qo;               // position of the tile's first token
+    const int wcol = col0 + (w % CW) * 32;            // the wave's first column
+    const bool wave_on = wcol < cols_total;
+    const int w_last = min(cols_total, wcol + 32) - 1;
+    const int pos_first = ctx + wcol / rep, pos_last = ctx + max(w_last, 0) / rep;
+    const int kend = kend_of(now), last_page = pages_of(now) - 1;
+    const int klow = klow_of(now), kbeg = klow & ~(BLK - 1);   // no column sees keys in [keep, klow)
+    const int nk = (min(a.keep, kbeg) + BLK - 1) / BLK;
+    const int nb = nk + (kend - kbeg + BLK - 1) / BLK;
+    auto block_key = [&](int b) SF_INLINE { return b < nk ? b * BLK : kbeg + (b - nk) * BLK; };
+    const int col = wcol + r;
+    const bool valid = col < cols_total;
+    const int tok = valid ? token_of(col) : 0, head = (NMAP * g + mp) * rep + (valid ? col - tok * rep : 0);
+    const int64_t row = row0 + qo + tok;
+    const int qpos = valid ? ctx + tok : -1;          // no key is visible to a column that is not there
+    const int qlow = window_start(qpos, a.window);
+    float m = kNegBig, l = 0.f;   // l: of the lane's keys
+    if (a.sink) {   // the sink is the state the online softmax starts from (log2 units)
+      m = a.sink_val != nullptr ? a.sink_val[head] * kLog2e : 0.f;
+      l = h == 0 ? 1.f : 0.f;
+    }
+    f32x16 O[NV];
+#pragma unroll
+    for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) O[vt][i] = 0.f;
+
     // keys at or past kend read a clamped page or stale slots, keys in front of the window whatever is there: their
     // scores are masked and their V zeroed (0 x NaN)
-    const int key = k0 + 16 * sg, at = key & (bs - 1);   // (a page may hold several blocks)
-    const int pg = __builtin_amdgcn_readfirstlane(lds_bt[min(key >> a.bs_shift, last_page)]);
-    const __bf16* kb = k_cache + ((static_cast<int64_t>(pg) * G + NMAP * g) * bs + at) * DK;
-    const __bf16* vb = v_cache + (static_cast<int64_t>(pg) * GV + gv) * DV * bs + at;
+    u32x4 vr[VU];
+    auto seen = [&](int t) SF_INLINE { return t < kend && (!WIN || t >= klow || t < a.keep); };
+    auto edge = [&](int k0) SF_INLINE { return k0 + BLK > kend || (WIN && k0 < klow && k0 + BLK > a.keep); };
+    // (a block with such keys takes the way through registers: fetched here, put down by put_block_v)
+    auto send_block_v = [&](int k0, __bf16* to) SF_INLINE {
+      const __bf16* vb = v_at(__builtin_amdgcn_readfirstlane(bt[min((k0 + 16 * sg) >> a.bs_shift, last_page)]), k0);
 #pragma unroll
-    for (int e = 0; e < NMAP; ++e)
-#pragma unroll
-      for (int u = 0; u < KU; ++u)
-        kr[e][u] = *reinterpret_cast<const u32x4*>(kb + e * bs * DK + k_src[u]);
-#pragma unroll
-    for (int u = 0; u < VU; ++u) vr[u] = *reinterpret_cast<const u32x4*>(vb + v_src[u]);
-  };
-  auto store_block = [&](int buf, int k0) {
-#pragma unroll
-    for (int e = 0; e < NMAP; ++e)
-#pragma unroll
-      for (int u = 0; u < KU; ++u)
-        *reinterpret_cast<u32x4*>(&lds_k[buf][e][k_dst[u]]) = kr[e][u];
-    const int key = k0 + 16 * sg + 8 * (lane & 1);
-    if (key + 8 > kend || (WIN && key < klow && key + 8 > a.keep)) {
-      auto seen = [&](int t) { return t < kend && (!WIN || t >= klow || t < a.keep); };
+      for (int u = 0; u < VU; ++u) {
+        if (!edge(k0)) send_v(vb, to, u);
+        else if (VU * WPG == VN || u * WPG + part < VN)
+          vr[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb) + v_src[u]);
+      }
+    };
+    auto put_block_v = [&](int k0, __bf16* to) SF_INLINE {
+      if (!edge(k0)) return;
+      const int key = k0 + 16 * sg + v_half;
 #pragma unroll
       for (int u = 0; u < VU; ++u)
+        if (VU * WPG == VN || u * WPG + part < VN) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          vr[u][j] &= (seen(key + 2 * j) ? 0x0000ffffu : 0u) | (seen(key + 2 * j + 1) ? 0xffff0000u : 0u);
-    }
-#pragma unroll
-    for (int u = 0; u < VU; ++u) *reinterpret_cast<u32x4*>(&lds_v[buf][v_dst[u]]) = vr[u];
-  };
+          for (int j = 0; j < 4; ++j)
+            vr[u][j] &= (seen(key + 2 * j) ? 0x0000ffffu : 0u) | (seen(key + 2 * j + 1) ? 0xffff0000u : 0u);
+          *reinterpret_cast<u32x4*>(to + v_lds + u * WPG * 512 + lane * 8) = vr[u];
+        }
+    };
 
-  const float scale2 = a.scale * kLog2e;
-  // A row of the score products: key with bits 2 and 3 swapped
-  const int krow = (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);
-  // keys at or below the window start of the wave's latest column are outside somebody's window
-  const int edge_lo = a.window > 0 ? pos_last - a.window : -1;
-  const int low_first = window_start(pos_first, a.window);   // no column of the wave sees keys below
-
-  load_block(block_key(0));
-  store_block(0, block_key(0));
-  __syncthreads();
-  for (int b = 0; b < nb; ++b) {
-    const int buf = b & 1, k0 = block_key(b);
-    const bool more = b + 1 < nb;
-    bool issued = false;
-    if (wave_on && k0 <= pos_last && (k0 + kBlock > low_first || k0 < a.keep)) {
-      f32x16 S[2];
-      __builtin_amdgcn_s_setprio(1);
+    // keys at or below the window start of the wave's latest column are outside somebody's window
+    const int edge_lo = a.window > 0 ? pos_last - a.window : -1;
+    const int low_first = window_start(pos_first, a.window);   // no column of the wave sees keys below
+    float carry = 1.f;   // pair form: of the second tile's maximum over the first one's, until the value products
+    auto needed = [&](int b) SF_INLINE {
+      const int k0 = block_key(b);
+      return b >= 0 && b < nb && wave_on && k0 <= pos_last && (k0 + BLK > low_first || k0 < a.keep);
+    };
+    auto scores = [&](const __bf16* from, f32x16 (&S)[KT]) SF_INLINE {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < KT; ++t) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
 #pragma unroll
-        for (int st = 0; st < ND; ++st) {
-          const bf16x8 kf =
-              *reinterpret_cast<const bf16x8*>(&lds_k[buf][mp][(32 * t + krow) * KS + 16 * st + 8 * h]);
-          S[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[st], S[t], 0, 0, 0);
-        }
+        for (int st = 0; st < ND; ++st) S[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf(from, t, st), qf[st], S[t], 0, 0, 0);
       }
-      if (more) load_block(block_key(b + 1));   // in flight behind the softmax and the value products
-      issued = true;
-      // register i of tile t holds key k0 + 8 h + 32 t + 16 (i >> 3) + (i & 7)
-      if (k0 + kBlock - 1 > pos_first || (WIN && k0 <= edge_lo)) {
+    };
+    auto rescale = [&](float alpha) SF_INLINE {
+#pragma unroll
+      for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) O[vt][i] *= alpha;
+    };
+    auto values = [&](const __bf16* from, const bf16x8 (&P)[2 * KT], bool split) SF_INLINE {
+#pragma unroll
+      for (int e = 0; e < MT; ++e) {
+        if (e > 0 && split && __any(carry != 1.f)) rescale(carry);
+#pragma unroll
+        for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+          for (int ks = 2 * e * TPM; ks < 2 * (e + 1) * TPM; ++ks)
+            O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf(from, vt, ks), P[ks], O[vt], 0, 0, 0);
+      }
+    };
+    auto weights = [&](int b, f32x16 (&S)[KT], bf16x8 (&P)[2 * KT]) SF_INLINE {
+      const int k0 = block_key(b);
+      if (k0 + BLK - 1 > pos_first || (WIN && k0 <= edge_lo)) {
+        // register i of tile t holds key k0 + 8 h + 32 t + 16 (i >> 3) + (i & 7)
         const int hi = qpos + 1 - k0 - 8 * h, lo = qlow - k0 - 8 * h, kp = a.keep - k0 - 8 * h;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < KT; ++t)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             const int o = 32 * t + 16 * (i >> 3) + (i & 7);
             if (o >= hi || (WIN && o < lo && o >= kp)) S[t][i] = -INFINITY;
           }
       }
-      // maxima of the block: one, or in the pair form's first blocks one per tile (kSplitBlocks)
-      constexpr int MT = NMAP, TPM = 2 / MT;
       float tmax[MT], mt[MT], psum[MT];
 #pragma unroll
       for (int e = 0; e < MT; ++e) {
-        tmax[e] = S[e * TPM][0];
+        tmax[e] = kNegBig;   // (all keys masked: below every maximum, never taken)
 #pragma unroll
         for (int t = e * TPM; t < (e + 1) * TPM; ++t)
 #pragma unroll
           for (int i = 0; i < 16; ++i) tmax[e] = fmaxf(tmax[e], S[t][i]);
       }
 #pragma unroll
-      for (int e = 0; e < MT; ++e) tmax[e] = fmaxf(tmax[e], xor32(tmax[e], x32)) * scale2;
+      for (int e = 0; e < MT; ++e) tmax[e] = both(tmax[e]) * scale2;
       if (MT > 1 && b >= kSplitBlocks) tmax[0] = fmaxf(tmax[0], tmax[MT - 1]);
-      auto rescale = [&](float alpha) {
+      mt[0] = fmaxf(tmax[0], m);
+      if (__any(mt[0] > m)) {
+        const float alpha = __builtin_amdgcn_exp2f(m - mt[0]);
         l *= alpha;
-#pragma unroll
-        for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) O[vt][i] *= alpha;
-      };
-      bool grow = tmax[0] > m;   // (scale > 0; all keys masked: -inf, never)
-      mt[0] = grow ? tmax[0] : m;
-      if (__any(grow)) rescale(__builtin_amdgcn_exp2f(m - mt[0]));
-      grow = MT > 1 && tmax[MT - 1] > mt[0];
-      mt[MT - 1] = grow ? tmax[MT - 1] : mt[0];
+        rescale(alpha);
+      }
+      mt[MT - 1] = MT > 1 ? fmaxf(tmax[MT - 1], mt[0]) : mt[0];
       m = mt[MT - 1];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          S[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i], scale2, -mt[t / TPM]));
-      bf16x8 pf[4];
 #pragma unroll
       for (int e = 0; e < MT; ++e) psum[e] = 0.f;   // of the weights as the value products take them, rounded
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+      for (int ks = 0; ks < 2 * KT; ++ks) {
         u32x4 wv;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          wv[j] = __builtin_bit_cast(unsigned int, __builtin_convertvector(
-                      (f32x2{S[ks >> 1][8 * (ks & 1) + 2 * j], S[ks >> 1][8 * (ks & 1) + 2 * j + 1]}),
-                      bf16x2));
-        pf[ks] = __builtin_bit_cast(bf16x8, wv);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          psum[(ks >> 1) / TPM] += __builtin_bit_cast(float, wv[j] << 16) + __builtin_bit_cast(float, wv[j] & 0xffff0000u);
-      }
-#pragma unroll
-      for (int e = 0; e < MT; ++e) {
-        if (e > 0 && __any(grow)) rescale(__builtin_amdgcn_exp2f(mt[0] - m));
-        l += psum[e];
-#pragma unroll
-        for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-          for (int ks = 2 * e * TPM; ks < 2 * (e + 1) * TPM; ++ks) {
-            const bf16x8 vf = *reinterpret_cast<const bf16x8*>(&lds_v[buf][(32 * vt + r) * kVS + 16 * ks + 8 * h]);
-            O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[ks], O[vt], 0, 0, 0);
-          }
-      }
-      __builtin_amdgcn_s_setprio(0);
-    }
-    if (more) {
-      if (!issued) load_block(block_key(b + 1));
-      store_block(buf ^ 1, block_key(b + 1));
-    }
-    __syncthreads();
-  }
-
-  l += xor32(l, x32);
-  if constexpr (NMAP == 2) {
-    // the second map's waves hand lam / l * O to the first map's through LDS (the K / V buffers are free)
-    static_assert(sizeof(lds_k) + sizeof(lds_v) >= CW * 64 * 16 * NV * sizeof(float), "room for the second map");
-    f32x4* xch = reinterpret_cast<f32x4*>(lds) + (w % CW) * 4 * NV * 64 + lane;
-    const float il = l > 0.f ? (mp == 0 ? 1.0f : a.lam) / l : 0.f;
-    if (mp == 1) {
-#pragma unroll
-      for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4)
-          xch[(vt * 4 + i4) * 64] = f32x4{O[vt][4 * i4] * il, O[vt][4 * i4 + 1] * il,
-                                          O[vt][4 * i4 + 2] * il, O[vt][4 * i4 + 3] * il};
-    }
-    __syncthreads();
-    if (mp == 1 || !valid) return;   // both halves of a column are valid together
-    const int ho = g * rep + col % rep;
-    float ss = 0.f;
-#pragma unroll
-    for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const f32x4 o2 = xch[(vt * 4 + i4) * 64];
-#pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float o = O[vt][4 * i4 + j] * il - o2[j];
-          O[vt][4 * i4 + j] = o;
-          ss += o * o;
+          const int t = ks >> 1, i = 8 * (ks & 1) + 2 * j;
+          const f32x2 x{__builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i], scale2, -mt[t / TPM])),
+                        __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i + 1], scale2, -mt[t / TPM]))};
+          wv[j] = __builtin_bit_cast(unsigned int, __builtin_convertvector(x, bf16x2));
+          psum[t / TPM] += __builtin_bit_cast(float, wv[j] << 16) + __builtin_bit_cast(float, wv[j] & 0xffff0000u);
+        }
+        P[ks] = __builtin_bit_cast(bf16x8, wv);
+      }
+      l += psum[0];
+      if (MT > 1) {
+        carry = __builtin_amdgcn_exp2f(mt[0] - m);
+        l = l * carry + psum[MT - 1];
+      }
+    };
+    // One block's scores, the weights of the one before and the value products of the one before that: a product and a
+    // few vector instructions in turn
+    auto quick = [&](auto parted, bool one_max, const __bf16* kr, const __bf16* vr, __bf16* kw, __bf16* vw, int bk, int bv, const f32x16 (&Si)[KT],
+                     f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT], bf16x8 (&Po)[2 * KT]) SF_INLINE {
+      constexpr int NP = 2 * KT * NV, NF = NP + KT * ND, LA = KT == 1 ? 2 : 3;
+      constexpr bool MSUM = KT > 1;   // the weights' sums by products with a half (one tile: the registers are not there)
+      constexpr int NS = NF + (MSUM ? 2 * KT : 0);
+      constexpr int WE = (MSUM ? 56 : 88) * KT, WR = 16 * NV;
+      constexpr int NB = std::min(std::max(NP, NS * WE / (WE + WR)), NS - 4 * KT - 1);   // slots of the exponentials; then O's factors
+      constexpr int SUM0 = NB + 1;                            // the weights' sums: products with a half, every other slot
+      static_assert(!MSUM || SUM0 + 4 * KT <= NS, "room for the sums");
+      // two maxima: the first tile's value products of all channels, a factor, the second tile's
+      constexpr bool PARTED = decltype(parted)::value;
+      constexpr int KP = PARTED ? 2 : 2 * KT;   // value products of a channel tile in a row
+      auto vt_of = [](int n) { return n % (KP * NV) / (2 * KP) * 2 + n % 2; };
+      auto ks_of = [](int n) { return n / (KP * NV) * KP + n % (2 * KP) / 2; };
+      bf16x8 fr[NF];
+      auto frag = [&](int n) SF_INLINE { fr[n] = n < NP ? vf(vr, vt_of(n), ks_of(n)) : kf(kr, (n - NP) % KT, (n - NP) / KT); };
+      const int kpg = bt[min((bk + 16 * sg) >> a.bs_shift, last_page)], vpg = bt[min((bv + 16 * sg) >> a.bs_shift, last_page)];
+#pragma unroll
+      for (int n = 0; n < LA; ++n) frag(n);
+      __builtin_amdgcn_sched_barrier(0);
+      float tm[2 * KT];
+#pragma unroll
+      for (int c = 0; c < 2 * KT; ++c) {
+        tm[c] = kNegBig;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) tm[c] = fmaxf(tm[c], Si[c >> 1][8 * (c & 1) + i]);
+      }
+      float top[2] = {fmaxf(tm[0], tm[1]), fmaxf(tm[2 * KT - 2], tm[2 * KT - 1])};
+      if (!PARTED || one_max) top[0] = fmaxf(top[0], top[1]);
+      const float m0 = fmaxf(both(top[0]) * scale2, m), alpha = __builtin_amdgcn_exp2f(m - m0);
+      const float before = carry;
+      m = m0;
+      if constexpr (PARTED) {
+        m = fmaxf(both(top[1]) * scale2, m0);
+        carry = __builtin_amdgcn_exp2f(m0 - m);
+      }
+      const float mt[2] = {m0, m};
+      l *= alpha;
+      const __bf16 *kb = nullptr, *vb = nullptr;
+      unsigned int wv[8 * KT];
+      f32x16 sums;
+      float ps[2] = {0.f, 0.f};
+      bf16x8 half;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) half[j] = static_cast<__bf16>(0.5f);   // (the lane's and lane ^ 32's l are added at the end)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        sums[i] = 0.f;
+#pragma unroll
+        for (int t = 0; t < KT; ++t) So[t][i] = 0.f;
+      }
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        __builtin_amdgcn_sched_barrier(0);
+        const bool summing = MSUM && n >= SUM0 && n < SUM0 + 4 * KT && (n - SUM0) % 2 == 0;
+        const int f = !MSUM || n < SUM0 ? n : n < SUM0 + 4 * KT ? SUM0 + (n - SUM0) / 2 : n - 2 * KT;   // fragment of this slot
+        if (!summing && f + LA < NF) frag(f + LA);
+        if (summing) {
+          const int ks = (n - SUM0) / 2;
+          if (PARTED && ks == 2) sums[0] *= carry;
+          sums = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              half, __builtin_bit_cast(bf16x8, (u32x4{wv[4 * ks], wv[4 * ks + 1], wv[4 * ks + 2], wv[4 * ks + 3]})), sums, 0, 0, 0);
+          hold(sums);
+        } else if (f < NP) {
+          const int vt = vt_of(f);
+          O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], Pi[ks_of(f)], O[vt], 0, 0, 0);
+          hold(O[vt]);
+        } else {
+          const int t = (f - NP) % KT;
+          So[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], qf[(f - NP) / KT], So[t], 0, 0, 0);
+          hold(So[t]);
+        }
+        if (n == 1) {
+          kb = k_at(__builtin_amdgcn_readfirstlane(kpg), bk);
+          vb = v_at(__builtin_amdgcn_readfirstlane(vpg), bv);
+        }
+        // the next blocks on their way
+        if (n >= 2 && n < 2 + NMAP * KU) send_k(kb, kw, n - 2);
+        if (n >= 2 + NMAP * KU && n < 2 + NMAP * KU + VU) send_v(vb, vw, n - 2 - NMAP * KU);
+        if constexpr (PARTED) {   // O of two channel tiles between their products of the first and of the second tile
+          constexpr int G2 = 2 * KP;
+          if (n >= G2 && n < G2 + KP * NV) {
+            const int pair2 = (n - G2) / G2 * 2, at = (n - G2) % G2;
+#pragma unroll
+            for (int c = 32 * at / G2; c < 32 * (at + 1) / G2; ++c) O[pair2 + c / 16][c % 16] *= before;
+            hold(O[pair2]);
+            hold(O[pair2 + 1]);
+          }
+        }
+        if (n < NB) {
+#pragma unroll
+          for (int u = 8 * KT * n / NB; u < 8 * KT * (n + 1) / NB; ++u) {
+            const int t = u / 8, i = 2 * (u % 8);
+            const float mx = PARTED ? mt[t] : m;
+            const f32x2 x{__builtin_amdgcn_exp2f(__builtin_fmaf(Si[t][i], scale2, -mx)),
+                          __builtin_amdgcn_exp2f(__builtin_fmaf(Si[t][i + 1], scale2, -mx))};
+            wv[u] = __builtin_bit_cast(unsigned int, __builtin_convertvector(x, bf16x2));
+            if constexpr (!MSUM)
+              ps[u % 2] += __builtin_bit_cast(float, wv[u] << 16) + __builtin_bit_cast(float, wv[u] & 0xffff0000u);
+            hold(wv[u]);
+          }
+        } else {
+#pragma unroll
+          for (int c = WR * (n - NB) / (NS - NB); c < WR * (n - NB + 1) / (NS - NB); ++c) {
+            O[c / 16][c % 16] *= alpha;
+            hold(static_cast<float>(O[c / 16][c % 16]));
+          }
         }
       }
-    ss += __shfl_xor(ss, 32, kWave);
-    const float f = a.post / sqrtf(ss / static_cast<float>(DV) + a.eps);
-    const __bf16* gt = a.gate != nullptr ? static_cast<const __bf16*>(a.gate) + row * a.gate_stride +
-                                               static_cast<int64_t>(ho) * DV : nullptr;
-    __bf16* o = static_cast<__bf16*>(out) + (row * (H / 2) + ho) * DV;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int vt = 0; vt < NV; ++vt)
+      for (int ks = 0; ks < 2 * KT; ++ks)
+        Po[ks] = __builtin_bit_cast(bf16x8, (u32x4{wv[4 * ks], wv[4 * ks + 1], wv[4 * ks + 2], wv[4 * ks + 3]}));
+      l = !MSUM ? l + (ps[0] + ps[1]) : PARTED ? l * carry + sums[0] : l + sums[0];
+    };
+
+    // ---- step i: scores of block i, weights of block i - 1, value products of block i - 2; K of block i + 1 and V of
+    // block i - 1 on their way to the other buffers
+    f32x16 S[KT];
+    bf16x8 P[2 * KT];
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int ch = vt * 32 + 8 * i4 + 4 * h;
-        bf16x4 gv4, ev;
-        if (gt != nullptr) gv4 = *reinterpret_cast<const bf16x4*>(gt + ch);
+    for (int t = 0; t < KT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          ev[j] = static_cast<__bf16>(O[vt][4 * i4 + j] * f *
-                                      (gt != nullptr ? sigmoidf_(static_cast<float>(gv4[j])) : 1.0f));
-        *reinterpret_cast<bf16x4*>(o + ch) = ev;
-      }
-    return;
-  }
-  if (!valid) return;
-  const float inv = (l > 0.f ? 1.0f / l : 0.f) * head_gate_of<__bf16>(a, row, head);
-  const int64_t o = (row * H + head) * DV;
+      for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
 #pragma unroll
-  for (int vt = 0; vt < NV; ++vt)
+    for (int ks = 0; ks < 2 * KT; ++ks) P[ks] = bf16x8{};
+    auto kbuf = [&](int i) SF_INLINE { return lds_k + (i & 1) * KB; };
+    auto vbuf = [&](int i) SF_INLINE { return lds_v + (i & 1) * VB; };
+    // steps [quick0, quick1): block i - 1 has no masked key, block i is needed
+    const int above = WIN ? max(edge_lo, low_first) : -1;   // (block i - 2 has a key that the wave sees)
+    const int quick0 = max(nk + 2, nk + ((above + BLK - kbeg) / BLK) + 1);
+    const int quick1 = wave_on ? nk + min(min(nb - nk, (pos_first + 1 - kbeg + BLK) / BLK), (pos_last - kbeg) / BLK + 1) : 0;
+    auto quick_step = [&](auto parted, int i, const f32x16 (&Si)[KT], f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT],
+                          bf16x8 (&Po)[2 * KT]) SF_INLINE {
+      quick(parted, i - 1 >= kSplitBlocks, kbuf(i), vbuf(i), kbuf(i + 1), vbuf(i + 1), kbeg + (i + 1 - nk) * BLK,
+            kbeg + (i - 1 - nk) * BLK, Si, So, Pi, Po);
+      wait_sent();
+      __syncthreads();
+    };
+    auto quick_two = [&](auto parted, int i) SF_INLINE {
+      f32x16 S2[KT];
+      bf16x8 P2[2 * KT];
+      quick_step(parted, i, S, S2, P, P2);
+      quick_step(parted, i + 1, S2, S, P2, P);
+    };
+    for (int i = 0; i < nb; ++i) {
+      if constexpr (MT > 1)
+        for (; i >= quick0 && i + 1 < quick1 && i - 2 < kSplitBlocks; i += 2) quick_two(std::true_type(), i);
+      for (; i >= quick0 && i + 1 < quick1; i += 2) quick_two(std::false_type(), i);
+      if (i == nb) break;
+      if (i + 1 < nb) send_block_k(bt, last_page, block_key(i + 1), kbuf(i + 1));
+      if (i >= 1) send_block_v(block_key(i - 1), vbuf(i + 1));
+      if (MANY && i == 0 && more) send_pages(nxt, lds_bt[(turn & 1) ^ 1]);
+      if (needed(i - 2)) values(vbuf(i), P, i - 2 < kSplitBlocks);
+      if (needed(i - 1)) weights(i - 1, S, P);
+      if (needed(i)) scores(kbuf(i), S);
+      if (i >= 1) put_block_v(block_key(i - 1), vbuf(i + 1));
+      wait_sent();
+      __syncthreads();
+    }
+    // steps nb and nb + 1 have no scores; the next piece's queries and first keys are on their way
+    send_block_v(block_key(nb - 1), vbuf(nb + 1));
+    if (MANY && more) send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), lds_k);
+    if (needed(nb - 2)) values(vbuf(nb), P, nb - 2 < kSplitBlocks);
+    if (MANY) load_q(nxt);
+    if (needed(nb - 1)) weights(nb - 1, S, P);
+    put_block_v(block_key(nb - 1), vbuf(nb + 1));
+    if (MANY) hold_q();
+    wait_sent();
+    __syncthreads();
+    bf16x4 gates[8];   // of the wave's half of the channels
+    if constexpr (NMAP == 2) {
+      if (a.gate != nullptr) {
+        const __bf16* gt = static_cast<const __bf16*>(a.gate) + row * a.gate_stride +
+                           static_cast<int64_t>(g * rep + (valid ? col - tok * rep : 0)) * DV + mp * (DV / 2) + 4 * h;
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int64_t at = o + vt * 32 + 8 * i4 + 4 * h;
-      if (a.out_f32) {
-        f32x4 ev;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ev[j] = O[vt][4 * i4 + j] * inv;
-        *reinterpret_cast<f32x4*>(static_cast<float*>(out) + at) = ev;
-      } else {
-        bf16x4 ev;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ev[j] = static_cast<__bf16>(O[vt][4 * i4 + j] * inv);
-        *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(out) + at) = ev;
+        for (int c = 0; c < 8; ++c) gates[c] = *reinterpret_cast<const bf16x4*>(gt + 8 * c);
       }
     }
+    if (needed(nb - 1)) values(vbuf(nb + 1), P, nb - 1 < kSplitBlocks);
+
+    l += xor32(l, x32);
+    if constexpr (NMAP == 2) {
+      // The two waves of a column set finish half of its channels each: they hand each other lam / l * O of the second
+      // and O / l of the first map through LDS, add up their squares, and exchange the sums.
+      constexpr int HV = NV / 2;
+      static_assert(NMAP == 1 || sizeof(lds_x) >= NW * 64 * 16 * HV * sizeof(float), "room for both halves");
+      const float il = l > 0.f ? (mp == 0 ? 1.0f : a.lam) / l : 0.f;
+      f32x16 own[HV], theirs[HV];
+#pragma unroll
+      for (int hv = 0; hv < HV; ++hv)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          own[hv][i] = mp == 0 ? O[hv][i] : O[HV + hv][i];
+          theirs[hv][i] = mp == 0 ? O[HV + hv][i] : O[hv][i];
+        }
+      f32x4* const give = reinterpret_cast<f32x4*>(lds_x) + w * HV * 4 * 64 + lane;
+      const f32x4* const take = reinterpret_cast<const f32x4*>(lds_x) + (w ^ CW) * HV * 4 * 64 + lane;
+#pragma unroll
+      for (int hv = 0; hv < HV; ++hv)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          give[(hv * 4 + i4) * 64] = f32x4{theirs[hv][4 * i4] * il, theirs[hv][4 * i4 + 1] * il, theirs[hv][4 * i4 + 2] * il,
+                                           theirs[hv][4 * i4 + 3] * il};
+      __syncthreads();
+      float ss = 0.f;
+#pragma unroll
+      for (int hv = 0; hv < HV; ++hv)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const f32x4 o2 = take[(hv * 4 + i4) * 64];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float mine = own[hv][4 * i4 + j] * il, o = mp == 0 ? mine - o2[j] : o2[j] - mine;
+            own[hv][4 * i4 + j] = o;
+            ss += o * o;
+          }
+        }
+      ss += xor32(ss, x32);
+      if (h == 0) lds_ss[w][r] = ss;
+      __syncthreads();
+      ss += lds_ss[w ^ CW][r];
+      const float f = a.post / sqrtf(ss / static_cast<float>(DV) + a.eps);
+      const int ln = fresh(lane), er = ln & 31, eh = ln >> 5, el = ln >> 3, ec = ln & 7;
+      char* x = lds_x + w * 4096;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const f32x16& o = own[c / 4];
+        const int i = c % 4 * 4;
+        f32x4 e{o[i] * f, o[i + 1] * f, o[i + 2] * f, o[i + 3] * f};
+        if (a.gate != nullptr) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) e[j] *= sigmoidf_(static_cast<float>(gates[c][j]));
+        }
+        const u32x2 b{__builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2{e[0], e[1]}), bf16x2)),
+                      __builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2{e[2], e[3]}), bf16x2))};
+        *reinterpret_cast<u32x2*>(x + er * 128 + ((c ^ ((er >> 1) & 7)) * 16) + 8 * eh) = b;
+      }
+      __builtin_amdgcn_wave_barrier();
+      __bf16* ob = static_cast<__bf16*>(out) + (static_cast<int64_t>(row0 + qo) * (H / 2) + g * rep) * DV + 64 * mp + 8 * ec;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int rr = 8 * j + el, cc = wcol + rr;
+        const u32x4 e = *reinterpret_cast<const u32x4*>(x + rr * 128 + ((ec ^ ((rr >> 1) & 7)) * 16));
+        if (cc < cols_total)
+          *reinterpret_cast<u32x4*>(ob + (static_cast<int64_t>(token_of(cc)) * (H / 2 - rep) + cc) * DV) = e;
+      }
+    } else {
+      const float inv = valid && l > 0.f ? head_gate_of<__bf16>(a, row, head) / l : 0.f;
+      if (MANY) __syncthreads();
+      if (a.out_f32) {
+        if (valid) {
+          float* o = static_cast<float*>(out) + (row * H + head) * DV + 4 * h;
+#pragma unroll
+          for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4)
+              *reinterpret_cast<f32x4*>(o + vt * 32 + 8 * i4) =
+                  f32x4{O[vt][4 * i4] * inv, O[vt][4 * i4 + 1] * inv, O[vt][4 * i4 + 2] * inv, O[vt][4 * i4 + 3] * inv};
+        }
+      } else {
+        // 64 channels at a time through LDS, the wave's own 4 KB (32 rows of 128 bytes, chunks changing places), so that
+        // a store has whole rows: 8-byte pieces of 32 rows kept the memory pipe busy for 2 us per piece of work.  (What
+        // depends on the lane is worked out here: kept over a piece it was spilled, and its reload waited for the stores.)
+        const int ln = fresh(lane), er = ln & 31, eh = ln >> 5, el = ln >> 3, ec = ln & 7;
+        char* x = (MANY ? lds_x : reinterpret_cast<char*>(lds_k)) + w * 4096;
+        __bf16* ob = static_cast<__bf16*>(out) + (static_cast<int64_t>(row0 + qo) * H + g * rep) * DV + 8 * ec;
+#pragma unroll
+        for (int v2 = 0; v2 < NV / 2; ++v2) {
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            const int vt = 2 * v2 + c / 4, i = c % 4 * 4;
+            const u32x2 e{__builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2{O[vt][i] * inv, O[vt][i + 1] * inv}), bf16x2)),
+                          __builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2{O[vt][i + 2] * inv, O[vt][i + 3] * inv}), bf16x2))};
+            *reinterpret_cast<u32x2*>(x + er * 128 + ((c ^ ((er >> 1) & 7)) * 16) + 8 * eh) = e;
+          }
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int rr = 8 * j + el, cc = wcol + rr;
+            const u32x4 e = *reinterpret_cast<const u32x4*>(x + rr * 128 + ((ec ^ ((rr >> 1) & 7)) * 16));
+            const int t = token_of(cc);
+            if (cc < cols_total)
+              *reinterpret_cast<u32x4*>(ob + (static_cast<int64_t>(t) * (H - rep) + cc) * DV + 64 * v2) = e;
+          }
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
+    }
+    if (!MANY || !more) return;
+    now = nxt;
+  }
 }
 
-template <int ND, int NV, int NMAP, int NW, int WPS>
+template <int ND, int NV, int NMAP, int NW, int KT>
 bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, const AttnArgs& a,
-            int num_tiles, hipStream_t st) {
+            int num_tiles, int cus, hipStream_t st) {
   constexpr int COLS = NW / NMAP * 32;
-  const int chunks = (kTileTokens * (a.H / a.G) + COLS - 1) / COLS;
-  const unsigned grid = static_cast<unsigned>(num_tiles) * (a.G / NMAP) * chunks;
-  auto* kernel = a.window > 0 ? sink_flash_kernel<ND, NV, NMAP, NW, WPS, true>
-                              : sink_flash_kernel<ND, NV, NMAP, NW, WPS, false>;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NW * 64), 0, st, out, static_cast<const __bf16*>(q),
-                     static_cast<const __bf16*>(k_cache), static_cast<const __bf16*>(v_cache), a,
-                     num_tiles, chunks);
+  const int chunks = (kTileTokens * (a.H / a.G) + COLS - 1) / COLS, heads = a.G / NMAP;
+  const int pieces = num_tiles * chunks;
+  const int workers = NW == 8 ? std::min(pieces, std::max({1, cus / heads, (pieces + kPieces - 1) / kPieces})) : pieces;
+  auto* kernel = a.window > 0 ? sink_flash_kernel<ND, NV, NMAP, NW, KT, true> : sink_flash_kernel<ND, NV, NMAP, NW, KT, false>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(workers) * heads), dim3(NW * 64), 0, st, out,
+                     static_cast<const __bf16*>(q), static_cast<const __bf16*>(k_cache),
+                     static_cast<const __bf16*>(v_cache), a, num_tiles, chunks, workers);
   return true;
 }
 
 }  // namespace sf
 
 // The shapes of the served families (head width 128, the latent cache of 192 + 64 channels, narrow heads,
-// two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two)
-// and contexts past the LDS page list run sink_attention.hip's kernel.  Measured at 4 prompts of ~1850
-// tokens (us, old kernel -> this one; variants at the same shapes):
-//   128 / 128, 32 heads over 8:  463 -> 159 (8 waves per workgroup: +1 %; 64 columns per wave: +30 %)
-//   256 / 192, 32 heads over 1: 1052 -> 261 (4 waves +50 %: one wave per SIMD hides no latency)
-//   two maps 64 / 128, 8 over 2, 5 x 1165 tokens, window 1024: 126 -> 72 (both maps in each of 4 waves
-//     +45 %: few workgroups there, so a wave's own chain counts; 2 waves per SIMD +10 %, 4 spill)
-// The workgroups of the 256 / 192 form hold 8 tokens (the old kernel's 4): so far ahead a NaN value reaches back (a weight
-// of 0 times NaN), as it did there.
+// two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two), caches or results
+// that are not 16-byte aligned and contexts past the LDS page list run sink_attention.hip's kernel.
+//
+// Four or eight waves: pieces of 128 columns up to 6 per CU, and tiles that do not fill eight waves (24 over 8 heads: 192
+// of 256 columns), go four by four.  us, whole layer, before / four waves / eight: 32 + 8 heads, 256 pieces (2 x 500) 34.5 /
+// 30.1 / 37.1; 768 (6 x 500) 58.1 / 54.3 / 56.1; 1220 (5 x 1000) 95.2 / 82.3 / 87.8; 1904 (4 x 2048) 198.1 / 182.7 / 180.0;
+// 24 + 8 heads 624 (3 x 777) 47.8 / 42.3 / 47.9, 1400 (2 x 3000) 177.7 / 146.0 / 157.4.  The latent form keeps 32 keys per
+// block: 64 scores and weights more than fill its registers (O and Q are 160).
+// The workgroups of the latent form hold 8 tokens: so far ahead a NaN value reaches back (a weight of 0 times NaN).
 bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void* v_cache,
                        const AttnArgs& a, int num_tiles, hipStream_t st) {
-  if (a.block_size < 16 || a.bt_width > sf::kPages || !(a.scale > 0.f)) return false;
-#define SF(D, V, MAPS, NW, WPS)                              \
+  if (a.block_size < 16 || a.bt_width > sf::kPages || !(a.scale > 0.f) ||
+      (reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(out)) % 16)
+    return false;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return false;
+  const int columns = kTileTokens * (a.H / a.G);
+  const bool few = columns % 256 != 0 || static_cast<int64_t>(num_tiles) * ((columns + 127) / 128) * a.G <= 6 * cus;
+#define SF(D, V, MAPS, NW, KT)                              \
   if (a.dim == D && a.vdim == V && (a.pair ? 2 : 1) == MAPS) \
-    return sf::launch<D / 16, V / 32, MAPS, NW, WPS>(out, q, k_cache, v_cache, a, num_tiles, st);
-  SF(64, 64, 1, 4, 2)
-  SF(128, 128, 1, 4, 2)
-  SF(256, 192, 1, 8, 2)
-  SF(64, 128, 2, 8, 3)
+    return sf::launch<D / 16, V / 32, MAPS, NW, KT>(out, q, k_cache, v_cache, a, num_tiles, cus, st);
+  if (few) {
+    SF(64, 64, 1, 4, 2)
+    SF(128, 128, 1, 4, 2)
+  }
+  SF(64, 64, 1, 8, 2)
+  SF(128, 128, 1, 8, 2)
+  SF(256, 192, 1, 8, 1)
+  SF(64, 128, 2, 8, 2)
 #undef SF
   return false;
 }

@@ -1124,6 +1124,41 @@ def test_two_maps_largest_weights_exact():
     assert float(err.pow(2).mean().sqrt()) < 4e-4
 
 
+@pytest.mark.parametrize("H,G,d,dv,S", [(32, 8, 128, 128, 90), (16, 4, 64, 64, 140), (5, 1, 256, 192, 170),
+                                        (8, 4, 64, 128, 170), (32, 32, 64, 128, 1100), (3, 1, 256, 192, 1100)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 5)])
+def test_flash_many_pieces(H, G, d, dv, S, window, keep):
+    """More tiles than a launch has workgroups: each takes several in turn, long and short ones, sorted up to 1024 of them;
+    more than 64 per workgroup and head; tiles past a portion's end; fp32 results (of the form without two maps)."""
+    rng = np.random.default_rng(S + window)
+    many = S > 1000
+    lens = rng.choice([1, 2, 5], S).tolist() if many else rng.choice([3, 64, 65, 100, 129, 200], S).tolist()
+    starts = rng.choice([0, 1, 40], S).tolist() if many else rng.choice([0, 0, 17, 63, 300], S).tolist()
+    md = ragged(lens, starts, list(range(S)), width=40)
+    for name, extra in (("tile_seq", [0, S - 1]), ("tile_qoff", [512, 512])):
+        md[name] = torch.cat([md[name], torch.tensor(extra, dtype=torch.int32)])
+    T, nb, pair = int(md["seq_qstart"][-1]), md["num_pages"], (d, dv) == (64, 128)
+    gen = torch.Generator().manual_seed(S)
+    q = torch.randn(T, H, d, generator=gen).to(torch.bfloat16)
+    k = torch.randn(nb, G, 16, d, generator=gen).to(torch.bfloat16)
+    v = torch.randn(nb, G // 2 if pair else G, dv, 16, generator=gen).to(torch.bfloat16)
+    gate = torch.randn(T, H // 2 * dv, generator=gen).to(torch.bfloat16)
+
+    def run(m, *t, **more):
+        q, k, v, gate = t
+        args = (q, k, v, m["block_tables"], m["seq_kvlen"], m["seq_qstart"], m["tile_seq"], m["tile_qoff"])
+        if pair:
+            return mx.differential_attention(*args, d ** -0.5, 0.4, 0.3, 1e-5, gate, 0, 0, window, keep)
+        return mx.sink_attention(*args, 0.2, True, window=window, keep_first=keep, **more)
+
+    want, g = run(md, q, k, v, gate), cuda(md)
+    dev = [t.cuda() for t in (q, k, v, gate)]
+    # as the edges' tests
+    for more in ({}, {} if pair else {"out_dtype": torch.float32}):
+        got = run(g, *dev, **more)
+        assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
+
+
 @pytest.mark.parametrize("bs", [64, 128, 512])
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 70)])
 def test_flash_attention_wide_pages(window, keep, bs):
