@@ -10,21 +10,21 @@
 // columns 32w..32w+31 (column c: token c / G, head c % G).  Every K/V tile is staged ONCE in
 // LDS per workgroup and read by all 128 columns (G x the reuse of a per-head kernel).
 //
-// Per 32-key block, per wave (cdna_hip_programming.md §3 "swapped QK^T"):
+// Per 64-key block (two 32-key sub-tiles), per wave ("swapped QK^T"):
 //   S^T[32 keys x 32 cols] = K[32 x 128] . Q^T[128 x 32]       8 x mfma_f32_32x32x16
-//     A = K rows from LDS (16 B reads, rows padded to 272 B: conflict-free), B = Q (registers);
-//     the accumulator has the column on the lane, so the online-softmax row statistics are
-//     lane-local over 16 registers plus one xor-32 exchange;
+//     A = K rows from LDS, B = Q (registers); the accumulator has the column on the lane, so the online-softmax row
+//     statistics are lane-local over 16 registers plus one xor-32 exchange;
 //   O^T[128 x 32] += V^T[128 x 32 keys] . P^T[32 keys x 32]    8 x mfma_f32_32x32x16
-//     B = P^T straight from the S^T accumulator registers (pairs packed to 16 bit; the k order
-//     inside a step is permuted, and the V^T A-operand reads follow the same permutation),
-//     A = V^T rows from LDS (one 16 B read per fragment from a key-permuted, padded image).
-// 64-key blocks (two 32-key sub-tiles).  O^T is rescaled only when a running max grew by more
-// than 2^8 (defer-max).
-// Pipelining: the next block's K/V are loaded global -> registers while the current block
-// computes, then written to the other LDS buffer; one workgroup barrier per block.  The
-// sequence's block-table slice is staged in LDS once so K/V addresses need no dependent
-// global load inside the loop.  Causal masking touches only the diagonal blocks.
+//     B = P^T straight from the S^T accumulator registers (pairs packed to 16 bit), A = V^T rows from LDS.
+// O^T is rescaled only when a running max grew by more than 2^8 (defer-max).
+// Pipelining: step i takes the scores of block i, the weights of block i - 1 and the value products of block i - 2, which
+// do not depend on each other, and deals them out by hand (`quick`): a product (32 cycles of the matrix core), then the
+// vector instructions that fit behind it.  Left to the compiler, products and softmax ran one after the other in every
+// wave.  Blocks on the diagonal and both ends go part by part.  K and V of the next blocks go straight from memory to LDS in
+// the meantime: no registers, one wait and one workgroup barrier per block.  The sequence's block-table slice is staged in
+// LDS once so K/V addresses need no dependent global load inside the loop.
+// Layer times, us, before -> now: 32 + 8 heads 4 x 2k tokens 176.0 -> 167.1 (37.6 of it the rotation), 1 x 2000 70.1 -> 59.8,
+// 16 x 500 92.3 -> 86.9; 24 + 8 heads 3 x 777 41.7 -> 39.7.  Bound: matrix and vector units together, at a clock that gives way.
 #include "common.h"
 #include "kernels.h"
 
@@ -34,22 +34,18 @@ namespace fp {
 constexpr int kD = 128;
 constexpr int kNS = 2;                   // 32-key sub-tiles per block
 constexpr int kKB = 32 * kNS;            // keys per block
-constexpr int kKStride = kD + 8;         // K tile row: 272 B (16 B reads conflict-free)
-// V^T tile row: 144 B (16-B aligned rows; 36-dword stride: the PV operand's ds_read_b128 and
-// the staging ds_write_b64 pairs are bank-conflict-free).  Inside every 16-key group the keys
-// are stored permuted - key 8 a + 4 h + b at column 8 h + 4 a + b - so the 8 keys one lane
-// needs for a PV fragment (keys 4 h .. 4 h + 3 and 8 + 4 h .. 8 + 4 h + 3, the order of the P^T
-// registers) are one contiguous 16 B read: one ds_read_b128 (4 LDS cycles) instead of a
-// ds_read2_b64 (8).
-constexpr int kVStride = kKB + 8;
-constexpr int kKTile = kKB * kKStride;   // elements
-constexpr int kVTile = kD * kVStride;
+// LDS images: K rows as they are (256 B), V as [16-key group][channel][16 keys]; the 16-byte chunks of a K row and the
+// halves of a V row change places (row & 15, channel bit 3) so that the fragments' ds_read_b128 have no bank conflicts.
+constexpr int kKTile = kKB * kD;         // elements
+constexpr int kVTile = kD * kKB;
 constexpr int kBtLds = 2048;             // block-table entries staged in LDS
 constexpr float kNegInf = -__builtin_huge_valf();
 constexpr float kRescale = 8.f;  // defer-max threshold (log2 units)
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+typedef __attribute__((address_space(3))) void* lds_ptr;
+#define FP_INLINE __attribute__((always_inline))
 
 template <typename T>
 struct Mf32;
@@ -89,6 +85,8 @@ struct FlashParams {
   int split_blocks;  // key blocks per split at least (atta_set_flash_split_blocks)
   float* part;    // [tile, Hkv, nsplit] slots of kPartBytes
   int* counters;  // [tile * Hkv], zero between launches (the last arriver re-arms)
+  int wide_out;   // rows of out start on 16-byte borders
+  int wide_in;    // the caches do: otherwise they go through registers, block by block
 };
 // one split's partial: 128 columns x 128 fp32 O values, then 128 (m, l) pairs
 constexpr uint32_t kPartOBytes = 128 * kD * 4;
@@ -110,23 +108,48 @@ __device__ __forceinline__ uint32_t pack2<__bf16>(float a, float b) {
 }
 
 // lane l <-> lane l ^ 32 exchange: one ds_bpermute with the byte index hoisted out of the loop
-// (__shfl_xor recomputed it per call: 7 VALU).  Not v_permlane32_swap: with both operands the
-// same value the compiler folded its two results into one (sum -> 2 * r0), a wrong softmax sum.
+// (__shfl_xor recomputed it per call: 7 VALU).
 __device__ __forceinline__ float xor32(float v, int idx4) {
   return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(idx4, __builtin_bit_cast(int, v)));
 }
+// larger value of the lane's and lane ^ 32's, without a trip through LDS.  (As an instruction: with both operands the same
+// value the compiler folded the builtin's two results into one.)
+__device__ __forceinline__ float both_max(float v) {
+  float a = v, b = v;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+#endif
+  return fmaxf(a, b);
+}
+// 16 bytes per lane from base + offset to 1 KB of LDS, without registers; there after wait_sent().  (After the builtin the
+// compiler makes every read of LDS wait for all transfers.)
+__device__ __forceinline__ void send16(const void* base, uint32_t offset, void* to) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(at) : "m0", "memory");
+#endif
+}
+__device__ __forceinline__ void wait_sent() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+}
+// the value is there at this point of the program
+template <typename X>
+__device__ __forceinline__ void hold(const X& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" ::"v"(x));
+#endif
+}
 
-// NW = 4: every wave stages 16 keys of both K and V; NW = 8 (two workgroup halves): waves
-// 0-3 stage K, waves 4-7 stage V, so each staged K/V block serves 256 columns and a wave issues
-// half the staging instructions.
+// NW = 8 (two workgroup halves): each staged K/V block serves 256 columns and a wave sends half as much.
 template <typename T, int G, int NW>
-__global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashParams p) {
+__global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p) {
   using MF = Mf32<T>;
   using frag = typename MF::frag;
   constexpr int kTokPerWave = 32 / G;
   constexpr int kTokPerWg = NW * kTokPerWave;
-  __shared__ __attribute__((aligned(16))) uint16_t lds_k[2][kKTile];
-  __shared__ __attribute__((aligned(16))) uint16_t lds_v[2][kVTile];
+  __shared__ __attribute__((aligned(1024))) uint16_t lds_k[2 * kKTile], lds_v[2 * kVTile];
   __shared__ int lds_bt[kBtLds];
 
   const int tid = threadIdx.x;
@@ -190,86 +213,79 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
   }
   __syncthreads();  // lds_bt ready
 
-  // ---- global -> register staging of one K/V block --------------------------------------
-  // Wave w stages keys 16 w .. 16 w + 15 of the block for BOTH tensors: with BS >= 16 those
-  // keys sit in one page, so the page lookup and the keys' place in the page are wave-uniform
-  // (one LDS read + readfirstlane, a scalar base) and every lane offset is a loop constant - the
-  // per-lane 64-bit address arithmetic of 8 independent lookups was ~70 VALU per block and wave.
-  //   K: lane l, chunk u -> key row 16 w + 4 u + (l >> 4), dims 8 (l & 15): each
-  //      instruction reads 4 contiguous 256 B rows (1 KiB);
-  //   V: lane l, chunk u -> d-row 32 u + (l >> 1), keys 16 w + 8 (l & 1) .. + 7: each
-  //      instruction reads 32 d-rows x 16 keys (1 KiB contiguous at BS = 16).
-  constexpr int kChunks = kKB * 16 / 256;   // per thread, per tensor
-  static_assert(kKB == 64 && kChunks == 4, "wave w stages keys 16 w .. 16 w + 15");
-  const int pshift = p.bs_shift + 7;        // log2(BS * kD) elements per (page, head)
+#pragma unroll
+  for (int st = 0; st < 8; ++st) hold(qf[st]);   // (there before the loop, which would wait for its transfers with them)
+
+  // ---- staging of one K/V block: memory -> LDS, past the registers ----------------------
+  // A wave sends keys of ONE 16-key group for both tensors: with BS >= 16 they sit in one page, so the page lookup and
+  // the keys' place in the page are wave-uniform (one LDS read + readfirstlane, a scalar base) and every lane offset is a
+  // constant.  A transfer is 1 KiB of contiguous memory: 4 K rows, or 32 channels x 16 keys (at BS = 16).
+  // Keys past the workgroup's range (>= wg_end) read a clamped page or the unused tail slots of the last page - stale
+  // bytes of whatever sequence held that page before.  Their scores are masked (P = 0), and their V^T columns are zeroed:
+  // that block's V goes through registers (put_v), so that a non-finite stale value cannot turn 0 * V into NaN.
+  constexpr int WPG = NW / 4, U = 4 / WPG;   // waves per group, transfers per wave and tensor
+  const int sg = wid & 3, part = wid >> 2;
   const int last_page = npages - 1;
-  // staging key group of this wave (16 keys) and which tensors it stages
-  const int sg = NW == 8 ? (wid & 3) : wid;
-  constexpr bool kBoth = NW == 4;
-  const bool stage_k = kBoth || wid < 4;
-  const bool stage_v = kBoth || wid >= 4;
-  const int k_lane = (lane >> 4) * kD + 8 * (lane & 15);
-  const int v_lane = (lane >> 1) * BS + 8 * (lane & 1);
-  const int k_lds = (16 * sg + (lane >> 4)) * kKStride + 8 * (lane & 15);
-  const int v_lds = (lane >> 1) * kVStride + 16 * sg + 4 * (lane & 1);  // permuted: see kVStride
-  // LDS only (the launcher rejects bt_stride > kBtLds): a select between the LDS copy and the
-  // global table compiled to FLAT loads, whose vmcnt wait put a dependent global round trip
-  // in front of every block's K/V loads.  Keys past the workgroup's range (>= wg_end) read a
-  // clamped page or the unused tail slots of the last page - stale bytes of whatever sequence
-  // held that page before.  Their scores are masked (P = 0), and their V^T columns are zeroed
-  // at staging (store_block), so a non-finite stale value cannot turn 0 * V into NaN
-  // (no invariant on the cache contents is needed).
-  u32x4 kr[kBoth ? kChunks : 1], vr[kChunks];  // NW = 8: one register set (vr) per wave
-  auto load_block = [&](int kb) {
-    const int key = kb * kKB + 16 * sg, at = key & (BS - 1);   // (a page may hold several blocks)
-    const int pi = min(key >> p.bs_shift, last_page);
-    const int pg = __builtin_amdgcn_readfirstlane(lds_bt[pi]);
-    const uint64_t off = static_cast<uint64_t>(static_cast<uint32_t>(pg * p.n_kv_heads + hk)) << pshift;
-    const uint16_t* kb_ = p.k_cache + off + at * kD;
-    const uint16_t* vb_ = p.v_cache + off + at;
-    if constexpr (kBoth) {
+  uint32_t k_src[U], v_src[U];   // bytes
+  const int v_half = 8 * ((lane ^ (lane >> 4)) & 1);
 #pragma unroll
-      for (int u = 0; u < kChunks; ++u)
-        kr[u] = *reinterpret_cast<const u32x4*>(kb_ + k_lane + u * 4 * kD);
+  for (int u = 0; u < U; ++u) {
+    const int row = 4 * (u * WPG + part) + (lane >> 4);
+    k_src[u] = 2u * (row * kD + ((lane & 15) ^ row) * 8);
+    v_src[u] = 2u * ((32 * (u * WPG + part) + (lane >> 1)) * BS + v_half);
+  }
+  const int k_lds = 16 * sg * kD + part * 512, v_lds = sg * kD * 16 + part * 512;
+  const uint16_t* k_base = p.k_cache + (static_cast<uint64_t>(hk) << (p.bs_shift + 7));
+  const uint16_t* v_base = p.v_cache + (static_cast<uint64_t>(hk) << (p.bs_shift + 7));
+  const uint32_t page = static_cast<uint32_t>(p.n_kv_heads) << (p.bs_shift + 7);   // elements of a page, all heads
+  auto page_at = [&](int k0) FP_INLINE { return lds_bt[min((k0 + 16 * sg) >> p.bs_shift, last_page)]; };
+  auto k_at = [&](int pg, int k0) FP_INLINE {
+    return k_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * page + ((k0 + 16 * sg) & (BS - 1)) * kD;
+  };
+  auto v_at = [&](int pg, int k0) FP_INLINE {
+    return v_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * page + ((k0 + 16 * sg) & (BS - 1));
+  };
+  auto send_k = [&](const uint16_t* kb, uint16_t* to, int u) FP_INLINE { send16(kb, k_src[u], to + k_lds + u * WPG * 512); };
+  auto send_v = [&](const uint16_t* vb, uint16_t* to, int u) FP_INLINE { send16(vb, v_src[u], to + v_lds + u * WPG * 512); };
+  u32x4 vr[U];
+  auto send_block_k = [&](int k0, uint16_t* to) FP_INLINE {
+    const uint16_t* kb = k_at(__builtin_amdgcn_readfirstlane(page_at(k0)), k0);
 #pragma unroll
-      for (int u = 0; u < kChunks; ++u)
-        vr[u] = *reinterpret_cast<const u32x4*>(vb_ + v_lane + u * 32 * BS);
-    } else {
-      // wave-uniform choice of tensor; the same registers carry K rows or V rows
-#pragma unroll
-      for (int u = 0; u < kChunks; ++u)
-        vr[u] = stage_k ? *reinterpret_cast<const u32x4*>(kb_ + k_lane + u * 4 * kD)
-                        : *reinterpret_cast<const u32x4*>(vb_ + v_lane + u * 32 * BS);
+    for (int u = 0; u < U; ++u) {
+      if (p.wide_in) send_k(kb, to, u);
+      else *reinterpret_cast<u32x4*>(to + k_lds + u * WPG * 512 + lane * 8) =
+               *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(kb) + k_src[u]);
     }
   };
-  auto store_block = [&](int buf, int kb) {
-    if (stage_k) {
+  auto send_block_v = [&](int k0, uint16_t* to) FP_INLINE {
+    const uint16_t* vb = v_at(__builtin_amdgcn_readfirstlane(page_at(k0)), k0);
 #pragma unroll
-      for (int u = 0; u < kChunks; ++u)
-        *reinterpret_cast<u32x4*>(&lds_k[buf][k_lds + u * 4 * kKStride]) =
-            kBoth ? kr[kBoth ? u : 0] : vr[u];
+    for (int u = 0; u < U; ++u) {
+      if (p.wide_in && k0 + kKB <= wg_end) send_v(vb, to, u);
+      else vr[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb) + v_src[u]);
     }
-    if (!stage_v) return;
-    // this lane's 8 V keys: kb * kKB + 16 sg + 8 (lane & 1) + j; only the last block can
-    // reach past wg_end (uniform per workgroup except at that edge)
-    const int vkey = kb * kKB + 16 * sg + 8 * (lane & 1);
-    if (vkey + 8 > wg_end) {
+  };
+  auto put_v = [&](int k0, uint16_t* to) FP_INLINE {
+    if (p.wide_in && k0 + kKB <= wg_end) return;
+    const int key = k0 + 16 * sg + v_half;
 #pragma unroll
-      for (int u = 0; u < kChunks; ++u)
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const unsigned lo = vkey + 2 * j < wg_end ? 0x0000ffffu : 0u;
-          const unsigned hi = vkey + 2 * j + 1 < wg_end ? 0xffff0000u : 0u;
-          vr[u][j] &= (lo | hi);
-        }
+      for (int j = 0; j < 4; ++j)
+        vr[u][j] &= (key + 2 * j < wg_end ? 0x0000ffffu : 0u) | (key + 2 * j + 1 < wg_end ? 0xffff0000u : 0u);
+      *reinterpret_cast<u32x4*>(to + v_lds + u * WPG * 512 + lane * 8) = vr[u];
     }
+  };
+  // ---- fragments.  A row of the score products: key with bits 2 and 3 swapped, so that register i of a tile holds key
+  // 16 (i >> 3) + 8 h + (i & 7) and a V^T fragment is one plain 16-byte read
+  const int krow = (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);
+  int kofs[8];
 #pragma unroll
-    for (int u = 0; u < kChunks; ++u) {
-      // keys 8 g .. 8 g + 3 -> columns 4 g .., keys 8 g + 4 .. 8 g + 7 -> columns 8 + 4 g ..
-      uint16_t* dst = &lds_v[buf][v_lds + u * 32 * kVStride];
-      reinterpret_cast<u32x2*>(dst)[0] = u32x2{vr[u][0], vr[u][1]};
-      reinterpret_cast<u32x2*>(dst + 8)[0] = u32x2{vr[u][2], vr[u][3]};
-    }
+  for (int st = 0; st < 8; ++st) kofs[st] = krow * kD + ((2 * st + h) ^ (krow & 15)) * 8;
+  const int vofs = r * 16 + 8 * (h ^ ((r >> 3) & 1));
+  auto kf = [&](const uint16_t* b, int t, int st) FP_INLINE { return *reinterpret_cast<const frag*>(b + 32 * t * kD + kofs[st]); };
+  auto vf = [&](const uint16_t* b, int dt, int ks) FP_INLINE {
+    return *reinterpret_cast<const frag*>(b + vofs + ks * kD * 16 + dt * 512);
   };
 
   f32x16 o[4];
@@ -277,129 +293,176 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
-  float m_run = kNegInf, l_run = 0.f;
+  float m_run = kNegInf, l_run = 0.f;   // l_run: of the lane's keys
 
-  if (kb0 < kb1) {
-    load_block(kb0);
-    store_block(0, kb0);
+  // defer-max: the running max m_run moves only when some column's max grew by more than kRescale (log2 units), so
+  // P = 2^(s - m_run) stays <= 2^kRescale; O and l are rescaled only then - with the max nearly settled after the first
+  // block, the multiplies of the rescale were paid on most blocks.  O, l and P of a block always use the same m_run, so
+  // the result is exact up to rounding.  Answers the factor of the columns that moved.
+  auto raise = [&](const f32x16 (&S)[kNS], float& alpha) FP_INLINE {
+    float tm[4];   // running max on the raw scores (scale > 0)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      tm[c] = kNegInf;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) tm[c] = fmaxf(tm[c], S[c >> 1][8 * (c & 1) + i]);
+    }
+    const float m_cand = fmaxf(m_run, both_max(fmaxf(fmaxf(tm[0], tm[1]), fmaxf(tm[2], tm[3]))) * p.scale_log2);
+    const bool grow = m_cand > m_run + kRescale;  // m_run == -inf: any finite m_cand
+    const float m_new = grow ? m_cand : m_run;
+    alpha = __builtin_amdgcn_exp2f(m_run - ((m_new == kNegInf) ? 0.f : m_new));
+    if (!grow) alpha = 1.f;
+    m_run = m_new;
+    return grow;
+  };
+  auto rescale = [&](float alpha) FP_INLINE {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+  };
+  // softmax in the log2 domain with the scale folded into one fma per element: p = 2^(s * scale_log2 - m); weights 2 u
+  // and 2 u + 1 of the block, and their place in the row sum's two chains
+  auto weight2 = [&](const f32x16 (&S)[kNS], int u, float neg_m, float& s0, float& s1) FP_INLINE {
+    const int t = u / 8, i = 2 * (u % 8);
+    const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i], p.scale_log2, neg_m));
+    const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][i + 1], p.scale_log2, neg_m));
+    s0 += x;
+    s1 += y;
+    return pack2<T>(x, y);
+  };
+  auto scores = [&](const uint16_t* kl, f32x16 (&S)[kNS]) FP_INLINE {
+#pragma unroll
+    for (int t = 0; t < kNS; ++t) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
+#pragma unroll
+      for (int st = 0; st < 8; ++st) S[t] = MF::mma(kf(kl, t, st), qf[st], S[t]);
+    }
+  };
+  auto values = [&](const uint16_t* vl, const u32x4 (&P)[4]) FP_INLINE {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) o[dt] = MF::mma(vf(vl, dt, ks), __builtin_bit_cast(frag, P[ks]), o[dt]);
+  };
+  auto weights = [&](int k0, f32x16 (&S)[kNS], u32x4 (&P)[4]) FP_INLINE {
+    // mask: only blocks crossing the diagonal of the wave's first token (wave-uniform branch)
+    if (k0 + kKB > ctx0 + w_first + 1) {
+      const int lim = c_end - k0 - 8 * h;
+#pragma unroll
+      for (int t = 0; t < kNS; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (32 * t + 16 * (i >> 3) + (i & 7) >= lim) S[t][i] = kNegInf;
+    }
+    float alpha, s0 = 0.f, s1 = 0.f;
+    if (__any(raise(S, alpha))) {
+      l_run *= alpha;
+      rescale(alpha);
+    }
+    const float neg_m = m_run == kNegInf ? 0.f : -m_run;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) P[u / 4][u % 4] = weight2(S, u, neg_m, s0, s1);
+    l_run += s0 + s1;
+  };
+  // One block's scores, the weights of the one before and the value products of the one before that: a product (32 cycles of
+  // the matrix core), then the vector instructions that fit behind it.  The same sums in the same order as the parts above.
+  auto quick = [&](const uint16_t* kl, const uint16_t* vl, uint16_t* kw, uint16_t* vw, int bk, int bv, const f32x16 (&Si)[kNS],
+                   f32x16 (&So)[kNS], const u32x4 (&Pi)[4], u32x4 (&Po)[4]) FP_INLINE {
+    constexpr int NP = 16, NF = 32, LA = 3, NB = 30;   // NB: slots of the exponentials
+    frag fr[NF];
+    auto read = [&](int n) FP_INLINE { fr[n] = n < NP ? vf(vl, n / 8 * 2 + n % 2, n % 8 / 2) : kf(kl, n % 2, (n - NP) / 2); };
+    const int kpg = page_at(bk), vpg = page_at(bv);
+#pragma unroll
+    for (int n = 0; n < LA; ++n) read(n);
+    __builtin_amdgcn_sched_barrier(0);
+    float alpha, s0 = 0.f, s1 = 0.f;
+    const bool grow = raise(Si, alpha);
+    const float neg_m = m_run == kNegInf ? 0.f : -m_run;
+    const uint16_t *kb = nullptr, *vb = nullptr;
+#pragma unroll
+    for (int t = 0; t < kNS; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) So[t][i] = 0.f;
+#pragma unroll
+    for (int n = 0; n < NF; ++n) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (n + LA < NF) read(n + LA);
+      if (n < NP) {
+        const int dt = n / 8 * 2 + n % 2;
+        o[dt] = MF::mma(fr[n], __builtin_bit_cast(frag, Pi[n % 8 / 2]), o[dt]);
+        hold(o[dt]);
+      } else {
+        So[n % 2] = MF::mma(fr[n], qf[(n - NP) / 2], So[n % 2]);
+        hold(So[n % 2]);
+      }
+      if (n == 1) {
+        kb = k_at(__builtin_amdgcn_readfirstlane(kpg), bk);
+        vb = v_at(__builtin_amdgcn_readfirstlane(vpg), bv);
+      }
+      if (n >= 2 && n < 2 + U) send_k(kb, kw, n - 2);
+      if (n >= 2 + U && n < 2 + 2 * U) send_v(vb, vw, n - 2 - U);
+#pragma unroll
+      for (int u = 16 * n / NB; n < NB && u < 16 * (n + 1) / NB; ++u) {
+        const uint32_t x = weight2(Si, u, neg_m, s0, s1);
+        hold(x);
+        Po[u / 4][u % 4] = x;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (__any(grow)) {
+      l_run *= alpha;
+      rescale(alpha);
+    }
+    l_run += s0 + s1;
+  };
+
+  // ---- step i: scores of block kb0 + i, weights of the block before, value products of the one before that; the next K
+  // and this V on their way to the other buffers
+  const int nb = kb1 - kb0, kfirst = kb0 * kKB;
+  auto kbuf = [&](int i) FP_INLINE { return lds_k + (i & 1) * kKTile; };
+  auto vbuf = [&](int i) FP_INLINE { return lds_v + (i & 1) * kVTile; };
+  auto needed = [&](int i) FP_INLINE { return i >= 0 && i < nb && kfirst + i * kKB < w_end; };   // wave-uniform
+  f32x16 sacc[kNS];
+  u32x4 pw[4];
+#pragma unroll
+  for (int t = 0; t < kNS; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sacc[t][i] = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) pw[ks] = u32x4{0u, 0u, 0u, 0u};
+  if (nb > 0) {
+    send_block_k(kfirst, kbuf(0));
+    wait_sent();
   }
   __syncthreads();
-
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const int buf = (kb - kb0) & 1;
-    const bool more = kb + 1 < kb1;
-    const int k0 = kb * kKB;
-    bool issued = false;
-    if (k0 < w_end) {  // wave-uniform: the wave has visible keys in this block
-      const uint16_t* kl = lds_k[buf];
-      const uint16_t* vl = lds_v[buf];
-      // S^T = K . Q^T, one 32x32 accumulator per 32-key sub-tile.  The wave keeps the issue
-      // priority from here to the end of its value products, so that the SIMD's other wave falls
-      // behind and fills the gaps instead of running the same phase in step: 8B prompts of 4 x 2k
-      // tokens, with the rope kernel: 189.9 -> 187.4 us.
-      __builtin_amdgcn_s_setprio(1);
-      f32x16 sacc[kNS];
-#pragma unroll
-      for (int t = 0; t < kNS; ++t) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[t][i] = 0.f;
-#pragma unroll
-        for (int st = 0; st < 8; ++st) {
-          const frag kf =
-              *reinterpret_cast<const frag*>(kl + (32 * t + r) * kKStride + 16 * st + 8 * h);
-          sacc[t] = MF::mma(kf, qf[st], sacc[t]);
-        }
-      }
-      // next block's K/V -> registers, issued after QK^T (guide §5.5 T14): in flight during
-      // softmax + PV.  Issued at the top of the loop instead, the first QK^T MFMA (whose
-      // accumulator the compiler had overlapped with the loads' address registers) waited
-      // vmcnt(0) for them: every block paid the whole load latency.
-      if (more) load_block(kb + 1);
-      issued = true;
-      // mask: only blocks crossing the diagonal of the wave's first token (wave-uniform
-      // branch); element (t, i) holds key k0 + 4 h + 32 t + (i & 3) + 8 (i >> 2), a compile-
-      // time offset from the lane's base, so a compare with one per-lane limit suffices
-      if (k0 + kKB > ctx0 + w_first + 1) {
-        const int lim = c_end - k0 - 4 * h;
-#pragma unroll
-        for (int t = 0; t < kNS; ++t)
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if (32 * t + (i & 3) + 8 * (i >> 2) >= lim) sacc[t][i] = kNegInf;
-      }
-      // running max on the raw scores (scale > 0), softmax in the log2 domain with the scale
-      // folded into one fma per element: p = 2^(s * scale_log2 - m)
-      float tmax = kNegInf;
-#pragma unroll
-      for (int t = 0; t < kNS; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, sacc[t][i]);
-      tmax = fmaxf(tmax, xor32(tmax, x32));
-      // defer-max (guide §5.5 T13): the running max m_run moves only when some column's max
-      // grew by more than kRescale (log2 units), so P = 2^(s - m_run) stays <= 2^kRescale;
-      // O and l are rescaled only then - with the max nearly settled after the first block,
-      // the multiplies of the rescale were paid on most blocks.  O, l and P of a
-      // block always use the same m_run, so the result is exact up to rounding.
-      const float m_cand = fmaxf(m_run, tmax * p.scale_log2);
-      const bool grow = m_cand > m_run + kRescale;  // m_run == -inf: any finite m_cand
-      if (__any(grow)) {
-        const float m_new = grow ? m_cand : m_run;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - ((m_new == kNegInf) ? 0.f : m_new));
-        l_run *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-        m_run = m_new;
-      }
-      const float m_use = (m_run == kNegInf) ? 0.f : m_run;
-      // exponent arguments and the row sum in two chains
-      typedef float f32x2_t __attribute__((ext_vector_type(2)));
-      const f32x2_t sc2 = {p.scale_log2, p.scale_log2};
-      const f32x2_t nm2 = {-m_use, -m_use};
-      f32x2_t ps2 = {0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < kNS; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-          const f32x2_t a = __builtin_elementwise_fma(f32x2_t{sacc[t][i], sacc[t][i + 1]}, sc2, nm2);
-          const f32x2_t e = {__builtin_amdgcn_exp2f(a[0]), __builtin_amdgcn_exp2f(a[1])};
-          sacc[t][i] = e[0];
-          sacc[t][i + 1] = e[1];
-          ps2 += e;
-        }
-      float psum = ps2[0] + ps2[1];
-      psum += xor32(psum, x32);
-      l_run += psum;
-      // P^T fragments per 16-key step: registers 8s..8s+7 of the sub-tile packed pairwise;
-      // O^T += V^T . P^T (A element j of half h = key 16 s + 8 (j >> 2) + 4 h + (j & 3))
-#pragma unroll
-      for (int t = 0; t < kNS; ++t) {
-        frag pf[2];
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          u32x4 w;
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            w[j] = pack2<T>(sacc[t][8 * st + 2 * j], sacc[t][8 * st + 2 * j + 1]);
-          pf[st] = __builtin_bit_cast(frag, w);
-        }
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const uint16_t* vrow = vl + (32 * dt + r) * kVStride + 32 * t + 8 * h;
-#pragma unroll
-          for (int st = 0; st < 2; ++st) {
-            const frag vf = *reinterpret_cast<const frag*>(vrow + 16 * st);
-            o[dt] = MF::mma(vf, pf[st], o[dt]);
-          }
-        }
-      }
-      __builtin_amdgcn_s_setprio(0);
+  // steps [2, quick1): the block before has no masked key, this one is needed
+  const int quick1 = w_end > 0 && p.wide_in ? min(min(nb, (ctx0 + w_first + 1 - kfirst) / kKB + 1), (w_end - 1 - kfirst) / kKB + 1) : 0;
+  auto quick_step = [&](int i, const f32x16 (&Si)[kNS], f32x16 (&So)[kNS], const u32x4 (&Pi)[4], u32x4 (&Po)[4]) FP_INLINE {
+    quick(kbuf(i), vbuf(i), kbuf(i + 1), vbuf(i + 1), kfirst + (i + 1) * kKB, kfirst + (i - 1) * kKB, Si, So, Pi, Po);
+    wait_sent();
+    __syncthreads();
+  };
+  for (int i = 0; nb > 0 && i <= nb; ++i) {
+    for (; i >= 2 && i + 1 < quick1; i += 2) {
+      f32x16 s2[kNS];
+      u32x4 p2[4];
+      quick_step(i, sacc, s2, pw, p2);
+      quick_step(i + 1, s2, sacc, p2, pw);
     }
-    if (more && !issued) load_block(kb + 1);  // waves with no visible key in this block
-    if (more) store_block(buf ^ 1, kb + 1);
+    const int k0 = kfirst + (i - 1) * kKB;
+    if (i + 1 < nb) send_block_k(k0 + 2 * kKB, kbuf(i + 1));
+    if (i >= 1) send_block_v(k0, vbuf(i + 1));
+    if (needed(i - 2)) values(vbuf(i), pw);
+    if (needed(i - 1)) weights(k0, sacc, pw);
+    if (needed(i)) scores(kbuf(i), sacc);
+    if (i >= 1) put_v(k0, vbuf(i + 1));
+    wait_sent();
     __syncthreads();
   }
+  if (needed(nb - 1)) values(vbuf(nb + 1), pw);
+  l_run += xor32(l_run, x32);
 
   if (ns > 1) {
     // ---- split-KV hand-over: publish (O, m, l) with device-scope stores, count arrivals; the
@@ -474,20 +537,37 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void flash_prefill_kernel(FlashPar
     }
   }
 
-  // ---- epilogue: O = O^T / l, lane (col r, half h) holds d = 32 dt + (i & 3) + 8 (i >> 2) + 4 h
-  if (c_valid) {
-    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    uint16_t* op = p.out + static_cast<int64_t>(qstart + c_tok) * p.out_stride +
-                   static_cast<int64_t>(c_head) * kD + 4 * h;
+  // ---- epilogue: O = O^T / l, lane (col r, half h) holds d = 32 dt + (i & 3) + 8 (i >> 2) + 4 h; 64 channels at a time
+  // through LDS (the wave's own 4 KB; K is read no more), so that a store has whole rows: 8-byte pieces of 32 rows keep the
+  // memory pipe busy
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  auto two = [&](int dt, int i) FP_INLINE {
+    return u32x2{pack2<T>(o[dt][i] * inv, o[dt][i + 1] * inv), pack2<T>(o[dt][i + 2] * inv, o[dt][i + 3] * inv)};
+  };
+  uint16_t* const op = p.out + static_cast<int64_t>(qstart + qoff + wid * kTokPerWave) * p.out_stride + static_cast<int64_t>(hk) * G * kD;
+  if (p.wide_out) {
+    char* x = reinterpret_cast<char*>(lds_k) + wid * 4096;
+#pragma unroll
+    for (int d2 = 0; d2 < 2; ++d2) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        *reinterpret_cast<u32x2*>(x + r * 128 + ((c ^ ((r >> 1) & 7)) * 16) + 8 * h) = two(2 * d2 + c / 4, c % 4 * 4);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int rr = 8 * j + (lane >> 3), tok = rr / G;
+        const u32x4 e = *reinterpret_cast<const u32x4*>(x + rr * 128 + (((lane & 7) ^ ((rr >> 1) & 7)) * 16));
+        if (rr < kTokPerWave * G && w_first + tok < qlen)
+          *reinterpret_cast<u32x4*>(op + tok * p.out_stride + (rr - tok * G) * kD + 64 * d2 + 8 * (lane & 7)) = e;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else if (c_valid) {
+    uint16_t* oc = op + (r / G) * p.out_stride + (r % G) * kD + 4 * h;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u32x2 w;
-        w[0] = pack2<T>(o[dt][4 * g + 0] * inv, o[dt][4 * g + 1] * inv);
-        w[1] = pack2<T>(o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv);
-        *reinterpret_cast<u32x2*>(op + 32 * dt + 8 * g) = w;
-      }
+      for (int g = 0; g < 4; ++g) *reinterpret_cast<u32x2*>(oc + 32 * dt + 8 * g) = two(dt, 4 * g);
   }
 }
 
@@ -561,6 +641,8 @@ int atta_flash_prefill(void* out, const void* q, const void* k_cache, const void
   prm.split_blocks = g_split_blocks;
   prm.part = part;
   prm.counters = counters;
+  prm.wide_in = (reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) % 16 == 0;
+  prm.wide_out = out_stride % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
   dim3 grid(num_tiles * n_kv_heads * nsplit);
   const int rc = dtype == 0 ? fp::launch<__bf16>(G, grid, stream, prm)
                             : fp::launch<_Float16>(G, grid, stream, prm);

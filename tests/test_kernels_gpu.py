@@ -158,6 +158,26 @@ def test_flash_prefill_split_kv(splits, hq, hkv):
                                        torch.zeros(1, device="cuda")).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (24, 8)])
+def test_flash_prefill_odd_alignment(hq, hkv):
+    """Caches and results whose rows start between 16-byte borders take the ways through registers and in 8-byte pieces:
+    bit for bit the results of aligned ones."""
+    torch.manual_seed(5)
+    seqs = [(400, 400), (193, 17), (700, 130)]
+    k, v, bt, kvlen, qstart, T = _make_paged(seqs, hkv, 16, torch.bfloat16)
+    q = torch.randn(T, hq, 128, dtype=torch.bfloat16, device="cuda")
+    ts, to = _tiles(seqs, ops.prefill_tile_tokens(hq // hkv, "flash"))
+
+    def shifted(t):
+        x = torch.empty(t.numel() + 4, dtype=t.dtype, device="cuda")[4:].view(t.shape)
+        return x.copy_(t)
+
+    want = ops.attention_prefill(q, k, v, bt, kvlen, qstart, ts, to, 0.1, impl="flash", kv_splits=1)
+    out = shifted(torch.zeros_like(q))
+    got = ops.attention_prefill(q, shifted(k), shifted(v), bt, kvlen, qstart, ts, to, 0.1, out=out, impl="flash", kv_splits=1)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("impl", ["flash", "v1"])
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("hq,hkv", [(32, 8), (64, 8), (8, 1), (4, 1), (16, 16), (24, 8)])
