@@ -2307,3 +2307,32 @@ def test_forget_gate_results_in_bf16():
         want.append((s64 * qq[:, t, :, :, None]).sum(2))
     want = torch.stack(want, 1).reshape(S * n, H, d)
     assert float((got.double().view_as(want) - want).norm() / want.norm()) < 7.38e-8
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n", [16, 47, 600])
+def test_chunked_pairs_beyond_the_range(n, d):
+    """16-bit q and k that are finite and whose product is not: infinities where the token-by-token form has them, and the
+    rows before it as they are without it."""
+    torch.manual_seed(d)
+    H, hit = 2, n - 9
+    md = ragged([n], [0], [0], width=40)
+    at_g = [md[x].cuda() for x in ("positions", "seq_qstart", "seq_slot")]
+    q, k, v = (torch.randn(n, H * d).to(torch.bfloat16) for _ in range(3))
+    v[hit] = torch.where(v[hit] < 0, v[hit] - 1, v[hit] + 1)   # (q . k v overflows where q . k does)
+    pw, tab, st = mx.retention_powers([0.9, 0.99], "cuda"), torch.zeros(n, 0).cuda(), torch.zeros(1, H, d, d)
+
+    def run(q, k):
+        return mx.retention(q.cuda(), k.cuda(), v.cuda(), pw, tab, st.clone().cuda(), *at_g, H, d, d).cpu()
+    fine = run(q, k)
+    q[hit, 3::d], k[hit, 3::d] = 1e20, 1e20
+    got = run(q, k)
+    want = mref.retention(q, k, v, pw[:, 1].cpu(), tab.cpu(), st.clone(), md["positions"], md["seq_qstart"],
+                          md["seq_slot"], H, d, d)
+    assert torch.equal(got[:hit], fine[:hit])
+    for a, b in ((got[:, 0], want[:, 0]), (got[:, 1], want[:, 1])):
+        assert torch.isinf(b[hit]).all() and torch.equal(a[hit], b[hit])
+        fin = torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), fin)
+        bound = n * 2.0 ** -24 * float(b[fin].double().abs().max())   # a rounding per token
+        assert float((a[fin].double() - b[fin].double()).abs().max()) <= max(bound, 1e-5)
