@@ -17,7 +17,10 @@
 // help); latent, 16 rows of 2000: 26 -> 12.1; two maps 21 -> 10.
 //
 // Join: four waves per (row, head) take every fourth partition, with the first four of them loaded before their
-// weights are known: 6.2 -> 3.7 us, latent 10.7 -> 4.4, two maps 7.1 -> 5.7.
+// weights are known: 6.2 -> 3.7 us, latent 10.7 -> 4.4, two maps 7.1 -> 5.7.  One look at the partitions' maxima and sums,
+// of both maps at once, in place of two or four in turn: layers, 16 rows of 2000, latent 28.7 -> 28.5 us, two maps
+// 31.4 -> 30.9, small, 6 rows of 1300, 19.2 -> 18.5.  (The partition kernel with the pages fetched beside the context's
+// length, one trip less, is slower: latent 28.7 -> 29.5, 32 + 8 heads 39.3 -> 39.7.)
 #include "sink_attention.h"
 
 namespace mixk {
@@ -195,28 +198,45 @@ sink_join_kernel(void* __restrict__ out, AttnArgs a) {
   const int kvlen = a.seq_kvlen[s];
   if (kvlen <= 0) return;
   const int np = live_parts(a, kvlen), vdim = a.vdim, ps = vdim + 2, rep = a.H / a.G;
-  float inv[NMAP];
+  auto head_of = [&](int mp) { return NMAP == 2 ? (2 * (ho / rep) + mp) * rep + ho % rep : ho; };   // G counts a K head per map
+  auto base_of = [&](int mp) { return a.part + (static_cast<int64_t>(s) * a.H + head_of(mp)) * a.max_parts * ps; };
+  // a lane's partition among the first 64: its maximum and sum; with the values of the first four per wave all of a chain's
+  // loads, of both maps, in one trip
+  float inv[NMAP], ahead[NMAP][kAhead][NJ], top[NMAP], sum[NMAP];
 #pragma unroll
   for (int mp = 0; mp < NMAP; ++mp) {
-    const int h = NMAP == 2 ? (2 * (ho / rep) + mp) * rep + ho % rep : ho;   // G counts a K head per map
-    const float* base = a.part + (static_cast<int64_t>(s) * a.H + h) * a.max_parts * ps;
-    float ahead[kAhead][NJ], acc[NJ];
+    const float* base = base_of(mp);
+    const float* e = base + static_cast<int64_t>(min(lane, np - 1)) * ps + vdim;
+    top[mp] = e[0];
+    sum[mp] = e[1];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i)
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
-        ahead[i][j] = base[static_cast<int64_t>(min(w + 4 * i, np - 1)) * ps + min(lane + kWave * j, vdim - 1)];
+        ahead[mp][i][j] = base[static_cast<int64_t>(min(w + 4 * i, np - 1)) * ps + min(lane + kWave * j, vdim - 1)];
+  }
+#pragma unroll
+  for (int mp = 0; mp < NMAP; ++mp) {
+    const int h = head_of(mp);
+    const float* base = base_of(mp);
+    float acc[NJ];
     const float sink_score = a.sink && a.sink_val != nullptr ? a.sink_val[h] : 0.f;
     float M = a.sink ? sink_score : kNegBig, L = 0.f;
-    for (int p = lane; p < np; p += kWave) M = fmaxf(M, base[static_cast<int64_t>(p) * ps + vdim]);
+    M = fmaxf(M, top[mp]);   // (lanes past the last partition hold it again)
+    for (int p = lane + kWave; p < np; p += kWave) M = fmaxf(M, base[static_cast<int64_t>(p) * ps + vdim]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, kWave));
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[j] = 0.f;
     for (int p0 = 0; p0 < np; p0 += kWave) {
-      const float* e = base + static_cast<int64_t>(min(p0 + lane, np - 1)) * ps + vdim;
-      const float wp = p0 + lane < np ? expf(e[0] - M) : 0.f;
-      L += p0 + lane < np ? e[1] * wp : 0.f;   // (a partition past the end may hold anything)
+      float e0 = top[mp], e1 = sum[mp];
+      if (p0 > 0) {
+        const float* e = base + static_cast<int64_t>(min(p0 + lane, np - 1)) * ps + vdim;
+        e0 = e[0];
+        e1 = e[1];
+      }
+      const float wp = p0 + lane < np ? expf(e0 - M) : 0.f;
+      L += p0 + lane < np ? e1 * wp : 0.f;   // (a partition past the end may hold anything)
       auto weight = [&](int i) {
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wp), i));
       };
@@ -226,7 +246,7 @@ sink_join_kernel(void* __restrict__ out, AttnArgs a) {
         for (int k = 0; k < kAhead; ++k, i += 4)
           if (i < np)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[j] += ahead[k][j] * weight(i);
+            for (int j = 0; j < NJ; ++j) acc[j] += ahead[mp][k][j] * weight(i);
 #pragma unroll 4
       for (; i < min(kWave, np - p0); i += 4)
 #pragma unroll

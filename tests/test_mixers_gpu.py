@@ -1836,6 +1836,34 @@ def test_decode_two_maps_edges(dt, H, G, window, keep):
     assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
 
 
+@pytest.mark.parametrize("H,G,d,dv,pair", [(6, 2, 128, 128, False), (5, 1, 256, 192, False), (8, 2, 64, 128, True)])
+@pytest.mark.parametrize("window,keep,bs", [(0, 0, 16), (0, 5, 64), (8400, 70, 16)])
+def test_decode_table_entries_past_the_context(H, G, d, dv, pair, window, keep, bs):
+    """Table entries behind a context's last page are no pages; a table that ends with the longest context; more
+    partitions than the join's first look takes (64)."""
+    torch.manual_seed(d + bs)
+    kv = [1, 17, 129, 320, 8193, 8500]
+    md = ragged([1] * len(kv), [x - 1 for x in kv], list(range(len(kv))), bs=bs, width=-(-max(kv) // bs))
+    nb = md["num_pages"]
+    wrong = md["block_tables"].clone()
+    for i, n in enumerate(kv):
+        wrong[i, -(-n // bs):] = 2 ** 31 - 1 - i
+    q, gate = torch.randn(len(kv), H * (2 if pair else 1), d).bfloat16(), torch.randn(len(kv), H * dv).bfloat16()
+    k, v = torch.randn(nb, G * (2 if pair else 1), bs, d).bfloat16(), torch.randn(nb, G, dv, bs).bfloat16()
+    empty = torch.zeros(0, dtype=torch.int32)
+
+    def run(m, table, q, k, v, gate, e):
+        at = (q, k, v, table, m["seq_kvlen"], m["seq_qstart"], e, e, d ** -0.5)
+        if pair:
+            return mx.differential_attention(*at, 0.4, 0.3, 1e-5, gate, len(kv), max(kv), window, keep)
+        return mx.sink_attention(*at, True, len(kv), max(kv), window=window, keep_first=keep)
+
+    want = run(md, md["block_tables"], q, k, v, gate, empty)
+    got = run(cuda(md), *(t.cuda() for t in (wrong, q, k, v, gate, empty)))
+    # weights and results are rounded to 8 bits once each, |v| <= 4.5 (as in the edges' tests)
+    assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("gs", [8, 64, 72, 128, 136, 256, 512, 520, 100])
 @pytest.mark.parametrize("full", [False, True])
