@@ -21,7 +21,7 @@
 //     C  O^T[16 channels x 16 tokens] += V^T . mixed^T (V^T rows straight from the pages).
 //   B needs A of all waves and C needs B of all waves; C of a tile and A of the next share one
 //   barrier interval, so a tile costs two barriers (which order LDS only: the V fragments of the
-//   tile are in flight during B, the first K fragments of the next one late in C).  The LDS images
+//   tile are in flight during B, the first K fragments of the next one during C).  The LDS images
 //   are XOR-swizzled (sg_place) to spread the accesses of every phase over the banks.
 //   A launch with few query tiles is split over the keys (sg_shares): every share writes fp32 partial
 //   rows, a join kernel adds them.
@@ -161,10 +161,15 @@ __device__ __forceinline__ void sg_barrier() {
 // Forms with few heads fit twice on a CU.
 constexpr int sg_waves(int HW, int NV) { return HW * NV <= 8 ? 4 : 2; }
 
-// V fragments in flight: what the registers leave.
+// V fragments in flight during the mix: what the registers leave.
 constexpr int sg_v_flight(int HW, int NV) {
   return HW * NV >= 32 ? NV / 4 : (HW * NV == 8 && NV == 8 ? NV / 2 : NV);
 }
+// Behind the mix there is room again for the next group of V fragments and the next tile's first keys: on their way
+// before this group's products, not just before their own use, where every wave waited for them.  Kernel's layer, us,
+// before / now: 24 + 8 heads 3 x 700 90.0 / 85.4, 3000 260 / 237; 32 + 8 heads 4 x 1000 225 / 210.  Two groups ahead spill
+// (248).  Forms with four waves per SIMD have half the registers (8 heads of 128, 2500 rows: 133, with a group ahead 155).
+constexpr int sg_v_ahead(int HW, int NV) { return sg_waves(HW, NV) == 2 ? 1 : 0; }
 
 template <int HW, int ND, int NV, bool CAP, bool ONE>   // dim <= 32 ND, vdim <= 16 NV, H <= 8 HW
 __global__ void __launch_bounds__(512, sg_waves(HW, NV))
@@ -173,7 +178,7 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
                               const __bf16* __restrict__ v_cache, SigArgs a) {
   constexpr int QL = sg_q_lds(HW, ND), QR = HW - QL;     // heads with Q in LDS / in registers
   constexpr int QS = 32 * ND;                            // LDS row of one token's Q
-  constexpr int NF = sg_v_flight(HW, NV);
+  constexpr int NF = sg_v_flight(HW, NV), NG = NV / NF, AHEAD = sg_v_ahead(HW, NV);   // V fragments by groups of NF
   extern __shared__ __attribute__((aligned(16))) char sg_smem[];
   constexpr int SL = sg_slots(HW), kSlots = 8 * SL, CH = 2 * SL;   // CH: slots per chunk
   typedef __attribute__((ext_vector_type(SL))) __bf16 slots_t;           // a wave's slots
@@ -245,7 +250,6 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
       tf[ht][j] = static_cast<__bf16>(ok ? a.talk[ho * H + hi] : 0.f);
     }
   }
-  const int nht = ((H - 1) / HW * SL + HW + 15) / 16;   // output slot tiles in use
   auto mix = [](chunk_t x, chunk_t t, sg_f32x4 d) {
     if constexpr (SL == 4) {
       return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, t, d, 0, 0, 0);
@@ -289,6 +293,22 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
     }
     return S;
   };
+  // a (key, token)'s weights of the wave's heads, high and low part, converted two at a time (32 + 8 heads 4 x 1000 203 ->
+  // 199 us).  A form without masks for the tiles in front of the first token spills: 257.
+  auto put_weights = [&](const float (&x)[SL], int key, int rr) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 two_t;
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    unsigned int hi[SL / 2], lo[SL / 2];
+#pragma unroll
+    for (int j = 0; j < SL / 2; ++j) {
+      hi[j] = __builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2{x[2 * j], x[2 * j + 1]}), two_t));
+      const f32x2 rest{x[2 * j] - __builtin_bit_cast(float, hi[j] << 16), x[2 * j + 1] - __builtin_bit_cast(float, hi[j] & 0xffff0000u)};
+      lo[j] = __builtin_bit_cast(unsigned int, __builtin_convertvector(rest, two_t));
+    }
+    const int o = sg_place<CH>(key, rr, w >> 1) + (w & 1) * SL;
+    __builtin_memcpy(__builtin_assume_aligned(w_hi + o, 2 * SL), hi, sizeof(hi));
+    __builtin_memcpy(__builtin_assume_aligned(w_lo + o, 2 * SL), lo, sizeof(lo));
+  };
   // weights of keys k0 + 16 sub .. + 15 for the wave's heads, into the LDS image
   auto weights = [&](int k0, int sub, const sg_f32x4 (&S)[HW]) {
     const int kb = k0 + sub * 16 + 4 * c;
@@ -296,20 +316,16 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
     const int rr = fresh(r);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      slots_t hi, lo;
+      float x[SL];
 #pragma unroll
       for (int hh = 0; hh < SL; ++hh) {
-        float x = 0.f;
+        x[hh] = 0.f;
         if (hh < HW) {
-          x = sig_weight<CAP>(S[hh < HW ? hh : 0][i], k1, k2, k3[hh < HW ? hh : 0]);
-          if (edge && kb + i > qpos) x = 0.f;
+          x[hh] = sig_weight<CAP>(S[hh < HW ? hh : 0][i], k1, k2, k3[hh < HW ? hh : 0]);
+          if (edge && kb + i > qpos) x[hh] = 0.f;
         }
-        hi[hh] = static_cast<__bf16>(x);
-        lo[hh] = static_cast<__bf16>(x - static_cast<float>(hi[hh]));
       }
-      const int o = sg_place<CH>(sub * 16 + 4 * c + i, rr, w >> 1) + (w & 1) * SL;
-      *reinterpret_cast<slots_t*>(w_hi + o) = hi;
-      *reinterpret_cast<slots_t*>(w_lo + o) = lo;
+      put_weights(x, sub * 16 + 4 * c + i, rr);
     }
   };
 
@@ -365,64 +381,73 @@ sigmoid_attention_mfma_kernel(__bf16* __restrict__ out, const __bf16* __restrict
   for (int k0 = kfirst; k0 < kstop; k0 += kSgKeys) {
     const int nk = k0 + kSgKeys, t8 = k0 + 8 * c;
     const __bf16* vb = v_cache + pv * vpage + (min(t8, last) & bmask & ~7) + static_cast<int64_t>(r) * bs;
-    sg_bf16x8 vf[NF];
-    auto load_v = [&](int vt0) {
+    sg_bf16x8 vf[1 + AHEAD][NF];
+    auto load_v = [&](int g) {
 #pragma unroll
       for (int e = 0; e < NF; ++e)
-        vf[e] = ld_frag(vb + static_cast<int64_t>(g0 * vdim + min(vt0 + e, nv - 1) * 16) * bs);
+        vf[g % (1 + AHEAD)][e] = ld_frag(vb + static_cast<int64_t>(g0 * vdim + min(g * NF + e, nv - 1) * 16) * bs);
     };
     if (ONE && wave_on) load_v(0);
     pv = page_at(nk + 8 * c);
     sg_barrier();
     const int rb = fresh(r);
-    // B: the wave mixes the pairs of tokens 2 w and 2 w + 1
+    // B: the wave mixes the pairs of tokens 2 w and 2 w + 1, 16 keys of a token at a time: the next ones' weights are on
+    // their way and the last ones' results go to LDS beside the products.  (A chain of eight reads, products and stores
+    // before: 24 + 8 heads 3 x 700 85.4 -> 82.5 us, 3000 237 -> 225, 32 + 8 heads 4 x 1000 210 -> 203.  All reads in front
+    // spill: 101, 283, 229.)
+    chunk_t ah[2], al[2];
+    sg_f32x4 D[2][kSlots / 16];
+    auto read_weights = [&](int u) {
+      const int o = sg_place<CH>((u & 1) * 16 + rb, 2 * w + (u >> 1), c);
+      al[u & 1] = *reinterpret_cast<const chunk_t*>(w_lo + o);
+      ah[u & 1] = *reinterpret_cast<const chunk_t*>(w_hi + o);
+    };
+    auto put_mixed = [&](int u) {
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const int t = 2 * w + tt;
+      for (int ht = 0; ht < kSlots / 16; ++ht) {
+        sg_bf16x4 e;
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const int o = sg_place<CH>(half * 16 + rb, t, c);
-        const chunk_t ah = *reinterpret_cast<const chunk_t*>(w_hi + o);
-        const chunk_t al = *reinterpret_cast<const chunk_t*>(w_lo + o);
-#pragma unroll
-        for (int ht = 0; ht < kSlots / 16; ++ht) {
-          if (ht < nht) {
-            sg_f32x4 D = {0.f, 0.f, 0.f, 0.f};
-            D = mix(al, tf[ht], D);
-            D = mix(ah, tf[ht], D);
-            sg_bf16x4 e;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) e[i] = static_cast<__bf16>(D[i]);
-            *reinterpret_cast<sg_bf16x4*>(mixed + sg_place<8>(ht * 16 + rb, t, half * 2 + (c >> 1)) +
-                                          (c & 1) * 4) = e;
-          }
-        }
+        for (int i = 0; i < 4; ++i) e[i] = static_cast<__bf16>(D[u & 1][ht][i]);
+        *reinterpret_cast<sg_bf16x4*>(mixed + sg_place<8>(ht * 16 + rb, 2 * w + (u >> 1), (u & 1) * 2 + (c >> 1)) + (c & 1) * 4) = e;
       }
+    };
+    read_weights(0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (u < 3) read_weights(u + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ht = 0; ht < kSlots / 16; ++ht) D[u & 1][ht] = mix(al[u & 1], tf[ht], sg_f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int ht = 0; ht < kSlots / 16; ++ht) D[u & 1][ht] = mix(ah[u & 1], tf[ht], D[u & 1][ht]);
+      if (u > 0) put_mixed(u - 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    put_mixed(3);
     sg_barrier();
     if (wave_on) {   // C
       const bool tail = nk > kend;
       const int rc = fresh(r);
       if (ONE) {
 #pragma unroll
-        for (int vt0 = 0; vt0 < NV; vt0 += NF) {
-          if (vt0 > 0) load_v(vt0);
-          if (vt0 + NF >= NV && NF < NV) load_k(ka, pk0, nk + r, g0);
+        for (int g = 0; g < NG; ++g) {
+          if (g + AHEAD > 0 && g + AHEAD < NG) load_v(g + AHEAD);
+          if (g == (NG - 1 > AHEAD ? NG - 1 - AHEAD : 0)) load_k(ka, pk0, nk + r, g0);   // (behind the last V)
+          if constexpr (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+          sg_bf16x8 (&v)[NF] = vf[g % (1 + AHEAD)];
           if (tail) {
 #pragma unroll
-            for (int e = 0; e < NF; ++e) vf[e] = keep_keys(vf[e], t8, kend);
+            for (int e = 0; e < NF; ++e) v[e] = keep_keys(v[e], t8, kend);
           }
 #pragma unroll
           for (int hh = 0; hh < HW; ++hh) {
             const sg_bf16x8 pf = ld_frag(mixed + sg_place<8>(SL * w + hh, rc, c));
 #pragma unroll
             for (int e = 0; e < NF; ++e)
-              O[hh][vt0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[e], pf, O[hh][vt0 + e], 0, 0, 0);
+              O[hh][g * NF + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[e], pf, O[hh][g * NF + e], 0, 0, 0);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (NF == NV) load_k(ka, pk0, nk + r, g0);
-        __builtin_amdgcn_sched_barrier(0);
       } else {
 #pragma unroll
         for (int hh = 0; hh < HW; ++hh) {
