@@ -123,10 +123,15 @@ __device__ __forceinline__ float both_max(float v) {
 }
 // 16 bytes per lane from base + offset to 1 KB of LDS, without registers; there after wait_sent().  (After the builtin the
 // compiler makes every read of LDS wait for all transfers.)
+// The base goes through a scalar move: five wait states belong between a vector instruction that writes a scalar register,
+// such as the reload of a spilled one, and a memory instruction that reads it, and the compiler does not put them in front
+// of assembly.  (The same in mixers/sink_flash.hip, a library of its own.)
 __device__ __forceinline__ void send16(const void* base, uint32_t offset, void* to) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(at) : "m0", "memory");
+  uint64_t from;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+               : "=&s"(from) : "v"(offset), "s"(base), "s"(at) : "m0", "memory");
 #endif
 }
 __device__ __forceinline__ void wait_sent() {

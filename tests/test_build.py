@@ -1,5 +1,6 @@
 """The in-tree native libraries build for gfx950 and load on a CPU-only host (catches
 undefined symbols / missing registrations before a GPU box ever sees them)."""
+import re
 import types
 
 import torch
@@ -123,3 +124,18 @@ def test_hip_units_are_compiled_without_packed_fp32(tmp_path, monkeypatch):
     for c in units:
         at = c.index("-packed-fp32-ops")
         assert c[at - 3:at] == ["-Xclang", "-target-feature", "-Xclang"]
+
+
+def test_transfers_to_lds_read_their_base_behind_a_scalar_move():
+    """A memory instruction in assembly that takes its address from a scalar register: the compiler does not keep the five
+    wait states behind a vector instruction that wrote it (a reload of a spilled register), so the assembly moves it first."""
+    found = 0
+    for src in [*build.kernel_sources(), *build.mixer_sources()]:
+        for text in re.findall(r'asm volatile\("((?:[^"\\]|\\.)*)"', src.read_text()):
+            lines = text.split("\\n\\t")
+            for i, line in enumerate(lines):
+                if re.match(r"(global|buffer|scratch)_", line):
+                    found += 1
+                    base = line.split()[-1]
+                    assert any(re.match(rf"s_mov_b64 {base},", x) for x in lines[:i]), (src.name, text)
+    assert found == 3
