@@ -2,7 +2,7 @@
 // sink_attention.hip, same masks, sink, gates and pair epilogue (see there for what they mean).
 //
 // A piece of work = up to NW x 32 columns of one 64-token tile, a column = (query token, query head of the KV head's
-// group); its workgroup walks blocks of 32 KT keys:
+// group); its workgroup walks blocks of 64 keys:
 //   S^T[32 keys x 32 cols] = K . Q^T    (mfma 32x32x16, A = K rows from LDS, B = Q in registers)
 //   O^T[vdim x 32 cols]   += V^T . P^T  (A = V^T rows from LDS, B = P^T from the S^T registers)
 // A lane holds one column of S^T, so the softmax statistics are lane-local plus one exchange with
@@ -34,6 +34,7 @@
 // now: 32 + 8 heads of 128 159 -> 138, latent 257 -> 221, two maps (8 heads, 5 x 1165, window 1024) 72 -> 50.
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "sink_attention.h"
 
@@ -50,6 +51,7 @@ typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
+constexpr int KT = 2;                    // tiles of 32 keys per block
 constexpr int kPages = 2048;             // page-table entries in LDS
 constexpr int kSortTiles = 1024;         // tiles that a workgroup puts in order
 constexpr int kPieces = 64;              // pieces of work per workgroup in LDS
@@ -114,8 +116,14 @@ __device__ __forceinline__ void hold(const X& x) {
 #endif
 }
 
-// DK = 16 ND (q / k width), DV = 32 NV (value width), blocks of 32 KT keys.
-template <int ND, int NV, int NMAP, int NW, int KT, bool WIN>
+// f(0), f(1), ... as constants (a loop of so much in a turn is not unrolled)
+template <int... N, typename F>
+__device__ __forceinline__ void each(std::integer_sequence<int, N...>, const F& f) {
+  (f(std::integral_constant<int, N>()), ...);
+}
+
+// DK = 16 ND (q / k width), DV = 32 NV (value width).
+template <int ND, int NV, int NMAP, int NW, bool WIN>
 __global__ void __launch_bounds__(NW * 64, 2)
 sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __bf16* __restrict__ k_cache,
                   const __bf16* __restrict__ v_cache, AttnArgs a, int num_tiles, int chunks, int workers) {
@@ -128,9 +136,14 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   constexpr int RB = CK < 16 ? 16 / CK : 1;         // K rows per 256 bytes
   constexpr int KB = NMAP * BLK * DK, VB = DV * BLK;   // elements of a buffer
   constexpr int MT = NMAP, TPM = KT / MT;           // maxima per block, tiles per maximum
-  static_assert(NMAP == 1 || (NW == 8 && KT == 2), "pair form: four waves per map");
+  // Queries of 256 and values of 192 channels take 160 registers, and two tiles' scores beside the ones before them all of the
+  // others: the tiles take turns, a tile's scores in the registers of the same tile of the block before.
+  constexpr bool TURNS = ND > 8;
+  static_assert(NMAP == 1 || NW == 8, "pair form: four waves per map");
   __shared__ __attribute__((aligned(1024))) __bf16 lds_k[2 * KB], lds_v[2 * VB];
-  __shared__ __attribute__((aligned(1024))) char lds_x[MANY ? (NMAP == 2 ? 65536 : 32768) : 16];
+  // (results of one map go through the values' buffers, where these are large enough)
+  constexpr bool XV = MANY && NMAP == 1 && 4 * VB >= 4096 * NW;
+  __shared__ __attribute__((aligned(1024))) char lds_x[MANY && !XV ? (NMAP == 2 ? 65536 : 32768) : 16];
   __shared__ float lds_ss[NMAP == 2 ? NW : 1][32];
   __shared__ int lds_bt[MANY ? 2 : 1][kPages];
   __shared__ int lds_piece[MANY ? kPieces : 1][8];
@@ -154,15 +167,14 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   // [group][channel][16 keys]; the 16-byte chunks of a K row and the halves of a V row change places so that the
   // fragments' reads have no bank conflicts
   const int sg = w % GR, part = w / GR;
-  uint32_t k_src[KU], v_src[VU];   // bytes
+  uint32_t k_src[TURNS ? 1 : KU];   // bytes (TURNS: the others are worked out where they are used)
 #pragma unroll
-  for (int u = 0; u < KU; ++u) {
+  for (int u = 0; u < (TURNS ? 1 : KU); ++u) {
     const int row = (u * WPG + part) * (64 / CK) + lane / CK;   // of the group
     k_src[u] = 2u * (row * DK + ((lane % CK) ^ ((row / RB) & (CK - 1) & 15)) * 8);
   }
   const int v_half = 8 * ((lane ^ (lane >> 4)) & 1);
-#pragma unroll
-  for (int u = 0; u < VU; ++u) v_src[u] = 2u * ((32 * (u * WPG + part) + (lane >> 1)) * bs + v_half);
+  const uint32_t v_src = 2u * ((32 * part + (lane >> 1)) * bs + v_half);
   const int k_lds = 16 * sg * DK + part * 512, v_lds = sg * DV * 16 + part * 512;
   const __bf16* k_base = k_cache + static_cast<int64_t>(NMAP * g) * bs * DK;
   const __bf16* v_base = v_cache + static_cast<int64_t>(gv) * DV * bs;
@@ -174,21 +186,29 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     return v_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * v_page + ((k0 + 16 * sg) & (bs - 1));
   };
   auto send_k = [&](const __bf16* kb, __bf16* to, int u) SF_INLINE {
-    if (KU * WPG == KN || (u % KU) * WPG + part < KN)
+    if constexpr (TURNS) {   // rows 4 further on: bits 2 and 3 of the chunk's place
+      static_assert(!TURNS || (NMAP == 1 && CK == 32 && WPG == 2), "four rows per transfer of the group's waves");
+      send16(kb + 4 * u * DK, fresh(k_src[0]) ^ (64u * u), to + k_lds + u * WPG * 512);
+    } else if (KU * WPG == KN || (u % KU) * WPG + part < KN) {
       send16(kb + (u / KU) * bs * DK, k_src[u % KU], to + (u / KU) * BLK * DK + k_lds + (u % KU) * WPG * 512);
+    }
   };
   auto send_v = [&](const __bf16* vb, __bf16* to, int u) SF_INLINE {
-    if (VU * WPG == VN || u * WPG + part < VN) send16(vb, v_src[u], to + v_lds + u * WPG * 512);
+    if (VU * WPG == VN || u * WPG + part < VN) send16(vb + 32 * u * WPG * bs, v_src, to + v_lds + u * WPG * 512);
   };
   // ---- fragments.  A row of the score products: key with bits 2 and 3 swapped
   const int krow = (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);
   const int kfrag = mp * BLK * DK + krow * DK, vfrag = r * 16 + 8 * (h ^ ((r >> 3) & 1));
   constexpr int KO = ND < 8 ? ND : 8;
-  int kofs[KO];
+  const int kplace = kfrag + (h ^ ((krow / RB) & (CK - 1) & 15)) * 8;   // of step 0; of the others:
+  typedef int Places[KO];
+  auto places = [&](Places& to) SF_INLINE {
+    const int k = TURNS ? fresh(kplace) : kplace;
 #pragma unroll
-  for (int st = 0; st < KO; ++st) kofs[st] = kfrag + ((2 * st + h) ^ ((krow / RB) & (CK - 1) & 15)) * 8;
-  auto kf = [&](const __bf16* b, int t, int st) SF_INLINE {
-    return *reinterpret_cast<const bf16x8*>(b + 32 * t * DK + kofs[st % 8] + st / 8 * 128);
+    for (int st = 0; st < KO; ++st) to[st] = k ^ (16 * st);
+  };
+  auto kf = [&](const __bf16* b, const Places& at, int t, int st) SF_INLINE {
+    return *reinterpret_cast<const bf16x8*>(b + 32 * t * DK + at[st % 8] + st / 8 * 128);
   };
   auto vf = [&](const __bf16* b, int vt, int ks) SF_INLINE {
     return *reinterpret_cast<const bf16x8*>(b + vfrag + ks * DV * 16 + vt * 512);
@@ -345,12 +365,22 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     const int nk = (min(a.keep, kbeg) + BLK - 1) / BLK;
     const int nb = nk + (kend - kbeg + BLK - 1) / BLK;
     auto block_key = [&](int b) SF_INLINE { return b < nk ? b * BLK : kbeg + (b - nk) * BLK; };
-    const int col = wcol + r;
-    const bool valid = col < cols_total;
-    const int tok = valid ? token_of(col) : 0, head = (NMAP * g + mp) * rep + (valid ? col - tok * rep : 0);
-    const int64_t row = row0 + qo + tok;
-    const int qpos = valid ? ctx + tok : -1;          // no key is visible to a column that is not there
-    const int qlow = window_start(qpos, a.window);
+    // the lane's column (worked out anew where it is used)
+    struct Column {
+      bool valid;
+      int tok, member;   // member: of the KV head's group
+    };
+    auto column = [&](int ln) SF_INLINE {
+      Column c;
+      const int col = wcol + (ln & 31);
+      c.valid = col < cols_total;
+      c.tok = c.valid ? token_of(col) : 0;
+      c.member = c.valid ? col - c.tok * rep : 0;
+      return c;
+    };
+    const Column c0 = column(lane);
+    const int head = (NMAP * g + mp) * rep + c0.member;
+    const int qpos = c0.valid ? ctx + c0.tok : -1;    // no key is visible to a column that is not there
     float m = kNegBig, l = 0.f;   // l: of the lane's keys
     if (a.sink) {   // the sink is the state the online softmax starts from (log2 units)
       m = a.sink_val != nullptr ? a.sink_val[head] * kLog2e : 0.f;
@@ -374,7 +404,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       for (int u = 0; u < VU; ++u) {
         if (!edge(k0)) send_v(vb, to, u);
         else if (VU * WPG == VN || u * WPG + part < VN)
-          vr[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb) + v_src[u]);
+          vr[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb + 32 * u * WPG * bs) + v_src);
       }
     };
     auto put_block_v = [&](int k0, __bf16* to) SF_INLINE {
@@ -399,12 +429,14 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       return b >= 0 && b < nb && wave_on && k0 <= pos_last && (k0 + BLK > low_first || k0 < a.keep);
     };
     auto scores = [&](const __bf16* from, f32x16 (&S)[KT]) SF_INLINE {
+      Places at;
+      places(at);
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
 #pragma unroll
-        for (int st = 0; st < ND; ++st) S[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf(from, t, st), qf[st], S[t], 0, 0, 0);
+        for (int st = 0; st < ND; ++st) S[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf(from, at, t, st), qf[st], S[t], 0, 0, 0);
       }
     };
     auto rescale = [&](float alpha) SF_INLINE {
@@ -428,7 +460,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       const int k0 = block_key(b);
       if (k0 + BLK - 1 > pos_first || (WIN && k0 <= edge_lo)) {
         // register i of tile t holds key k0 + 8 h + 32 t + 16 (i >> 3) + (i & 7)
-        const int hi = qpos + 1 - k0 - 8 * h, lo = qlow - k0 - 8 * h, kp = a.keep - k0 - 8 * h;
+        const int hi = qpos + 1 - k0 - 8 * h, lo = window_start(qpos, a.window) - k0 - 8 * h, kp = a.keep - k0 - 8 * h;
 #pragma unroll
         for (int t = 0; t < KT; ++t)
 #pragma unroll
@@ -480,10 +512,10 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     };
     // One block's scores, the weights of the one before and the value products of the one before that: a product and a
     // few vector instructions in turn
-    auto quick = [&](auto parted, bool one_max, const __bf16* kr, const __bf16* vr, __bf16* kw, __bf16* vw, int bk, int bv, const f32x16 (&Si)[KT],
+    auto quick = [&](auto parted, const Places& at, bool one_max, const __bf16* kr, const __bf16* vr, __bf16* kw, __bf16* vw, int bk, int bv, const f32x16 (&Si)[KT],
                      f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT], bf16x8 (&Po)[2 * KT]) SF_INLINE {
-      constexpr int NP = 2 * KT * NV, NF = NP + KT * ND, LA = KT == 1 ? 2 : 3;
-      constexpr bool MSUM = KT > 1;   // the weights' sums by products with a half (one tile: the registers are not there)
+      constexpr int NP = 2 * KT * NV, NF = NP + KT * ND, LA = TURNS ? 2 : 3;
+      constexpr bool MSUM = !TURNS;   // the weights' sums by products with a half
       constexpr int NS = NF + (MSUM ? 2 * KT : 0);
       constexpr int WE = (MSUM ? 56 : 88) * KT, WR = 16 * NV;
       constexpr int NB = std::min(std::max(NP, NS * WE / (WE + WR)), NS - 4 * KT - 1);   // slots of the exponentials; then O's factors
@@ -495,7 +527,11 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       auto vt_of = [](int n) { return n % (KP * NV) / (2 * KP) * 2 + n % 2; };
       auto ks_of = [](int n) { return n / (KP * NV) * KP + n % (2 * KP) / 2; };
       bf16x8 fr[NF];
-      auto frag = [&](int n) SF_INLINE { fr[n] = n < NP ? vf(vr, vt_of(n), ks_of(n)) : kf(kr, (n - NP) % KT, (n - NP) / KT); };
+      auto tile_of = [](int n) { return TURNS ? (n - NP) / ND : (n - NP) % KT; };
+      auto step_of = [](int n) { return TURNS ? (n - NP) % ND : (n - NP) / KT; };
+      // (TURNS: a tile's weights are done before the products that take its scores' registers)
+      static_assert(!TURNS || (NB <= KT * NP && NB <= NP + ND), "scores and weights of a tile in the same registers");
+      auto frag = [&](int n) SF_INLINE { fr[n] = n < NP ? vf(vr, vt_of(n), ks_of(n)) : kf(kr, at, tile_of(n), step_of(n)); };
       const int kpg = bt[min((bk + 16 * sg) >> a.bs_shift, last_page)], vpg = bt[min((bv + 16 * sg) >> a.bs_shift, last_page)];
 #pragma unroll
       for (int n = 0; n < LA; ++n) frag(n);
@@ -529,10 +565,10 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       for (int i = 0; i < 16; ++i) {
         sums[i] = 0.f;
 #pragma unroll
-        for (int t = 0; t < KT; ++t) So[t][i] = 0.f;
+        for (int t = 0; t < KT && !TURNS; ++t) So[t][i] = 0.f;
       }
-#pragma unroll
-      for (int n = 0; n < NS; ++n) {
+      each(std::make_integer_sequence<int, NS>(), [&](auto slot) SF_INLINE {
+        constexpr int n = slot;
         __builtin_amdgcn_sched_barrier(0);
         const bool summing = MSUM && n >= SUM0 && n < SUM0 + 4 * KT && (n - SUM0) % 2 == 0;
         const int f = !MSUM || n < SUM0 ? n : n < SUM0 + 4 * KT ? SUM0 + (n - SUM0) / 2 : n - 2 * KT;   // fragment of this slot
@@ -548,8 +584,8 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
           O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], Pi[ks_of(f)], O[vt], 0, 0, 0);
           hold(O[vt]);
         } else {
-          const int t = (f - NP) % KT;
-          So[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], qf[(f - NP) / KT], So[t], 0, 0, 0);
+          const int t = tile_of(f), st = step_of(f);
+          So[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], qf[st], TURNS && st == 0 ? f32x16{} : So[t], 0, 0, 0);
           hold(So[t]);
         }
         if (n == 1) {
@@ -588,7 +624,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
             hold(static_cast<float>(O[c / 16][c % 16]));
           }
         }
-      }
+      });
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < 2 * KT; ++ks)
@@ -612,23 +648,28 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     const int above = WIN ? max(edge_lo, low_first) : -1;   // (block i - 2 has a key that the wave sees)
     const int quick0 = max(nk + 2, nk + ((above + BLK - kbeg) / BLK) + 1);
     const int quick1 = wave_on ? nk + min(min(nb - nk, (pos_first + 1 - kbeg + BLK) / BLK), (pos_last - kbeg) / BLK + 1) : 0;
-    auto quick_step = [&](auto parted, int i, const f32x16 (&Si)[KT], f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT],
+    auto quick_step = [&](auto parted, const Places& at, int i, const f32x16 (&Si)[KT], f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT],
                           bf16x8 (&Po)[2 * KT]) SF_INLINE {
-      quick(parted, i - 1 >= kSplitBlocks, kbuf(i), vbuf(i), kbuf(i + 1), vbuf(i + 1), kbeg + (i + 1 - nk) * BLK,
+      quick(parted, at, i - 1 >= kSplitBlocks, kbuf(i), vbuf(i), kbuf(i + 1), vbuf(i + 1), kbeg + (i + 1 - nk) * BLK,
             kbeg + (i - 1 - nk) * BLK, Si, So, Pi, Po);
       wait_sent();
       __syncthreads();
     };
-    auto quick_two = [&](auto parted, int i) SF_INLINE {
-      f32x16 S2[KT];
+    auto quick_two = [&](auto parted, const Places& at, int i) SF_INLINE {
+      f32x16 other[KT];
+      f32x16 (&S2)[KT] = TURNS ? S : other;
       bf16x8 P2[2 * KT];
-      quick_step(parted, i, S, S2, P, P2);
-      quick_step(parted, i + 1, S2, S, P2, P);
+      quick_step(parted, at, i, S, S2, P, P2);
+      quick_step(parted, at, i + 1, S2, S, P2, P);
     };
     for (int i = 0; i < nb; ++i) {
-      if constexpr (MT > 1)
-        for (; i >= quick0 && i + 1 < quick1 && i - 2 < kSplitBlocks; i += 2) quick_two(std::true_type(), i);
-      for (; i >= quick0 && i + 1 < quick1; i += 2) quick_two(std::false_type(), i);
+      if (i >= quick0 && i + 1 < quick1) {
+        Places at;
+        places(at);
+        if constexpr (MT > 1)
+          for (; i + 1 < quick1 && i - 2 < kSplitBlocks; i += 2) quick_two(std::true_type(), at, i);
+        for (; i + 1 < quick1; i += 2) quick_two(std::false_type(), at, i);
+      }
       if (i == nb) break;
       if (i + 1 < nb) send_block_k(bt, last_page, block_key(i + 1), kbuf(i + 1));
       if (i >= 1) send_block_v(block_key(i - 1), vbuf(i + 1));
@@ -653,10 +694,12 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     bf16x4 gates[8];   // of the wave's half of the channels
     if constexpr (NMAP == 2) {
       if (a.gate != nullptr) {
-        const __bf16* gt = static_cast<const __bf16*>(a.gate) + row * a.gate_stride +
-                           static_cast<int64_t>(g * rep + (valid ? col - tok * rep : 0)) * DV + mp * (DV / 2) + 4 * h;
+        const int ln = fresh(lane);
+        const Column c = column(ln);
+        const __bf16* gt = static_cast<const __bf16*>(a.gate) + static_cast<int64_t>(row0 + qo + c.tok) * a.gate_stride +
+                           static_cast<int64_t>(g * rep + c.member) * DV + mp * (DV / 2) + 4 * (ln >> 5);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) gates[c] = *reinterpret_cast<const bf16x4*>(gt + 8 * c);
+        for (int j = 0; j < 8; ++j) gates[j] = *reinterpret_cast<const bf16x4*>(gt + 8 * j);
       }
     }
     if (needed(nb - 1)) values(vbuf(nb + 1), P, nb - 1 < kSplitBlocks);
@@ -728,11 +771,15 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
           *reinterpret_cast<u32x4*>(ob + (static_cast<int64_t>(token_of(cc)) * (H / 2 - rep) + cc) * DV) = e;
       }
     } else {
-      const float inv = valid && l > 0.f ? head_gate_of<__bf16>(a, row, head) / l : 0.f;
+      const int ln = fresh(lane), er = ln & 31, eh = ln >> 5, el = ln >> 3, ec = ln & 7;
+      const Column c = column(ln);
+      const int64_t row = row0 + qo + c.tok;
+      const int head = g * rep + c.member;
+      const float inv = c.valid && l > 0.f ? head_gate_of<__bf16>(a, row, head) / l : 0.f;
       if (MANY) __syncthreads();
       if (a.out_f32) {
-        if (valid) {
-          float* o = static_cast<float*>(out) + (row * H + head) * DV + 4 * h;
+        if (c.valid) {
+          float* o = static_cast<float*>(out) + (row * H + head) * DV + 4 * eh;
 #pragma unroll
           for (int vt = 0; vt < NV; ++vt)
 #pragma unroll
@@ -744,8 +791,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
         // 64 channels at a time through LDS, the wave's own 4 KB (32 rows of 128 bytes, chunks changing places), so that
         // a store has whole rows: 8-byte pieces of 32 rows kept the memory pipe busy for 2 us per piece of work.  (What
         // depends on the lane is worked out here: kept over a piece it was spilled, and its reload waited for the stores.)
-        const int ln = fresh(lane), er = ln & 31, eh = ln >> 5, el = ln >> 3, ec = ln & 7;
-        char* x = (MANY ? lds_x : reinterpret_cast<char*>(lds_k)) + w * 4096;
+        char* x = (XV ? reinterpret_cast<char*>(lds_v) : MANY ? lds_x : reinterpret_cast<char*>(lds_k)) + w * 4096;
         __bf16* ob = static_cast<__bf16*>(out) + (static_cast<int64_t>(row0 + qo) * H + g * rep) * DV + 8 * ec;
 #pragma unroll
         for (int v2 = 0; v2 < NV / 2; ++v2) {
@@ -774,14 +820,14 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   }
 }
 
-template <int ND, int NV, int NMAP, int NW, int KT>
+template <int ND, int NV, int NMAP, int NW>
 bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, const AttnArgs& a,
             int num_tiles, int cus, hipStream_t st) {
   constexpr int COLS = NW / NMAP * 32;
   const int chunks = (kTileTokens * (a.H / a.G) + COLS - 1) / COLS, heads = a.G / NMAP;
   const int pieces = num_tiles * chunks;
   const int workers = NW == 8 ? std::min(pieces, std::max({1, cus / heads, (pieces + kPieces - 1) / kPieces})) : pieces;
-  auto* kernel = a.window > 0 ? sink_flash_kernel<ND, NV, NMAP, NW, KT, true> : sink_flash_kernel<ND, NV, NMAP, NW, KT, false>;
+  auto* kernel = a.window > 0 ? sink_flash_kernel<ND, NV, NMAP, NW, true> : sink_flash_kernel<ND, NV, NMAP, NW, false>;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(workers) * heads), dim3(NW * 64), 0, st, out,
                      static_cast<const __bf16*>(q), static_cast<const __bf16*>(k_cache),
                      static_cast<const __bf16*>(v_cache), a, num_tiles, chunks, workers);
@@ -797,8 +843,7 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
 // Four or eight waves: pieces of 128 columns up to 6 per CU, and tiles that do not fill eight waves (24 over 8 heads: 192
 // of 256 columns), go four by four.  us, whole layer, before / four waves / eight: 32 + 8 heads, 256 pieces (2 x 500) 34.5 /
 // 30.1 / 37.1; 768 (6 x 500) 58.1 / 54.3 / 56.1; 1220 (5 x 1000) 95.2 / 82.3 / 87.8; 1904 (4 x 2048) 198.1 / 182.7 / 180.0;
-// 24 + 8 heads 624 (3 x 777) 47.8 / 42.3 / 47.9, 1400 (2 x 3000) 177.7 / 146.0 / 157.4.  The latent form keeps 32 keys per
-// block: 64 scores and weights more than fill its registers (O and Q are 160).
+// 24 + 8 heads 624 (3 x 777) 47.8 / 42.3 / 47.9, 1400 (2 x 3000) 177.7 / 146.0 / 157.4.
 // The workgroups of the latent form hold 8 tokens: so far ahead a NaN value reaches back (a weight of 0 times NaN).
 bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void* v_cache,
                        const AttnArgs& a, int num_tiles, hipStream_t st) {
@@ -810,17 +855,17 @@ bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void
     return false;
   const int columns = kTileTokens * (a.H / a.G);
   const bool few = columns % 256 != 0 || static_cast<int64_t>(num_tiles) * ((columns + 127) / 128) * a.G <= 6 * cus;
-#define SF(D, V, MAPS, NW, KT)                              \
+#define SF(D, V, MAPS, NW)                                   \
   if (a.dim == D && a.vdim == V && (a.pair ? 2 : 1) == MAPS) \
-    return sf::launch<D / 16, V / 32, MAPS, NW, KT>(out, q, k_cache, v_cache, a, num_tiles, cus, st);
+    return sf::launch<D / 16, V / 32, MAPS, NW>(out, q, k_cache, v_cache, a, num_tiles, cus, st);
   if (few) {
-    SF(64, 64, 1, 4, 2)
-    SF(128, 128, 1, 4, 2)
+    SF(64, 64, 1, 4)
+    SF(128, 128, 1, 4)
   }
-  SF(64, 64, 1, 8, 2)
-  SF(128, 128, 1, 8, 2)
-  SF(256, 192, 1, 8, 1)
-  SF(64, 128, 2, 8, 2)
+  SF(64, 64, 1, 8)
+  SF(128, 128, 1, 8)
+  SF(256, 192, 1, 8)
+  SF(64, 128, 2, 8)
 #undef SF
   return false;
 }

@@ -1199,6 +1199,38 @@ def test_flash_window_without_expired_keys(H, G, d, dv, window, keep):
     assert torch.allclose(got.cpu().float(), want.float(), atol=4e-2, rtol=4e-2)
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(8, 4, 64, 64), (8, 2, 128, 128), (5, 1, 256, 192)])
+def test_flash_weights_of_64_keys(H, G, d, dv):
+    """A weight is rounded to 8 bits against the largest score of its own 64 keys and of all before them, in every form:
+    fp32 results are those of such weights but for the scores' rounding in 32 bits."""
+    torch.manual_seed(d)
+    n, scale = 500, 1.2 * d ** -0.5
+    md = ragged([n], [0], [0], width=32)
+    nb = md["num_pages"]
+    q = torch.randn(n, H, d).to(torch.bfloat16)
+    k, v = torch.randn(nb, G, 16, d).to(torch.bfloat16), torch.randn(nb, G, dv, 16).to(torch.bfloat16)
+    sink = torch.randn(H)
+    g = cuda(md)
+    got = mx.sink_attention(q.cuda(), k.cuda(), v.cuda(), g["block_tables"], g["seq_kvlen"], g["seq_qstart"], g["tile_seq"],
+                            g["tile_qoff"], scale, True, sink_values=sink.cuda(), out_dtype=torch.float32).cpu().double()
+    pages = md["block_tables"][0, :-(-n // 16)].long()
+    ks = k[pages].permute(1, 0, 2, 3).reshape(G, -1, d)[:, :n].double().repeat_interleave(H // G, 0)
+    vs = v[pages].permute(1, 0, 3, 2).reshape(G, -1, dv)[:, :n].double().repeat_interleave(H // G, 0)
+    s = torch.bmm(q.double().transpose(0, 1), ks.transpose(1, 2).contiguous()) * (scale / np.log(2))
+    s.masked_fill_(torch.ones(n, n, dtype=torch.bool).triu(1), float("-inf"))
+    m = (sink.double() / np.log(2)).view(H, 1).expand(H, n)
+    l, o = torch.ones(H, n, dtype=torch.float64), torch.zeros(H, n, dv, dtype=torch.float64)
+    for b in range(0, n, 64):
+        top = torch.maximum(m, s[:, :, b:b + 64].amax(-1))
+        p = torch.exp2(s[:, :, b:b + 64] - top[..., None]).to(torch.bfloat16).double()
+        f = torch.exp2(m - top)
+        l, o, m = l * f + p.sum(-1), o * f[..., None] + torch.bmm(p, vs[:, b:b + 64]), top
+    want = (o / l[..., None]).transpose(0, 1)
+    # scores of up to 16 (log2 units) are off by 2^-20 or so: a weight in 2^11 rounds the other way, by 2^-8.  (Maxima per 32
+    # keys: 1e-3.)
+    assert float((got - want).norm() / want.norm()) < 1.5e-4
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
