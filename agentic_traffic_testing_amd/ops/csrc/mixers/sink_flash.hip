@@ -26,6 +26,12 @@
 // behind the present one's last steps.  Batches whose pieces of 128 columns number up to six per CU run one piece per
 // workgroup of four waves, two workgroups per CU (the rule, with both sides measured, at launch_sink_flash).
 //
+// Short prompts: with its start and its masked blocks a piece of one block is latency from end to end, so its first values
+// come with its first keys, its queries behind its first pages, and the parts' products have their operands on the way and go
+// on different sums in turn.  Kernel, us, one part after the other / pipeline without this / now: one prompt of 17 tokens,
+// 32 + 8 heads 6.0 / 6.8 / 6.3, latent 14.9 / 14.7 / 12.3, 16 + 4 heads of 64 4.8 / 5.4 / 5.2; of 188 tokens 10.4 / 10.7 / 9.6,
+// 21.8 / 22.4 / 18.3, 7.6 / 8.2 / 7.8; 475 tokens on 2000 cached ones 71 / 45 / 44, 138 / 115 / 94, 50 / 34 / 33.
+//
 // Pair form: a workgroup's first four waves carry the first map, the other four the second one, over the
 // same columns and one V block; at the end each wave finishes half of the channels.
 //
@@ -63,38 +69,44 @@ constexpr int kSplitBlocks = 4;
 constexpr float kLog2e = 1.44269504088896341f;
 #define SF_INLINE __attribute__((always_inline))
 
-__device__ __forceinline__ float xor32(float v, int idx4) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(idx4, __builtin_bit_cast(int, v)));
-}
-// larger value of the lane's and lane ^ 32's (the builtin's two results are taken for one where both operands are the
-// same value)
-__device__ __forceinline__ float both(float v) {
+// larger value, or the sum, of the lane's and lane ^ 32's (the builtin's two results are taken for one where both operands
+// are the same value)
+__device__ __forceinline__ f32x2 halves(float v) {
   float a = v, b = v;
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
 #endif
-  return fmaxf(a, b);
+  return f32x2{a, b};
 }
-// 16 (send4: 4) bytes per lane from base + offset to 64 lanes' LDS from `to` on, without registers; there after
-// wait_sent().  (After the builtin the compiler makes every read of LDS wait for all transfers.)
-// The base goes through a scalar move: five wait states belong between a vector instruction that writes a scalar register,
-// such as the reload of a spilled one, and a memory instruction that reads it, and the compiler does not put them in front
-// of assembly.  (The same in flash_prefill.hip, a library of its own.)
-__device__ __forceinline__ void send16(const void* base, uint32_t offset, void* to) {
+__device__ __forceinline__ float both(float v) {
+  const f32x2 x = halves(v);
+  return fmaxf(x[0], x[1]);
+}
+__device__ __forceinline__ float both_sum(float v) {
+  const f32x2 x = halves(v);
+  return x[0] + x[1];
+}
+// 16 (send4: 4) bytes per lane from base + offset to 64 lanes' LDS from address `to` on, without registers; there after
+// wait_sent().  (After the builtin the compiler makes every read of LDS wait for all transfers.)  The base goes through a
+// scalar move: five wait states belong between a vector instruction that writes a scalar register, such as the reload of
+// a spilled one, and a memory instruction that reads it, and the compiler does not put them in front of assembly.  (The
+// same in flash_prefill.hip, a library of its own.)
+__device__ __forceinline__ void send16(const void* base, uint32_t offset, uint32_t to) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
   uint64_t from;
   asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
-               : "=&s"(from) : "v"(offset), "s"(base), "s"(at) : "m0", "memory");
+               : "=&s"(from) : "v"(offset), "s"(base), "s"(to) : "m0", "memory");
 #endif
 }
-__device__ __forceinline__ void send4(const void* base, uint32_t offset, void* to) {
+__device__ __forceinline__ void send4(const void* base, uint32_t offset, uint32_t to) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
   uint64_t from;
   asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dword %1, %0"
-               : "=&s"(from) : "v"(offset), "s"(base), "s"(at) : "m0", "memory");
+               : "=&s"(from) : "v"(offset), "s"(base), "s"(to) : "m0", "memory");
 #endif
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(const_cast<void*>(p))));
 }
 __device__ __forceinline__ void wait_sent() {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -157,7 +169,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   const int gv = NMAP == 2 ? g : g / a.v_share;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 31, h = lane >> 5, x32 = (lane ^ 32) << 2;
+  const int r = lane & 31, h = lane >> 5;
   const int mp = NMAP == 2 ? w / CW : 0;            // the wave's map
   const float scale2 = a.scale * kLog2e;
   const uint32_t per = 0xffffffffu / rep + 1;       // (columns x rep < 2^32; rep 1: 0)
@@ -174,7 +186,9 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     k_src[u] = 2u * (row * DK + ((lane % CK) ^ ((row / RB) & (CK - 1) & 15)) * 8);
   }
   const int v_half = 8 * ((lane ^ (lane >> 4)) & 1);
-  const uint32_t v_src = 2u * ((32 * part + (lane >> 1)) * bs + v_half);
+  uint32_t v_src[TURNS ? 1 : VU];
+#pragma unroll
+  for (int u = 0; u < (TURNS ? 1 : VU); ++u) v_src[u] = 2u * ((32 * (u * WPG + part) + (lane >> 1)) * bs + v_half);
   const int k_lds = 16 * sg * DK + part * 512, v_lds = sg * DV * 16 + part * 512;
   const __bf16* k_base = k_cache + static_cast<int64_t>(NMAP * g) * bs * DK;
   const __bf16* v_base = v_cache + static_cast<int64_t>(gv) * DV * bs;
@@ -185,27 +199,37 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   auto v_at = [&](int pg, int k0) SF_INLINE {
     return v_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * v_page + ((k0 + 16 * sg) & (bs - 1));
   };
-  auto send_k = [&](const __bf16* kb, __bf16* to, int u) SF_INLINE {
+  // (`b`: which of the two buffers, its lowest bit)
+  const uint32_t k_to = lds_address(lds_k) + 2 * k_lds, v_to = lds_address(lds_v) + 2 * v_lds;
+  auto send_k = [&](const __bf16* kb, int b, int u) SF_INLINE {
+    const uint32_t to = k_to + (b & 1) * 2 * KB + u % KU * WPG * 1024 + u / KU * 2 * BLK * DK;
     if constexpr (TURNS) {   // rows 4 further on: bits 2 and 3 of the chunk's place
       static_assert(!TURNS || (NMAP == 1 && CK == 32 && WPG == 2), "four rows per transfer of the group's waves");
-      send16(kb + 4 * u * DK, fresh(k_src[0]) ^ (64u * u), to + k_lds + u * WPG * 512);
+      send16(kb + 4 * u * DK, fresh(k_src[0]) ^ (64u * u), to);
     } else if (KU * WPG == KN || (u % KU) * WPG + part < KN) {
-      send16(kb + (u / KU) * bs * DK, k_src[u % KU], to + (u / KU) * BLK * DK + k_lds + (u % KU) * WPG * 512);
+      send16(kb + (u / KU) * bs * DK, k_src[u % KU], to);
     }
   };
-  auto send_v = [&](const __bf16* vb, __bf16* to, int u) SF_INLINE {
-    if (VU * WPG == VN || u * WPG + part < VN) send16(vb + 32 * u * WPG * bs, v_src, to + v_lds + u * WPG * 512);
+  auto send_v = [&](const __bf16* vb, int b, int u) SF_INLINE {
+    const uint32_t to = v_to + (b & 1) * 2 * VB + u * WPG * 1024;
+    if (VU * WPG == VN || u * WPG + part < VN) send16(TURNS ? vb + 32 * u * WPG * bs : vb, v_src[TURNS ? 0 : u], to);
   };
   // ---- fragments.  A row of the score products: key with bits 2 and 3 swapped
-  const int krow = (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);
-  const int kfrag = mp * BLK * DK + krow * DK, vfrag = r * 16 + 8 * (h ^ ((r >> 3) & 1));
+  const int vfrag = r * 16 + 8 * (h ^ ((r >> 3) & 1));
   constexpr int KO = ND < 8 ? ND : 8;
-  const int kplace = kfrag + (h ^ ((krow / RB) & (CK - 1) & 15)) * 8;   // of step 0; of the others:
-  typedef int Places[KO];
-  auto places = [&](Places& to) SF_INLINE {
-    const int k = TURNS ? fresh(kplace) : kplace;
+  typedef int Places[KO];   // of the first steps of a row
+  auto places_of = [&](int ln, Places& to) SF_INLINE {
+    const int row = (ln & 19) | ((ln & 4) << 1) | ((ln & 8) >> 1);
+    const int at = mp * BLK * DK + row * DK + ((ln >> 5) ^ ((row / RB) & (CK - 1) & 15)) * 8;
 #pragma unroll
-    for (int st = 0; st < KO; ++st) to[st] = k ^ (16 * st);
+    for (int st = 0; st < KO; ++st) to[st] = at ^ (16 * st);
+  };
+  Places kept;
+  if (!TURNS) places_of(lane, kept);
+  auto places = [&](Places& to) SF_INLINE {   // (TURNS: no registers to keep them)
+    if (TURNS) return places_of(fresh(lane), to);
+#pragma unroll
+    for (int st = 0; st < KO; ++st) to[st] = kept[st];
   };
   auto kf = [&](const __bf16* b, const Places& at, int t, int st) SF_INLINE {
     return *reinterpret_cast<const bf16x8*>(b + 32 * t * DK + at[st % 8] + st / 8 * 128);
@@ -225,7 +249,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   };
   auto cols_of = [&](const Piece& p) SF_INLINE { return min(kTileTokens, p.n - p.qo) * rep; };
   auto kend_of = [&](const Piece& p) SF_INLINE {
-    return p.kvlen - p.n + p.qo + (min(cols_of(p), p.col0 + COLS) - 1) / rep + 1;
+    return p.kvlen - p.n + p.qo + token_of(min(cols_of(p), p.col0 + COLS) - 1) + 1;
   };
   auto fetch = [&](int item) SF_INLINE {
     Piece p;
@@ -236,11 +260,14 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     if (p.n <= 0 || p.kvlen <= 0 || p.qo >= p.n || p.col0 >= min(kTileTokens, p.n - p.qo) * rep) p.n = 0;
     return p;
   };
-  if constexpr (MANY) {
+  // (one piece each: no trip through LDS)
+  const bool many = MANY && pieces > workers;
+  const Piece only = fetch(pieces - 1 - worker);
+  if (many) {
     // Long ones first: a piece's rank among the tiles' numbers of blocks, found by bisection of the keys (blocks, then
     // place in the list: no two are alike), which every wave holds for itself
     constexpr int KR = kSortTiles / 64;
-    if (pieces > workers && num_tiles <= kSortTiles) {
+    if (num_tiles <= kSortTiles) {
       unsigned int key[KR];
       Piece own[KR];
       const int most = (a.bt_width << a.bs_shift) / BLK + 2;
@@ -287,46 +314,45 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   }
   // the next piece with work, from number k on
   auto next_piece = [&](int& k, Piece& p) SF_INLINE {
-    if constexpr (!MANY) {
-      if (k > 0) return false;
-      p = fetch(pieces - 1 - worker);
-      return p.n > 0;
-    } else {
-      // (each workgroup begins at another of its pieces: queries and results of all of them do not come at once)
-      for (; k < mine; ++k) {
-        const int* e = lds_piece[(k + worker) % mine];
-        p.n = __builtin_amdgcn_readfirstlane(e[4]);
-        if (p.n == 0) continue;
-        p.s = __builtin_amdgcn_readfirstlane(e[0]), p.qo = __builtin_amdgcn_readfirstlane(e[1]);
-        p.col0 = __builtin_amdgcn_readfirstlane(e[2]), p.row0 = __builtin_amdgcn_readfirstlane(e[3]);
-        p.kvlen = __builtin_amdgcn_readfirstlane(e[5]);
-        return true;
-      }
-      return false;
+    if (!many) {
+      p = only;
+      return k == 0 && p.n > 0;
     }
+    // (each workgroup begins at another of its pieces: queries and results of all of them do not come at once)
+    for (; k < mine; ++k) {
+      const int* e = lds_piece[MANY ? (k + worker) % mine : 0];
+      p.n = __builtin_amdgcn_readfirstlane(e[4]);
+      if (p.n == 0) continue;
+      p.s = __builtin_amdgcn_readfirstlane(e[0]), p.qo = __builtin_amdgcn_readfirstlane(e[1]);
+      p.col0 = __builtin_amdgcn_readfirstlane(e[2]), p.row0 = __builtin_amdgcn_readfirstlane(e[3]);
+      p.kvlen = __builtin_amdgcn_readfirstlane(e[5]);
+      return true;
+    }
+    return false;
   };
   // ---- what a piece needs before its first step
   auto pages_of = [&](const Piece& p) SF_INLINE { return min((kend_of(p) + bs - 1) >> a.bs_shift, kPages); };   // (the launcher bounds the table)
   // key blocks: the kept keys in front of the window, then from the window's start (block-aligned)
-  auto klow_of = [&](const Piece& p) SF_INLINE { return window_start(p.kvlen - p.n + p.qo + p.col0 / rep, a.window); };
+  auto klow_of = [&](const Piece& p) SF_INLINE { return window_start(p.kvlen - p.n + p.qo + token_of(p.col0), a.window); };
   auto first_key = [&](const Piece& p) SF_INLINE { return min(a.keep, klow_of(p) & ~(BLK - 1)) > 0 ? 0 : klow_of(p) & ~(BLK - 1); };
-  auto send_pages = [&](const Piece& p, int* bt) SF_INLINE {
+  auto send_pages = [&](const Piece& p, int from, int list) SF_INLINE {   // of the page list from entry `from` on, into list 0 or 1
     const int* btg = a.block_tables + static_cast<int64_t>(p.s) * a.bt_width;
-    const int npages = pages_of(p);
-    for (int i = w * 64; i < npages; i += NW * 64)
-      if (i + lane < npages) send4(btg, 4u * (i + lane), bt + i);
+    const int npages = pages_of(p), ln = fresh(lane);
+    for (int i = from + w * 64; i < npages; i += NW * 64)
+      if (i + ln < npages) send4(btg, 4u * (i + ln), lds_address(lds_bt) + 4 * (list * kPages + i));
   };
-  auto send_block_k = [&](const int* bt, int last_page, int k0, __bf16* to) SF_INLINE {
+  auto send_block_k = [&](const int* bt, int last_page, int k0, int b) SF_INLINE {
     const __bf16* kb = k_at(__builtin_amdgcn_readfirstlane(bt[min((k0 + 16 * sg) >> a.bs_shift, last_page)]), k0);
 #pragma unroll
-    for (int u = 0; u < NMAP * KU; ++u) send_k(kb, to, u);
+    for (int u = 0; u < NMAP * KU; ++u) send_k(kb, b, u);
   };
   bf16x8 qf[ND];
-  auto load_q = [&](const Piece& p) SF_INLINE {
+  auto load_q = [&](const Piece& p, bool real) SF_INLINE {
     const int ln = fresh(lane), col = p.col0 + (w % CW) * 32 + (ln & 31);
     const bool valid = col < cols_of(p);
     const int tok = valid ? token_of(col) : 0, head = (NMAP * g + mp) * rep + (valid ? col - tok * rep : 0);
-    const __bf16* qp = q + (p.row0 + p.qo + tok) * a.q_stride + static_cast<int64_t>(head) * DK + 8 * (ln >> 5);
+    // (`real` false: nobody reads them; one row, whose lines are one)
+    const __bf16* qp = q + (real ? (p.row0 + p.qo + tok) * a.q_stride + static_cast<int64_t>(head) * DK + 8 * (ln >> 5) : 0);
 #pragma unroll
     for (int st = 0; st < ND; ++st) qf[st] = *reinterpret_cast<const bf16x8*>(qp + 16 * st);
   };
@@ -339,18 +365,22 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
 #pragma unroll
     for (int st = 0; st < ND; ++st) hold(qf[st]);
   };
-  send_pages(now, lds_bt[0]);
-  load_q(now);
-  hold_q();
-  wait_sent();
+  {   // queries on their way behind the first pages, which do not wait for them
+    const int* btg = a.block_tables + static_cast<int64_t>(now.s) * a.bt_width;
+    const int npages = pages_of(now), page = btg[max(min(tid, npages - 1), 0)];
+    load_q(now, true);
+    if (tid < npages) lds_bt[0][tid] = page;
+    if (npages > NW * 64) {
+      send_pages(now, NW * 64, 0);
+      wait_sent();
+    }
+  }
   __syncthreads();
-  send_block_k(lds_bt[0], pages_of(now) - 1, first_key(now), lds_k);
-  wait_sent();
-  __syncthreads();
+  send_block_k(lds_bt[0], pages_of(now) - 1, first_key(now), 0);
 
   for (int turn = 0;; ++turn) {
     ++pn;
-    nxt = now;   // (after the last one its queries are read once more, for nothing)
+    nxt = now;
     const bool more = next_piece(pn, nxt);
     const int* const bt = lds_bt[MANY ? turn & 1 : 0];
     const int qo = now.qo, row0 = now.row0, kvlen = now.kvlen, col0 = now.col0;
@@ -359,7 +389,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     const int wcol = col0 + (w % CW) * 32;            // the wave's first column
     const bool wave_on = wcol < cols_total;
     const int w_last = min(cols_total, wcol + 32) - 1;
-    const int pos_first = ctx + wcol / rep, pos_last = ctx + max(w_last, 0) / rep;
+    const int pos_first = ctx + token_of(wcol), pos_last = ctx + token_of(max(w_last, 0));
     const int kend = kend_of(now), last_page = pages_of(now) - 1;
     const int klow = klow_of(now), kbeg = klow & ~(BLK - 1);   // no column sees keys in [keep, klow)
     const int nk = (min(a.keep, kbeg) + BLK - 1) / BLK;
@@ -378,13 +408,12 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       c.member = c.valid ? col - c.tok * rep : 0;
       return c;
     };
-    const Column c0 = column(lane);
+    const Column c0 = column(fresh(lane));
     const int head = (NMAP * g + mp) * rep + c0.member;
-    const int qpos = c0.valid ? ctx + c0.tok : -1;    // no key is visible to a column that is not there
     float m = kNegBig, l = 0.f;   // l: of the lane's keys
     if (a.sink) {   // the sink is the state the online softmax starts from (log2 units)
       m = a.sink_val != nullptr ? a.sink_val[head] * kLog2e : 0.f;
-      l = h == 0 ? 1.f : 0.f;
+      l = fresh(lane) < 32 ? 1.f : 0.f;
     }
     f32x16 O[NV];
 #pragma unroll
@@ -393,31 +422,22 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       for (int i = 0; i < 16; ++i) O[vt][i] = 0.f;
 
     // keys at or past kend read a clamped page or stale slots, keys in front of the window whatever is there: their
-    // scores are masked and their V zeroed (0 x NaN)
-    u32x4 vr[VU];
+    // scores are masked and their V zeroed (0 x NaN) once it is there, by the wave that fetched it
     auto seen = [&](int t) SF_INLINE { return t < kend && (!WIN || t >= klow || t < a.keep); };
-    auto edge = [&](int k0) SF_INLINE { return k0 + BLK > kend || (WIN && k0 < klow && k0 + BLK > a.keep); };
-    // (a block with such keys takes the way through registers: fetched here, put down by put_block_v)
-    auto send_block_v = [&](int k0, __bf16* to) SF_INLINE {
+    auto send_block_v = [&](int k0, int b) SF_INLINE {
       const __bf16* vb = v_at(__builtin_amdgcn_readfirstlane(bt[min((k0 + 16 * sg) >> a.bs_shift, last_page)]), k0);
 #pragma unroll
-      for (int u = 0; u < VU; ++u) {
-        if (!edge(k0)) send_v(vb, to, u);
-        else if (VU * WPG == VN || u * WPG + part < VN)
-          vr[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb + 32 * u * WPG * bs) + v_src);
-      }
+      for (int u = 0; u < VU; ++u) send_v(vb, b, u);
     };
-    auto put_block_v = [&](int k0, __bf16* to) SF_INLINE {
-      if (!edge(k0)) return;
-      const int key = k0 + 16 * sg + v_half;
+    auto clear_block_v = [&](int k0, __bf16* to) SF_INLINE {
+      if (k0 + BLK <= kend && !(WIN && k0 < klow && k0 + BLK > a.keep)) return;
+      const int ln = fresh(lane), key = k0 + 16 * sg + 8 * ((ln ^ (ln >> 4)) & 1);
+      u32x4 seen2;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) seen2[j] = (seen(key + 2 * j) ? 0x0000ffffu : 0u) | (seen(key + 2 * j + 1) ? 0xffff0000u : 0u);
 #pragma unroll
       for (int u = 0; u < VU; ++u)
-        if (VU * WPG == VN || u * WPG + part < VN) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            vr[u][j] &= (seen(key + 2 * j) ? 0x0000ffffu : 0u) | (seen(key + 2 * j + 1) ? 0xffff0000u : 0u);
-          *reinterpret_cast<u32x4*>(to + v_lds + u * WPG * 512 + lane * 8) = vr[u];
-        }
+        if (VU * WPG == VN || u * WPG + part < VN) *reinterpret_cast<u32x4*>(to + v_lds + u * WPG * 512 + ln * 8) &= seen2;
     };
 
     // keys at or below the window start of the wave's latest column are outside somebody's window
@@ -428,16 +448,22 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       const int k0 = block_key(b);
       return b >= 0 && b < nb && wave_on && k0 <= pos_last && (k0 + BLK > low_first || k0 < a.keep);
     };
+    // (products with their operands on the way, on different sums in turn: left to the compiler each waited for its own)
     auto scores = [&](const __bf16* from, f32x16 (&S)[KT]) SF_INLINE {
       Places at;
       places(at);
+      constexpr int N = KT * ND, LA = TURNS ? 3 : 4;
+      bf16x8 fr[N];
+      auto read = [&](int n) SF_INLINE { fr[n] = kf(from, at, n % KT, n / KT); };
 #pragma unroll
-      for (int t = 0; t < KT; ++t) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
-#pragma unroll
-        for (int st = 0; st < ND; ++st) S[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf(from, at, t, st), qf[st], S[t], 0, 0, 0);
-      }
+      for (int n = 0; n < LA; ++n) read(n);
+      each(std::make_integer_sequence<int, N>(), [&](auto slot) SF_INLINE {
+        constexpr int n = slot;
+        __builtin_amdgcn_sched_barrier(0);
+        if (n + LA < N) read(n + LA);
+        S[n % KT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[n], qf[n / KT], n < KT ? f32x16{} : S[n % KT], 0, 0, 0);
+      });
+      __builtin_amdgcn_sched_barrier(0);
     };
     auto rescale = [&](float alpha) SF_INLINE {
 #pragma unroll
@@ -446,28 +472,44 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
         for (int i = 0; i < 16; ++i) O[vt][i] *= alpha;
     };
     auto values = [&](const __bf16* from, const bf16x8 (&P)[2 * KT], bool split) SF_INLINE {
-#pragma unroll
-      for (int e = 0; e < MT; ++e) {
+      constexpr int N = 2 * TPM * NV, LA = TURNS ? 3 : 4;
+      each(std::make_integer_sequence<int, MT>(), [&](auto half) SF_INLINE {
+        constexpr int e = half;
         if (e > 0 && split && __any(carry != 1.f)) rescale(carry);
+        bf16x8 fr[N];
+        auto read = [&](int n) SF_INLINE { fr[n] = vf(from, n % NV, 2 * e * TPM + n / NV); };
 #pragma unroll
-        for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-          for (int ks = 2 * e * TPM; ks < 2 * (e + 1) * TPM; ++ks)
-            O[vt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf(from, vt, ks), P[ks], O[vt], 0, 0, 0);
-      }
+        for (int n = 0; n < LA; ++n) read(n);
+        each(std::make_integer_sequence<int, N>(), [&](auto slot) SF_INLINE {
+          constexpr int n = slot;
+          __builtin_amdgcn_sched_barrier(0);
+          if (n + LA < N) read(n + LA);
+          O[n % NV] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[n], P[2 * e * TPM + n / NV], O[n % NV], 0, 0, 0);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
     };
     auto weights = [&](int b, f32x16 (&S)[KT], bf16x8 (&P)[2 * KT]) SF_INLINE {
       const int k0 = block_key(b);
       if (k0 + BLK - 1 > pos_first || (WIN && k0 <= edge_lo)) {
-        // register i of tile t holds key k0 + 8 h + 32 t + 16 (i >> 3) + (i & 7)
-        const int hi = qpos + 1 - k0 - 8 * h, lo = window_start(qpos, a.window) - k0 - 8 * h, kp = a.keep - k0 - 8 * h;
+        const int ln = fresh(lane);
+        const Column c = column(ln);
+        const int qpos = c.valid ? ctx + c.tok : -1;   // no key is visible to a column that is not there
+        // Register i of tile t holds key k0 + 8 h + 32 t + 16 (i >> 3) + (i & 7): bit 16 (i >> 3) + (i & 7) of a tile's
+        // word.  (A comparison per key, whose result waits in a scalar register: 800 cycles per block.)
+        auto below = [](int n) SF_INLINE { return n <= 0 ? 0u : n >= 32 ? ~0u : (1u << n) - 1; };
 #pragma unroll
-        for (int t = 0; t < KT; ++t)
+        for (int t = 0; t < KT; ++t) {
+          const int k8 = k0 + 8 * (ln >> 5) + 32 * t;
+          unsigned int out = ~below(qpos + 1 - k8);
+          if (WIN) out |= below(window_start(qpos, a.window) - k8) & ~below(a.keep - k8);
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const int o = 32 * t + 16 * (i >> 3) + (i & 7);
-            if (o >= hi || (WIN && o < lo && o >= kp)) S[t][i] = -INFINITY;
+            const float v = S[t][i];
+            const unsigned int x = __builtin_amdgcn_sbfe(out, 16 * (i >> 3) + (i & 7), 1);
+            S[t][i] = __builtin_bit_cast(float, (x & 0xff800000u) | (~x & __builtin_bit_cast(unsigned int, v)));
           }
+        }
       }
       float tmax[MT], mt[MT], psum[MT];
 #pragma unroll
@@ -512,7 +554,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     };
     // One block's scores, the weights of the one before and the value products of the one before that: a product and a
     // few vector instructions in turn
-    auto quick = [&](auto parted, const Places& at, bool one_max, const __bf16* kr, const __bf16* vr, __bf16* kw, __bf16* vw, int bk, int bv, const f32x16 (&Si)[KT],
+    auto quick = [&](auto parted, const Places& at, bool one_max, const __bf16* kr, const __bf16* vr, int b, int bk, int bv, const f32x16 (&Si)[KT],
                      f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT], bf16x8 (&Po)[2 * KT]) SF_INLINE {
       constexpr int NP = 2 * KT * NV, NF = NP + KT * ND, LA = TURNS ? 2 : 3;
       constexpr bool MSUM = !TURNS;   // the weights' sums by products with a half
@@ -593,8 +635,8 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
           vb = v_at(__builtin_amdgcn_readfirstlane(vpg), bv);
         }
         // the next blocks on their way
-        if (n >= 2 && n < 2 + NMAP * KU) send_k(kb, kw, n - 2);
-        if (n >= 2 + NMAP * KU && n < 2 + NMAP * KU + VU) send_v(vb, vw, n - 2 - NMAP * KU);
+        if (n >= 2 && n < 2 + NMAP * KU) send_k(kb, b, n - 2);
+        if (n >= 2 + NMAP * KU && n < 2 + NMAP * KU + VU) send_v(vb, b, n - 2 - NMAP * KU);
         if constexpr (PARTED) {   // O of two channel tiles between their products of the first and of the second tile
           constexpr int G2 = 2 * KP;
           if (n >= G2 && n < G2 + KP * NV) {
@@ -636,12 +678,6 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     // block i - 1 on their way to the other buffers
     f32x16 S[KT];
     bf16x8 P[2 * KT];
-#pragma unroll
-    for (int t = 0; t < KT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < 2 * KT; ++ks) P[ks] = bf16x8{};
     auto kbuf = [&](int i) SF_INLINE { return lds_k + (i & 1) * KB; };
     auto vbuf = [&](int i) SF_INLINE { return lds_v + (i & 1) * VB; };
     // steps [quick0, quick1): block i - 1 has no masked key, block i is needed
@@ -650,7 +686,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     const int quick1 = wave_on ? nk + min(min(nb - nk, (pos_first + 1 - kbeg + BLK) / BLK), (pos_last - kbeg) / BLK + 1) : 0;
     auto quick_step = [&](auto parted, const Places& at, int i, const f32x16 (&Si)[KT], f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT],
                           bf16x8 (&Po)[2 * KT]) SF_INLINE {
-      quick(parted, at, i - 1 >= kSplitBlocks, kbuf(i), vbuf(i), kbuf(i + 1), vbuf(i + 1), kbeg + (i + 1 - nk) * BLK,
+      quick(parted, at, i - 1 >= kSplitBlocks, kbuf(i), vbuf(i), i + 1, kbeg + (i + 1 - nk) * BLK,
             kbeg + (i - 1 - nk) * BLK, Si, So, Pi, Po);
       wait_sent();
       __syncthreads();
@@ -662,6 +698,14 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       quick_step(parted, at, i, S, S2, P, P2);
       quick_step(parted, at, i + 1, S2, S, P2, P);
     };
+    // (a workgroup's first values come with its first keys: a piece of few blocks waits once for both)
+    if (turn == 0) {
+      send_block_v(block_key(0), 0);
+      wait_sent();
+      hold_q();
+      clear_block_v(block_key(0), vbuf(0));
+      __syncthreads();
+    }
     for (int i = 0; i < nb; ++i) {
       if (i >= quick0 && i + 1 < quick1) {
         Places at;
@@ -671,25 +715,28 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
         for (; i + 1 < quick1; i += 2) quick_two(std::false_type(), at, i);
       }
       if (i == nb) break;
-      if (i + 1 < nb) send_block_k(bt, last_page, block_key(i + 1), kbuf(i + 1));
-      if (i >= 1) send_block_v(block_key(i - 1), vbuf(i + 1));
-      if (MANY && i == 0 && more) send_pages(nxt, lds_bt[(turn & 1) ^ 1]);
+      if (i + 1 < nb) send_block_k(bt, last_page, block_key(i + 1), i + 1);
+      const bool v_now = i > (turn == 0 ? 1 : 0);
+      if (v_now) send_block_v(block_key(i - 1), i + 1);
+      if (MANY && i == 0 && more) send_pages(nxt, 0, (turn & 1) ^ 1);
       if (needed(i - 2)) values(vbuf(i), P, i - 2 < kSplitBlocks);
       if (needed(i - 1)) weights(i - 1, S, P);
       if (needed(i)) scores(kbuf(i), S);
-      if (i >= 1) put_block_v(block_key(i - 1), vbuf(i + 1));
+      if (nb == 1 && turn == 0 && !(MANY && more)) break;   // (nothing on its way, and nothing that a wave writes next is read by another)
       wait_sent();
+      if (v_now) clear_block_v(block_key(i - 1), vbuf(i + 1));
       __syncthreads();
     }
     // steps nb and nb + 1 have no scores; the next piece's queries and first keys are on their way
-    send_block_v(block_key(nb - 1), vbuf(nb + 1));
-    if (MANY && more) send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), lds_k);
+    const bool v_now = nb > (turn == 0 ? 1 : 0);
+    if (v_now) send_block_v(block_key(nb - 1), nb + 1);
+    if (MANY && more) send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), 0);
     if (needed(nb - 2)) values(vbuf(nb), P, nb - 2 < kSplitBlocks);
-    if (MANY) load_q(nxt);
     if (needed(nb - 1)) weights(nb - 1, S, P);
-    put_block_v(block_key(nb - 1), vbuf(nb + 1));
+    if (MANY) load_q(nxt, more);
     if (MANY) hold_q();
     wait_sent();
+    if (v_now) clear_block_v(block_key(nb - 1), vbuf(nb + 1));
     __syncthreads();
     bf16x4 gates[8];   // of the wave's half of the channels
     if constexpr (NMAP == 2) {
@@ -704,7 +751,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     }
     if (needed(nb - 1)) values(vbuf(nb + 1), P, nb - 1 < kSplitBlocks);
 
-    l += xor32(l, x32);
+    l = both_sum(l);
     if constexpr (NMAP == 2) {
       // The two waves of a column set finish half of its channels each: they hand each other lam / l * O of the second
       // and O / l of the first map through LDS, add up their squares, and exchange the sums.
@@ -741,7 +788,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
             ss += o * o;
           }
         }
-      ss += xor32(ss, x32);
+      ss = both_sum(ss);
       if (h == 0) lds_ss[w][r] = ss;
       __syncthreads();
       ss += lds_ss[w ^ CW][r];

@@ -1231,6 +1231,33 @@ def test_flash_weights_of_64_keys(H, G, d, dv):
     assert float((got - want).norm() / want.norm()) < 1.5e-4
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(8, 4, 64, 64), (32, 8, 128, 128), (6, 2, 128, 128), (5, 1, 256, 192), (8, 4, 64, 128)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (300, 5), (450, 70), (1024, 4), (1000, 130)])
+def test_flash_long_windows(H, G, d, dv, window, keep):
+    """Windows and contexts of many blocks, where most steps are the dealt-out ones, kept keys in front of them (none, one,
+    two and three blocks), odd and even numbers of steps; a page list of more entries than a workgroup has threads."""
+    torch.manual_seed(d + H + window)
+    lens, starts = [700, 129, 64, 3, 65, 1], [0, 1301, 1990, 8300, 448, 0]
+    md = ragged(lens, starts, list(range(6)), width=520)
+    nb, T, pair = md["num_pages"], sum(lens), (d, dv) == (64, 128)
+    q = torch.randn(T, H, d).to(torch.bfloat16)
+    k = torch.randn(nb, G, 16, d).to(torch.bfloat16)
+    v = torch.randn(nb, G // 2 if pair else G, dv, 16).to(torch.bfloat16)
+    gate = torch.randn(T, H // 2 * dv).to(torch.bfloat16)
+
+    def run(m, to):
+        args = (to(q), to(k), to(v), m["block_tables"], m["seq_kvlen"], m["seq_qstart"], m["tile_seq"], m["tile_qoff"])
+        if pair:
+            return mx.differential_attention(*args, d ** -0.5, 0.4, 0.3, 1e-5, to(gate), 0, 0, window, keep)
+        return mx.sink_attention(*args, d ** -0.5, True, window=window, keep_first=keep, out_dtype=torch.float32)
+
+    want, got = run(md, lambda t: t).double(), run(cuda(md), lambda t: t.cuda()).cpu().double()
+    # A weight of 8 bits is off by at most 2^-9 of itself, the sum that it is divided by is that of the rounded ones; results
+    # of two maps in bf16, by the same again on both sides, and their difference is divided by its own size, at least half of
+    # a map's.  (A row's sum, its maximum or one key's weight that is off by a hundredth would be 1e-2.)
+    assert float((got - want).norm() / want.norm()) < (4 if pair else 1) * 2.0 ** -9
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
