@@ -1,6 +1,5 @@
 // Prefill flash attention over the paged KV cache, LDS-staged K/V tiles on 32x32x16 MFMA
-// (replaces the attention vLLM runs under engine.generate(), reference
-// llm/serve_llm.py:527-531).  Varlen batches, causal with a context offset (chunked prefill
+// (the attention that vLLM runs under engine.generate(), reference llm/serve_llm.py:527-531).  Varlen batches, causal with a context offset (chunked prefill
 // and prefix-cache hits: query token i of a sequence sits at position kvlen - qlen + i),
 // GQA G = Hq / Hkv in {1, 2, 3, 4, 8}, head_dim 128, bf16 / fp16 (G = 3: Llama-3.2-3B, 24 q /
 // 8 kv heads; a wave's last 32 mod 3 = 2 columns idle).
@@ -23,8 +22,18 @@
 // wave.  Blocks on the diagonal and both ends go part by part.  K and V of the next blocks go straight from memory to LDS in
 // the meantime: no registers, one wait and one workgroup barrier per block.  The sequence's block-table slice is staged in
 // LDS once so K/V addresses need no dependent global load inside the loop.
-// Layer times, us, before -> now: 32 + 8 heads 4 x 2k tokens 176.0 -> 167.1 (37.6 of it the rotation), 1 x 2000 70.1 -> 59.8,
-// 16 x 500 92.3 -> 86.9; 24 + 8 heads 3 x 777 41.7 -> 39.7.  Bound: matrix and vector units together, at a clock that gives way.
+// Short prompts and chunks behind a cached prefix: with its start and its masked blocks a workgroup of one block is latency
+// from end to end, so the first V comes with the first K, the queries behind the first pages, and the parts' products have
+// their operands on the way and go on different sums in turn.
+// Kernel, us, 32 + 8 heads, one part after the other / pipeline without this / now; bound by the chain of loads and parts: 17
+// tokens 5.6 / 6.6 / 6.2, 85 7.2 / 8.4 / 7.7, 188 9.5 / 10.5 / 9.4, 475 16.6 / 14.9 / 13.9; behind cached ones: 5 x 17 on 600
+// 17.5 / 15.9 / 15.0, 5 x 85 on 500 18.6 / 18.3 / 16.5, 188 on 512 20.8 / 17.9 / 16.7, 475 on 2000 40.9 / 36.0 / 34.1, 17 on 4096
+// (split) 29.8 / 29.6 / 28.3; bound by matrix and vector units together, at a clock that gives way: 16 x 100 14.3 / 13.6 / 12.4,
+// 1 x 2000 56 / 48.4 / 46.3, 4 x 2k 146 / 139 / 132.  24 + 8 heads: 17 tokens 5.2 / 6.5 / 6.2, 188 9.6 / 10.9 / 9.7, 4 x 2k
+// 122 / 116 / 110.
+#include <type_traits>
+#include <utility>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -44,6 +53,7 @@ constexpr float kRescale = 8.f;  // defer-max threshold (log2 units)
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;   // in memory, wherever it begins
 typedef __attribute__((address_space(3))) void* lds_ptr;
 #define FP_INLINE __attribute__((always_inline))
 
@@ -121,18 +131,25 @@ __device__ __forceinline__ float both_max(float v) {
 #endif
   return fmaxf(a, b);
 }
-// 16 bytes per lane from base + offset to 1 KB of LDS, without registers; there after wait_sent().  (After the builtin the
-// compiler makes every read of LDS wait for all transfers.)
-// The base goes through a scalar move: five wait states belong between a vector instruction that writes a scalar register,
-// such as the reload of a spilled one, and a memory instruction that reads it, and the compiler does not put them in front
-// of assembly.  (The same in mixers/sink_flash.hip, a library of its own.)
-__device__ __forceinline__ void send16(const void* base, uint32_t offset, void* to) {
+// 16 bytes per lane from base + offset to 1 KB of LDS from address `to` on, without registers; there after wait_sent().
+// (After the builtin the compiler makes every read of LDS wait for all transfers.)  The base goes through a scalar move:
+// five wait states belong between a vector instruction that writes a scalar register, such as the reload of a spilled one,
+// and a memory instruction that reads it, and the compiler does not put them in front of assembly.  (The same in
+// mixers/sink_flash.hip, a library of its own.)
+__device__ __forceinline__ void send16(const void* base, uint32_t offset, uint32_t to) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(to))));
   uint64_t from;
   asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
-               : "=&s"(from) : "v"(offset), "s"(base), "s"(at) : "m0", "memory");
+               : "=&s"(from) : "v"(offset), "s"(base), "s"(to) : "m0", "memory");
 #endif
+}
+// the same by way of registers: from memory off 16-byte borders
+__device__ __forceinline__ void copy16(const void* base, uint32_t offset, uint32_t to, int lane) {
+  typedef __attribute__((address_space(3))) u32x4* lds_u32x4;
+  *(lds_u32x4)(to + 16u * lane) = *reinterpret_cast<const u32x4_any*>(static_cast<const char*>(base) + offset);
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)(const_cast<void*>(p))));
 }
 __device__ __forceinline__ void wait_sent() {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -145,6 +162,19 @@ __device__ __forceinline__ void hold(const X& x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("" ::"v"(x));
 #endif
+}
+
+// the value, computed anew from here on (not kept in a register until then)
+__device__ __forceinline__ int fresh(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v));
+#endif
+  return v;
+}
+// f(0), f(1), ... as constants
+template <int... N, typename F>
+__device__ __forceinline__ void each(std::integer_sequence<int, N...>, const F& f) {
+  (f(std::integral_constant<int, N>()), ...);
 }
 
 // NW = 8 (two workgroup halves): each staged K/V block serves 256 columns and a wave sends half as much.
@@ -205,7 +235,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
 
   // ---- block table slice -> LDS -------------------------------------------------------
   const int npages = min((wg_end + BS - 1) >> p.bs_shift, kBtLds);
-  for (int i = tid; i < npages; i += NW * 64) lds_bt[i] = bt[i];
+  const int page0 = bt[max(min(tid, npages - 1), 0)];   // (the first ones do not wait for the queries behind them)
 
   // ---- Q (B operand): Q[col r][16 st + 8 h .. +8], 8 k-steps over D ----------------------
   frag qf[8];
@@ -216,18 +246,17 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     for (int st = 0; st < 8; ++st)
       qf[st] = c_valid ? *reinterpret_cast<const frag*>(qp + 16 * st) : frag{};
   }
+  if (tid < npages) lds_bt[tid] = page0;
+  for (int i = tid + NW * 64; i < npages; i += NW * 64) lds_bt[i] = bt[i];
   __syncthreads();  // lds_bt ready
-
-#pragma unroll
-  for (int st = 0; st < 8; ++st) hold(qf[st]);   // (there before the loop, which would wait for its transfers with them)
 
   // ---- staging of one K/V block: memory -> LDS, past the registers ----------------------
   // A wave sends keys of ONE 16-key group for both tensors: with BS >= 16 they sit in one page, so the page lookup and
   // the keys' place in the page are wave-uniform (one LDS read + readfirstlane, a scalar base) and every lane offset is a
   // constant.  A transfer is 1 KiB of contiguous memory: 4 K rows, or 32 channels x 16 keys (at BS = 16).
   // Keys past the workgroup's range (>= wg_end) read a clamped page or the unused tail slots of the last page - stale
-  // bytes of whatever sequence held that page before.  Their scores are masked (P = 0), and their V^T columns are zeroed:
-  // that block's V goes through registers (put_v), so that a non-finite stale value cannot turn 0 * V into NaN.
+  // bytes of whatever sequence held that page before.  Their scores are masked (P = 0), and their V^T columns are zeroed once
+  // they are there, by the wave that sent them, so that a non-finite stale value cannot turn 0 * V into NaN.
   constexpr int WPG = NW / 4, U = 4 / WPG;   // waves per group, transfers per wave and tensor
   const int sg = wid & 3, part = wid >> 2;
   const int last_page = npages - 1;
@@ -250,36 +279,47 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
   auto v_at = [&](int pg, int k0) FP_INLINE {
     return v_base + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * page + ((k0 + 16 * sg) & (BS - 1));
   };
-  auto send_k = [&](const uint16_t* kb, uint16_t* to, int u) FP_INLINE { send16(kb, k_src[u], to + k_lds + u * WPG * 512); };
-  auto send_v = [&](const uint16_t* vb, uint16_t* to, int u) FP_INLINE { send16(vb, v_src[u], to + v_lds + u * WPG * 512); };
-  u32x4 vr[U];
-  auto send_block_k = [&](int k0, uint16_t* to) FP_INLINE {
+  // (`b`: which of the two buffers, its lowest bit)
+  const uint32_t k_to = lds_address(lds_k) + 2 * k_lds, v_to = lds_address(lds_v) + 2 * v_lds;
+  auto move16 = [&](const uint16_t* base, uint32_t offset, uint32_t to, bool direct) FP_INLINE {
+    if (direct) send16(base, offset, to);
+    else copy16(base, offset, to, fresh(lane));
+  };
+  auto send_k = [&](const uint16_t* kb, int b, int u, bool direct) FP_INLINE {
+    move16(kb, k_src[u], k_to + (b & 1) * 2 * kKTile + u * WPG * 1024, direct);
+  };
+  auto send_v = [&](const uint16_t* vb, int b, int u, bool direct) FP_INLINE {
+    move16(vb, v_src[u], v_to + (b & 1) * 2 * kVTile + u * WPG * 1024, direct);
+  };
+  auto send_block_k = [&](int k0, int b) FP_INLINE {
     const uint16_t* kb = k_at(__builtin_amdgcn_readfirstlane(page_at(k0)), k0);
+    if (__builtin_expect(p.wide_in, 1)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (p.wide_in) send_k(kb, to, u);
-      else *reinterpret_cast<u32x4*>(to + k_lds + u * WPG * 512 + lane * 8) =
-               *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(kb) + k_src[u]);
+      for (int u = 0; u < U; ++u) send_k(kb, b, u, true);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) send_k(kb, b, u, false);
     }
   };
-  auto send_block_v = [&](int k0, uint16_t* to) FP_INLINE {
+  auto send_block_v = [&](int k0, int b) FP_INLINE {
     const uint16_t* vb = v_at(__builtin_amdgcn_readfirstlane(page_at(k0)), k0);
+    if (__builtin_expect(p.wide_in, 1)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (p.wide_in && k0 + kKB <= wg_end) send_v(vb, to, u);
-      else vr[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb) + v_src[u]);
+      for (int u = 0; u < U; ++u) send_v(vb, b, u, true);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) send_v(vb, b, u, false);
     }
   };
-  auto put_v = [&](int k0, uint16_t* to) FP_INLINE {
-    if (p.wide_in && k0 + kKB <= wg_end) return;
-    const int key = k0 + 16 * sg + v_half;
+  auto clear_block_v = [&](int k0, int b) FP_INLINE {
+    if (k0 + kKB <= wg_end) return;
+    const int ln = fresh(lane), key = k0 + 16 * sg + 8 * ((ln ^ (ln >> 4)) & 1);
+    u32x4 mask;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int j = 0; j < 4; ++j) mask[j] = (key + 2 * j < wg_end ? 0x0000ffffu : 0u) | (key + 2 * j + 1 < wg_end ? 0xffff0000u : 0u);
+    uint16_t* to = lds_v + (b & 1) * kVTile + v_lds + ln * 8;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        vr[u][j] &= (key + 2 * j < wg_end ? 0x0000ffffu : 0u) | (key + 2 * j + 1 < wg_end ? 0xffff0000u : 0u);
-      *reinterpret_cast<u32x4*>(to + v_lds + u * WPG * 512 + lane * 8) = vr[u];
-    }
+    for (int u = 0; u < U; ++u) *reinterpret_cast<u32x4*>(to + u * WPG * 512) &= mask;
   };
   // ---- fragments.  A row of the score products: key with bits 2 and 3 swapped, so that register i of a tile holds key
   // 16 (i >> 3) + 8 h + (i & 7) and a V^T fragment is one plain 16-byte read
@@ -336,30 +376,51 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     s1 += y;
     return pack2<T>(x, y);
   };
+  // (products with their operands on the way, on different sums in turn: left to the compiler each waited for its own)
   auto scores = [&](const uint16_t* kl, f32x16 (&S)[kNS]) FP_INLINE {
+    constexpr int N = 8 * kNS, LA = 4;
+    frag fr[N];
+    auto read = [&](int n) FP_INLINE { fr[n] = kf(kl, n % kNS, n / kNS); };
 #pragma unroll
-    for (int t = 0; t < kNS; ++t) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) S[t][i] = 0.f;
-#pragma unroll
-      for (int st = 0; st < 8; ++st) S[t] = MF::mma(kf(kl, t, st), qf[st], S[t]);
-    }
+    for (int n = 0; n < LA; ++n) read(n);
+    each(std::make_integer_sequence<int, N>(), [&](auto slot) FP_INLINE {
+      constexpr int n = slot;
+      __builtin_amdgcn_sched_barrier(0);
+      if (n + LA < N) read(n + LA);
+      S[n % kNS] = MF::mma(fr[n], qf[n / kNS], n < kNS ? f32x16{} : S[n % kNS]);
+    });
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto values = [&](const uint16_t* vl, const u32x4 (&P)[4]) FP_INLINE {
+    constexpr int N = 16, LA = 4;
+    frag fr[N];
+    auto read = [&](int n) FP_INLINE { fr[n] = vf(vl, n % 4, n / 4); };
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) o[dt] = MF::mma(vf(vl, dt, ks), __builtin_bit_cast(frag, P[ks]), o[dt]);
+    for (int n = 0; n < LA; ++n) read(n);
+    each(std::make_integer_sequence<int, N>(), [&](auto slot) FP_INLINE {
+      constexpr int n = slot;
+      __builtin_amdgcn_sched_barrier(0);
+      if (n + LA < N) read(n + LA);
+      o[n % 4] = MF::mma(fr[n], __builtin_bit_cast(frag, P[n / 4]), o[n % 4]);
+    });
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto weights = [&](int k0, f32x16 (&S)[kNS], u32x4 (&P)[4]) FP_INLINE {
-    // mask: only blocks crossing the diagonal of the wave's first token (wave-uniform branch)
+    // mask: only blocks crossing the diagonal of the wave's first token (wave-uniform branch).  Register i of a tile holds
+    // its key 16 (i >> 3) + 8 h + (i & 7): a bit of a word per tile.  (A comparison per key, whose result waits in a scalar
+    // register: 800 cycles per block.)
     if (k0 + kKB > ctx0 + w_first + 1) {
-      const int lim = c_end - k0 - 8 * h;
 #pragma unroll
-      for (int t = 0; t < kNS; ++t)
+      for (int t = 0; t < kNS; ++t) {
+        const int n = c_end - k0 - 8 * h - 32 * t;
+        const unsigned int out = n <= 0 ? ~0u : n >= 32 ? 0u : ~0u << n;
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * t + 16 * (i >> 3) + (i & 7) >= lim) S[t][i] = kNegInf;
+        for (int i = 0; i < 16; ++i) {
+          const float v = S[t][i];
+          const unsigned int x = __builtin_amdgcn_sbfe(out, 16 * (i >> 3) + (i & 7), 1);
+          S[t][i] = __builtin_bit_cast(float, (x & 0xff800000u) | (~x & __builtin_bit_cast(unsigned int, v)));
+        }
+      }
     }
     float alpha, s0 = 0.f, s1 = 0.f;
     if (__any(raise(S, alpha))) {
@@ -373,7 +434,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
   };
   // One block's scores, the weights of the one before and the value products of the one before that: a product (32 cycles of
   // the matrix core), then the vector instructions that fit behind it.  The same sums in the same order as the parts above.
-  auto quick = [&](const uint16_t* kl, const uint16_t* vl, uint16_t* kw, uint16_t* vw, int bk, int bv, const f32x16 (&Si)[kNS],
+  auto quick = [&](const uint16_t* kl, const uint16_t* vl, int b, int bk, int bv, const f32x16 (&Si)[kNS],
                    f32x16 (&So)[kNS], const u32x4 (&Pi)[4], u32x4 (&Po)[4]) FP_INLINE {
     constexpr int NP = 16, NF = 32, LA = 3, NB = 30;   // NB: slots of the exponentials
     frag fr[NF];
@@ -406,8 +467,8 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
         kb = k_at(__builtin_amdgcn_readfirstlane(kpg), bk);
         vb = v_at(__builtin_amdgcn_readfirstlane(vpg), bv);
       }
-      if (n >= 2 && n < 2 + U) send_k(kb, kw, n - 2);
-      if (n >= 2 + U && n < 2 + 2 * U) send_v(vb, vw, n - 2 - U);
+      if (n >= 2 && n < 2 + U) send_k(kb, b, n - 2, true);
+      if (n >= 2 + U && n < 2 + 2 * U) send_v(vb, b, n - 2 - U, true);
 #pragma unroll
       for (int u = 16 * n / NB; n < NB && u < 16 * (n + 1) / NB; ++u) {
         const uint32_t x = weight2(Si, u, neg_m, s0, s1);
@@ -431,21 +492,19 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
   auto needed = [&](int i) FP_INLINE { return i >= 0 && i < nb && kfirst + i * kKB < w_end; };   // wave-uniform
   f32x16 sacc[kNS];
   u32x4 pw[4];
-#pragma unroll
-  for (int t = 0; t < kNS; ++t)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) sacc[t][i] = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) pw[ks] = u32x4{0u, 0u, 0u, 0u};
-  if (nb > 0) {
-    send_block_k(kfirst, kbuf(0));
-    wait_sent();
+  if (nb > 0) {   // (the first V with the first K: a workgroup of few blocks waits once for both)
+    send_block_k(kfirst, 0);
+    send_block_v(kfirst, 0);
   }
+#pragma unroll
+  for (int st = 0; st < 8; ++st) hold(qf[st]);   // (there before the loop, which would wait for its transfers with them)
+  wait_sent();
+  if (nb > 0) clear_block_v(kfirst, 0);
   __syncthreads();
   // steps [2, quick1): the block before has no masked key, this one is needed
   const int quick1 = w_end > 0 && p.wide_in ? min(min(nb, (ctx0 + w_first + 1 - kfirst) / kKB + 1), (w_end - 1 - kfirst) / kKB + 1) : 0;
   auto quick_step = [&](int i, const f32x16 (&Si)[kNS], f32x16 (&So)[kNS], const u32x4 (&Pi)[4], u32x4 (&Po)[4]) FP_INLINE {
-    quick(kbuf(i), vbuf(i), kbuf(i + 1), vbuf(i + 1), kfirst + (i + 1) * kKB, kfirst + (i - 1) * kKB, Si, So, Pi, Po);
+    quick(kbuf(i), vbuf(i), i + 1, kfirst + (i + 1) * kKB, kfirst + (i - 1) * kKB, Si, So, Pi, Po);
     wait_sent();
     __syncthreads();
   };
@@ -457,13 +516,14 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
       quick_step(i + 1, s2, sacc, p2, pw);
     }
     const int k0 = kfirst + (i - 1) * kKB;
-    if (i + 1 < nb) send_block_k(k0 + 2 * kKB, kbuf(i + 1));
-    if (i >= 1) send_block_v(k0, vbuf(i + 1));
+    if (i + 1 < nb) send_block_k(k0 + 2 * kKB, i + 1);
+    if (i >= 2) send_block_v(k0, i + 1);
     if (needed(i - 2)) values(vbuf(i), pw);
     if (needed(i - 1)) weights(k0, sacc, pw);
     if (needed(i)) scores(kbuf(i), sacc);
-    if (i >= 1) put_v(k0, vbuf(i + 1));
+    if (nb == 1 && i == 0) continue;   // (nothing on its way, and nothing that a wave writes next is read by another)
     wait_sent();
+    if (i >= 2) clear_block_v(k0, i + 1);
     __syncthreads();
   }
   if (needed(nb - 1)) values(vbuf(nb + 1), pw);
