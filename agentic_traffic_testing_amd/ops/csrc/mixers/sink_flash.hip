@@ -489,6 +489,10 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
         __builtin_amdgcn_sched_barrier(0);
       });
     };
+    // a maximum and what it makes of the sums so far (a sink may be infinite or NaN: an infinity stays the maximum, and its
+    // own factor is 1; a NaN stays)
+    auto higher = [](float t, float m) SF_INLINE { return t > m ? t : m; };
+    auto factor = [](float t, float m) SF_INLINE { return t > m ? __builtin_amdgcn_exp2f(m - t) : 1.f; };
     auto weights = [&](int b, f32x16 (&S)[KT], bf16x8 (&P)[2 * KT]) SF_INLINE {
       const int k0 = block_key(b);
       if (k0 + BLK - 1 > pos_first || (WIN && k0 <= edge_lo)) {
@@ -514,22 +518,22 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       float tmax[MT], mt[MT], psum[MT];
 #pragma unroll
       for (int e = 0; e < MT; ++e) {
-        tmax[e] = kNegBig;   // (all keys masked: below every maximum, never taken)
+        tmax[e] = -INFINITY;
 #pragma unroll
         for (int t = e * TPM; t < (e + 1) * TPM; ++t)
 #pragma unroll
           for (int i = 0; i < 16; ++i) tmax[e] = fmaxf(tmax[e], S[t][i]);
       }
 #pragma unroll
-      for (int e = 0; e < MT; ++e) tmax[e] = both(tmax[e]) * scale2;
+      for (int e = 0; e < MT; ++e) tmax[e] = fmaxf(both(tmax[e]) * scale2, kNegBig);   // (all keys masked: never above a maximum)
       if (MT > 1 && b >= kSplitBlocks) tmax[0] = fmaxf(tmax[0], tmax[MT - 1]);
-      mt[0] = fmaxf(tmax[0], m);
-      if (__any(mt[0] > m)) {
-        const float alpha = __builtin_amdgcn_exp2f(m - mt[0]);
+      mt[0] = higher(tmax[0], m);
+      if (__any(tmax[0] > m)) {
+        const float alpha = factor(tmax[0], m);
         l *= alpha;
         rescale(alpha);
       }
-      mt[MT - 1] = MT > 1 ? fmaxf(tmax[MT - 1], mt[0]) : mt[0];
+      mt[MT - 1] = MT > 1 ? higher(tmax[MT - 1], mt[0]) : mt[0];
       m = mt[MT - 1];
 #pragma unroll
       for (int e = 0; e < MT; ++e) psum[e] = 0.f;   // of the weights as the value products take them, rounded
@@ -548,7 +552,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       }
       l += psum[0];
       if (MT > 1) {
-        carry = __builtin_amdgcn_exp2f(mt[0] - m);
+        carry = factor(tmax[MT - 1], mt[0]);
         l = l * carry + psum[MT - 1];
       }
     };
@@ -587,12 +591,13 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       }
       float top[2] = {fmaxf(tm[0], tm[1]), fmaxf(tm[2 * KT - 2], tm[2 * KT - 1])};
       if (!PARTED || one_max) top[0] = fmaxf(top[0], top[1]);
-      const float m0 = fmaxf(both(top[0]) * scale2, m), alpha = __builtin_amdgcn_exp2f(m - m0);
+      const float t0 = both(top[0]) * scale2, m0 = higher(t0, m), alpha = factor(t0, m);
       const float before = carry;
       m = m0;
       if constexpr (PARTED) {
-        m = fmaxf(both(top[1]) * scale2, m0);
-        carry = __builtin_amdgcn_exp2f(m0 - m);
+        const float t1 = both(top[1]) * scale2;
+        m = higher(t1, m0);
+        carry = factor(t1, m0);
       }
       const float mt[2] = {m0, m};
       l *= alpha;

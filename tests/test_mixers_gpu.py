@@ -1258,6 +1258,30 @@ def test_flash_long_windows(H, G, d, dv, window, keep):
     assert float((got - want).norm() / want.norm()) < (4 if pair else 1) * 2.0 ** -9
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(8, 4, 64, 64), (8, 2, 128, 128), (5, 1, 256, 192)])
+@pytest.mark.parametrize("window", [0, 400])
+def test_flash_sinks_that_are_no_numbers(H, G, d, dv, window):
+    """A head's sink of +inf takes all of the weight, of -inf none, a NaN makes the head's results NaN; other heads do not see it."""
+    torch.manual_seed(d + window)
+    lens = [700, 17, 65]
+    md = ragged(lens, [0, 0, 640], [0, 1, 2], width=64)
+    nb, T = md["num_pages"], sum(lens)
+    q = torch.randn(T, H, d).to(torch.bfloat16)
+    k, v = torch.randn(nb, G, 16, d).to(torch.bfloat16), torch.randn(nb, G, dv, 16).to(torch.bfloat16)
+    sink = torch.randn(H)
+    sink[0], sink[2], sink[4] = float("inf"), float("-inf"), float("nan")
+    plain = torch.where(torch.isfinite(sink), sink, torch.full((H,), -1e4))   # (exp of it is 0)
+    g = cuda(md)
+    got = mx.sink_attention(q.cuda(), k.cuda(), v.cuda(), g["block_tables"], g["seq_kvlen"], g["seq_qstart"], g["tile_seq"],
+                            g["tile_qoff"], d ** -0.5, True, sink_values=sink.cuda(), window=window).cpu().float()
+    want = mref.sink_attention(q, k, v, md["block_tables"], md["seq_kvlen"], md["seq_qstart"], d ** -0.5, True, plain,
+                               window).float()
+    assert torch.equal(got[:, 0], torch.zeros(T, dv)) and torch.isnan(got[:, 4]).all()
+    rest = [h for h in range(H) if h not in (0, 4)]
+    # as the edges' tests
+    assert torch.allclose(got[:, rest], want[:, rest], atol=4e-2, rtol=4e-2)
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
