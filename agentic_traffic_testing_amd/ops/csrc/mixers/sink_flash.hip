@@ -21,10 +21,10 @@
 //
 // Work: the hardware hands workgroups to the shader engines strictly in turn, a free place in one waits for its turn, and a
 // workgroup's start (page list, queries, first keys: a chain of loads) costs 3 - 4 us; both together left CUs idle a fifth
-// of the time.  So large batches run one workgroup of eight waves per CU that takes several pieces: sorted by length and
-// dealt back and forth (their sums come out equal within 3 %), the next piece's page list, queries and first keys on their way
-// behind the present one's last steps.  Batches whose pieces of 128 columns number up to six per CU run one piece per
-// workgroup of four waves, two workgroups per CU (the rule, with both sides measured, at launch_sink_flash).
+// of the time.  So the latent form and the one of two maps, whose registers let a CU hold eight waves, run one workgroup of
+// eight waves per CU that takes several pieces: sorted by length and dealt back and forth (their sums come out equal
+// within 3 %), the next piece's page list, queries and first keys on their way behind the present one's last steps.  The
+// others run one piece per workgroup of four waves, two workgroups per CU (figures at launch_sink_flash).
 //
 // Short prompts: with its start and its masked blocks a piece of one block is latency from end to end, so its first values
 // come with its first keys, its queries behind its first pages, and the parts' products have their operands on the way and go
@@ -153,9 +153,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   constexpr bool TURNS = ND > 8;
   static_assert(NMAP == 1 || NW == 8, "pair form: four waves per map");
   __shared__ __attribute__((aligned(1024))) __bf16 lds_k[2 * KB], lds_v[2 * VB];
-  // (results of one map go through the values' buffers, where these are large enough)
-  constexpr bool XV = MANY && NMAP == 1 && 4 * VB >= 4096 * NW;
-  __shared__ __attribute__((aligned(1024))) char lds_x[MANY && !XV ? (NMAP == 2 ? 65536 : 32768) : 16];
+  __shared__ __attribute__((aligned(1024))) char lds_x[NMAP == 2 ? 65536 : 16];
   __shared__ float lds_ss[NMAP == 2 ? NW : 1][32];
   __shared__ int lds_bt[MANY ? 2 : 1][kPages];
   __shared__ int lds_piece[MANY ? kPieces : 1][8];
@@ -843,7 +841,8 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
         // 64 channels at a time through LDS, the wave's own 4 KB (32 rows of 128 bytes, chunks changing places), so that
         // a store has whole rows: 8-byte pieces of 32 rows kept the memory pipe busy for 2 us per piece of work.  (What
         // depends on the lane is worked out here: kept over a piece it was spilled, and its reload waited for the stores.)
-        char* x = (XV ? reinterpret_cast<char*>(lds_v) : MANY ? lds_x : reinterpret_cast<char*>(lds_k)) + w * 4096;
+        static_assert(NMAP == 2 || 4 * (MANY ? VB : KB) >= 4096 * NW, "room for the rows");
+        char* x = reinterpret_cast<char*>(MANY ? lds_v : lds_k) + w * 4096;
         __bf16* ob = static_cast<__bf16*>(out) + (static_cast<int64_t>(row0 + qo) * H + g * rep) * DV + 8 * ec;
 #pragma unroll
         for (int v2 = 0; v2 < NV / 2; ++v2) {
@@ -892,11 +891,11 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
 // two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two), caches or results
 // that are not 16-byte aligned and contexts past the LDS page list run sink_attention.hip's kernel.
 //
-// Four or eight waves: pieces of 128 columns up to 6 per CU, and tiles that do not fill eight waves (24 over 8 heads: 192
-// of 256 columns), go four by four.  us, whole layer, before / four waves / eight: 32 + 8 heads, 256 pieces (2 x 500) 34.5 /
-// 30.1 / 37.1; 768 (6 x 500) 58.1 / 54.3 / 56.1; 1220 (5 x 1000) 95.2 / 82.3 / 87.8; 1904 (4 x 2048) 198.1 / 182.7 / 180.0;
-// 24 + 8 heads 624 (3 x 777) 47.8 / 42.3 / 47.9, 1400 (2 x 3000) 177.7 / 146.0 / 157.4.
-// The workgroups of the latent form hold 8 tokens: so far ahead a NaN value reaches back (a weight of 0 times NaN).
+// One map of 64 or 128 goes by four waves, one piece each, two workgroups per CU.  Eight, with several pieces per workgroup in
+// turn, were better by 2 % at best, and a NaN value of a later token (a weight of 0 times NaN) reached back twice as far once
+// a batch was large.  us, four / eight waves: 32 + 8 heads, 4 x 2k 136 / 136, 3 x 2500 172 / 168, 2 x 4000 246 / 245, 8 x 1000 86 / 89,
+// 16 x 500 56 / 61, 60 x 100 39 / 44; in a window of 1024 4 x 2k 115 / 122, 2 x 4000 132 / 145; 64 wide 4 x 2k 55.9 / 54.9.
+// A value reaches back 128 columns, 32 tokens at four heads per group (latent: 8).
 bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void* v_cache,
                        const AttnArgs& a, int num_tiles, hipStream_t st) {
   if (a.block_size < 16 || a.bt_width > sf::kPages || !(a.scale > 0.f) ||
@@ -905,17 +904,11 @@ bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return false;
-  const int columns = kTileTokens * (a.H / a.G);
-  const bool few = columns % 256 != 0 || static_cast<int64_t>(num_tiles) * ((columns + 127) / 128) * a.G <= 6 * cus;
 #define SF(D, V, MAPS, NW)                                   \
   if (a.dim == D && a.vdim == V && (a.pair ? 2 : 1) == MAPS) \
     return sf::launch<D / 16, V / 32, MAPS, NW>(out, q, k_cache, v_cache, a, num_tiles, cus, st);
-  if (few) {
-    SF(64, 64, 1, 4)
-    SF(128, 128, 1, 4)
-  }
-  SF(64, 64, 1, 8)
-  SF(128, 128, 1, 8)
+  SF(64, 64, 1, 4)
+  SF(128, 128, 1, 4)
   SF(256, 192, 1, 8)
   SF(64, 128, 2, 8)
 #undef SF

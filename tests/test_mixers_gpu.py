@@ -1282,6 +1282,32 @@ def test_flash_sinks_that_are_no_numbers(H, G, d, dv, window):
     assert torch.allclose(got[:, rest], want[:, rest], atol=4e-2, rtol=4e-2)
 
 
+@pytest.mark.parametrize("H,G,d,dv,reach", [(32, 8, 128, 128, 32), (16, 4, 64, 64, 32), (32, 1, 256, 192, 8)])
+@pytest.mark.parametrize("seqs", [3, 120])
+def test_flash_values_of_other_tokens(H, G, d, dv, reach, seqs):
+    """A NaN value reaches the tokens that see it and no further than the others of their 128 columns (256 of the latent
+    form), backwards and, out of a window, forwards, however many prompts there are."""
+    torch.manual_seed(d + seqs)
+    window = 20
+    md = ragged([64] * seqs, [0] * seqs, list(range(seqs)), width=4)
+    nb = md["num_pages"]
+    q = torch.randn(64 * seqs, H, d).to(torch.bfloat16).cuda()
+    k, v = torch.randn(nb, G, 16, d).to(torch.bfloat16).cuda(), torch.randn(nb, G, dv, 16).to(torch.bfloat16).cuda()
+    g = cuda(md)
+
+    def run(v, window):
+        return mx.sink_attention(q, k, v, g["block_tables"], g["seq_kvlen"], g["seq_qstart"], g["tile_seq"], g["tile_qoff"],
+                                 d ** -0.5, True, window=window).view(seqs, 64, H, dv)
+
+    late, early = v.clone(), v.clone()
+    for s in range(seqs):
+        late[md["block_tables"][s, 2], :, :, 40 % 16] = float("nan")
+        early[md["block_tables"][s, 0], :, :, 5] = float("nan")
+    assert torch.equal(run(late, 0)[:, :40 // reach * reach], run(v, 0)[:, :40 // reach * reach])
+    first = -(-(5 + window) // reach) * reach   # all of these tokens' windows begin behind key 5
+    assert torch.equal(run(early, window)[:, first:], run(v, window)[:, first:])
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
