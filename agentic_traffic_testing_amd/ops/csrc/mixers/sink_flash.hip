@@ -55,6 +55,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;   // in memory, wherever it begins
+typedef f32x4 __attribute__((aligned(4))) f32x4_any;
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
 constexpr int KT = 2;                    // tiles of 32 keys per block
@@ -98,6 +100,11 @@ __device__ __forceinline__ void send16(const void* base, uint32_t offset, uint32
                : "=&s"(from) : "v"(offset), "s"(base), "s"(to) : "m0", "memory");
 #endif
 }
+// the same by way of registers: from memory off 16-byte borders
+__device__ __forceinline__ void copy16(const void* base, uint32_t offset, uint32_t to, int lane) {
+  typedef __attribute__((address_space(3))) u32x4* lds_u32x4;
+  *(lds_u32x4)(to + 16u * lane) = *reinterpret_cast<const u32x4_any*>(static_cast<const char*>(base) + offset);
+}
 __device__ __forceinline__ void send4(const void* base, uint32_t offset, uint32_t to) {
 #if defined(__HIP_DEVICE_COMPILE__)
   uint64_t from;
@@ -134,8 +141,9 @@ __device__ __forceinline__ void each(std::integer_sequence<int, N...>, const F& 
   (f(std::integral_constant<int, N>()), ...);
 }
 
-// DK = 16 ND (q / k width), DV = 32 NV (value width).
-template <int ND, int NV, int NMAP, int NW, bool WIN>
+// DK = 16 ND (q / k width), DV = 32 NV (value width).  BORDERS: the caches begin on 16-byte borders, as transfers past the
+// registers need them; otherwise blocks go through registers, part by part.
+template <int ND, int NV, int NMAP, int NW, bool WIN, bool BORDERS>
 __global__ void __launch_bounds__(NW * 64, 2)
 sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __bf16* __restrict__ k_cache,
                   const __bf16* __restrict__ v_cache, AttnArgs a, int num_tiles, int chunks, int workers) {
@@ -199,18 +207,22 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   };
   // (`b`: which of the two buffers, its lowest bit)
   const uint32_t k_to = lds_address(lds_k) + 2 * k_lds, v_to = lds_address(lds_v) + 2 * v_lds;
+  auto move16 = [&](const __bf16* base, uint32_t offset, uint32_t to) SF_INLINE {
+    if constexpr (BORDERS) send16(base, offset, to);
+    else copy16(base, offset, to, fresh(lane));
+  };
   auto send_k = [&](const __bf16* kb, int b, int u) SF_INLINE {
     const uint32_t to = k_to + (b & 1) * 2 * KB + u % KU * WPG * 1024 + u / KU * 2 * BLK * DK;
     if constexpr (TURNS) {   // rows 4 further on: bits 2 and 3 of the chunk's place
       static_assert(!TURNS || (NMAP == 1 && CK == 32 && WPG == 2), "four rows per transfer of the group's waves");
-      send16(kb + 4 * u * DK, fresh(k_src[0]) ^ (64u * u), to);
+      move16(kb + 4 * u * DK, fresh(k_src[0]) ^ (64u * u), to);
     } else if (KU * WPG == KN || (u % KU) * WPG + part < KN) {
-      send16(kb + (u / KU) * bs * DK, k_src[u % KU], to);
+      move16(kb + (u / KU) * bs * DK, k_src[u % KU], to);
     }
   };
   auto send_v = [&](const __bf16* vb, int b, int u) SF_INLINE {
     const uint32_t to = v_to + (b & 1) * 2 * VB + u * WPG * 1024;
-    if (VU * WPG == VN || u * WPG + part < VN) send16(TURNS ? vb + 32 * u * WPG * bs : vb, v_src[TURNS ? 0 : u], to);
+    if (VU * WPG == VN || u * WPG + part < VN) move16(TURNS ? vb + 32 * u * WPG * bs : vb, v_src[TURNS ? 0 : u], to);
   };
   // ---- fragments.  A row of the score products: key with bits 2 and 3 swapped
   const int vfrag = r * 16 + 8 * (h ^ ((r >> 3) & 1));
@@ -686,7 +698,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     // steps [quick0, quick1): block i - 1 has no masked key, block i is needed
     const int above = WIN ? max(edge_lo, low_first) : -1;   // (block i - 2 has a key that the wave sees)
     const int quick0 = max(nk + 2, nk + ((above + BLK - kbeg) / BLK) + 1);
-    const int quick1 = wave_on ? nk + min(min(nb - nk, (pos_first + 1 - kbeg + BLK) / BLK), (pos_last - kbeg) / BLK + 1) : 0;
+    const int quick1 = BORDERS && wave_on ? nk + min(min(nb - nk, (pos_first + 1 - kbeg + BLK) / BLK), (pos_last - kbeg) / BLK + 1) : 0;
     auto quick_step = [&](auto parted, const Places& at, int i, const f32x16 (&Si)[KT], f32x16 (&So)[KT], const bf16x8 (&Pi)[2 * KT],
                           bf16x8 (&Po)[2 * KT]) SF_INLINE {
       quick(parted, at, i - 1 >= kSplitBlocks, kbuf(i), vbuf(i), i + 1, kbeg + (i + 1 - nk) * BLK,
@@ -710,7 +722,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       __syncthreads();
     }
     for (int i = 0; i < nb; ++i) {
-      if (i >= quick0 && i + 1 < quick1) {
+      if (BORDERS && i >= quick0 && i + 1 < quick1) {
         Places at;
         places(at);
         if constexpr (MT > 1)
@@ -818,7 +830,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
         const int rr = 8 * j + el, cc = wcol + rr;
         const u32x4 e = *reinterpret_cast<const u32x4*>(x + rr * 128 + ((ec ^ ((rr >> 1) & 7)) * 16));
         if (cc < cols_total)
-          *reinterpret_cast<u32x4*>(ob + (static_cast<int64_t>(token_of(cc)) * (H / 2 - rep) + cc) * DV) = e;
+          *reinterpret_cast<u32x4_any*>(ob + (static_cast<int64_t>(token_of(cc)) * (H / 2 - rep) + cc) * DV) = e;
       }
     } else {
       const int ln = fresh(lane), er = ln & 31, eh = ln >> 5, el = ln >> 3, ec = ln & 7;
@@ -834,7 +846,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
           for (int vt = 0; vt < NV; ++vt)
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4)
-              *reinterpret_cast<f32x4*>(o + vt * 32 + 8 * i4) =
+              *reinterpret_cast<f32x4_any*>(o + vt * 32 + 8 * i4) =
                   f32x4{O[vt][4 * i4] * inv, O[vt][4 * i4 + 1] * inv, O[vt][4 * i4 + 2] * inv, O[vt][4 * i4 + 3] * inv};
         }
       } else {
@@ -860,7 +872,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
             const u32x4 e = *reinterpret_cast<const u32x4*>(x + rr * 128 + ((ec ^ ((rr >> 1) & 7)) * 16));
             const int t = token_of(cc);
             if (cc < cols_total)
-              *reinterpret_cast<u32x4*>(ob + (static_cast<int64_t>(t) * (H - rep) + cc) * DV + 64 * v2) = e;
+              *reinterpret_cast<u32x4_any*>(ob + (static_cast<int64_t>(t) * (H - rep) + cc) * DV + 64 * v2) = e;
           }
           __builtin_amdgcn_wave_barrier();
         }
@@ -878,7 +890,10 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
   const int chunks = (kTileTokens * (a.H / a.G) + COLS - 1) / COLS, heads = a.G / NMAP;
   const int pieces = num_tiles * chunks;
   const int workers = NW == 8 ? std::min(pieces, std::max({1, cus / heads, (pieces + kPieces - 1) / kPieces})) : pieces;
-  auto* kernel = a.window > 0 ? sink_flash_kernel<ND, NV, NMAP, NW, true> : sink_flash_kernel<ND, NV, NMAP, NW, false>;
+  const bool borders = (reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) % 16 == 0;
+  auto* kernel = !borders       ? sink_flash_kernel<ND, NV, NMAP, NW, true, false>
+                 : a.window > 0 ? sink_flash_kernel<ND, NV, NMAP, NW, true, true>
+                                : sink_flash_kernel<ND, NV, NMAP, NW, false, true>;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(workers) * heads), dim3(NW * 64), 0, st, out,
                      static_cast<const __bf16*>(q), static_cast<const __bf16*>(k_cache),
                      static_cast<const __bf16*>(v_cache), a, num_tiles, chunks, workers);
@@ -888,8 +903,8 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
 }  // namespace sf
 
 // The shapes of the served families (head width 128, the latent cache of 192 + 64 channels, narrow heads,
-// two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two), caches or results
-// that are not 16-byte aligned and contexts past the LDS page list run sink_attention.hip's kernel.
+// two maps of 64 over values of 128); other shapes, pages below 16 tokens (a 16-key group would span two) and contexts past the
+// LDS page list run sink_attention.hip's kernel.
 //
 // One map of 64 or 128 goes by four waves, one piece each, two workgroups per CU.  Eight, with several pieces per workgroup in
 // turn, were better by 2 % at best, and a NaN value of a later token (a weight of 0 times NaN) reached back twice as far once
@@ -898,9 +913,7 @@ bool launch(void* out, const void* q, const void* k_cache, const void* v_cache, 
 // A value reaches back 128 columns, 32 tokens at four heads per group (latent: 8).
 bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void* v_cache,
                        const AttnArgs& a, int num_tiles, hipStream_t st) {
-  if (a.block_size < 16 || a.bt_width > sf::kPages || !(a.scale > 0.f) ||
-      (reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(out)) % 16)
-    return false;
+  if (a.block_size < 16 || a.bt_width > sf::kPages || !(a.scale > 0.f)) return false;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return false;

@@ -1308,6 +1308,44 @@ def test_flash_values_of_other_tokens(H, G, d, dv, reach, seqs):
     assert torch.equal(run(early, window)[:, first:], run(v, window)[:, first:])
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(8, 4, 64, 64), (8, 2, 128, 128), (5, 1, 256, 192), (8, 4, 64, 128)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (300, 70)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_flash_off_16_byte_borders(H, G, d, dv, window, keep, dtype):
+    """Caches that begin between 16-byte borders take the same kernel, part by part: the results of aligned ones but for the
+    weights' sums, with one block and many, and more pieces of work than a launch of the latent form has workgroups.
+    Results between the borders: bit for bit those of aligned ones."""
+    torch.manual_seed(d + window)
+    lens, starts = [700, 129, 64, 3, 65, 1, 400] + [70] * 130, [0, 501, 990, 0, 448, 0, 0] + [0] * 130
+    md = cuda(ragged(lens, starts, list(range(len(lens))), width=80))
+    nb, T, pair = md["num_pages"], sum(lens), (d, dv) == (64, 128)
+    if pair and dtype == torch.float32:
+        pytest.skip("the results of two maps are of q's type")
+    q = torch.randn(T, H, d).to(torch.bfloat16).cuda()
+    k = torch.randn(nb, G, 16, d).to(torch.bfloat16).cuda()
+    v = torch.randn(nb, G // 2 if pair else G, dv, 16).to(torch.bfloat16).cuda()
+
+    def shifted(t, by):
+        x = torch.empty(t.numel() + by, dtype=t.dtype, device="cuda")[by:].view(t.shape)
+        return x.copy_(t)
+
+    def run(k, v, by):
+        out = shifted(torch.zeros(T, H // 2 if pair else H, dv, dtype=dtype, device="cuda"), by)
+        mx._native().sink_attention(out, q, k, v, md["block_tables"], md["seq_kvlen"], md["seq_qstart"], md["tile_seq"],
+                                    md["tile_qoff"], d ** -0.5, not pair, 0, 1, None, True, None, window, None, keep,
+                                    [0.4, 0.7, 1e-5] if pair else None)
+        return out
+
+    want = run(k, v, 0)
+    assert torch.equal(run(k, v, 1), want)
+    # A row's sum goes through up to 40 roundings in another order: 40 x 2^-24 of a result.  In 16 bits one in 2^15 / 40 then
+    # rounds the other way, by 2^-8.  Two maps: twice that.  (Maxima over other blocks of keys, as in the general kernel: 1e-3.)
+    limit = 2.4e-6 if dtype == torch.float32 else (2 if pair else 1) * 2.0 ** -8 * (40 * 2.0 ** -15) ** 0.5
+    for kk, vv, by in ((shifted(k, 4), v, 0), (k, shifted(v, 1), 1), (shifted(k, 1), shifted(v, 4), 4)):
+        got = run(kk, vv, by).double()
+        assert float((got - want.double()).norm() / want.double().norm()) < limit
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
@@ -1948,17 +1986,18 @@ def test_decode_two_maps_edges(dt, H, G, window, keep):
 @pytest.mark.parametrize("H,G,d,dv,pair", [(6, 2, 128, 128, False), (5, 1, 256, 192, False), (8, 2, 64, 128, True)])
 @pytest.mark.parametrize("window,keep,bs", [(0, 0, 16), (0, 5, 64), (8400, 70, 16)])
 def test_decode_table_entries_past_the_context(H, G, d, dv, pair, window, keep, bs):
-    """Table entries behind a context's last page are no pages; a table that ends with the longest context; more
+    """Table entries behind a context's last page name a page that nobody may use (in range, all NaN); a table that ends with the longest context; more
     partitions than the join's first look takes (64)."""
     torch.manual_seed(d + bs)
     kv = [1, 17, 129, 320, 8193, 8500]
     md = ragged([1] * len(kv), [x - 1 for x in kv], list(range(len(kv))), bs=bs, width=-(-max(kv) // bs))
-    nb = md["num_pages"]
+    nb = md["num_pages"] + 1
     wrong = md["block_tables"].clone()
     for i, n in enumerate(kv):
-        wrong[i, -(-n // bs):] = 2 ** 31 - 1 - i
+        wrong[i, -(-n // bs):] = nb - 1
     q, gate = torch.randn(len(kv), H * (2 if pair else 1), d).bfloat16(), torch.randn(len(kv), H * dv).bfloat16()
     k, v = torch.randn(nb, G * (2 if pair else 1), bs, d).bfloat16(), torch.randn(nb, G, dv, bs).bfloat16()
+    k[-1], v[-1] = float("nan"), float("nan")
     empty = torch.zeros(0, dtype=torch.int32)
 
     def run(m, table, q, k, v, gate, e):
