@@ -22,15 +22,16 @@
 // wave.  Blocks on the diagonal and both ends go part by part.  K and V of the next blocks go straight from memory to LDS in
 // the meantime: no registers, one wait and one workgroup barrier per block.  The sequence's block-table slice is staged in
 // LDS once so K/V addresses need no dependent global load inside the loop.
-// Short prompts and chunks behind a cached prefix: with its start and its masked blocks a workgroup of one block is latency
-// from end to end, so the first V comes with the first K, the queries behind the first pages, and the parts' products have
-// their operands on the way and go on different sums in turn.
+// Short prompts and chunks behind a cached prefix: with its start and its masked blocks a workgroup of few blocks is latency
+// from end to end, so the first V comes with the first K, the queries are asked for behind the page list and not waited for
+// with it (1000 of 12500 cycles at 17 tokens), the parts' products have their operands on the way and go on different sums
+// in turn, and one block or two go without steps, their code in a row (another 1200: fetches of instructions).
 // Kernel, us, 32 + 8 heads, one part after the other / pipeline without this / now; bound by the chain of loads and parts: 17
-// tokens 5.6 / 6.6 / 6.2, 85 7.2 / 8.4 / 7.7, 188 9.5 / 10.5 / 9.4, 475 16.6 / 14.9 / 13.9; behind cached ones: 5 x 17 on 600
-// 17.5 / 15.9 / 15.0, 5 x 85 on 500 18.6 / 18.3 / 16.5, 188 on 512 20.8 / 17.9 / 16.7, 475 on 2000 40.9 / 36.0 / 34.1, 17 on 4096
-// (split) 29.8 / 29.6 / 28.3; bound by matrix and vector units together, at a clock that gives way: 16 x 100 14.3 / 13.6 / 12.4,
-// 1 x 2000 56 / 48.4 / 46.3, 4 x 2k 146 / 139 / 132.  24 + 8 heads: 17 tokens 5.2 / 6.5 / 6.2, 188 9.6 / 10.9 / 9.7, 4 x 2k
-// 122 / 116 / 110.
+// tokens 6.3 / 7.3 / 6.2, 85 8.0 / 9.0 / 7.4, 188 10.3 / 11.2 / 10.0, 475 17.5 / 15.5 / 14.6; behind cached ones: 5 x 17 on 600
+// 17.9 / 16.2 / 15.4, 5 x 85 on 500 19.4 / 19.0 / 17.2, 188 on 512 21.0 / 18.0 / 17.0, 475 on 2000 43.4 / 37.2 / 35.3, 17 on 4096
+// (split) 29.5 / 29.6 / 28.0; bound by matrix and vector units together, at a clock that gives way: 16 x 100 14.5 / 13.7 / 12.6,
+// 1 x 2000 61 / 49 / 47.6, 4 x 2k 155 / 144 / 140.  24 + 8 heads: 17 tokens 6.0 / 7.1 / 6.3, 85 8.8 / 9.6 / 7.7, 4 x 2k
+// 129 / 124 / 114.
 #include <type_traits>
 #include <utility>
 
@@ -235,9 +236,10 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
 
   // ---- block table slice -> LDS -------------------------------------------------------
   const int npages = min((wg_end + BS - 1) >> p.bs_shift, kBtLds);
-  const int page0 = bt[max(min(tid, npages - 1), 0)];   // (the first ones do not wait for the queries behind them)
+  for (int i = tid; i < npages; i += NW * 64) lds_bt[i] = bt[i];
 
   // ---- Q (B operand): Q[col r][16 st + 8 h .. +8], 8 k-steps over D ----------------------
+  // (behind the page list, which would wait with them: loads under a condition)
   frag qf[8];
   {
     const uint16_t* qp = p.q + static_cast<int64_t>(qstart + (c_valid ? c_tok : 0)) * p.q_stride +
@@ -246,8 +248,6 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     for (int st = 0; st < 8; ++st)
       qf[st] = c_valid ? *reinterpret_cast<const frag*>(qp + 16 * st) : frag{};
   }
-  if (tid < npages) lds_bt[tid] = page0;
-  for (int i = tid + NW * 64; i < npages; i += NW * 64) lds_bt[i] = bt[i];
   __syncthreads();  // lds_bt ready
 
   // ---- staging of one K/V block: memory -> LDS, past the registers ----------------------
@@ -492,14 +492,19 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
   auto needed = [&](int i) FP_INLINE { return i >= 0 && i < nb && kfirst + i * kKB < w_end; };   // wave-uniform
   f32x16 sacc[kNS];
   u32x4 pw[4];
-  if (nb > 0) {   // (the first V with the first K: a workgroup of few blocks waits once for both)
+  if (nb > 0) {   // (the first V with the first K: a workgroup of one block or two waits once for all of them)
     send_block_k(kfirst, 0);
     send_block_v(kfirst, 0);
+    if (__builtin_expect(nb == 2, 0)) {
+      send_block_k(kfirst + kKB, 1);
+      send_block_v(kfirst + kKB, 1);
+    }
   }
 #pragma unroll
   for (int st = 0; st < 8; ++st) hold(qf[st]);   // (there before the loop, which would wait for its transfers with them)
   wait_sent();
   if (nb > 0) clear_block_v(kfirst, 0);
+  if (__builtin_expect(nb == 2, 0)) clear_block_v(kfirst + kKB, 1);
   __syncthreads();
   // steps [2, quick1): the block before has no masked key, this one is needed
   const int quick1 = w_end > 0 && p.wide_in ? min(min(nb, (ctx0 + w_first + 1 - kfirst) / kKB + 1), (w_end - 1 - kfirst) / kKB + 1) : 0;
@@ -508,7 +513,18 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     wait_sent();
     __syncthreads();
   };
-  for (int i = 0; nb > 0 && i <= nb; ++i) {
+  // (One block or two: all there, code in a row.  Steps lie on both sides of the dealt-out ones, and each place that is come to
+  // for the first time costs a fetch of instructions.)
+  if (nb <= 2) {
+    for (int i = 0; i < nb; ++i)
+      if (needed(i)) {
+        scores(kbuf(i), sacc);
+        weights(kfirst + i * kKB, sacc, pw);
+        values(vbuf(i), pw);
+      }
+    __syncthreads();   // (the results' way out is K's buffers)
+  }
+  for (int i = 0; nb > 2 && i <= nb; ++i) {
     for (; i >= 2 && i + 1 < quick1; i += 2) {
       f32x16 s2[kNS];
       u32x4 p2[4];
@@ -521,15 +537,14 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     if (needed(i - 2)) values(vbuf(i), pw);
     if (needed(i - 1)) weights(k0, sacc, pw);
     if (needed(i)) scores(kbuf(i), sacc);
-    if (nb == 1 && i == 0) continue;   // (nothing on its way, and nothing that a wave writes next is read by another)
     wait_sent();
     if (i >= 2) clear_block_v(k0, i + 1);
     __syncthreads();
   }
-  if (needed(nb - 1)) values(vbuf(nb + 1), pw);
+  if (nb > 2 && needed(nb - 1)) values(vbuf(nb + 1), pw);
   l_run += xor32(l_run, x32);
 
-  if (ns > 1) {
+  if (__builtin_expect(ns > 1, 0)) {
     // ---- split-KV hand-over: publish (O, m, l) with device-scope stores, count arrivals; the
     // last workgroup of the tile merges every split's partial into its own registers
     __shared__ int fl_last;
@@ -610,7 +625,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     return u32x2{pack2<T>(o[dt][i] * inv, o[dt][i + 1] * inv), pack2<T>(o[dt][i + 2] * inv, o[dt][i + 3] * inv)};
   };
   uint16_t* const op = p.out + static_cast<int64_t>(qstart + qoff + wid * kTokPerWave) * p.out_stride + static_cast<int64_t>(hk) * G * kD;
-  if (p.wide_out) {
+  if (__builtin_expect(p.wide_out, 1)) {
     char* x = reinterpret_cast<char*>(lds_k) + wid * 4096;
 #pragma unroll
     for (int d2 = 0; d2 < 2; ++d2) {

@@ -158,6 +158,25 @@ def test_flash_prefill_split_kv(splits, hq, hkv):
                                        torch.zeros(1, device="cuda")).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (24, 8), (8, 8)])
+def test_flash_prefill_few_blocks(hq, hkv, dtype):
+    """Workgroups of one, two and three blocks of 64 keys, whole and ragged, with and without cached keys; what lies behind
+    a context in its last page is NaN."""
+    torch.manual_seed(7)
+    seqs = [(n, q) for n in (1, 17, 63, 64, 65, 127, 128, 129, 192) for q in sorted({n, min(n, 5)})]
+    k, v, bt, kvlen, qstart, T = _make_paged(seqs, hkv, 16, dtype)
+    q = torch.randn(T, hq, 128, dtype=dtype, device="cuda")
+    ts, to = _tiles(seqs, ops.prefill_tile_tokens(hq // hkv, "flash"))
+    exp = ref.paged_attention(q, k, v, bt.clamp(min=0), kvlen, qstart, 0.09).double()
+    for i, (n, _) in enumerate(seqs):
+        if n % 16:
+            k[bt[i, n // 16], :, n % 16:], v[bt[i, n // 16], :, :, n % 16:] = float("nan"), float("nan")
+    got = ops.attention_prefill(q, k, v, bt, kvlen, qstart, ts, to, 0.09, impl="flash", kv_splits=1).double()
+    # weights and results are rounded once each, by at most half a step of the type
+    assert float((got - exp).norm() / exp.norm()) < 2 * torch.finfo(dtype).eps / 2
+
+
 @pytest.mark.parametrize("hq,hkv", [(32, 8), (24, 8)])
 def test_flash_prefill_odd_alignment(hq, hkv):
     """Caches and results whose rows start between 16-byte borders take the ways through registers and in 8-byte pieces:
