@@ -26,11 +26,13 @@
 // within 3 %), the next piece's page list, queries and first keys on their way behind the present one's last steps.  The
 // others run one piece per workgroup of four waves, two workgroups per CU (figures at launch_sink_flash).
 //
-// Short prompts: with its start and its masked blocks a piece of one block is latency from end to end, so its first values
-// come with its first keys, its queries behind its first pages, and the parts' products have their operands on the way and go
-// on different sums in turn.  Kernel, us, one part after the other / pipeline without this / now: one prompt of 17 tokens,
-// 32 + 8 heads 6.0 / 6.8 / 6.3, latent 14.9 / 14.7 / 12.3, 16 + 4 heads of 64 4.8 / 5.4 / 5.2; of 188 tokens 10.4 / 10.7 / 9.6,
-// 21.8 / 22.4 / 18.3, 7.6 / 8.2 / 7.8; 475 tokens on 2000 cached ones 71 / 45 / 44, 138 / 115 / 94, 50 / 34 / 33.
+// Short prompts: with its start and its masked blocks a piece of few blocks is latency from end to end, so its first values
+// come with its first keys, its queries behind its first pages, the parts' products have their operands on the way and go
+// on different sums in turn, and a workgroup's only piece of one block or two goes without steps, its code in a row.  Kernel,
+// us, one part after the other / pipeline without this / now: one prompt of 17 tokens, 32 + 8 heads 6.6 / 7.3 / 6.4, latent
+// 15.3 / 15.0 / 11.7, 16 + 4 heads of 64 5.6 / 6.0 / 5.4, two maps of 8 9.4 / 11.4 / 8.9; of 85 tokens 8.4 / 9.2 / 7.8,
+// 18.3 / 19.1 / 14.1, 6.6 / 7.3 / 6.4, 11.5 / 14.0 / 11.1; of 188 11.1 / 11.2 / 10.0, 22.0 / 22.2 / 18.6, 8.2 / 8.8 / 8.2,
+// 14.1 / 16.7 / 14.6; 475 tokens on 2000 cached ones 72 / 47 / 47, 139 / 116 / 96, 50 / 34 / 33, 50 / 45 / 39.
 //
 // Pair form: a workgroup's first four waves carry the first map, the other four the second one, over the
 // same columns and one V block; at the end each wave finishes half of the channels.
@@ -713,15 +715,42 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       quick_step(parted, at, i, S, S2, P, P2);
       quick_step(parted, at, i + 1, S2, S, P2, P);
     };
-    // (a workgroup's first values come with its first keys: a piece of few blocks waits once for both)
+    bf16x4 gates[8];   // pair form: of the wave's half of the channels
+    auto load_gates = [&]() SF_INLINE {
+      if (NMAP == 1 || a.gate == nullptr) return;
+      const int ln = fresh(lane);
+      const Column c = column(ln);
+      const __bf16* gt = static_cast<const __bf16*>(a.gate) + static_cast<int64_t>(row0 + qo + c.tok) * a.gate_stride +
+                         static_cast<int64_t>(g * rep + c.member) * DV + mp * (DV / 2) + 4 * (ln >> 5);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) gates[j] = *reinterpret_cast<const bf16x4*>(gt + 8 * j);
+    };
+    // A workgroup of one block or two waits once, for all keys and values, and takes them in a row: the steps' parts lie on
+    // both sides of the dealt-out ones, and each place that is come to for the first time costs a fetch of instructions.
+    const bool brief = turn == 0 && nb <= 2 && !(MANY && more);
     if (turn == 0) {
       send_block_v(block_key(0), 0);
+      if (__builtin_expect(brief && nb == 2, 0)) {
+        send_block_k(bt, last_page, block_key(1), 1);
+        send_block_v(block_key(1), 1);
+      }
       wait_sent();
       hold_q();
       clear_block_v(block_key(0), vbuf(0));
+      if (__builtin_expect(brief && nb == 2, 0)) clear_block_v(block_key(1), vbuf(1));
       __syncthreads();
     }
-    for (int i = 0; i < nb; ++i) {
+    if (__builtin_expect(brief, 0)) {
+      load_gates();
+      for (int i = 0; i < nb; ++i)
+        if (needed(i)) {
+          scores(kbuf(i), S);
+          weights(i, S, P);
+          values(vbuf(i), P, i < kSplitBlocks);
+        }
+      if (!MANY) __syncthreads();   // (the results' way out is K's buffers)
+    }
+    for (int i = 0; !brief && i < nb; ++i) {
       if (BORDERS && i >= quick0 && i + 1 < quick1) {
         Places at;
         places(at);
@@ -737,34 +766,25 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       if (needed(i - 2)) values(vbuf(i), P, i - 2 < kSplitBlocks);
       if (needed(i - 1)) weights(i - 1, S, P);
       if (needed(i)) scores(kbuf(i), S);
-      if (nb == 1 && turn == 0 && !(MANY && more)) break;   // (nothing on its way, and nothing that a wave writes next is read by another)
       wait_sent();
       if (v_now) clear_block_v(block_key(i - 1), vbuf(i + 1));
       __syncthreads();
     }
     // steps nb and nb + 1 have no scores; the next piece's queries and first keys are on their way
-    const bool v_now = nb > (turn == 0 ? 1 : 0);
-    if (v_now) send_block_v(block_key(nb - 1), nb + 1);
-    if (MANY && more) send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), 0);
-    if (needed(nb - 2)) values(vbuf(nb), P, nb - 2 < kSplitBlocks);
-    if (needed(nb - 1)) weights(nb - 1, S, P);
-    if (MANY) load_q(nxt, more);
-    if (MANY) hold_q();
-    wait_sent();
-    if (v_now) clear_block_v(block_key(nb - 1), vbuf(nb + 1));
-    __syncthreads();
-    bf16x4 gates[8];   // of the wave's half of the channels
-    if constexpr (NMAP == 2) {
-      if (a.gate != nullptr) {
-        const int ln = fresh(lane);
-        const Column c = column(ln);
-        const __bf16* gt = static_cast<const __bf16*>(a.gate) + static_cast<int64_t>(row0 + qo + c.tok) * a.gate_stride +
-                           static_cast<int64_t>(g * rep + c.member) * DV + mp * (DV / 2) + 4 * (ln >> 5);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gates[j] = *reinterpret_cast<const bf16x4*>(gt + 8 * j);
-      }
+    if (__builtin_expect(!brief, 1)) {
+      const bool v_now = nb > (turn == 0 ? 1 : 0);
+      if (v_now) send_block_v(block_key(nb - 1), nb + 1);
+      if (MANY && more) send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), 0);
+      if (needed(nb - 2)) values(vbuf(nb), P, nb - 2 < kSplitBlocks);
+      if (needed(nb - 1)) weights(nb - 1, S, P);
+      if (MANY) load_q(nxt, more);
+      if (MANY) hold_q();
+      wait_sent();
+      if (v_now) clear_block_v(block_key(nb - 1), vbuf(nb + 1));
+      __syncthreads();
+      load_gates();
+      if (needed(nb - 1)) values(vbuf(nb + 1), P, nb - 1 < kSplitBlocks);
     }
-    if (needed(nb - 1)) values(vbuf(nb + 1), P, nb - 1 < kSplitBlocks);
 
     l = both_sum(l);
     if constexpr (NMAP == 2) {

@@ -1258,6 +1258,38 @@ def test_flash_long_windows(H, G, d, dv, window, keep):
     assert float((got - want).norm() / want.norm()) < (4 if pair else 1) * 2.0 ** -9
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(8, 4, 64, 64), (32, 8, 128, 128), (6, 2, 128, 128), (5, 1, 256, 192), (8, 4, 64, 128)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (20, 5), (50, 70), (64, 0)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_flash_few_blocks(H, G, d, dv, window, keep, gated):
+    """Pieces of one, two and three blocks, whole and ragged, with kept keys in front of the window; what lies behind a
+    context in its last page is NaN."""
+    torch.manual_seed(d + H + window)
+    lens, starts = [1, 17, 63, 64, 65, 100, 128, 129, 30], [0, 0, 1, 64, 63, 28, 0, 300, 130]
+    md = ragged(lens, starts, list(range(9)), width=32)
+    nb, T, pair = md["num_pages"], sum(lens), (d, dv) == (64, 128)
+    q = torch.randn(T, H, d).to(torch.bfloat16)
+    k = torch.randn(nb, G, 16, d).to(torch.bfloat16)
+    v = torch.randn(nb, G // 2 if pair else G, dv, 16).to(torch.bfloat16)
+    gate = torch.randn(T, H // 2 * dv if pair else H).to(torch.bfloat16) if gated else None
+
+    def run(m, to):
+        args = (to(q), to(k), to(v), m["block_tables"], m["seq_kvlen"], m["seq_qstart"], m["tile_seq"], m["tile_qoff"])
+        g = None if gate is None else to(gate)
+        if pair:
+            return mx.differential_attention(*args, d ** -0.5, 0.4, 0.3, 1e-5, g, 0, 0, window, keep)
+        return mx.sink_attention(*args, d ** -0.5, True, window=window, gate=g, keep_first=keep, out_dtype=torch.float32)
+
+    want = run(md, lambda t: t).double()
+    for i, n in enumerate(md["seq_kvlen"].tolist()):
+        if n % 16:
+            page = md["block_tables"][i, n // 16]
+            k[page, :, n % 16:], v[page, :, :, n % 16:] = float("nan"), float("nan")
+    got = run(cuda(md), lambda t: t.cuda()).cpu().double()
+    # as with long windows
+    assert float((got - want).norm() / want.norm()) < (4 if pair else 1) * 2.0 ** -9
+
+
 @pytest.mark.parametrize("H,G,d,dv", [(8, 4, 64, 64), (8, 2, 128, 128), (5, 1, 256, 192)])
 @pytest.mark.parametrize("window", [0, 400])
 def test_flash_sinks_that_are_no_numbers(H, G, d, dv, window):
