@@ -18,8 +18,8 @@
 //
 // Join: four waves per (row, head) take every fourth partition, with the first four of them loaded before their
 // weights are known: 6.2 -> 3.7 us, latent 10.7 -> 4.4, two maps 7.1 -> 5.7.  One look at the partitions' maxima and sums,
-// of both maps at once, in place of two or four in turn: layers, 16 rows of 2000, latent 28.7 -> 28.5 us, two maps
-// 31.4 -> 30.9, small, 6 rows of 1300, 19.2 -> 18.5.  (The partition kernel with the pages fetched beside the context's
+// of both maps at once, in place of two or four in turn: layers, 16 rows of 2000, two maps 31.4 -> 30.9 us, small, 6 rows of
+// 1300, 19.2 -> 18.5, latent as before within 1 %.  (The partition kernel with the pages fetched beside the context's
 // length, one trip less, is slower: latent 28.7 -> 29.5, 32 + 8 heads 39.3 -> 39.7.)
 #include "sink_attention.h"
 

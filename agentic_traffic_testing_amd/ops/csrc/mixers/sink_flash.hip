@@ -14,10 +14,10 @@
 // Pipeline: step i takes the scores of block i, the weights of block i - 1 and the value products of block i - 2, so that
 // matrix and vector work of one step do not depend on each other, and `quick` deals them out by hand: a product (32 cycles
 // of the matrix core), then as many vector instructions as fit behind it.  Left to the compiler the two ran one after the
-// other, also across the two waves of a SIMD (5000 cycles per block and pair of waves; 3350 now, 2300 of them products).  Steps
-// with masks, at the window's edges and at both ends go part by part.  K of block i + 1 and V of block i - 1 travel straight
-// from memory to LDS in the meantime: no registers, one wait and one barrier per step.  A wave moves keys of ONE 16-key
-// group, which lie in one page (pages of 16 tokens or more), so its page and the group's place in it are scalars.
+// other, also across the two waves of a SIMD.  Steps with masks, at the window's edges and at both ends go part by part.  K
+// of block i + 1 and V of block i - 1 travel straight from memory to LDS in the meantime: no registers, one wait and one
+// barrier per step.  A wave moves keys of ONE 16-key group, which lie in one page (pages of 16 tokens or more), so its page
+// and the group's place in it are scalars.
 //
 // Work: the hardware hands workgroups to the shader engines strictly in turn, a free place in one waits for its turn, and a
 // workgroup's start (page list, queries, first keys: a chain of loads) costs 3 - 4 us; both together left CUs idle a fifth
@@ -37,9 +37,10 @@
 // Pair form: a workgroup's first four waves carry the first map, the other four the second one, over the
 // same columns and one V block; at the end each wave finishes half of the channels.
 //
-// Bound (128 wide): matrix cores 60 - 70 % and vector units 60 % busy inside the steps, at 2.0 - 2.1 GHz: with both busy the
-// clock gives way (the kernel before, half as busy: 2.2 GHz; products alone: 1.85 GHz).  4 prompts of ~1.9k tokens, us, before ->
-// now: 32 + 8 heads of 128 159 -> 138, latent 257 -> 221, two maps (8 heads, 5 x 1165, window 1024) 72 -> 50.
+// Bound: matrix cores and vector units together, over the whole kernel 44 and 48 % busy (128 wide; latent 46 and 45, two maps 18
+// and 43, with few pieces per CU), at a clock that gives way.  4 prompts of ~1.9k tokens, us, one part after the other /
+// pipeline with 32 keys per block of the latent form / now: 32 + 8 heads of 128 159 / 137 / 135, latent 257 / 227 / 204, two maps
+// (8 heads, 5 x 1165, window 1024) 72 / 49 / 48.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
