@@ -25,13 +25,13 @@
 // Short prompts and chunks behind a cached prefix: with its start and its masked blocks a workgroup of few blocks is latency
 // from end to end, so the first V comes with the first K, the queries are asked for behind the page list and not waited for
 // with it (1000 of 12500 cycles at 17 tokens), the parts' products have their operands on the way and go on different sums
-// in turn, and one block or two go without steps, their code in a row (another 1200: fetches of instructions).
+// in turn, and up to three blocks go without steps, their code in a row (another 1200 of them: fetches of instructions).
 // Kernel, us, 32 + 8 heads, one part after the other / pipeline without this / now; bound by the chain of loads and parts: 17
-// tokens 6.3 / 7.3 / 6.2, 85 8.0 / 9.0 / 7.4, 188 10.3 / 11.2 / 10.0, 475 17.5 / 15.5 / 14.6; behind cached ones: 5 x 17 on 600
-// 17.9 / 16.2 / 15.4, 5 x 85 on 500 19.4 / 19.0 / 17.2, 188 on 512 21.0 / 18.0 / 17.0, 475 on 2000 43.4 / 37.2 / 35.3, 17 on 4096
-// (split) 29.5 / 29.6 / 28.0; bound by matrix and vector units together, at a clock that gives way: 16 x 100 14.5 / 13.7 / 12.6,
-// 1 x 2000 61 / 49 / 47.6, 4 x 2k 155 / 144 / 140.  24 + 8 heads: 17 tokens 6.0 / 7.1 / 6.3, 85 8.8 / 9.6 / 7.7, 4 x 2k
-// 129 / 124 / 114.
+// tokens 6.3 / 7.3 / 6.0, 85 8.1 / 9.0 / 7.3, 188 10.3 / 11.2 / 8.9, 475 17.6 / 15.5 / 14.4; behind cached ones: 5 x 17 on 600
+// 17.9 / 16.2 / 15.0, 5 x 85 on 500 19.6 / 19.0 / 17.2, 188 on 512 21.2 / 18.0 / 17.1, 475 on 2000 43.3 / 37.2 / 35.3, 17 on 4096
+// (split) 29.0 / 29.6 / 27.4; bound by matrix and vector units together, at a clock that gives way: 16 x 100 14.5 / 13.7 / 12.7,
+// 1 x 2000 61 / 49 / 48, 4 x 2k 157 / 144 / 136.  24 + 8 heads: 17 tokens 6.1 / 7.1 / 6.1, 85 8.9 / 9.6 / 7.7, 188 10.3 / 11.4 /
+// 9.1, 4 x 2k 130 / 124 / 115.
 #include <type_traits>
 #include <utility>
 
@@ -50,6 +50,9 @@ constexpr int kKTile = kKB * kD;         // elements
 constexpr int kVTile = kD * kKB;
 constexpr int kBtLds = 2048;             // block-table entries staged in LDS
 constexpr float kNegInf = -__builtin_huge_valf();
+// Workgroups of so many blocks take them one after the other.  Cycles of one of 3 / 4 / 6 blocks, alone on its CU: in steps
+// 17700 / 20400 / 24700, one after the other 15400 / 20100 / 25700.
+constexpr int kBrief = 3;
 constexpr float kRescale = 8.f;  // defer-max threshold (log2 units)
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -492,10 +495,11 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
   auto needed = [&](int i) FP_INLINE { return i >= 0 && i < nb && kfirst + i * kKB < w_end; };   // wave-uniform
   f32x16 sacc[kNS];
   u32x4 pw[4];
-  if (nb > 0) {   // (the first V with the first K: a workgroup of one block or two waits once for all of them)
+  const bool brief = nb <= kBrief;
+  if (nb > 0) {   // (the first V with the first K: a workgroup of few blocks waits once for both, and for the second ones)
     send_block_k(kfirst, 0);
     send_block_v(kfirst, 0);
-    if (__builtin_expect(nb == 2, 0)) {
+    if (__builtin_expect(brief && nb > 1, 0)) {
       send_block_k(kfirst + kKB, 1);
       send_block_v(kfirst + kKB, 1);
     }
@@ -504,7 +508,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
   for (int st = 0; st < 8; ++st) hold(qf[st]);   // (there before the loop, which would wait for its transfers with them)
   wait_sent();
   if (nb > 0) clear_block_v(kfirst, 0);
-  if (__builtin_expect(nb == 2, 0)) clear_block_v(kfirst + kKB, 1);
+  if (__builtin_expect(brief && nb > 1, 0)) clear_block_v(kfirst + kKB, 1);
   __syncthreads();
   // steps [2, quick1): the block before has no masked key, this one is needed
   const int quick1 = w_end > 0 && p.wide_in ? min(min(nb, (ctx0 + w_first + 1 - kfirst) / kKB + 1), (w_end - 1 - kfirst) / kKB + 1) : 0;
@@ -513,18 +517,30 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     wait_sent();
     __syncthreads();
   };
-  // (One block or two: all there, code in a row.  Steps lie on both sides of the dealt-out ones, and each place that is come to
-  // for the first time costs a fetch of instructions.)
-  if (nb <= 2) {
-    for (int i = 0; i < nb; ++i)
+  // (Few blocks: one after the other, code in a row, the third's keys and values on their way behind the second.  Steps lie on
+  // both sides of the dealt-out ones, and each place that is come to for the first time costs a fetch of instructions.)
+  if (brief) {
+    for (int i = 0; i < nb; ++i) {
       if (needed(i)) {
         scores(kbuf(i), sacc);
         weights(kfirst + i * kKB, sacc, pw);
         values(vbuf(i), pw);
       }
+      if (__builtin_expect(nb > 2, 0)) {
+        if (i == 1) {
+          wait_sent();
+          clear_block_v(kfirst + 2 * kKB, 0);
+        }
+        __syncthreads();
+        if (i == 0) {
+          send_block_k(kfirst + 2 * kKB, 0);
+          send_block_v(kfirst + 2 * kKB, 0);
+        }
+      }
+    }
     __syncthreads();   // (the results' way out is K's buffers)
   }
-  for (int i = 0; nb > 2 && i <= nb; ++i) {
+  for (int i = 0; !brief && i <= nb; ++i) {
     for (; i >= 2 && i + 1 < quick1; i += 2) {
       f32x16 s2[kNS];
       u32x4 p2[4];
@@ -541,7 +557,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_prefill_kernel(FlashParams p
     if (i >= 2) clear_block_v(k0, i + 1);
     __syncthreads();
   }
-  if (nb > 2 && needed(nb - 1)) values(vbuf(nb + 1), pw);
+  if (!brief && needed(nb - 1)) values(vbuf(nb + 1), pw);
   l_run += xor32(l_run, x32);
 
   if (__builtin_expect(ns > 1, 0)) {
