@@ -28,11 +28,12 @@
 //
 // Short prompts: with its start and its masked blocks a piece of few blocks is latency from end to end, so its first values
 // come with its first keys, its queries behind its first pages, the parts' products have their operands on the way and go
-// on different sums in turn, and a workgroup's only piece of one block or two goes without steps, its code in a row.  Kernel,
-// us, one part after the other / pipeline without this / now: one prompt of 17 tokens, 32 + 8 heads 6.6 / 7.3 / 6.4, latent
-// 15.3 / 15.0 / 11.7, 16 + 4 heads of 64 5.6 / 6.0 / 5.4, two maps of 8 9.4 / 11.4 / 8.9; of 85 tokens 8.4 / 9.2 / 7.8,
-// 18.3 / 19.1 / 14.1, 6.6 / 7.3 / 6.4, 11.5 / 14.0 / 11.1; of 188 11.1 / 11.2 / 10.0, 22.0 / 22.2 / 18.6, 8.2 / 8.8 / 8.2,
-// 14.1 / 16.7 / 14.6; 475 tokens on 2000 cached ones 72 / 47 / 47, 139 / 116 / 96, 50 / 34 / 33, 50 / 45 / 39.
+// on different sums in turn, and a piece of up to three blocks goes without steps, its code in a row.  Kernel, us, one part
+// after the other / pipeline without this / now: one prompt of 17 tokens, 32 + 8 heads 6.7 / 7.3 / 6.2, latent 15.3 / 15.0 / 12.0,
+// 16 + 4 heads of 64 5.6 / 6.0 / 5.3, two maps of 8 9.4 / 11.4 / 9.0; of 85 tokens 8.6 / 9.2 / 7.6, 18.6 / 19.1 / 14.5, 6.8 / 7.3 /
+// 6.3, 11.4 / 14.0 / 11.0; of 188 11.2 / 11.2 / 9.1, 22.0 / 22.2 / 17.5, 8.3 / 8.8 / 7.4, 14.0 / 16.7 / 13.3; two maps, several
+// pieces per workgroup, 32 heads 14 x 220 59.4 / 64.5 / 60.1, 16 x 85 30.1 / 32.2 / 30.1; 475 tokens on 2000 cached ones 72 / 47 / 46,
+// 139 / 116 / 97, 50 / 34 / 33, 50 / 45 / 39.
 //
 // Pair form: a workgroup's first four waves carry the first map, the other four the second one, over the
 // same columns and one V block; at the end each wave finishes half of the channels.
@@ -65,6 +66,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int KT = 2;                    // tiles of 32 keys per block
 constexpr int kPages = 2048;             // page-table entries in LDS
 constexpr int kSortTiles = 1024;         // tiles that a workgroup puts in order
+constexpr int kBrief = 3;                // pieces of so many blocks take them one after the other (the line as measured in flash_prefill.hip)
 constexpr int kPieces = 64;              // pieces of work per workgroup in LDS
 // Pair form: in the first blocks each of the two tiles has its own maximum.  Largest weights are rounded to exactly 1;
 // with a maximum per 64 keys there are fewer of them than per 32, half of the difference from the first block, 90 %
@@ -391,6 +393,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
   __syncthreads();
   send_block_k(lds_bt[0], pages_of(now) - 1, first_key(now), 0);
 
+  bool was_brief = false;   // the piece before: the present one's first keys and queries are still on their way
   for (int turn = 0;; ++turn) {
     ++pn;
     nxt = now;
@@ -726,30 +729,50 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
 #pragma unroll
       for (int j = 0; j < 8; ++j) gates[j] = *reinterpret_cast<const bf16x4*>(gt + 8 * j);
     };
-    // A workgroup of one block or two waits once, for all keys and values, and takes them in a row: the steps' parts lie on
-    // both sides of the dealt-out ones, and each place that is come to for the first time costs a fetch of instructions.
-    const bool brief = turn == 0 && nb <= 2 && !(MANY && more);
-    if (turn == 0) {
-      send_block_v(block_key(0), 0);
-      if (__builtin_expect(brief && nb == 2, 0)) {
+    // A piece of few blocks takes them one after the other, code in a row, the first two after one wait, the third's keys and
+    // values on their way behind the second: the pipeline would be filled and emptied for them, its steps' parts lie on both
+    // sides of the dealt-out ones, and each place that is come to for the first time costs a fetch of instructions.
+    const bool brief = nb <= kBrief, v_first = turn == 0 || brief;
+    if (v_first || was_brief) {
+      if (MANY && NMAP == 1 && turn > 0) __syncthreads();   // (V's buffers were the results' way out)
+      if (v_first) send_block_v(block_key(0), 0);
+      if (__builtin_expect(brief && nb > 1, 0)) {
         send_block_k(bt, last_page, block_key(1), 1);
         send_block_v(block_key(1), 1);
       }
+      if (MANY && brief && more) send_pages(nxt, 0, (turn & 1) ^ 1);
       wait_sent();
       hold_q();
-      clear_block_v(block_key(0), vbuf(0));
-      if (__builtin_expect(brief && nb == 2, 0)) clear_block_v(block_key(1), vbuf(1));
+      if (v_first) clear_block_v(block_key(0), vbuf(0));
+      if (__builtin_expect(brief && nb > 1, 0)) clear_block_v(block_key(1), vbuf(1));
       __syncthreads();
     }
+    was_brief = brief;
     if (__builtin_expect(brief, 0)) {
       load_gates();
-      for (int i = 0; i < nb; ++i)
+      for (int i = 0; i < nb; ++i) {
         if (needed(i)) {
           scores(kbuf(i), S);
           weights(i, S, P);
           values(vbuf(i), P, i < kSplitBlocks);
         }
-      if (!MANY) __syncthreads();   // (the results' way out is K's buffers)
+        if (__builtin_expect(nb > 2, 0)) {
+          if (i == 1) {
+            wait_sent();
+            clear_block_v(block_key(2), vbuf(0));
+          }
+          __syncthreads();
+          if (i == 0) {
+            send_block_k(bt, last_page, block_key(2), 0);
+            send_block_v(block_key(2), 0);
+          }
+        }
+      }
+      if (!MANY || more) __syncthreads();   // (the results' way out is K's buffers)
+      if (MANY && more) {   // on their way behind the results
+        send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), 0);
+        load_q(nxt, true);
+      }
     }
     for (int i = 0; !brief && i < nb; ++i) {
       if (BORDERS && i >= quick0 && i + 1 < quick1) {
@@ -761,7 +784,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
       }
       if (i == nb) break;
       if (i + 1 < nb) send_block_k(bt, last_page, block_key(i + 1), i + 1);
-      const bool v_now = i > (turn == 0 ? 1 : 0);
+      const bool v_now = i > (v_first ? 1 : 0);
       if (v_now) send_block_v(block_key(i - 1), i + 1);
       if (MANY && i == 0 && more) send_pages(nxt, 0, (turn & 1) ^ 1);
       if (needed(i - 2)) values(vbuf(i), P, i - 2 < kSplitBlocks);
@@ -773,7 +796,7 @@ sink_flash_kernel(void* __restrict__ out, const __bf16* __restrict__ q, const __
     }
     // steps nb and nb + 1 have no scores; the next piece's queries and first keys are on their way
     if (__builtin_expect(!brief, 1)) {
-      const bool v_now = nb > (turn == 0 ? 1 : 0);
+      const bool v_now = nb > (v_first ? 1 : 0);
       if (v_now) send_block_v(block_key(nb - 1), nb + 1);
       if (MANY && more) send_block_k(lds_bt[(turn & 1) ^ 1], pages_of(nxt) - 1, first_key(nxt), 0);
       if (needed(nb - 2)) values(vbuf(nb), P, nb - 2 < kSplitBlocks);
