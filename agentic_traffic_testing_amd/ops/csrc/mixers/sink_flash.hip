@@ -38,10 +38,10 @@
 // Pair form: a workgroup's first four waves carry the first map, the other four the second one, over the
 // same columns and one V block; at the end each wave finishes half of the channels.
 //
-// Bound: matrix cores and vector units together, over the whole kernel 44 and 48 % busy (128 wide; latent 46 and 45, two maps 18
-// and 43, with few pieces per CU), at a clock that gives way.  4 prompts of ~1.9k tokens, us, one part after the other /
-// pipeline with 32 keys per block of the latent form / now: 32 + 8 heads of 128 159 / 137 / 135, latent 257 / 227 / 204, two maps
-// (8 heads, 5 x 1165, window 1024) 72 / 49 / 48.
+// Bound: matrix cores and vector units together, over the whole kernel 44 and 48 % busy (128 wide; latent 47 and 45, two maps 18
+// and 42, with few pieces per CU), at a clock that gives way.  4 prompts of ~1.9k tokens, us, one part after the other /
+// pipeline with 32 keys per block of the latent form / now: 32 + 8 heads of 128 159 / 137 / 139, latent 257 / 227 / 208, two maps
+// (8 heads, 5 x 1165, window 1024) 72 / 49 / 48, the last ones on a card that is 3 % slower (128 wide the last two are alike).
 #include <algorithm>
 #include <type_traits>
 #include <utility>
