@@ -139,3 +139,15 @@ def test_transfers_to_lds_read_their_base_behind_a_scalar_move():
                     base = line.split()[-1]
                     assert any(re.match(rf"s_mov_b64 {base},", x) for x in lines[:i]), (src.name, text)
     assert found == 3
+
+
+def test_flash_kernels_share_their_assembly():
+    """The two flash kernels are in libraries of their own and have the same assembly: what is mended in one is in the other."""
+    def texts(name):
+        src = next(p for p in [*build.kernel_sources(), *build.mixer_sources()] if p.name == name).read_text()
+        return set(re.findall(r'asm volatile\(("(?:[^"\\]|\\.)*"(?:\s*"(?:[^"\\]|\\.)*")*)', src))
+
+    llama, mixers = texts("flash_prefill.hip"), texts("sink_flash.hip")
+    assert len(llama) >= 3
+    # (4-byte transfers are the mixers' alone)
+    assert mixers - llama == {t for t in mixers if "global_load_lds_dword %1" in t} and llama <= mixers
