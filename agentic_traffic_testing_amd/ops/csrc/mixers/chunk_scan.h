@@ -1,4 +1,4 @@
-// Chunked form of the recurrences S = diag(a) S + k u^T, o = S^T q (chunk_scan.hip).
+// Chunked form of the recurrences S = diag(a) S + k u^T, o = S^T q (chunk_scan_kernels.h).
 #pragma once
 
 #include "mix_common.h"
@@ -55,7 +55,7 @@ constexpr int scan_record_floats(int mode, int dk) {
   return scan_rec_decay(mode) + (scan_keeps_decays(mode) ? kScanChunk * scan_decay_width(dk) : 0);
 }
 // A long portion in few heads leaves most of the chip idle: with one number or one per channel as the decay it is cut
-// into segments that run side by side, in two passes (chunk_scan.hip).  `chunks`: a segment's length with which the
+// into segments that run side by side, in two passes (chunk_scan_kernels.h).  `chunks`: a segment's length with which the
 // batch makes about 256 workgroups (one per CU: the registers allow no second one), at least 7 and a 16th of the batch
 // (a segment's start is put together from all segments before it; us with at least 10 / 7, 8 heads: 350 rows forget gate
 // 55 / 46, state space 42 / 35, retention 49 / 40, 600 rows 53 / 48, 40 / 36, 46 / 41).  A batch of less than 20 chunks is

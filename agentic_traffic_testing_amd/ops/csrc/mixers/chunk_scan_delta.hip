@@ -1,0 +1,3 @@
+#include "chunk_scan_kernels.h"
+
+template int mixk::cs::launch_mode<mixk::kModeDelta>(const mixk::ChunkArgs&, int, hipStream_t);

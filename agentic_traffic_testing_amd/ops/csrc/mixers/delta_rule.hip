@@ -1,5 +1,5 @@
 // Gated delta rule over ragged batches of portions, state carried per sequence in fp32.  Most batches run the
-// kernels of chunk_scan.hip and step_scan.hip; the kernel here takes portions whose keys are wider than a chunk's, and
+// kernels of chunk_scan_kernels.h and step_scan.hip; the kernel here takes portions whose keys are wider than a chunk's, and
 // short ones with per-channel decays (scan_route).
 //
 // Per head, with S [dim, vdim] the state, per token:

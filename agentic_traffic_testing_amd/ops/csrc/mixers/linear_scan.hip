@@ -1,5 +1,5 @@
 // Gated linear recurrence over ragged batches of portions, state carried per sequence in fp32.  Most batches run the
-// kernels of chunk_scan.hip and step_scan.hip; the kernel here takes portions whose keys are wider than a chunk's,
+// kernels of chunk_scan_kernels.h and step_scan.hip; the kernel here takes portions whose keys are wider than a chunk's,
 // and short ones (scan_route).
 //
 // Per head, with S [dk, dv] the state, per token:

@@ -5,7 +5,7 @@
 // q and k are rotated here (rotate-half pairs (i, i + n_freq) over the first 2 n_freq channels,
 // cos / sin from the step's table) and k times dk^-1/2, so everything after the projections is fp32.
 // A portion whose first position is 0 starts from the zero state whatever its slot holds.
-// Kernels: chunk_scan.hip (portions), step_scan.hip (decode rows, short portions, keys wider than 128).
+// Kernels: chunk_scan_kernels.h (portions), step_scan.hip (decode rows, short portions, keys wider than 128).
 #include "chunk_scan.h"
 #include "mixers.h"
 
