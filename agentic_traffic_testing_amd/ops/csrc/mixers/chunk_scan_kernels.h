@@ -17,29 +17,30 @@
 // * scores kernel: one wave per (chunk, head) prepares what does not need the state - A, T and the
 //   per-token scales - into a record in scratch.  All chunks at once, off the serial chain.
 // * walk kernel: a workgroup walks the chunks of one (sequence, head), or of two heads with the same keys, for 64 or 128
-//   value columns (walk_shape).  Four or eight waves hold 16 columns of S each, in accumulators: the accumulator tiles of
+//   value columns (walk_shape).  Four waves hold 16 or 32 columns of S each (eight 16, by rows at any address), in accumulators: the accumulator tiles of
 //   16 x 16 are, split, at once the operands of the products with S, so S, W and U never leave registers, and a wave does
 //   not wait for another one's products.  The others prepare the chunks' operands in LDS, one step ahead (one barrier per
 //   chunk), with their loads one or two steps ahead of that.
 //
-// Bound of the walk: vector instructions.  fp32 matrix products run on the vector units (the walk with 16x16x4 products:
-// matrix busy 36 - 42 %, vector busy 50 %, and twelve waves per CU bring no more than eight), bf16 ones beside them (here:
-// vector 59 and matrix 30 % for the delta rule per channel, 68 and 20 for the forget gate, 48 and 22, 51 and 14 in the second
-// pass of state space and retention; LDS 7 - 17 %; scores kernels of the first two vector 54 and 51, matrix 11 and 7 %).  So the
-// products with the state are made of bf16 parts: three parts hold the 24 bits of a number, six products of parts leave
+// Bound of the walk: the chain of a chunk's products, parts and LDS reads in a wave that has a SIMD's matrix unit to itself,
+// and the operands' vector work beside it.  fp32 matrix products run on the vector units (the walk with 16x16x4 products:
+// matrix busy 36 - 42 %, vector busy 50 %, and twelve waves per CU bring no more than eight), bf16 ones beside them.
+// So the products with the state are made of bf16 parts: three parts hold the 24 bits of a number, six products of parts leave
 // errors below fp32 products' (they add eight terms between roundings, those four), and a sum over 128 rows takes 24
-// instructions of 16 cycles and 176 vector ones for the state's parts instead of 32 of 32 cycles.
-// The delta rule's waves have a SIMD to themselves but for the operands', and their own chain counts: the parts of the next
-// rows are made between the products (385 -> 369 us in the first line; not for two such waves per SIMD, where vector work
-// in program order between products holds them up: 3 % more).
+// instructions of 16 cycles instead of 32 of 32 cycles.  What a part leaves of its number is a matrix product too (Identity):
+// the parts of 128 rows take 48 vector instructions in place of 176.
+// The products' waves go through full chunks in an order of their own (`full` below), 32 columns per wave where the operands
+// serve 128, so that every operand read from LDS is used twice.  Walk, us, before / with parts by products / in order:
+// delta rule per channel, 4 x 1.9k tokens 257 / 241 / 222, forget gate, 16 x 460 158 / 148 / 129; without the operands'
+// waves' work 207 / 196 and 125 / 119, without the products' 165 / 135 and 114 / 104.
 // Per-channel decays are worked out once, by the scores kernel, and kept in the records (8 KB per 16 tokens and head
 // written and read twice, against 26 instructions per decay in two more places): forget gate 280 -> 262 us, delta rule
 // 377 -> 373.
 // Measured: the token-by-token kernels, fp32 products with 64 columns per workgroup, bf16 parts, and with the scores' halves of
 // channels, pairs inside four tokens and values in one part where they are exact (us, scores + walk; 32 heads of 128, bf16
 // unless noted):
-//   delta rule, per-channel decay, 4 x ~1850 tokens: 1798, 130 + 343, 132 + 262, 99 + 256
-//   forget gate, 16 x ~460 tokens:                    777, 111 + 308, 98 + 168, 83 + 158
+//   delta rule, per-channel decay, 4 x ~1850 tokens: 1798, 130 + 343, 132 + 262, 99 + 256, today 99 + 222
+//   forget gate, 16 x ~460 tokens:                    777, 111 + 308, 98 + 168, 83 + 158, today 83 + 129
 //   state space, 96 heads of 128 x 64, 1023 tokens, fp32: 250, 21 + 94, 22 + 64, 19 + 63 in five segments of head pairs
 //   retention, one portion of 1500 tokens (+ 11 rows): 260, 21 + 88, 22 + 69, 21 + 65 in eight segments, the rows inside the
 //   scores launch
@@ -100,17 +101,50 @@ __device__ __forceinline__ float join(unsigned p0, unsigned p1, unsigned p2, boo
   return b != b ? a : copysignf(__FLT_MAX__, a);   // (a finite number that part 0 rounds to infinity: the largest)
 }
 __device__ __forceinline__ float abs_sum(const f32x4 x) { return (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3])); }
-// ... of eight numbers, in eleven steps of four instructions to go between matrix products
-struct SplitSteps {
-  float r[8], b[8];
-  __device__ __forceinline__ void step(int i, u32x4 (&p)[3]) {   // (i known when compiled)
+// The same for four numbers per lane, what a part leaves by the matrix cores: minus the identity times the part, added to
+// the numbers.  Their layout as 16 x 16 numbers is that of the part as an operand of 16 rows, and one product (16 cycles
+// beside the vector units) takes the place of four instructions that unpack the part and four that subtract it; the
+// difference has at most 24 bits, and it is exact.  A number without parts leaves NaN in the lane's and the column's
+// other three lanes' parts 1 and 2, so it is for numbers whose products are looked at by column, or that have parts.
+struct Identity {
+  u32x2 minus;   // row m, columns 4 gr ... + 3
+  __device__ __forceinline__ explicit Identity(int lane) {
+    const int i = (lane & 15) - 4 * (lane >> 4);
+    minus = u32x2{i == 0 ? 0xbf80u : i == 1 ? 0xbf800000u : 0u, i == 2 ? 0xbf80u : i == 3 ? 0xbf800000u : 0u};
+  }
+  __device__ __forceinline__ f32x4 rest(const f32x4 x, unsigned p0, unsigned p1) const {
+    typedef __attribute__((ext_vector_type(4))) short s16x4;
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, minus), __builtin_bit_cast(s16x4, u32x2{p0, p1}),
+                                                     x, 0, 0, 0);
+  }
+  template <int FIRST = 0>
+  __device__ __forceinline__ void split(f32x4 x, unsigned (&p)[3][2]) const {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int part = i / 5, at = 2 * e + (i + part) % 2;
-      if (i % 5 == 0) p[part][e] = pack_bf16(r[2 * e], r[2 * e + 1]);
-      else if (i % 5 == 1) b[2 * e] = bf16_low(p[part][e]);
-      else if (i % 5 == 2) b[2 * e + 1] = bf16_high(p[part][e]);
-      else r[at] -= b[at];
+    for (int i = FIRST; i < 3; ++i) {
+      p[i][0] = pack_bf16(x[0], x[1]);
+      p[i][1] = pack_bf16(x[2], x[3]);
+      if (i < 2) x = rest(x, p[i][0], p[i][1]);
+    }
+  }
+};
+// Part 0 of products a b, and what it leaves of them unrounded, which the other parts then hold (as a product rounded first,
+// per-channel delta rule in 32 bits, results 8 % further from 64 bits).
+__device__ __forceinline__ f32x4 split_product(const f32x4 a, const f32x4 b, unsigned (&p0)[2]) {
+  p0[0] = pack_bf16(a[0] * b[0], a[1] * b[1]);
+  p0[1] = pack_bf16(a[2] * b[2], a[3] * b[3]);
+  return f32x4{__builtin_fmaf(a[0], b[0], -bf16_low(p0[0])), __builtin_fmaf(a[1], b[1], -bf16_high(p0[0])),
+               __builtin_fmaf(a[2], b[2], -bf16_low(p0[1])), __builtin_fmaf(a[3], b[3], -bf16_high(p0[1]))};
+}
+// ... of eight numbers, in eleven steps to go between matrix products
+struct SplitSteps {
+  f32x4 r[2];
+  __device__ __forceinline__ void step(int i, u32x4 (&p)[3], const Identity& id) {   // (i known when compiled)
+    const int part = i / 5, j = i % 5;
+    if (j == 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[part][e] = pack_bf16(r[e >> 1][2 * (e & 1)], r[e >> 1][2 * (e & 1) + 1]);
+    } else if (j < 3) {
+      r[j - 1] = id.rest(r[j - 1], p[part][2 * (j - 1)], p[part][2 * (j - 1) + 1]);
     }
   }
 };
@@ -1017,11 +1051,12 @@ template <int MODE, int DK, bool EXACT>
 struct WalkBuf {
   static constexpr bool DELTA = MODE >= kModeDelta, CH = per_channel<MODE>();
   static constexpr int COLS = DELTA ? kWalkCols : 2 * kWalkCols, HEADS = MODE == kModeStateSpace ? 2 : 1;
-  // rows in three parts, channels in the order that a product over 32 rows of S takes them (place())
-  __bf16 qe[3][16][DK + 8];                           // P_i q_i; one number as the decay: q_i
-  __bf16 ke[DELTA ? 3 : 1][DELTA ? 16 : 1][DK + 8];   // P_i k_i; k_i
+  // rows in three parts, per four tokens and channel as the lane that prepares them holds them; the reads transpose
+  typedef u32x2 Rows[3][4][DK + 16];
+  Rows qe;                              // P_i q_i; one number as the decay: q_i
+  u32x2 ke[DELTA ? 3 : 1][DELTA ? 4 : 1][DK + 16];   // P_i k_i; k_i
   // D_end,j k_j; not EXACT and one number as the decay: k_j.  Per four tokens and channel two parts of each
-  u32x4 kt01[4][DK];                    // parts 0 and 1; EXACT: 0, and zeros
+  std::conditional_t<EXACT, u32x2, u32x4> kt01[4][DK];   // parts 0 and 1; EXACT: 0
   u32x4 kt20[4][DK];                    // ... 2 and 0; EXACT: 2 and 1
   __bf16 amat[EXACT ? 2 : 1][16][4][8]; // EXACT: A per row and four tokens: part 0, and zeros; parts 2 and 1
   f32x4 v[4][COLS];                     // per four tokens and column
@@ -1046,7 +1081,7 @@ struct WalkLds {
 // state (of which it leaves a copy, since pass 2 overwrites it) to the state at its end; the others but the last from
 // zero to what they add to the state, with the decay over them.  Pass 2 puts the state at a segment's start together
 // from these and walks it; the last segment writes the sequence's state.
-template <typename T, int MODE, int DK, int VEC, int PASS>
+template <typename T, int MODE, int DK, int VEC, int PASS, int CT>
 __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkLds<MODE, DK, exact_values<T, MODE>()>& lds) {
   constexpr int NT = DK / 16, kDecay = scan_rec_decay(MODE);
   const int REC = scan_record_floats(MODE, VEC ? DK : a.dk), DS = scan_decay_width(VEC ? DK : a.dk);   // (scan_scores_kernel)
@@ -1060,12 +1095,13 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
   constexpr int BUFS = WalkLds<MODE, DK, EXACT>::BUFS, OW = operand_waves(MODE, DK);
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int waves = (blockDim.x >> 6) - OW;   // of the products
+  const Identity id(lane);
+  const int waves = (blockDim.x >> 6) - OW, tiles = CT * waves;   // of the products; columns in 16s
   const int hb = a.H / a.walk_heads, cb = blockIdx.x / hb, h0 = blockIdx.x % hb * a.walk_heads;
-  // wave w: 16 columns of a head
+  // wave w: 16 CT columns of a head
   const bool two = a.walk_heads == 2;
-  const int h = two && w < waves ? h0 + (w >> 2) : h0;
-  const int col0 = DELTA || two ? cb * kWalkCols + 16 * (w & 3) : 16 * (cb * waves + w);
+  const int h = two && w < waves ? h0 + (CT * w >> 2) : h0;
+  const int col0 = DELTA || two ? cb * kWalkCols + 16 * (CT * w & 3) : 16 * (cb * tiles + CT * w);
   const int s = sg.s, slot = a.seq_slot[s];
   int first = a.seq_qstart[s], n = a.seq_qstart[s + 1] - first;
   if (slot < 0 || n < a.min_rows) return;
@@ -1136,7 +1172,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           }
       };
       if (tid < 512) {
-        if (waves == 8) put_together(std::integral_constant<int, 2>{});
+        if (tiles == 8) put_together(std::integral_constant<int, 2>{});
         else put_together(std::integral_constant<int, 1>{});
       }
       lds_barrier();
@@ -1145,50 +1181,57 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 
   if (w < waves) {
     // ---- products
+    __builtin_amdgcn_s_setprio(1);   // (their chain is the longer one: walk of the per-channel delta rule 224 -> 222 us)
     const int m = lane & 15, gr = lane >> 4;
-    const int col = col0 + m;
-    const bool on = col < a.dv;
     float* st = a.state + (static_cast<int64_t>(slot) * a.H + h) * a.dk * a.dv;
-    f32x4 S[NT];
+    f32x4 S[CT][NT];
     // (the last segment of a cut portion holds the copy of the sequence's state)
     const float* from = PASS == 2 ? seg_state(sg.P - 1, h) : st;
-    const bool blank = PASS == 1 && sg.j > 0, fresh = PASS != 2 && a.positions[first] == 0;
+    const bool blank = PASS == 1 && sg.j > 0, fresh = (PASS == 0 || sg.j == 0) && a.positions[first] == 0;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * t + 4 * gr + i;
-        const bool in = on && d < a.dk;
-        if (PASS == 2 && sg.j > 0) {
-          const float x = lds.start[DELTA ? 0 : d][16 * w + m];
-          S[t][i] = in ? x : 0.f;
-        } else {
-          const float x = from[static_cast<int64_t>(min(d, a.dk - 1)) * a.dv + min(col, a.dv - 1)];
-          S[t][i] = !fresh && !blank && in ? x : 0.f;
-        }
-      }
-    if (PASS == 2 && sg.j > 0) lds_barrier();   // (the operands' buffers are the same memory)
-    auto store_state = [&](float* p) {
-      int c = col, r = 4 * gr;   // (new values: the addresses of the loads would be kept over the chunks)
-      asm volatile("" : "+v"(c), "+v"(r));
-      if (c < a.dv)
+      for (int t = 0; t < NT; ++t) S[ct][t] = zero;
+    if (!fresh && !blank)   // (uniform)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        const int col = col0 + 16 * ct + m;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int d = 16 * t + r + i;
-            if (d < a.dk) p[static_cast<int64_t>(d) * a.dv + c] = S[t][i];
+            const int d = 16 * t + 4 * gr + i;
+            const bool in = col < a.dv && d < a.dk;
+            const float x = PASS == 2 && sg.j > 0 ? lds.start[DELTA ? 0 : d][16 * (CT * w + ct) + m]
+                                                  : from[static_cast<int64_t>(min(d, a.dk - 1)) * a.dv + min(col, a.dv - 1)];
+            S[ct][t][i] = in ? x : 0.f;
           }
+      }
+    if (PASS == 2 && sg.j > 0) lds_barrier();   // (the operands' buffers are the same memory)
+    auto store_state = [&](float* p) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        int c = col0 + 16 * ct + m, r = 4 * gr;   // (new values: the addresses of the loads would be kept over the chunks)
+        asm volatile("" : "+v"(c), "+v"(r));
+        if (c < a.dv)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int d = 16 * t + r + i;
+              if (d < a.dk) p[static_cast<int64_t>(d) * a.dv + c] = S[ct][t][i];
+            }
+      }
     };
-    if (PASS == 1 && sg.j == 0) store_state(seg_state(sg.P - 1, h));
+    if (PASS == 1 && sg.j == 0 && !fresh) store_state(seg_state(sg.P - 1, h));
     float* op = a.out + (static_cast<int64_t>(first) * a.H + h) * a.dv;
     const int o_stride = a.H * a.dv;
     const float skip = MODE == kModeStateSpace ? a.p2[h] : 0.f;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     ChunkDecay fixed;
     if (MODE == kModeRetention) fixed.set(a.p0 + h * kPowers);
     float over = 1.f;   // one number as the decay: over the chunks so far
-    const int head = Buf::HEADS == 2 && two ? w >> 2 : 0;
+    const int head = Buf::HEADS == 2 && two ? CT * w >> 2 : 0;
     // of the record: A or T (row m; the fp64 product's results want the rows in another order), and the scales of the
     // tokens 4 gr ...
     auto matrix = [&](const Buf& b, int at) {
@@ -1203,10 +1246,23 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     struct Sum {
       f32x4 big, small[2];
     };
-    auto add = [&](Sum& x, const __bf16 (&rows)[3][16][DK + 8], const u32x4 (&p)[3], int s) {
+    // The rows of the 16 tokens, 32 channels in the order that a product over 32 rows of S takes them (of two tiles of S the
+    // rows 4 gr + i).  The read transposes pieces of four tokens in groups of 16 lanes, four channels of all tokens; a lane's
+    // own piece is at (token group m % 4, channel m / 4).
+    auto row = [&](const u32x2 (&x)[4][DK + 16], int s) {
+      typedef __attribute__((ext_vector_type(4))) short s16x4;
+      auto get = [&](int t) {
+        const u32x2* at = &x[m & 3][32 * s + 16 * t + 4 * gr + (m >> 2)];
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                             (__attribute__((address_space(3))) s16x4*)(void*)const_cast<u32x2*>(at)));
+      };
+      const u32x2 lo = get(0), hi = get(1);
+      return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    };
+    auto add = [&](Sum& x, const typename Buf::Rows& rows, const u32x4 (&p)[3], int s) {
       u32x4 r[3];
 #pragma unroll
-      for (int e = 0; e < 3; ++e) r[e] = *reinterpret_cast<const u32x4*>(&rows[e][m][32 * s + 8 * gr]);
+      for (int e = 0; e < 3; ++e) r[e] = row(rows[e], s);
       x.small[0] = mma(r[0], p[2], x.small[0]);
       x.small[1] = mma(r[2], p[0], x.small[1]);
       x.big = mma(r[0], p[0], x.big);
@@ -1221,7 +1277,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     };
     // The same in fp32, where parts are missing or the sum of rows that are not scaled is not finite; here they are (`scales`:
     // the scales in the record).
-    auto sum_fp32 = [&](const Buf& b, const __bf16 (&rows)[3][16][DK + 8], int scales) {
+    auto sum_fp32 = [&](const Buf& b, const typename Buf::Rows& rows, int scales, const f32x4 (&S)[NT]) {
       const float sc = MODE == kModeForget ? 1.f : b.scale[head][scales - kRecQ + m];
       f32x4 x = zero;
 #pragma unroll
@@ -1229,23 +1285,25 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           __builtin_amdgcn_sched_barrier(0);
-          const int at = 32 * (t >> 1) + 8 * gr + 4 * (t & 1) + i;
           unsigned r[3];
 #pragma unroll
-          for (int e = 0; e < 3; ++e) r[e] = *reinterpret_cast<const unsigned short*>(&rows[e][m][at]);
+          for (int e = 0; e < 3; ++e)
+            r[e] = reinterpret_cast<const unsigned short*>(&rows[e][m >> 2][16 * t + 4 * gr + i])[m & 3];
           x = mma(join(r[0], r[1], r[2], false) * sc, S[t][i], x);
         }
       return x;
     };
     // the rows 32 s ... of S in parts
-    auto state_parts = [&](u32x4 (&p)[3], int s) {
+    auto state_parts = [&](u32x4 (&p)[3], int s, const f32x4 (&S)[NT]) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f32x4& t = S[2 * s + (e >> 1)];
-        unsigned x[3];
-        split(t[2 * (e & 1)], t[2 * (e & 1) + 1], x[0], x[1], x[2]);
+      for (int t = 0; t < 2; ++t) {
+        unsigned x[3][2];
+        id.split(S[2 * s + t], x);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) p[i][e] = x[i];
+        for (int i = 0; i < 3; ++i) {
+          p[i][2 * t] = x[i][0];
+          p[i][2 * t + 1] = x[i][1];
+        }
       }
     };
     // U in parts, as the other operand of 16 tokens: half of a product's 32 terms, the other half takes other parts
@@ -1254,16 +1312,21 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       u32x4 p0, p10, p1, p02;
     };
     // EXACT: the number itself, beside part 0, or the parts 2 and 1, of the keys and of A.
-    auto parts = [](const f32x4 x) {
-      if constexpr (EXACT) {
-        const unsigned u = pack_bf16(x[0], x[1]), v = pack_bf16(x[2], x[3]);
-        return Parts{u32x4{u, v, 0, 0}, u32x4{}, u32x4{}, u32x4{u, v, u, v}};
-      }
-      unsigned u[3][2];
-      split(x[0], x[1], u[0][0], u[1][0], u[2][0]);
-      split(x[2], x[3], u[0][1], u[1][1], u[2][1]);
+    auto as_parts = [](const unsigned (&u)[3][2]) {
       return Parts{u32x4{u[0][0], u[0][1], 0, 0}, u32x4{u[1][0], u[1][1], u[0][0], u[0][1]},
                    u32x4{0, 0, u[1][0], u[1][1]}, u32x4{u[0][0], u[0][1], u[2][0], u[2][1]}};
+    };
+    // of V, scaled as the state gets it
+    auto parts = [&](const f32x4 V, const f32x4 by) {
+      if constexpr (EXACT) {
+        const unsigned u = pack_bf16(V[0], V[1]), v = pack_bf16(V[2], V[3]);
+        return Parts{u32x4{u, v, 0, 0}, u32x4{}, u32x4{}, u32x4{u, v, u, v}};
+      } else {
+        unsigned u[3][2];
+        if constexpr (CH) id.split(V, u);
+        else id.template split<1>(split_product(V, by, u[0]), u);
+        return as_parts(u);
+      }
     };
     auto abs = [](const f32x4 x) { return f32x4{fabsf(x[0]), fabsf(x[1]), fabsf(x[2]), fabsf(x[3])}; };
     // numbers that split() takes, and sums that were not of others; `U`: as the state gets them
@@ -1272,32 +1335,61 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       return !__any(!(abs_sum(U) + abs_sum(R) + keys <= 0.5f * kSplitMax));
     };
     auto finite = [](float x) { return fabsf(x) < HUGE_VALF; };
+    // The product of the first parts.  EXACT: of 16 terms; where a product of 32 terms adds to it, a vector instruction is in
+    // between (the compiler leaves too few cycles for the sum of one straight into the other).
+    typedef std::conditional_t<EXACT, u32x2, u32x4> Kt;
+    auto first_parts = [](const Kt& x, const Parts& u, const f32x4 D) {
+      if constexpr (EXACT) {
+        typedef __attribute__((ext_vector_type(4))) short s16x4;
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, x),
+                                                         __builtin_bit_cast(s16x4, u32x2{u.p0[0], u.p0[1]}), D, 0, 0, 0);
+      } else {
+        return mma(x, u.p0, D);
+      }
+    };
+    auto decay_rows = [&](const Buf& b, float end, int t) {
+      if (CH) return *reinterpret_cast<const f32x4*>(&b.end[CH ? 16 * t + 4 * gr : 0]);
+      return f32x4{end, end, end, end};
+    };
     // A tile of S where U or the keys are not ordinary: as advance(), and what comes out not finite in fp32, with kt scaled
     // and not U.
-    auto advance_odd = [&](const Buf& b, const f32x4 V, const Parts& u, float end, int t, const u32x4 x, const u32x4 y, f32x4 D) {
+    auto advance_odd = [&](const Buf& b, const f32x4 V, const Parts& u, float end, int t, const Kt x, const u32x4 y, f32x4 D,
+                           f32x4 (&S)[NT]) {
       const f32x4 sc = CH || EXACT ? f32x4{1.f, 1.f, 1.f, 1.f} : scale(b, kRecKt);
-      f32x4 f = {end, end, end, end};
-      if (CH) f = *reinterpret_cast<const f32x4*>(&b.end[CH ? 16 * t + 4 * gr : 0]);
+      const f32x4 f = decay_rows(b, end, t);
       f32x4 other = S[t] * f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) other = mma(join(x[i >> 1], (EXACT ? y : x)[2 + (i >> 1)], y[i >> 1], i & 1) * sc[i], V[i], other);
+      for (int i = 0; i < 4; ++i) {
+        const unsigned p1 = EXACT ? y[2 + (i >> 1)] : x[(2 + (i >> 1)) % (sizeof(Kt) / 4)];
+        other = mma(join(x[i >> 1], p1, y[i >> 1], i & 1) * sc[i], V[i], other);
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) D[i] = __builtin_fmaf(S[t][i], f[i], D[i]);
-      D = mma(x, u.p0, D);
+      D = first_parts(x, u, D);
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[t][i] = finite(D[i]) ? D[i] : other[i];
+    };
+    // the smaller parts' products
+    auto small_parts = [&](const Kt& x, const u32x4& y, const Parts& u) {
+      f32x4 D = mma(y, u.p02, zero);
+      if constexpr (!EXACT) {
+        D = mma(x, u.p1, D);
+        D = mma(x, u.p10, D);
+      }
+      return D;
     };
     // S = P_end S + kt U.  A product adds eight terms and the sum so far at a time, less exactly the wider their range; so
     // the first parts' come by themselves and last, on top of what the state's decay leaves, in the tokens' order: what
     // decays have made small is rounded while it is alone.  (Error of 16 tokens whose decay is 1 / 0.5 each, 1e-8, fp32
     // products / with parts 0 x 0 and 1 x 0 in one product / here: 8.5 / 5.1 / 3.8 and 2.9 / 4.2 / 3.3.)
-    // `U`: scaled, `V`: as it is; `is_odd`: U or the keys are not ordinary
-    auto advance = [&](const Buf& b, const f32x4 V, const f32x4 U, float end, auto is_odd) {
-      const Parts u = parts(EXACT ? V : U);
+    // `V`: not scaled; `is_odd`: U or the keys are not ordinary
+    auto advance = [&](const Buf& b, const f32x4 V, float end, auto is_odd, f32x4 (&S)[NT]) {
+      const Parts u = parts(V, CH || EXACT ? zero : scale(b, kRecKt));
       bool odd = false;
       // Two tiles at a time, whose products do not wait for each other, and the next two's operands on their way (left to
       // itself the compiler loads all of them first, and spills).
-      u32x4 hm[2][2], lh[2][2];
+      Kt hm[2][2];
+      u32x4 lh[2][2];
       auto ahead = [&](int t) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -1313,28 +1405,21 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         if (t + 2 < NT) ahead(t + 2);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int e = 0; e < 2; ++e) D[e] = mma(lh[p][e], u.p02, zero);
-        if constexpr (!EXACT) {
-#pragma unroll
-          for (int e = 0; e < 2; ++e) D[e] = mma(hm[p][e], u.p1, D[e]);
-#pragma unroll
-          for (int e = 0; e < 2; ++e) D[e] = mma(hm[p][e], u.p10, D[e]);
-        }
+        for (int e = 0; e < 2; ++e) D[e] = small_parts(hm[p][e], lh[p][e], u);
         if (t == 0) odd = is_odd();   // (here the latency of a check is hidden)
         if (__builtin_expect(odd, 0)) {
 #pragma unroll
-          for (int e = 0; e < 2; ++e) advance_odd(b, V, u, end, t + e, hm[p][e], lh[p][e], D[e]);
+          for (int e = 0; e < 2; ++e) advance_odd(b, V, u, end, t + e, hm[p][e], lh[p][e], D[e], S);
           continue;
         }
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          f32x4 f = {end, end, end, end};
-          if (CH) f = *reinterpret_cast<const f32x4*>(&b.end[CH ? 16 * (t + e) + 4 * gr : 0]);
+          const f32x4 f = decay_rows(b, end, t + e);
 #pragma unroll
           for (int i = 0; i < 4; ++i) S[t + e][i] = __builtin_fmaf(S[t + e][i], f[i], D[e][i]);
         }
 #pragma unroll
-        for (int e = 0; e < 2; ++e) S[t + e] = mma(hm[p][e], u.p0, S[t + e]);
+        for (int e = 0; e < 2; ++e) S[t + e] = first_parts(hm[p][e], u, S[t + e]);
       }
     };
     auto replace = [&](f32x4& x, f32x4& scale, const f32x4 with) {   // what is not finite
@@ -1360,14 +1445,15 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     };
     // A V, the smaller parts of A first
     auto read_out_exact = [&](const Buf& b, const f32x4 V) {
-      const Parts u = parts(V);
+      const Parts u = parts(V, zero);
       u32x4 x[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) x[e] = *reinterpret_cast<const u32x4*>(&b.amat[EXACT ? e : 0][m][gr][0]);
       return mma(x[0], u.p0, mma(x[1], u.p02, zero));
     };
     // AV: EXACT, and ordinary: the sum A U
-    auto write = [&](const Buf& b, const f32x4 U, const f32x4 R, const f32x4 sq, const f32x4 V, int c, auto odd, const f32x4 AV) {
+    auto write = [&](const Buf& b, const f32x4 U, const f32x4 R, const f32x4 sq, const f32x4 V, int c, auto odd, const f32x4 AV, int col0) {
+      const int col = col0 + m;
       float* oc = op + static_cast<int64_t>(c) * kScanChunk * o_stride;
       f32x4 x = U, bad;
       if constexpr (odd) bad = take_nonfinite(x, lane);
@@ -1393,23 +1479,231 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 #pragma unroll
         for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = O[i];
       } else {
-        const int rows = on ? n - c * kScanChunk - 4 * gr : 0;
+        const int rows = col < a.dv ? n - c * kScanChunk - 4 * gr : 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           if (i < rows) at_bytes<float>(oc + i * o_stride, at) = O[i];
       }
     };
+    auto order = [] { __builtin_amdgcn_sched_barrier(0); };
+    // product i of rows r and a state's parts q
+    auto product = [&](Sum& x, const u32x4 (&r)[3], const u32x4 (&q)[3], int i) {
+      constexpr int kRow[] = {0, 2, 0, 1, 1, 0}, kState[] = {2, 0, 0, 1, 0, 1}, kSum[] = {0, 1, 2, 0, 1, 0};
+      f32x4& to = kSum[i] == 2 ? x.big : x.small[kSum[i] % 2];
+      to = mma(r[kRow[i]], q[kState[i]], to);
+    };
+    // beside product i of six: a part of the next rows, and what it leaves
+    auto part_beside = [&](SplitSteps& next, int i, u32x4 (&q)[3]) {
+      if (i % 2 == 0) {
+        next.step(5 * (i / 2), q, id);
+        if (i < 4) {
+          next.step(5 * (i / 2) + 1, q, id);
+          next.step(5 * (i / 2) + 2, q, id);
+        }
+      }
+    };
+    // Full chunks of full columns and ordinary numbers are walked in loops of their own.  A wave issues in order, and left to
+    // itself the compiler puts every load, part and product right in front of what waits for it; here all have been on their
+    // way for a few products.  A chunk that is not ordinary is left, untouched, to the loop behind (two ways in one loop cost
+    // a move per number of the state and chunk).
+    const int full = col0 + 16 * CT <= a.dv ? n / kScanChunk : 0;
+    int c = 0;
     lds_barrier();
     if constexpr (DELTA) {
+      SplitSteps next;
+      auto take = [&](int s) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) next.r[e] = S[0][(2 * s + e) % NT];
+      };
+      if constexpr (NT == 8) {
+        u32x4 p[3][3];   // of S's rows 0 - 31 and 96 - 127, 32 - 63, 64 - 95
+        state_parts(p[0], 0, S[0]);
+        for (; c < full; ++c) {
+          const Buf& b = lds.buf[c % BUFS];
+          const auto& key_rows = *reinterpret_cast<const typename Buf::Rows*>(&b.ke);
+          Sum Ws = {zero, {zero, zero}}, Rs = Ws;
+          u32x4 ra[3], rb[3], rc[3];
+          auto load = [&](u32x4 (&r)[3], const typename Buf::Rows& rows, int s, int e) { r[e] = row(rows[e], s); };
+          // six products of rows r and the parts q; beside them what `more` does in step i
+          auto products = [&](Sum& x, const u32x4 (&r)[3], const u32x4 (&q)[3], auto more) {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+              product(x, r, q, i);
+              order();
+              more(i);
+              order();
+            }
+          };
+#pragma unroll
+          for (int e = 0; e < 3; ++e) load(ra, key_rows, 0, e);
+#pragma unroll
+          for (int e = 0; e < 3; ++e) load(rc, b.qe, 0, e);
+#pragma unroll
+          for (int e = 0; e < 3; ++e) load(rb, key_rows, 1, e);
+          order();
+          take(1);   // (while the rows come)
+#pragma unroll
+          for (int i = 0; i < 11; ++i) {
+            next.step(i, p[1], id);
+            order();
+          }
+          take(2);
+          products(Ws, ra, p[0], [&](int i) { part_beside(next, i, p[2]); });
+          products(Rs, rc, p[0], [&](int i) { if (i < 3) load(ra, key_rows, 2, i); });
+          take(3);
+          products(Ws, rb, p[1], [&](int i) {
+            if (i < 3) load(rc, b.qe, 1, i);
+            part_beside(next, i, p[0]);
+          });
+          products(Ws, ra, p[2], [&](int i) { if (i < 3) load(rb, key_rows, 3, i); });
+          f32x4 M, v, sk, skt;
+          products(Ws, rb, p[0], [&](int i) {
+            if (i == 0) M = matrix(b, DELTA ? 256 : 0);
+            if (i == 1) v = b.v[gr][16 * w + m];
+            if (i == 2) sk = scale(b, kRecK);
+            if (i == 2) skt = CH ? zero : scale(b, kRecKt);
+            if (i >= 3) load(ra, b.qe, 2, i - 3);
+          });
+          // From here on W's sum, U and its parts one after the other, and between them the sum for the outputs.
+          f32x4 X, U, U2, rest;
+          float sum = 0.f;
+          unsigned u[3][2];
+          products(Rs, rc, p[1], [&](int i) {
+            if (i < 3) load(rb, b.qe, 3, i);
+            if (i == 1) X = Ws.big + (Ws.small[0] + Ws.small[1]);
+            if (i == 2) X = v - sk * X;
+            if (i == 3) U = mma(M[0], X[0], zero);
+            if (i == 3) U2 = mma(M[1], X[1], zero);
+            if (i == 5) U = mma(M[2], X[2], U);
+            if (i == 5) U2 = mma(M[3], X[3], U2);
+          });
+          products(Rs, ra, p[2], [&](int i) {
+            if (i == 0) sum = abs_sum(X) + (abs_sum(M) + (CH ? 0.f : b.scale[head][kRecNoParts - kRecQ]));
+            if (i == 2) {
+              U += U2;
+              if constexpr (CH) {
+                u[0][0] = pack_bf16(U[0], U[1]);
+                u[0][1] = pack_bf16(U[2], U[3]);
+                rest = id.rest(U, u[0][0], u[0][1]);
+              } else {
+                rest = split_product(U, skt, u[0]);
+              }
+            }
+            if (i == 5) {
+              u[1][0] = pack_bf16(rest[0], rest[1]);
+              u[1][1] = pack_bf16(rest[2], rest[3]);
+              rest = id.rest(rest, u[1][0], u[1][1]);
+            }
+          });
+          Kt hm[2][2];
+          u32x4 lh[2][2];
+          f32x4 f[2][2];
+          auto keys = [&](int t) {
+            const int q = t / 2 % 2;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              lh[q][e] = b.kt20[gr][16 * (t + e) + m];
+              hm[q][e] = b.kt01[gr][16 * (t + e) + m];
+              if (CH) f[q][e] = decay_rows(b, 0.f, t + e);
+            }
+          };
+          f32x4 A, sq;
+          products(Rs, rb, p[0], [&](int i) {
+            if (i == 0) keys(0);
+            if (i == 2) keys(2);
+            if (i == 3) {
+              u[2][0] = pack_bf16(rest[0], rest[1]);
+              u[2][1] = pack_bf16(rest[2], rest[3]);
+            }
+            if (i == 4) A = matrix(b, 0);
+            if (i == 5) sq = scale(b, kRecQ);
+          });
+          const Parts parts_u = as_parts(u);
+          const float end = decay_of(b);
+          f32x4 D[2][2];
+          auto small = [&](int t) {   // small_parts(), the two tiles in turn
+            const int q = t / 2 % 2, r = q;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              D[r][e] = mma(lh[q][e], parts_u.p02, zero);
+              order();
+            }
+            if constexpr (!EXACT) {
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                D[r][e] = mma(hm[q][e], parts_u.p1, D[r][e]);
+                order();
+              }
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                D[r][e] = mma(hm[q][e], parts_u.p10, D[r][e]);
+                order();
+              }
+            }
+          };
+          small(0);
+          const f32x4 R = total(Rs);
+          sum += abs_sum(R);
+          // (sums of 16 of these products and of 128 rows, scaled, are far from the ends of the range)
+          if (__builtin_expect(__any(!(sum <= 0x1p50f)), 0)) break;
+          f32x4 Y[2];
+#pragma unroll
+          for (int t = 0; t < NT; t += 2) {
+            const int q = t / 2 % 2, r = q;
+            order();
+            if (t + 2 < NT) small(t + 2);
+            order();
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) S[0][t + e][i] = __builtin_fmaf(S[0][t + e][i], CH ? f[q][e][i] : end, D[r][e][i]);
+            order();
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              S[0][t + e] = first_parts(hm[q][e], parts_u, S[0][t + e]);
+              order();
+            }
+            if (t + 4 < NT) keys(t + 4);
+            if (t < 4) {   // A U
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                Y[e] = mma(A[t + e], U[t + e], t == 0 ? zero : Y[e]);
+                order();
+              }
+            }
+            if (t == 2) {
+              take(0);
+              next.step(0, p[0], id);
+              next.step(1, p[0], id);
+              order();
+              next.step(2, p[0], id);
+            }
+            if (t == 4) {
+              next.step(5, p[0], id);
+              next.step(6, p[0], id);
+              order();
+              next.step(7, p[0], id);
+              Y[0] += Y[1];
+              float* oc = op + static_cast<int64_t>(c) * kScanChunk * o_stride;
+              const unsigned at = (4 * gr * o_stride + col0 + m) * sizeof(float);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = __builtin_fmaf(R[i], sq[i], Y[0][i]);
+            }
+          }
+          order();
+          next.step(10, p[0], id);
+          lds_barrier();
+        }
+      }
       u32x4 p[2][3];
-      state_parts(p[0], 0);
-      for (int c = 0; c < nc; ++c) {
+      state_parts(p[0], 0, S[0]);
+      for (; c < nc; ++c) {
         const Buf& b = lds.buf[c % BUFS];
         Sum Ws = {zero, {zero, zero}}, Rs = Ws;
         u32x4 rows[2][2][3];   // of ke and qe
+        const auto& key_rows = *reinterpret_cast<const typename Buf::Rows*>(&b.ke);
         auto ahead = [&](int s, int i) {
-          rows[s & 1][i / 3][i % 3] = *reinterpret_cast<const u32x4*>(
-              i < 3 ? &b.ke[DELTA ? i : 0][DELTA ? m : 0][32 * s + 8 * gr] : &b.qe[i - 3][m][32 * s + 8 * gr]);
+          rows[s & 1][i / 3][i % 3] = row(i < 3 ? key_rows[i] : b.qe[i - 3], s);
         };
 #pragma unroll
         for (int i = 0; i < 6; ++i) ahead(0, i);
@@ -1421,7 +1715,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           SplitSteps next;
           if (more)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) next.r[e] = S[(2 * s + 2 + (e >> 2)) % NT][e & 3];
+            for (int e = 0; e < 2; ++e) next.r[e] = S[0][(2 * s + 2 + e) % NT];
 #pragma unroll
           for (int i = 0; i < 12; ++i) {   // products of ke and qe in turn
             constexpr int kRow[] = {0, 2, 0, 1, 1, 0}, kState[] = {2, 0, 0, 1, 0, 1}, kSum[] = {0, 1, 2, 0, 1, 0};
@@ -1429,7 +1723,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             f32x4& to = kSum[i >> 1] == 2 ? x.big : x.small[kSum[i >> 1]];
             to = mma(rows[s & 1][i & 1][kRow[i >> 1]], p[s & 1][kState[i >> 1]], to);
             if (more && i < 6) ahead(s + 1, i);
-            if (more && i < 11) next.step(i, p[s + 1 & 1]);
+            if (more && i < 11) next.step(i, p[s + 1 & 1], id);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -1444,10 +1738,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           U = mma(M[2], X[2], U);
           U2 = mma(M[3], X[3], U2);
           U += U2;
-          const f32x4 Us = CH ? U : U * scale(b, kRecKt);
-          advance(b, U, Us, decay_of(b), [] { return decltype(odd)::value; });
-          write(b, U, R, sq, zero, c, odd, zero);
-          state_parts(p[0], 0);
+          advance(b, U, decay_of(b), [] { return decltype(odd)::value; }, S[0]);
+          write(b, U, R, sq, zero, c, odd, zero, col0);
+          state_parts(p[0], 0, S[0]);
         };
         // (sums of 16 of these products and of 128 rows, scaled, are far from the ends of the range)
         const float keys = CH ? 0.f : b.scale[head][kRecNoParts - kRecQ];
@@ -1455,8 +1748,8 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           finish(std::false_type{});
         } else {
           f32x4 one = {1.f, 1.f, 1.f, 1.f};
-          replace(R, sq, sum_fp32(b, b.qe, kRecQ));
-          replace(X, one, v - sum_fp32(b, *reinterpret_cast<const __bf16 (*)[3][16][DK + 8]>(&b.ke), kRecK));
+          replace(R, sq, sum_fp32(b, b.qe, kRecQ, S[0]));
+          replace(X, one, v - sum_fp32(b, key_rows, kRecK, S[0]));
           bad = take_nonfinite(X, lane);
           finish(std::true_type{});
         }
@@ -1465,44 +1758,199 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       if (nc & 1) lds_barrier();
       store_state(st);
     } else {
-      for (int c = 0; c < nc; ++c) {
-        const Buf& b = lds.buf[c % BUFS];
-        const f32x4 U = b.v[gr][16 * w + m], Us = CH || EXACT ? U : U * scale(b, kRecKt);
-        f32x4 R = zero, AV = zero;
-        if (PASS != 1) {
-          if constexpr (EXACT) AV = read_out_exact(b, U);
-          Sum Rs = {zero, {zero, zero}};
-#pragma unroll
-          for (int s = 0; s < NT / 2; ++s) {
-            u32x4 p[3];
-            state_parts(p, s);
-            add(Rs, b.qe, p, s);
-          }
-          R = total(Rs);
-        }
+      // The chunk's decay where it is one number, and over the chunks so far.
+      auto end_of = [&](const Buf& b, int c) {
         float end = decay_of(b);
         if (MODE == kModeRetention) {
           const float e = fixed.next();
           end = n - c * kScanChunk >= kScanChunk ? e : end;
         }
         if (PASS == 1 && !CH) over *= end;
+        return end;
+      };
+      auto worst = [&](const Buf& b) { return CH ? 0.f : b.scale[head][kRecNoParts - kRecQ]; };
+      for (; c < full; ++c) {
+        const Buf& b = lds.buf[c % BUFS];
+        f32x4 U[CT], f[2][2];
+        Kt hm[2][2];
+        u32x4 lh[2][2];
+        Parts u[CT];
+        auto keys = [&](int t) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            lh[t >> 1 & 1][e] = b.kt20[gr][16 * (t + e) + m];
+            hm[t >> 1 & 1][e] = b.kt01[gr][16 * (t + e) + m];
+            if (CH) f[t >> 1 & 1][e] = decay_rows(b, 0.f, t + e);
+          }
+        };
+        float sum = worst(b);
+        if constexpr (PASS != 1) {
+          u32x4 rows[2][3], p[2][CT][3], A[2];
+          Sum Rs[CT];
+          f32x4 AV[CT];
+          auto ahead = [&](int s, int e) { rows[s & 1][e] = row(b.qe[e], s); };
+#pragma unroll
+          for (int e = 0; e < 3; ++e) ahead(0, e);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            U[ct] = b.v[gr][16 * (CT * w + ct) + m];
+            Rs[ct] = {zero, {zero, zero}};
+          }
+          const f32x4 sq = scale(b, kRecQ), sk = CH || EXACT ? zero : scale(b, kRecKt);
+          f32x4 M = zero;
+          if constexpr (EXACT) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) A[e] = *reinterpret_cast<const u32x4*>(&b.amat[EXACT ? e : 0][m][gr][0]);
+          } else {
+            M = matrix(b, 0);
+          }
+          order();
+          SplitSteps next[CT];
+          auto take = [&](int s) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+              for (int e = 0; e < 2; ++e) next[ct].r[e] = S[ct][2 * s + e];
+          };
+          take(0);
+#pragma unroll
+          for (int i = 0; i < 11; ++i) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) next[ct].step(i, p[0][ct], id);
+            order();
+          }
+#pragma unroll
+          for (int s = 0; s < NT / 2; ++s) {
+            const bool more = s + 1 < NT / 2;
+            if (more) take(s + 1);
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+#pragma unroll
+              for (int ct = 0; ct < CT; ++ct) {
+                product(Rs[ct], rows[s & 1], p[s & 1][ct], i);
+                if (more) {
+                  if (ct == 0 && i < 3) ahead(s + 1, i);
+                  part_beside(next[ct], i, p[s + 1 & 1][ct]);
+                } else if (i == 0) {
+                  u[ct] = parts(U[ct], sk);
+                  sum += abs_sum(CH || EXACT ? U[ct] : U[ct] * sk);
+                  if (ct == 0) keys(0);
+                } else if (EXACT && i == 2) {
+                  AV[ct] = mma(A[1], u[ct].p02, zero);
+                } else if (EXACT && i == 4) {
+                  AV[ct] = mma(A[0], u[ct].p0, AV[ct]);
+                }
+                order();
+              }
+            }
+          }
+          f32x4 R[CT];
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            if constexpr (!EXACT && !F64) AV[ct] = read_out(M, U[ct]);
+            R[ct] = total(Rs[ct]);
+            sum += abs_sum(R[ct]);
+            if (EXACT) sum += abs_sum(AV[ct]);
+          }
+          if (__builtin_expect(__any(!(sum <= 0.5f * kSplitMax)), 0)) break;
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            f32x4 O;
+            if constexpr (F64) {
+              const auto X = read_out(M, U[ct]);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) O[i] = static_cast<float>(X[i] + R[ct][i]);
+            } else {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                O[i] = MODE == kModeForget ? AV[ct][i] + R[ct][i] : __builtin_fmaf(R[ct][i], sq[i], AV[ct][i]);
+            }
+            if (MODE == kModeStateSpace) O += skip * U[ct];
+            float* oc = op + static_cast<int64_t>(c) * kScanChunk * o_stride;
+            const unsigned at = (4 * gr * o_stride + col0 + 16 * ct + m) * sizeof(float);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = O[i];
+          }
+        } else {
+          keys(0);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            U[ct] = b.v[gr][16 * (CT * w + ct) + m];
+            const f32x4 sk = CH || EXACT ? zero : scale(b, kRecKt);
+            sum += abs_sum(CH || EXACT ? U[ct] : U[ct] * sk);
+            u[ct] = parts(U[ct], sk);
+          }
+          if (__builtin_expect(__any(!(sum <= 0.5f * kSplitMax)), 0)) break;
+        }
+        const float end = end_of(b, c);
         // The waves of a SIMD end their steps in different places: while one waits for the read-out's products, the other
         // one has those with kt, whose vector work and operands take longer.
-        if constexpr (PASS == 1) {
-          if (w >= 4) lds_barrier();
-          advance(b, U, Us, end, [&] { return !ordinary(b, Us, zero); });
-        } else if (__builtin_expect(ordinary(b, Us, EXACT ? abs(R) + abs(AV) : R), 1)) {
-          write(b, U, R, scale(b, kRecQ), U, c, std::false_type{}, AV);
-          if (w >= 4) lds_barrier();
-          advance(b, U, Us, end, [] { return false; });
-        } else {
-          f32x4 sq = scale(b, kRecQ);
-          replace(R, sq, sum_fp32(b, b.qe, kRecQ));
-          write(b, U, R, sq, U, c, std::true_type{}, AV);
-          if (w >= 4) lds_barrier();
-          advance(b, U, Us, end, [] { return true; });
+        if (CT == 1 && w >= 4) lds_barrier();
+        f32x4 D[2][2][CT];
+        auto small = [&](int t) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) D[t >> 1 & 1][e][ct] = small_parts(hm[t >> 1 & 1][e], lh[t >> 1 & 1][e], u[ct]);
+        };
+        small(0);
+#pragma unroll
+        for (int t = 0; t < NT; t += 2) {
+          const int q = t >> 1 & 1;
+          if (t + 2 < NT) keys(t + 2);
+          order();
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                S[ct][t + e][i] = __builtin_fmaf(S[ct][t + e][i], CH ? f[q][e][i] : end, D[q][e][ct][i]);
+          order();
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) S[ct][t + e] = first_parts(hm[q][e], u[ct], S[ct][t + e]);
+          if (t + 2 < NT) small(t + 2);
+          order();
         }
-        if (w < 4) lds_barrier();
+        if (CT == 2 || w < 4) lds_barrier();
+      }
+      for (; c < nc; ++c) {
+        const Buf& b = lds.buf[c % BUFS];
+        const float end = end_of(b, c);
+        auto chunk = [&](f32x4 (&S)[NT], int ct, bool sync) __attribute__((always_inline)) {
+          const f32x4 U = b.v[gr][16 * (CT * w + ct) + m], Us = CH || EXACT ? U : U * scale(b, kRecKt);
+          f32x4 R = zero, AV = zero;
+          if (PASS != 1) {
+            if constexpr (EXACT) AV = read_out_exact(b, U);
+            Sum Rs = {zero, {zero, zero}};
+#pragma unroll
+            for (int s = 0; s < NT / 2; ++s) {
+              u32x4 p[3];
+              state_parts(p, s, S);
+              add(Rs, b.qe, p, s);
+            }
+            R = total(Rs);
+          }
+          if constexpr (PASS == 1) {
+            if (sync) lds_barrier();
+            advance(b, U, end, [&] { return !ordinary(b, Us, zero); }, S);
+          } else if (__builtin_expect(ordinary(b, Us, EXACT ? abs(R) + abs(AV) : R), 1)) {
+            write(b, U, R, scale(b, kRecQ), U, c, std::false_type{}, AV, col0 + 16 * ct);
+            if (sync) lds_barrier();
+            advance(b, U, end, [] { return false; }, S);
+          } else {
+            f32x4 sq = scale(b, kRecQ);
+            replace(R, sq, sum_fp32(b, b.qe, kRecQ, S));
+            write(b, U, R, sq, U, c, std::true_type{}, AV, col0 + 16 * ct);
+            if (sync) lds_barrier();
+            advance(b, U, end, [] { return true; }, S);
+          }
+        };
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) chunk(S[ct], ct, CT == 1 && w >= 4);
+        if (CT == 2 || w < 4) lds_barrier();
       }
       if (nc & 1) lds_barrier();
       if (PASS == 1) {
@@ -1549,10 +1997,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
   constexpr bool KEYS = MODE != kModeForget, DEC = MODE == kModeDeltaChannel, SCALED = DEC || (EXACT && !CH), TURN = MODE == kModeRetention;
   unsigned oq[4], ok[4], od[DEC ? 4 : 1], ot[TURN ? 4 : 1], ov[4];
   const int ow = w - waves, vc = VC * ((16 * ow + (lane & 15)) % (Buf::COLS / VC));   // (of fewer columns some twice)
-  const int vhead = two ? vc >> 6 : 0, vcol = DELTA || two ? cb * kWalkCols + (vc & 63) : 16 * waves * cb + vc;
+  const int vhead = two ? vc >> 6 : 0, vcol = DELTA || two ? cb * kWalkCols + (vc & 63) : 16 * tiles * cb + vc;
   const int at_mat = 256 / OW * ow + lane % (256 / OW), at_scale = 64 / OW * ow + lane % (64 / OW);
   const unsigned mat_off = at_mat * sizeof(float), scale_off = (kRecQ + at_scale) * sizeof(float);
-  const int at_row = (c0 & ~31) | (c0 & 12) << 1 | (c0 & 16) >> 2 | (c0 & 3);   // 32 s + 16 t + 4 g + i: 32 s + 8 g + 4 t + i
   const int cl = min(c0, a.dk - CPW), nf = TURN ? a.n_freq : 0;
   const int fq = c0 < nf ? c0 : c0 < 2 * nf ? c0 - nf : 0, partner = (c0 < nf ? c0 + nf : fq) - cl;
   auto offsets = [&](int nt) {
@@ -1682,6 +2129,17 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     }
     const f32x4 kts = in.kt;
     load(in, c + AHEAD);
+    // numbers that have no parts, or may get beyond (decays are at most 1, the keys' scales make them so)
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < CPW; ++j) {
+        if (PASS != 1) sum += fabsf(q[i][j]);
+        sum += fabsf(k[i][j]);
+        if (CH && MODE != kModeForget) sum += d[i][j];   // (the forget gate's key holds it)
+      }
+    const bool odd = __any(!(sum <= 0.5f * kSplitMax));
     float f[CPW], behind[CPW];   // products of the decays of the lane groups before / behind this one
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
@@ -1693,53 +2151,93 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         behind[j] = (tg & 1 ? 1.f : near.upper) * (tg & 2 ? 1.f : far.upper);
       }
     }
-    auto put = [&](__bf16 (&rows)[3][16][DK + 8], const float (&x)[4][CPW]) {
+    // per channel of the lane: P_i q_i, P_i k_i and D_end,j k_j of its four tokens
+    constexpr int KE = PASS != 1 ? CPW : 0, KT = KE + (DELTA ? CPW : 0), N = KT + CPW;
+    f32x4 x[N];   // (with a product, first the one factor, then what part 0 leaves)
+    unsigned p[N][3][2];
+    auto factor = [&](int j) {   // of the rows
+      f32x4 y;
 #pragma unroll
-      for (int i = 0; i < 4; i += 3 - CPW) {
-        unsigned p[3];
-        if constexpr (CPW == 2) split(x[i][0], x[i][1], p[0], p[1], p[2]);
-        else split(x[i][0], x[i + 1][0], p[0], p[1], p[2]);
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-          if constexpr (CPW == 2) {
-            *reinterpret_cast<unsigned*>(&rows[e][4 * tg + i][at_row]) = p[e];
-          } else {
-            *reinterpret_cast<unsigned short*>(&rows[e][4 * tg + i][at_row]) = static_cast<unsigned short>(p[e]);
-            *reinterpret_cast<unsigned short*>(&rows[e][4 * tg + i + 1][at_row]) = static_cast<unsigned short>(p[e] >> 16);
-          }
-        }
+      for (int i = 0; i < 4; ++i) {
+        f[j] *= d[i][j];
+        y[i] = f[j];
       }
+      return y;
     };
-    float x[4][CPW], y[4][CPW];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) {
-        if (CH) f[j] *= d[i][j];
-        x[i][j] = CH ? q[i][j] * f[j] : q[i][j];
-        y[i][j] = CH ? k[i][j] * f[j] : k[i][j];
-      }
-    if constexpr (PASS != 1) put(b.qe, x);
-    if constexpr (DELTA) put(*reinterpret_cast<__bf16 (*)[3][16][DK + 8]>(&b.ke), y);
+    auto tokens = [](const float (&z)[4][CPW], int j) { return f32x4{z[0][j], z[1][j], z[2][j], z[3][j]}; };
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
-      if (CH && tg == 3) b.end[CH ? c0 + j : 0] = f[j];   // the whole chunk
-      if (PASS == 1) over[j] *= c < nc ? f[j] : 1.f;   // (a chunk for nobody has the last one's)
-      float x[4], e = behind[j];
-#pragma unroll
-      for (int i = 3; i >= 0; --i) {
-        x[i] = CH ? k[i][j] * (DELTA ? e * kts[i] : e) : SCALED ? k[i][j] * kts[i] : k[i][j];
-        if (CH) e *= d[i][j];
-      }
-      unsigned p[3][2];
-      split(x[0], x[1], p[0][0], p[1][0], p[2][0]);
-      split(x[2], x[3], p[0][1], p[1][1], p[2][1]);
-      if constexpr (EXACT) {
-        b.kt01[tg][c0 + j] = u32x4{p[0][0], p[0][1], 0, 0};
-        b.kt20[tg][c0 + j] = u32x4{p[2][0], p[2][1], p[1][0], p[1][1]};
+      if constexpr (CH) {
+        const f32x4 by = factor(j);
+        if (PASS != 1) x[j % N] = split_product(tokens(q, j), by, p[j % N][0]);
+        if (DELTA) x[(KE + j) % N] = split_product(tokens(k, j), by, p[(KE + j) % N][0]);
+        if (tg == 3) b.end[CH ? c0 + j : 0] = f[j];   // the whole chunk
       } else {
-        b.kt01[tg][c0 + j] = u32x4{p[0][0], p[0][1], p[1][0], p[1][1]};
-        b.kt20[tg][c0 + j] = u32x4{p[2][0], p[2][1], p[0][0], p[0][1]};
+        if (PASS != 1) x[j % N] = tokens(q, j);
+        if (DELTA) x[(KE + j) % N] = tokens(k, j);
+      }
+      if (PASS == 1) over[j] *= c < nc ? f[j] : 1.f;   // (a chunk for nobody has the last one's)
+      if constexpr (CH || SCALED) {
+        f32x4 by = kts;
+        float e = behind[j];
+        if (CH)
+#pragma unroll
+          for (int i = 3; i >= 0; --i) {
+            by[i] = DELTA ? e * kts[i] : e;
+            e *= d[i][j];
+          }
+        x[KT + j] = split_product(tokens(k, j), by, p[KT + j][0]);
+      } else {
+        x[KT + j] = tokens(k, j);
+      }
+    }
+    const auto from = [](int g) { return CH || (SCALED && g >= KT) ? 1 : 0; };   // the first part that is not there
+    if (__builtin_expect(odd, 0)) {
+#pragma unroll
+      for (int g = 0; g < N; ++g)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          float lo = x[g][2 * e], hi = x[g][2 * e + 1];
+#pragma unroll
+          for (int i = from(g); i < 3; ++i) {
+            p[g][i][e] = pack_bf16(lo, hi);
+            lo -= bf16_low(p[g][i][e]);
+            hi -= bf16_high(p[g][i][e]);
+          }
+        }
+    } else {   // all side by side: a product's result is there after the others' instructions
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int g = 0; g < N; ++g)
+          if (i >= from(g)) {
+            p[g][i][0] = pack_bf16(x[g][0], x[g][1]);
+            p[g][i][1] = pack_bf16(x[g][2], x[g][3]);
+            if (i < 2) x[g] = id.rest(x[g], p[g][i][0], p[g][i][1]);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    auto put = [&](u32x2 (&rows)[3][4][DK + 16], int g) {
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        if constexpr (CPW == 2)
+          *reinterpret_cast<u32x4*>(&rows[e][tg][c0]) = u32x4{p[g][e][0], p[g][e][1], p[(g + 1) % N][e][0], p[(g + 1) % N][e][1]};
+        else
+          rows[e][tg][c0] = u32x2{p[g][e][0], p[g][e][1]};
+      }
+    };
+    if constexpr (PASS != 1) put(b.qe, 0);
+    if constexpr (DELTA) put(b.ke, KE % N);
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) {
+      const unsigned (&y)[3][2] = p[KT + j];
+      if constexpr (EXACT) {
+        b.kt01[tg][c0 + j] = u32x2{y[0][0], y[0][1]};
+        b.kt20[tg][c0 + j] = u32x4{y[2][0], y[2][1], y[1][0], y[1][1]};
+      } else {
+        b.kt01[tg][c0 + j] = u32x4{y[0][0], y[0][1], y[1][0], y[1][1]};
+        b.kt20[tg][c0 + j] = u32x4{y[2][0], y[2][1], y[0][0], y[0][1]};
       }
     }
     lds_barrier();
@@ -1760,32 +2258,32 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     for (int j = 0; j < CPW; ++j) seg_decay(sg.j, h0)[c0 + j] = over[j];
 }
 
-template <typename T, int MODE, int DK, int VEC>
-__global__ void __launch_bounds__(kWalkThreads, 3)
+template <typename T, int MODE, int DK, int VEC, int CT>
+__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
 scan_walk_kernel(ChunkArgs a, int portion0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>()> lds;
   const Segment sg{find_portion(a, portion0 + static_cast<int>(blockIdx.y)), 0, 1, 0, 0};
-  if (sg.s >= 0) walk<T, MODE, DK, VEC, 0>(a, sg, lds);
+  if (sg.s >= 0) walk<T, MODE, DK, VEC, 0, CT>(a, sg, lds);
 }
 
 // segment0 + blockIdx.y = segment of the batch.  First kernel: pass 1, and the portions that are not cut.
-template <typename T, int MODE, int DK, int VEC>
-__global__ void __launch_bounds__(kWalkThreads, 3)
+template <typename T, int MODE, int DK, int VEC, int CT>
+__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
 scan_segments_kernel(ChunkArgs a, int segment0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>()> lds;
   const Segment sg = find_segment<false>(a, segment0 + blockIdx.y);
   if (sg.s < 0) return;
   if (sg.P == 1)
-    walk<T, MODE, DK, VEC, 0>(a, sg, lds);
+    walk<T, MODE, DK, VEC, 0, CT>(a, sg, lds);
   else if (sg.j < sg.P - 1 && sg.state + sg.P <= a.seg_states)   // (the bound holds: scan_segments)
-    walk<T, MODE, DK, VEC, 1>(a, sg, lds);
+    walk<T, MODE, DK, VEC, 1, CT>(a, sg, lds);
 }
-template <typename T, int MODE, int DK, int VEC>
-__global__ void __launch_bounds__(kWalkThreads, 3)
+template <typename T, int MODE, int DK, int VEC, int CT>
+__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
 scan_segments_end_kernel(ChunkArgs a, int segment0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>()> lds;
   const Segment sg = find_segment<true>(a, segment0 + blockIdx.y);
-  if (sg.s >= 0 && sg.state + sg.P <= a.seg_states) walk<T, MODE, DK, VEC, 2>(a, sg, lds);
+  if (sg.s >= 0 && sg.state + sg.P <= a.seg_states) walk<T, MODE, DK, VEC, 2, CT>(a, sg, lds);
 }
 
 template <typename T, int MODE, int DK, int VEC>
@@ -1807,22 +2305,28 @@ int launch(const ChunkArgs& a, hipStream_t st) {
   b.walk_heads = shape.heads;
   b.walk_portions = static_cast<int>(std::min<int64_t>(a.S, a.T / a.min_rows));
   const unsigned gx = a.H / shape.heads * ((a.dv + shape.cols - 1) / shape.cols);
-  const dim3 block(kWave * (shape.waves + operand_waves(MODE, DK)));
-  if constexpr (MODE < kModeDelta) {
-    if (a.seg_states > 0) {
-      // at most a segment per portion, and those of the cut ones
-      scan_grids(gx, static_cast<int64_t>(b.walk_portions) + a.seg_states, [&](dim3 grid, int first) {
-        hipLaunchKernelGGL((scan_segments_kernel<T, MODE, DK, VEC>), grid, block, 0, st, b, first);
-      });
-      scan_grids(gx, a.seg_states, [&](dim3 grid, int first) {
-        hipLaunchKernelGGL((scan_segments_end_kernel<T, MODE, DK, VEC>), grid, block, 0, st, b, first);
-      });
-      return static_cast<int>(hipGetLastError());
+  auto walk = [&](auto tiles) {
+    constexpr int CT = decltype(tiles)::value;
+    const dim3 block(kWave * (shape.waves / CT + operand_waves(MODE, DK)));
+    if constexpr (MODE < kModeDelta) {
+      if (a.seg_states > 0) {
+        // at most a segment per portion, and those of the cut ones
+        scan_grids(gx, static_cast<int64_t>(b.walk_portions) + a.seg_states, [&](dim3 grid, int first) {
+          hipLaunchKernelGGL((scan_segments_kernel<T, MODE, DK, VEC, CT>), grid, block, 0, st, b, first);
+        });
+        scan_grids(gx, a.seg_states, [&](dim3 grid, int first) {
+          hipLaunchKernelGGL((scan_segments_end_kernel<T, MODE, DK, VEC, CT>), grid, block, 0, st, b, first);
+        });
+        return;
+      }
     }
-  }
-  scan_grids(gx, b.walk_portions, [&](dim3 grid, int first) {
-    hipLaunchKernelGGL((scan_walk_kernel<T, MODE, DK, VEC>), grid, block, 0, st, b, first);
-  });
+    scan_grids(gx, b.walk_portions, [&](dim3 grid, int first) {
+      hipLaunchKernelGGL((scan_walk_kernel<T, MODE, DK, VEC, CT>), grid, block, 0, st, b, first);
+    });
+  };
+  constexpr bool WIDE = MODE < kModeDelta && VEC == 2;
+  if (WIDE && shape.waves == 8) walk(std::integral_constant<int, WIDE ? 2 : 1>{});
+  else walk(std::integral_constant<int, 1>{});
   return static_cast<int>(hipGetLastError());
 }
 
