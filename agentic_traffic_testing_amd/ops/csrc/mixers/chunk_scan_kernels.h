@@ -14,7 +14,7 @@
 // to the middle); h = 8, 4, 2, 1 covers all pairs j < i.  (16-bit inputs: h = 8 and 4, and the pairs inside four tokens as
 // sums on the vector units.)
 //
-// * scores kernel: one wave per (chunk, head) prepares what does not need the state - A, T and the
+// * scores kernel: a wave or two (score_pairs) per (chunk, head) prepare what does not need the state - A, T and the
 //   per-token scales - into a record in scratch.  All chunks at once, off the serial chain.
 // * walk kernel: a workgroup walks the chunks of one (sequence, head), or of two heads with the same keys, for 64 or 128
 //   value columns (walk_shape).  Four waves hold 16 or 32 columns of S each (eight 16, by rows at any address), in accumulators: the accumulator tiles of
@@ -39,8 +39,8 @@
 // Measured: the token-by-token kernels, fp32 products with 64 columns per workgroup, bf16 parts, and with the scores' halves of
 // channels, pairs inside four tokens and values in one part where they are exact (us, scores + walk; 32 heads of 128, bf16
 // unless noted):
-//   delta rule, per-channel decay, 4 x ~1850 tokens: 1798, 130 + 343, 132 + 262, 99 + 256, today 99 + 222
-//   forget gate, 16 x ~460 tokens:                    777, 111 + 308, 98 + 168, 83 + 158, today 83 + 129
+//   delta rule, per-channel decay, 4 x ~1850 tokens: 1798, 130 + 343, 132 + 262, 99 + 256, today 83 + 224
+//   forget gate, 16 x ~460 tokens:                    777, 111 + 308, 98 + 168, 83 + 158, today 71 + 129
 //   state space, 96 heads of 128 x 64, 1023 tokens, fp32: 250, 21 + 94, 22 + 64, 19 + 63 in five segments of head pairs
 //   retention, one portion of 1500 tokens (+ 11 rows): 260, 21 + 88, 22 + 69, 21 + 65 in eight segments, the rows inside the
 //   scores launch
@@ -403,13 +403,39 @@ __device__ __forceinline__ void queries_keys(const Raw<T, MODE, CPL>& r, const C
     }
 }
 
+// y += a[j] of lane LANE of each 16, times x[j], for N of them.  (The broadcast operand wants two idle cycles behind its last
+// write, which the compiler does not see here; from the builtin it makes a move and a multiply-add.)
+#define MIXK_TERM(A, X) "v_fmac_f32_dpp %0, " A ", " X " row_newbcast:%1 row_mask:0xf bank_mask:0xf\n\t"
+template <int LANE, int N>
+__device__ __forceinline__ void add_broadcast(float& y, const float* a, const float* x) {
+  if constexpr (N == 1)
+    asm("s_nop 1\n\t" MIXK_TERM("%2", "%3") : "+&v"(y) : "n"(LANE), "v"(a[0]), "v"(x[0]));
+  if constexpr (N == 2)
+    asm("s_nop 1\n\t" MIXK_TERM("%2", "%3") MIXK_TERM("%4", "%5")
+        : "+&v"(y) : "n"(LANE), "v"(a[0]), "v"(x[0]), "v"(a[1]), "v"(x[1]));
+  if constexpr (N == 3)
+    asm("s_nop 1\n\t" MIXK_TERM("%2", "%3") MIXK_TERM("%4", "%5") MIXK_TERM("%6", "%7")
+        : "+&v"(y) : "n"(LANE), "v"(a[0]), "v"(x[0]), "v"(a[1]), "v"(x[1]), "v"(a[2]), "v"(x[2]));
+  if constexpr (N == 4)
+    asm("s_nop 1\n\t" MIXK_TERM("%2", "%3") MIXK_TERM("%4", "%5") MIXK_TERM("%6", "%7") MIXK_TERM("%8", "%9")
+        : "+&v"(y) : "n"(LANE), "v"(a[0]), "v"(x[0]), "v"(a[1]), "v"(x[1]), "v"(a[2]), "v"(x[2]), "v"(a[3]), "v"(x[3]));
+}
+#undef MIXK_TERM
+
 // ---- scores -------------------------------------------------------------------------------------------
 constexpr int kScoreWaves = 4;
+// Per-channel decays of 16-bit inputs: two waves per chunk, half of its channels each; the sums come together at the end.  (A
+// lane with eight channels of q, k and the decays takes 195 - 209 registers, two waves per SIMD; with four, three and four.
+// Scores, us, one wave / two / two and T from broadcast operands: delta rule, 4 x 1.9k tokens 99 / 97 / 83 - vector units
+// busy 54 / - / 80 % -, forget gate, 16 x 460 84 / 71; with no more than 128 registers for the delta rule 111, spilled.)
+template <typename T, int MODE, int DK>
+constexpr bool score_pairs() { return per_channel<MODE>() && sizeof(T) == 2 && DK == 128; }
 
 template <typename T, int MODE, int DK, bool VEC>
-__global__ void __launch_bounds__(64 * kScoreWaves, 2)
+__global__ void __launch_bounds__(64 * kScoreWaves, (score_pairs<T, MODE, DK>() ? (MODE == kModeForget ? 4 : 3) : 2))
 scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
-  constexpr int CPL = DK / 16, kDecay = scan_rec_decay(MODE);
+  constexpr bool PAIRS = score_pairs<T, MODE, DK>();
+  constexpr int CPL = DK / 16 / (PAIRS ? 2 : 1), kDecay = scan_rec_decay(MODE);
   // (the kernels for any alignment take keys of all widths)
   const int REC = scan_record_floats(MODE, VEC ? DK : a.dk), DS = scan_decay_width(VEC ? DK : a.dk);
   constexpr bool DELTA = MODE >= kModeDelta, CH = per_channel<MODE>();
@@ -421,11 +447,12 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
   // Operand rows hold half of the channels at a time, in half the LDS, and what is worked out for them is not kept: more waves
   // per CU (rows of 128 channels, 62 and 79 KB per workgroup, let eight onto it).  us: delta rule per channel, 4 x 1.9k
   // tokens, 111 -> 101; forget gate, 16 x 460, 94 -> 85; state space in 32 bits, 1023, 21.1 -> 18.7; retention 21.1 -> 20.9.
-  constexpr int HALVES = DK == 128 && !EXACT ? 2 : 1, WIDE = DK / HALVES, CH_HALF = CPL / HALVES;
+  constexpr int HALVES = DK == 128 && !EXACT && !PAIRS ? 2 : 1, WIDE = DK / HALVES / (PAIRS ? 2 : 1), CH_HALF = CPL / HALVES;
   struct Lds {
     float row[ROWS][WIDE + 4];      // operand rows of the products
     float sq[16][20], sk[DELTA ? 16 : 1][20];   // A; L
     float sc[4][16];                // scale of q, of k, beta, scalar decay
+    float sum[PAIRS ? 3 : 1][16];   // of half of the channels: q . q, k . k, q . k
   };
   constexpr size_t LDS_BYTES = sizeof(Lds) * kScoreWaves > sizeof(ss::StepLds<MODE, DK / 16>)
                                    ? sizeof(Lds) * kScoreWaves : sizeof(ss::StepLds<MODE, DK / 16>);
@@ -442,10 +469,11 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
   Lds* lds_all = reinterpret_cast<Lds*>(lds_raw);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   Lds& s = lds_all[w];
-  const int64_t item = static_cast<int64_t>(blockIdx.x - step_blocks) * kScoreWaves + w;
-  // the wave's chunk and head; waves without one stay for nothing (there is no workgroup barrier)
+  // the wave's chunk and head, and with two waves its first channel; waves without a chunk stay for nothing but the pairs'
+  // barrier
+  const int64_t item = (static_cast<int64_t>(blockIdx.x - step_blocks) * kScoreWaves + w) / (PAIRS ? 2 : 1);
+  const int ch0 = PAIRS ? DK / 2 * (w & 1) : 0;
   const int slot = static_cast<int>(item / a.H), h = static_cast<int>(item % a.H);
-  if (slot >= a.n_slots) return;
   int lo = 0, hi = a.S - 1;   // last sequence whose first slot is at or below `slot`
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -453,7 +481,11 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
   }
   const int first = a.seq_qstart[lo], n = a.seq_qstart[lo + 1] - first;
   const int t0 = (slot - first / kScanChunk - lo) * kScanChunk;
-  if (n < a.min_rows || t0 >= n || a.seq_slot[lo] < 0) return;
+  const bool none = slot >= a.n_slots || n < a.min_rows || t0 >= n || a.seq_slot[lo] < 0;
+  if (none) {
+    if (PAIRS) lds_barrier();
+    return;
+  }
   const int nt = min(kScanChunk, n - t0);
   const int g = MODE == kModeForget ? h : h / (a.H / a.G);
   const int64_t row0 = first + t0;
@@ -499,15 +531,15 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
     }
   } else {
     Raw<T, MODE, CPL> r;
-    load_raw<VEC, T, MODE, CPL>(r, a, h, g, row0, nt, lane, m * CPL);
+    load_raw<VEC, T, MODE, CPL>(r, a, h, g, row0, nt, lane, ch0 + m * CPL);
     float b0[CPL], b1[CPL];
-    if constexpr (CH) decay_params<MODE, CPL>(a, h, m * CPL, b0, b1);
+    if constexpr (CH) decay_params<MODE, CPL>(a, h, ch0 + m * CPL, b0, b1);
     if (VEC && CH && nt == kScanChunk && a.dk == DK) {   // (uniform)
-      if constexpr (CH) decays<true, T, MODE, CPL>(r, a, nt, lane, m * CPL, b0, b1, d);
-      queries_keys<true, VEC, T, MODE, CPL>(r, a, g, row0, nt, lane, m * CPL, d, q, k);
+      if constexpr (CH) decays<true, T, MODE, CPL>(r, a, nt, lane, ch0 + m * CPL, b0, b1, d);
+      queries_keys<true, VEC, T, MODE, CPL>(r, a, g, row0, nt, lane, ch0 + m * CPL, d, q, k);
     } else {
-      if constexpr (CH) decays<false, T, MODE, CPL>(r, a, nt, lane, m * CPL, b0, b1, d);
-      queries_keys<false, VEC, T, MODE, CPL>(r, a, g, row0, nt, lane, m * CPL, d, q, k);
+      if constexpr (CH) decays<false, T, MODE, CPL>(r, a, nt, lane, ch0 + m * CPL, b0, b1, d);
+      queries_keys<false, VEC, T, MODE, CPL>(r, a, g, row0, nt, lane, ch0 + m * CPL, d, q, k);
     }
     if constexpr (!CH) {
       float sum = 0.f;
@@ -522,8 +554,8 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < CPL; j += 4)
-          if (VEC || m * CPL < DS)
-            *reinterpret_cast<f32x4*>(rec + kDecay + (4 * gr + i) * DS + m * CPL + j) =
+          if (VEC || ch0 + m * CPL < DS)
+            *reinterpret_cast<f32x4*>(rec + kDecay + (4 * gr + i) * DS + ch0 + m * CPL + j) =
                 f32x4{d[i][j], d[i][j + 1], d[i][j + 2], d[i][j + 3]};
   }
   // per-token numbers of token m: beta, scalar decay and its products, dt, inverse norms
@@ -567,19 +599,23 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
         kk = group_sum<16>(kk);
       }
       if (CH) qk = group_sum<16>(qk);
-      if (m == 0) {
+      if (PAIRS && m == 0) {
+        s.sum[0][4 * gr + i] = qq;
+        s.sum[PAIRS ? 1 : 0][4 * gr + i] = kk;
+        s.sum[PAIRS ? 2 : 0][4 * gr + i] = qk;
+      } else if (m == 0) {
         s.sc[0][4 * gr + i] = qq;
         s.sc[1][4 * gr + i] = kk;
         s.sc[3][4 * gr + i] = qk;
       }
     }
     wave_sync();
-    if (DELTA) {
+    if (DELTA && !PAIRS) {
       qi = 1.0f / (sqrtf(static_cast<float>(a.dk)) * sqrtf(s.sc[0][m] + 1e-6f));
       ki = 1.0f / sqrtf(s.sc[1][m] + 1e-6f);
     }
   }
-  const float diag = CH ? s.sc[3][m] : 0.f;
+  const float diag = CH && !PAIRS ? s.sc[3][m] : 0.f;
   // prefix and suffix products of the scalar decay, by every lane of the token (a fixed decay's powers come
   // from the table, rounded once: a slow head remembers thousands of tokens)
   const float* pw = MODE == kModeRetention ? a.p0 + h * kPowers : nullptr;
@@ -603,7 +639,7 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
     end = __shfl(pre, lane | 15, kWave);
   }
   wave_sync();
-  if (lane < 16) {
+  if (!PAIRS && lane < 16) {
     rec[kRecQ + lane] = qi * pre;
     rec[kRecK + lane] = ki * pre;
     rec[kRecKt + lane] = ki * dt * suf;
@@ -630,7 +666,7 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
   // (`rows` puts down a half's rows; with `self` also rows rb .. times themselves, into `own`)
   typedef std::conditional_t<sizeof(T) == 4, f64x4, f32x4> sums;
   auto product = [&](auto rows, int ra, int rb, int nb, auto self, sums& own) __attribute__((always_inline)) {
-    constexpr int N = sizeof(T) == 4 ? 2 : 8;
+    constexpr int N = sizeof(T) == 4 ? 2 : PAIRS ? 4 : 8;
     sums x[N], y[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = y[i] = sums{0, 0, 0, 0};
@@ -653,8 +689,9 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
             x[i & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i], bv[i], x[i & 1], 0, 0, 0);
             if constexpr (self) y[i & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(sv[i], bv[i], y[i & 1], 0, 0, 0);
           } else {
-            x[4 * (t & 1) + i] = mma(av[i], bv[i], x[4 * (t & 1) + i]);
-            if constexpr (self) y[4 * (t & 1) + i] = mma(sv[i], bv[i], y[4 * (t & 1) + i]);
+            const int e = (4 * t + i) % N;
+            x[e] = mma(av[i], bv[i], x[e]);
+            if constexpr (self) y[e] = mma(sv[i], bv[i], y[e]);
           }
         }
       }
@@ -666,6 +703,7 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
     }
     auto total = [](const sums* z) {
       if constexpr (sizeof(T) == 4) return z[0] + z[1];
+      else if constexpr (N == 4) return (z[0] + z[1]) + (z[2] + z[3]);
       else return ((z[0] + z[1]) + (z[2] + z[3])) + ((z[4] + z[5]) + (z[6] + z[7]));
     };
     own = total(y);
@@ -724,7 +762,7 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
       if (DELTA) s.sk[ti][m] = 0.f;
     }
     wave_sync();
-    if (lane < 16) s.sq[lane][lane] = diag * s.sc[0][lane] * s.sc[1][lane];
+    if (!PAIRS && lane < 16) s.sq[lane][lane] = diag * s.sc[0][lane] * s.sc[1][lane];
     // local products of the lane's four tokens, for the channels of a half: from the first on, and behind a token to the last
     struct Local {
       float pf[4][CH_HALF], sf[4][CH_HALF];
@@ -760,8 +798,8 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
             constexpr int HS = decltype(half)::value;
             if (u / HS == v / HS) {
               const int ti = (u / HS) * 2 * HS + HS + u % HS, tj = (v / HS) * 2 * HS + v % HS;
-              if (!DELTA || gr < 2) s.sq[ti][tj] = DELTA ? x[i] * s.sc[0][ti] * s.sc[1][tj] : x[i];
-              else s.sk[ti][tj] = x[i] * s.sc[1][ti] * s.sc[1][tj] * s.sc[2][ti];
+              if (!DELTA || gr < 2) s.sq[ti][tj] = DELTA && !PAIRS ? x[i] * s.sc[0][ti] * s.sc[1][tj] : x[i];
+              else s.sk[ti][tj] = PAIRS ? x[i] : x[i] * s.sc[1][ti] * s.sc[1][tj] * s.sc[2][ti];
             }
           };
           if (DELTA || gr < 2) pair(std::integral_constant<int, HA>{});
@@ -843,7 +881,7 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
       for (int e = 1; e < N; ++e) y = m == e ? x[e] : y;
       const int e = m < 6 ? m : m - 6, j = e < 3 ? 0 : e < 5 ? 1 : 2, i = e < 3 ? e + 1 : e < 5 ? e - 1 : 3;
       const int ti = 4 * gr + i, tj = 4 * gr + j;
-      if (DELTA) y *= s.sc[m < 6 ? 0 : 1][ti] * s.sc[1][tj] * (m < 6 ? 1.f : s.sc[2][ti]);
+      if (DELTA && !PAIRS) y *= s.sc[m < 6 ? 0 : 1][ti] * s.sc[1][tj] * (m < 6 ? 1.f : s.sc[2][ti]);
       if (m < N) (m < 6 ? s.sq : s.sk)[ti][tj] = y;
     }
     if constexpr (!FOURS) {
@@ -878,33 +916,74 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
       }
     }
   }
-  wave_sync();
-  *reinterpret_cast<f32x4*>(rec + m * 16 + 4 * gr) = *reinterpret_cast<const f32x4*>(&s.sq[m][4 * gr]);
-  if constexpr (DELTA) {
-    // (I + L) T = diag(beta), one column per lane (lanes 16 - 63 repeat the columns)
-    float x[16];
-    const float bc = s.sc[2][m];
+  if constexpr (PAIRS) {
+    lds_barrier();
+    const Lds &s0 = lds_all[w & ~1], &s1 = lds_all[w | 1];
+    auto sum = [&](int e) { return s0.sum[PAIRS ? e : 0][m] + s1.sum[PAIRS ? e : 0][m]; };
+    const float qk = sum(2);
+    if (DELTA) {
+      qi = 1.0f / (sqrtf(static_cast<float>(a.dk)) * sqrtf(sum(0) + 1e-6f));
+      ki = 1.0f / sqrtf(sum(1) + 1e-6f);
+    }
+    if (lane < 16) s.sc[1][lane] = ki;
+    wave_sync();
+    const f32x4 kj = *reinterpret_cast<const f32x4*>(&s.sc[1][4 * gr]);   // of the columns 4 gr ...
+    auto both = [&](const float (&x)[20], const float (&y)[20]) {
+      return *reinterpret_cast<const f32x4*>(&x[4 * gr]) + *reinterpret_cast<const f32x4*>(&y[4 * gr]);
+    };
+    if ((w & 1) == 0) {   // A and the scales
+      f32x4 x = both(s0.sq[m], s1.sq[m]);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float v = i == m ? bc : 0.f;
-#pragma unroll
-      for (int j4 = 0; j4 < i; j4 += 4) {
-        const f32x4 L = *reinterpret_cast<const f32x4*>(&s.sk[i][j4]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (j4 + e < i) v -= L[e] * x[j4 + e];
+      for (int i = 0; i < 4; ++i) x[i] = (4 * gr + i == m ? qk : x[i]) * qi * kj[i];
+      *reinterpret_cast<f32x4*>(rec + m * 16 + 4 * gr) = x;
+      if (lane < 16) {
+        rec[kRecQ + lane] = qi;
+        rec[kRecK + lane] = ki;
+        rec[kRecKt + lane] = ki;
+        rec[kRecEnd + lane] = lane == kRecNoParts - kRecEnd ? 0.f : 1.f;
       }
-      x[i] = v;
+      return;
     }
-    wave_sync();
+    if constexpr (DELTA) {   // L
+      f32x4 x = both(s0.sk[m], s1.sk[m]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {   // transpose through LDS: lane group gr stores rows 4 gr .. of its column
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        if (gr == b) s.sq[4 * b + i][m] = x[4 * b + i];
+      for (int i = 0; i < 4; ++i) x[i] = 4 * gr + i < m ? x[i] * ki * kj[i] * beta : 0.f;
+      *reinterpret_cast<f32x4*>(&s.sk[m][4 * gr]) = x;
+      wave_sync();
+    } else {
+      return;
     }
+  } else {
     wave_sync();
-    *reinterpret_cast<f32x4*>(rec + kRecT + m * 16 + 4 * gr) = *reinterpret_cast<const f32x4*>(&s.sq[m][4 * gr]);
+    *reinterpret_cast<f32x4*>(rec + m * 16 + 4 * gr) = *reinterpret_cast<const f32x4*>(&s.sq[m][4 * gr]);
+  }
+  if constexpr (DELTA) {
+    // (I + L) T = diag(beta), one column per lane (lanes 16 - 63 repeat the columns).  Lane m of each 16 has row m of L, and
+    // L_ij comes from there as the multiply-add's own broadcast operand (read from LDS it is waited for, row by row).
+    float L[16], x[16];
+#pragma unroll
+    for (int j = 0; j < 16; j += 4) {
+      const f32x4 l = *reinterpret_cast<const f32x4*>(&s.sk[m][j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) L[j + e] = -l[e];
+    }
+    const float bc = PAIRS ? beta : s.sc[2][m];
+    auto row_of = [&](auto self, auto i_) __attribute__((always_inline)) -> void {
+      constexpr int i = decltype(i_)::value, last = i & ~3;
+      x[i] = i == m ? bc : 0.f;
+#pragma unroll
+      for (int j = 0; j < last; j += 4) add_broadcast<i, 4>(x[i], L + j, x + j);
+      add_broadcast<i, i - last>(x[i], L + last, x + last);
+      if constexpr (i < 15) self(self, std::integral_constant<int, i + 1>{});
+    };
+    row_of(row_of, std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {   // lane group gr stores rows 4 gr .. of its column
+      float v = x[i];
+#pragma unroll
+      for (int b = 1; b < 4; ++b) v = gr == b ? x[4 * b + i] : v;
+      rec[kRecT + (4 * gr + i) * 16 + m] = v;
+    }
   }
 }
 
@@ -2295,7 +2374,8 @@ int launch(const ChunkArgs& a, hipStream_t st) {
   const bool apart = cols * a.H * a.S >= 2048;
   if (apart)
     if (const int rc = launch_step_scan(a, MODE, a.min_rows - 1, sizeof(T) == 4 ? 2 : 0, st)) return rc;
-  const int64_t steps = apart ? 0 : cols * a.H * a.S, blocks = steps + (items + kScoreWaves - 1) / kScoreWaves;
+  const int64_t score_waves = items * (score_pairs<T, MODE, DK>() ? 2 : 1);
+  const int64_t steps = apart ? 0 : cols * a.H * a.S, blocks = steps + (score_waves + kScoreWaves - 1) / kScoreWaves;
   if (blocks > 0x7fffffff) return -1;
   hipLaunchKernelGGL((scan_scores_kernel<T, MODE, DK, (VEC > 0)>), dim3(static_cast<unsigned>(blocks)),
                      dim3(64 * kScoreWaves), 0, st, a, static_cast<int>(steps), static_cast<int>(cols * a.H),
