@@ -103,6 +103,29 @@ def test_rope_cache(dtype, hq, hkv, T):
     close(v2, v1, 0.0)
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("hq,hkv", [(1, 1), (4, 2), (6, 2), (5, 1), (16, 2)])
+@pytest.mark.parametrize("T,bs,pad", [(16, 16, 0), (17, 16, 8), (31, 8, 16), (48, 32, 4)])
+def test_rope_cache_groups(dtype, hq, hkv, T, bs, pad):
+    """Tiles of 16 tokens, whole and not, by the size of a KV head's group (5: the kernel for any), rows inside wider ones (4
+    more: not aligned, the same), pages that a tile fills, enters midway and leaves."""
+    torch.manual_seed(T)
+    D, nb = 128, 128 // bs + 2
+    qkv = torch.randn(T, (hq + 2 * hkv) * D + pad, dtype=dtype, device="cuda")[:, :(hq + 2 * hkv) * D]
+    pos = torch.randint(0, 4000, (T,), dtype=torch.int32, device="cuda")
+    slots = torch.arange(T, dtype=torch.int32, device="cuda") + 3
+    slots[[0, T - 2]] = -1
+    cs = ref.rope_cos_sin(D, 8192, 500000.0, None, device="cuda")
+    k1, v1 = _rand_cache(nb, hkv, bs, D, dtype)
+    k2, v2 = k1.clone(), v1.clone()
+    q_exp = ref.rope_cache(qkv, pos, slots, cs, k1, v1, hq, hkv, D)
+    q_got = ops.rope_cache(qkv, pos, slots, cs, k2, v2, hq, hkv, D)
+    # a rotated number in 32 bits, rounded once: half a unit in its last place beside the reference's rounding
+    close(q_got, q_exp, 2e-2, 1e-2)
+    close(k2, k1, 2e-2, 1e-2)
+    close(v2, v1, 0.0)
+
+
 def _make_paged(seqs, hkv, bs, dtype, nb_extra=8, seed=0):
     """seqs: list of (kvlen, qlen). Returns caches, block tables, metadata on cuda."""
     g = torch.Generator().manual_seed(seed)
