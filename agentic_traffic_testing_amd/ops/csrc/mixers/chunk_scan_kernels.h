@@ -1125,30 +1125,39 @@ struct ChunkDecay {
 template <typename T, int MODE>
 constexpr bool exact_values() { return sizeof(T) == 2 && (MODE == kModeForget || MODE == kModeRetention); }
 
+// Queries and keys are exact in one part where they go into the products as they came, in 16 bits: their scales and the one
+// number of the decay come afterwards.  A sum over S's rows then takes three products in place of six, and kt U, as kt is the
+// keys, two per tile; no part is worked out, and a third of the operands goes through LDS.  Walk, us, three parts / one:
+// delta rule, 32 heads of 128, 4 x 1.9k tokens 206 / 156, state space, 128 heads of 128 x 64 43.5 + 82 / 32.5 + 67 (states
+// 7 % closer to 64 bits).
+template <typename T, int MODE>
+constexpr bool exact_rows() { return sizeof(T) == 2 && (MODE == kModeStateSpace || MODE == kModeDelta); }
+
 // A chunk's operands.
-template <int MODE, int DK, bool EXACT>
+template <int MODE, int DK, bool EXACT, bool ONE>
 struct WalkBuf {
   static constexpr bool DELTA = MODE >= kModeDelta, CH = per_channel<MODE>();
   static constexpr int COLS = DELTA ? kWalkCols : 2 * kWalkCols, HEADS = MODE == kModeStateSpace ? 2 : 1;
   // rows in three parts, per four tokens and channel as the lane that prepares them holds them; the reads transpose
-  typedef u32x2 Rows[3][4][DK + 16];
+  typedef u32x2 Rows[ONE ? 1 : 3][4][DK + 16];
   Rows qe;                              // P_i q_i; one number as the decay: q_i
-  u32x2 ke[DELTA ? 3 : 1][DELTA ? 4 : 1][DK + 16];   // P_i k_i; k_i
+  u32x2 ke[DELTA && !ONE ? 3 : 1][DELTA ? 4 : 1][DK + 16];   // P_i k_i; k_i
   // D_end,j k_j; not EXACT and one number as the decay: k_j.  Per four tokens and channel two parts of each
-  std::conditional_t<EXACT, u32x2, u32x4> kt01[4][DK];   // parts 0 and 1; EXACT: 0
-  u32x4 kt20[4][DK];                    // ... 2 and 0; EXACT: 2 and 1
+  // parts 0 and 1; EXACT: 0; ONE: the number, which a delta rule has in ke
+  std::conditional_t<EXACT || ONE, u32x2, u32x4> kt01[DELTA && ONE ? 1 : 4][DK];
+  u32x4 kt20[ONE ? 1 : 4][DK];          // ... 2 and 0; EXACT: 2 and 1
   __bf16 amat[EXACT ? 2 : 1][16][4][8]; // EXACT: A per row and four tokens: part 0, and zeros; parts 2 and 1
   f32x4 v[4][COLS];                     // per four tokens and column
   float mat[HEADS][DELTA ? 512 : 256];  // of the record: A, and T
   float scale[HEADS][64];               // ... kRecQ, kRecK, kRecKt, kRecEnd
   float end[CH ? DK : 4];               // P_end
 };
-template <int MODE, int DK, bool EXACT>
+template <int MODE, int DK, bool EXACT, bool ONE>
 struct WalkLds {
   static constexpr bool DELTA = MODE >= kModeDelta;
   static constexpr int BUFS = DELTA ? 2 : 3;
   union {
-    WalkBuf<MODE, DK, EXACT> buf[BUFS];
+    WalkBuf<MODE, DK, EXACT, ONE> buf[BUFS];
     float start[DELTA ? 1 : DK][2 * kWalkCols + 4];   // the state at a segment's start
   };
 };
@@ -1161,7 +1170,7 @@ struct WalkLds {
 // zero to what they add to the state, with the decay over them.  Pass 2 puts the state at a segment's start together
 // from these and walks it; the last segment writes the sequence's state.
 template <typename T, int MODE, int DK, int VEC, int PASS, int CT>
-__device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkLds<MODE, DK, exact_values<T, MODE>()>& lds) {
+__device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()>& lds) {
   constexpr int NT = DK / 16, kDecay = scan_rec_decay(MODE);
   const int REC = scan_record_floats(MODE, VEC ? DK : a.dk), DS = scan_decay_width(VEC ? DK : a.dk);   // (scan_scores_kernel)
   constexpr bool DELTA = MODE >= kModeDelta, CH = per_channel<MODE>();
@@ -1170,8 +1179,10 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
   // (token by token 0.78), with both at 0.74.  The others do not need it (state space: 6 us of 67).
   constexpr bool F64 = sizeof(T) == 4 && MODE == kModeForget;
   constexpr bool EXACT = exact_values<T, MODE>();
-  using Buf = WalkBuf<MODE, DK, EXACT>;
-  constexpr int BUFS = WalkLds<MODE, DK, EXACT>::BUFS, OW = operand_waves(MODE, DK);
+  constexpr bool ONE = exact_rows<T, MODE>();
+  constexpr int RP = ONE ? 1 : 3;   // parts of the rows
+  using Buf = WalkBuf<MODE, DK, EXACT, ONE>;
+  constexpr int BUFS = WalkLds<MODE, DK, EXACT, ONE>::BUFS, OW = operand_waves(MODE, DK);
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const Identity id(lane);
@@ -1338,16 +1349,19 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       const u32x2 lo = get(0), hi = get(1);
       return u32x4{lo[0], lo[1], hi[0], hi[1]};
     };
+    // product i of six of rows r and a state's parts q (ONE: of three)
+    auto product = [&](Sum& x, const u32x4 (&r)[3], const u32x4 (&q)[3], int i) {
+      constexpr int kRow[] = {0, 2, 0, 1, 1, 0}, kState[] = {2, 0, 0, 1, 0, 1}, kSum[] = {0, 1, 2, 0, 1, 0};
+      if (kRow[i] >= RP) return;
+      f32x4& to = kSum[i] == 2 ? x.big : x.small[kSum[i] % 2];
+      to = mma(r[kRow[i]], q[kState[i]], to);
+    };
     auto add = [&](Sum& x, const typename Buf::Rows& rows, const u32x4 (&p)[3], int s) {
       u32x4 r[3];
 #pragma unroll
-      for (int e = 0; e < 3; ++e) r[e] = row(rows[e], s);
-      x.small[0] = mma(r[0], p[2], x.small[0]);
-      x.small[1] = mma(r[2], p[0], x.small[1]);
-      x.big = mma(r[0], p[0], x.big);
-      x.small[0] = mma(r[1], p[1], x.small[0]);
-      x.small[1] = mma(r[1], p[0], x.small[1]);
-      x.small[0] = mma(r[0], p[1], x.small[0]);
+      for (int e = 0; e < RP; ++e) r[e] = row(rows[e], s);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) product(x, r, p, i);
     };
     auto total = [](const Sum& x) {
       f32x4 y = x.big + (x.small[0] + x.small[1]);
@@ -1366,9 +1380,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           __builtin_amdgcn_sched_barrier(0);
           unsigned r[3];
 #pragma unroll
-          for (int e = 0; e < 3; ++e)
+          for (int e = 0; e < RP; ++e)
             r[e] = reinterpret_cast<const unsigned short*>(&rows[e][m >> 2][16 * t + 4 * gr + i])[m & 3];
-          x = mma(join(r[0], r[1], r[2], false) * sc, S[t][i], x);
+          x = mma((ONE ? bf16_low(r[0]) : join(r[0], r[ONE ? 0 : 1], r[ONE ? 0 : 2], false)) * sc, S[t][i], x);
         }
       return x;
     };
@@ -1391,7 +1405,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       u32x4 p0, p10, p1, p02;
     };
     // EXACT: the number itself, beside part 0, or the parts 2 and 1, of the keys and of A.
+    // ONE: parts 2 and 1, of products with the keys twice.
     auto as_parts = [](const unsigned (&u)[3][2]) {
+      if constexpr (ONE) return Parts{u32x4{u[0][0], u[0][1], 0, 0}, u32x4{}, u32x4{}, u32x4{u[2][0], u[2][1], u[1][0], u[1][1]}};
       return Parts{u32x4{u[0][0], u[0][1], 0, 0}, u32x4{u[1][0], u[1][1], u[0][0], u[0][1]},
                    u32x4{0, 0, u[1][0], u[1][1]}, u32x4{u[0][0], u[0][1], u[2][0], u[2][1]}};
     };
@@ -1414,14 +1430,29 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       return !__any(!(abs_sum(U) + abs_sum(R) + keys <= 0.5f * kSplitMax));
     };
     auto finite = [](float x) { return fabsf(x) < HUGE_VALF; };
-    // The product of the first parts.  EXACT: of 16 terms; where a product of 32 terms adds to it, a vector instruction is in
-    // between (the compiler leaves too few cycles for the sum of one straight into the other).
-    typedef std::conditional_t<EXACT, u32x2, u32x4> Kt;
+    // The product of the first parts.  EXACT and ONE: of 16 terms and, but for retention, as many zeros (a product adds the sum
+    // so far to four terms and zeros at a time and rounds, one of 16 terms to more of them: states are 0.2 - 2 % further from
+    // 64 bits with it, retention's are not, and the walk 2 - 4 % faster).
+    // Where a product of 32 terms adds to one of 16, a vector instruction has to be in between: the compiler leaves too few
+    // cycles.
+    constexpr bool SHORT = MODE == kModeRetention;
+    typedef std::conditional_t<EXACT || ONE, u32x2, u32x4> Kt;
+    auto key_at = [&](const Buf& b, int t) -> Kt {
+      if constexpr (DELTA && ONE) return b.ke[0][DELTA ? gr : 0][16 * t + m];
+      else return b.kt01[gr][16 * t + m];
+    };
+    auto key_rest = [&](const Buf& b, int t) {
+      if constexpr (ONE) return u32x4{};
+      else return b.kt20[gr][16 * t + m];
+    };
     auto first_parts = [](const Kt& x, const Parts& u, const f32x4 D) {
-      if constexpr (EXACT) {
+      if constexpr (EXACT || ONE) {
         typedef __attribute__((ext_vector_type(4))) short s16x4;
-        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, x),
-                                                         __builtin_bit_cast(s16x4, u32x2{u.p0[0], u.p0[1]}), D, 0, 0, 0);
+        if constexpr (SHORT)
+          return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, x),
+                                                           __builtin_bit_cast(s16x4, u32x2{u.p0[0], u.p0[1]}), D, 0, 0, 0);
+        else
+          return mma(u32x4{x[0], x[1], 0, 0}, u.p0, D);
       } else {
         return mma(x, u.p0, D);
       }
@@ -1440,7 +1471,8 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const unsigned p1 = EXACT ? y[2 + (i >> 1)] : x[(2 + (i >> 1)) % (sizeof(Kt) / 4)];
-        other = mma(join(x[i >> 1], p1, y[i >> 1], i & 1) * sc[i], V[i], other);
+        const float k = ONE ? (i & 1 ? bf16_high(x[i >> 1]) : bf16_low(x[i >> 1])) : join(x[i >> 1], p1, y[i >> 1], i & 1);
+        other = mma(k * sc[i], V[i], other);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) D[i] = __builtin_fmaf(S[t][i], f[i], D[i]);
@@ -1450,8 +1482,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     };
     // the smaller parts' products
     auto small_parts = [&](const Kt& x, const u32x4& y, const Parts& u) {
+      if constexpr (ONE) return mma(u32x4{x[0], x[1], x[0], x[1]}, u.p02, zero);
       f32x4 D = mma(y, u.p02, zero);
-      if constexpr (!EXACT) {
+      if constexpr (!EXACT && !ONE) {
         D = mma(x, u.p1, D);
         D = mma(x, u.p10, D);
       }
@@ -1472,8 +1505,8 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       auto ahead = [&](int t) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          hm[t >> 1 & 1][e] = b.kt01[gr][16 * (t + e) + m];
-          lh[t >> 1 & 1][e] = b.kt20[gr][16 * (t + e) + m];
+          hm[t >> 1 & 1][e] = key_at(b, t + e);
+          lh[t >> 1 & 1][e] = key_rest(b, t + e);
         }
       };
       ahead(0);
@@ -1565,12 +1598,6 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       }
     };
     auto order = [] { __builtin_amdgcn_sched_barrier(0); };
-    // product i of rows r and a state's parts q
-    auto product = [&](Sum& x, const u32x4 (&r)[3], const u32x4 (&q)[3], int i) {
-      constexpr int kRow[] = {0, 2, 0, 1, 1, 0}, kState[] = {2, 0, 0, 1, 0, 1}, kSum[] = {0, 1, 2, 0, 1, 0};
-      f32x4& to = kSum[i] == 2 ? x.big : x.small[kSum[i] % 2];
-      to = mma(r[kRow[i]], q[kState[i]], to);
-    };
     // beside product i of six: a part of the next rows, and what it leaves
     auto part_beside = [&](SplitSteps& next, int i, u32x4 (&q)[3]) {
       if (i % 2 == 0) {
@@ -1614,11 +1641,11 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             }
           };
 #pragma unroll
-          for (int e = 0; e < 3; ++e) load(ra, key_rows, 0, e);
+          for (int e = 0; e < RP; ++e) load(ra, key_rows, 0, e);
 #pragma unroll
-          for (int e = 0; e < 3; ++e) load(rc, b.qe, 0, e);
+          for (int e = 0; e < RP; ++e) load(rc, b.qe, 0, e);
 #pragma unroll
-          for (int e = 0; e < 3; ++e) load(rb, key_rows, 1, e);
+          for (int e = 0; e < RP; ++e) load(rb, key_rows, 1, e);
           order();
           take(1);   // (while the rows come)
 #pragma unroll
@@ -1628,27 +1655,27 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           }
           take(2);
           products(Ws, ra, p[0], [&](int i) { part_beside(next, i, p[2]); });
-          products(Rs, rc, p[0], [&](int i) { if (i < 3) load(ra, key_rows, 2, i); });
+          products(Rs, rc, p[0], [&](int i) { if (i < RP) load(ra, key_rows, 2, i); });
           take(3);
           products(Ws, rb, p[1], [&](int i) {
-            if (i < 3) load(rc, b.qe, 1, i);
+            if (i < RP) load(rc, b.qe, 1, i);
             part_beside(next, i, p[0]);
           });
-          products(Ws, ra, p[2], [&](int i) { if (i < 3) load(rb, key_rows, 3, i); });
+          products(Ws, ra, p[2], [&](int i) { if (i < RP) load(rb, key_rows, 3, i); });
           f32x4 M, v, sk, skt;
           products(Ws, rb, p[0], [&](int i) {
             if (i == 0) M = matrix(b, DELTA ? 256 : 0);
             if (i == 1) v = b.v[gr][16 * w + m];
             if (i == 2) sk = scale(b, kRecK);
             if (i == 2) skt = CH ? zero : scale(b, kRecKt);
-            if (i >= 3) load(ra, b.qe, 2, i - 3);
+            if (i >= 3 && i - 3 < RP) load(ra, b.qe, 2, i - 3);
           });
           // From here on W's sum, U and its parts one after the other, and between them the sum for the outputs.
           f32x4 X, U, U2, rest;
           float sum = 0.f;
           unsigned u[3][2];
           products(Rs, rc, p[1], [&](int i) {
-            if (i < 3) load(rb, b.qe, 3, i);
+            if (i < RP) load(rb, b.qe, 3, i);
             if (i == 1) X = Ws.big + (Ws.small[0] + Ws.small[1]);
             if (i == 2) X = v - sk * X;
             if (i == 3) U = mma(M[0], X[0], zero);
@@ -1681,8 +1708,8 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             const int q = t / 2 % 2;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-              lh[q][e] = b.kt20[gr][16 * (t + e) + m];
-              hm[q][e] = b.kt01[gr][16 * (t + e) + m];
+              lh[q][e] = key_rest(b, t + e);
+              hm[q][e] = key_at(b, t + e);
               if (CH) f[q][e] = decay_rows(b, 0.f, t + e);
             }
           };
@@ -1704,10 +1731,11 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             const int q = t / 2 % 2, r = q;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-              D[r][e] = mma(lh[q][e], parts_u.p02, zero);
+              if constexpr (ONE) D[r][e] = small_parts(hm[q][e], lh[q][e], parts_u);
+              else D[r][e] = mma(lh[q][e], parts_u.p02, zero);
               order();
             }
-            if constexpr (!EXACT) {
+            if constexpr (!EXACT && !ONE) {
 #pragma unroll
               for (int e = 0; e < 2; ++e) {
                 D[r][e] = mma(hm[q][e], parts_u.p1, D[r][e]);
@@ -1782,7 +1810,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         u32x4 rows[2][2][3];   // of ke and qe
         const auto& key_rows = *reinterpret_cast<const typename Buf::Rows*>(&b.ke);
         auto ahead = [&](int s, int i) {
-          rows[s & 1][i / 3][i % 3] = row(i < 3 ? key_rows[i] : b.qe[i - 3], s);
+          if (i % 3 < RP) rows[s & 1][i / 3][i % 3] = row(i < 3 ? key_rows[i % 3 % RP] : b.qe[i % 3 % RP], s);
         };
 #pragma unroll
         for (int i = 0; i < 6; ++i) ahead(0, i);
@@ -1797,10 +1825,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             for (int e = 0; e < 2; ++e) next.r[e] = S[0][(2 * s + 2 + e) % NT];
 #pragma unroll
           for (int i = 0; i < 12; ++i) {   // products of ke and qe in turn
-            constexpr int kRow[] = {0, 2, 0, 1, 1, 0}, kState[] = {2, 0, 0, 1, 0, 1}, kSum[] = {0, 1, 2, 0, 1, 0};
-            Sum& x = i & 1 ? Rs : Ws;
-            f32x4& to = kSum[i >> 1] == 2 ? x.big : x.small[kSum[i >> 1]];
-            to = mma(rows[s & 1][i & 1][kRow[i >> 1]], p[s & 1][kState[i >> 1]], to);
+            product(i & 1 ? Rs : Ws, rows[s & 1][i & 1], p[s & 1], i >> 1);
             if (more && i < 6) ahead(s + 1, i);
             if (more && i < 11) next.step(i, p[s + 1 & 1], id);
             __builtin_amdgcn_sched_barrier(0);
@@ -1857,8 +1882,8 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         auto keys = [&](int t) {
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
-            lh[t >> 1 & 1][e] = b.kt20[gr][16 * (t + e) + m];
-            hm[t >> 1 & 1][e] = b.kt01[gr][16 * (t + e) + m];
+            lh[t >> 1 & 1][e] = key_rest(b, t + e);
+            hm[t >> 1 & 1][e] = key_at(b, t + e);
             if (CH) f[t >> 1 & 1][e] = decay_rows(b, 0.f, t + e);
           }
         };
@@ -1869,7 +1894,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           f32x4 AV[CT];
           auto ahead = [&](int s, int e) { rows[s & 1][e] = row(b.qe[e], s); };
 #pragma unroll
-          for (int e = 0; e < 3; ++e) ahead(0, e);
+          for (int e = 0; e < RP; ++e) ahead(0, e);
 #pragma unroll
           for (int ct = 0; ct < CT; ++ct) {
             U[ct] = b.v[gr][16 * (CT * w + ct) + m];
@@ -1908,7 +1933,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
               for (int ct = 0; ct < CT; ++ct) {
                 product(Rs[ct], rows[s & 1], p[s & 1][ct], i);
                 if (more) {
-                  if (ct == 0 && i < 3) ahead(s + 1, i);
+                  if (ct == 0 && i < RP) ahead(s + 1, i);
                   part_beside(next[ct], i, p[s + 1 & 1][ct]);
                 } else if (i == 0) {
                   u[ct] = parts(U[ct], sk);
@@ -2218,7 +2243,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         sum += fabsf(k[i][j]);
         if (CH && MODE != kModeForget) sum += d[i][j];   // (the forget gate's key holds it)
       }
-    const bool odd = __any(!(sum <= 0.5f * kSplitMax));
+    const bool odd = !ONE && __any(!(sum <= 0.5f * kSplitMax));
     float f[CPW], behind[CPW];   // products of the decays of the lane groups before / behind this one
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
@@ -2289,17 +2314,17 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       for (int i = 0; i < 3; ++i) {
 #pragma unroll
         for (int g = 0; g < N; ++g)
-          if (i >= from(g)) {
+          if (i >= from(g) && i < RP) {
             p[g][i][0] = pack_bf16(x[g][0], x[g][1]);
             p[g][i][1] = pack_bf16(x[g][2], x[g][3]);
-            if (i < 2) x[g] = id.rest(x[g], p[g][i][0], p[g][i][1]);
+            if (i + 1 < RP) x[g] = id.rest(x[g], p[g][i][0], p[g][i][1]);
           }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    auto put = [&](u32x2 (&rows)[3][4][DK + 16], int g) {
+    auto put = [&](u32x2 (&rows)[RP][4][DK + 16], int g) {
 #pragma unroll
-      for (int e = 0; e < 3; ++e) {
+      for (int e = 0; e < RP; ++e) {
         if constexpr (CPW == 2)
           *reinterpret_cast<u32x4*>(&rows[e][tg][c0]) = u32x4{p[g][e][0], p[g][e][1], p[(g + 1) % N][e][0], p[(g + 1) % N][e][1]};
         else
@@ -2311,7 +2336,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
       const unsigned (&y)[3][2] = p[KT + j];
-      if constexpr (EXACT) {
+      if constexpr (ONE) {
+        if constexpr (!DELTA) b.kt01[tg][c0 + j] = u32x2{y[0][0], y[0][1]};
+      } else if constexpr (EXACT) {
         b.kt01[tg][c0 + j] = u32x2{y[0][0], y[0][1]};
         b.kt20[tg][c0 + j] = u32x4{y[2][0], y[2][1], y[1][0], y[1][1]};
       } else {
@@ -2340,7 +2367,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 template <typename T, int MODE, int DK, int VEC, int CT>
 __global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
 scan_walk_kernel(ChunkArgs a, int portion0) {
-  __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>()> lds;
+  __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg{find_portion(a, portion0 + static_cast<int>(blockIdx.y)), 0, 1, 0, 0};
   if (sg.s >= 0) walk<T, MODE, DK, VEC, 0, CT>(a, sg, lds);
 }
@@ -2349,7 +2376,7 @@ scan_walk_kernel(ChunkArgs a, int portion0) {
 template <typename T, int MODE, int DK, int VEC, int CT>
 __global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
 scan_segments_kernel(ChunkArgs a, int segment0) {
-  __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>()> lds;
+  __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg = find_segment<false>(a, segment0 + blockIdx.y);
   if (sg.s < 0) return;
   if (sg.P == 1)
@@ -2360,7 +2387,7 @@ scan_segments_kernel(ChunkArgs a, int segment0) {
 template <typename T, int MODE, int DK, int VEC, int CT>
 __global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
 scan_segments_end_kernel(ChunkArgs a, int segment0) {
-  __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>()> lds;
+  __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg = find_segment<true>(a, segment0 + blockIdx.y);
   if (sg.s >= 0 && sg.state + sg.P <= a.seg_states) walk<T, MODE, DK, VEC, 2, CT>(a, sg, lds);
 }
