@@ -50,6 +50,10 @@ __device__ __forceinline__ int keep_parts(int keep, int wstart) {
 bool launch_sink_flash(void* out, const void* q, const void* k_cache, const void* v_cache,
                        const AttnArgs& a, int num_tiles, hipStream_t st);
 
+// Prompts and decode partitions in 32 bits on the matrix cores (sink_float.hip); false: not these shapes.
+bool launch_sink_float(void* out, const void* q, const void* k_cache, const void* v_cache, const AttnArgs& a,
+                       int num_tiles, int num_decode, int parts, hipStream_t st);
+
 // Partition kernel of the decode rows (sink_decode.hip); false: no instance for these shapes.
 bool launch_sink_decode(const void* q, const void* k_cache, const void* v_cache, const AttnArgs& a, int num_decode,
                         int parts, hipStream_t st);

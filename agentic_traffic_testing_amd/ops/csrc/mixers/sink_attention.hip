@@ -1,6 +1,6 @@
 // Causal paged softmax attention for any head widths, with an optional sink (one extra key of
 // score 0 and no value in every denominator).  K pages are [nb, G, BS, dim], V pages are
-// channel-major [nb, G, vdim, BS].  Three kernels:
+// channel-major [nb, G, vdim, BS].  Four kernels:
 //
 // * rows kernel (any dtype, any widths; fp32 scores, weights and accumulation): a workgroup of
 //   256 threads serves 16 "rows" against a stream of key tiles staged in LDS as fp32; thread
@@ -21,6 +21,7 @@
 //   8+4h..8+4h+3 for lane half h), and the V^T operand reads follow the same order.
 //   The served head widths run its flash form instead (sink_flash.hip; the rule stands there).
 // * decode of the served head widths: sink_decode.hip, with the join of the decode partials (all kernels).
+// * 32 bits (widths in multiples of 16, aligned), prompts and decode: sink_float.hip, for what the rows kernel does otherwise.
 //
 // A sliding window (`window` > 0: the query at position i sees keys j with 0 <= i - j < window)
 // moves the first key tile of a workgroup up to the window's start and masks the tiles that
@@ -716,6 +717,14 @@ extern "C" int mixk_sink_attention(void* out, const void* q, const void* k_cache
     num_tiles = 0;
     if (nd_mfma > 0) num_decode = 0;
     if (num_decode <= 0) return 0;
+  }
+  if (dtype == 2) {   // (sink_float.hip has the rule and both sides' times)
+    const int parts = decode_parts(max_decode_kv, a.window, a.keep);
+    if (num_decode > 0 && (parts > max_parts || parts < 1)) return -1;
+    if (launch_sink_float(out, q, k_cache, v_cache, a, num_tiles, num_decode, parts, st)) {
+      if (num_decode > 0) launch_sink_join(out, a, num_decode, dtype, st);
+      return static_cast<int>(hipGetLastError());
+    }
   }
   MIXK_DISPATCH(dtype, rc = launch_rows<T>(out, q, k_cache, v_cache, a, num_tiles, num_decode,
                                            max_decode_kv, st));

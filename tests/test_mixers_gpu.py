@@ -1405,6 +1405,44 @@ def test_flash_off_16_byte_borders(H, G, d, dv, window, keep, dtype):
         assert float((got - want.double()).norm() / want.double().norm()) < limit
 
 
+@pytest.mark.parametrize("H,G,share,d,dv", [(4, 4, 1, 16, 16), (6, 2, 1, 64, 64), (8, 4, 2, 48, 128), (4, 2, 1, 128, 112),
+                                            (5, 1, 1, 256, 192), (20, 1, 1, 240, 256)])
+@pytest.mark.parametrize("window,keep,bs", [(0, 0, 16), (100, 0, 48), (64, 70, 16), (300, 200, 64), (1, 3, 16)])
+def test_attention_in_32_bits_edges(H, G, share, d, dv, window, keep, bs):
+    """Matrix cores in 32 bits: portions around the blocks (16 tokens, 16 keys) and single rows around the partitions (128
+    keys), windows and kept keys that share a block; page slots that no key is in hold NaN.  Caches between 16-byte borders
+    take the general kernel: the same results."""
+    torch.manual_seed(d + window)
+    lens = [1, 1, 1, 1, 1, 15, 16, 17, 33, 130, 2]
+    starts = [0, 126, 128, 340, 639, 0, 0, 63, 638, 62, 15]
+    md = ragged(lens, starts, list(range(len(lens))), bs=bs, width=64)
+    T, nb = int(md["seq_qstart"][-1]), md["num_pages"]
+    q, gate, sink = torch.randn(T, H * d + 24), torch.randn(T, H), torch.randn(H)
+    k, v = torch.randn(nb, G, bs, d), torch.randn(nb, G // share, dv, bs)
+    used = torch.zeros(nb, bs, dtype=torch.bool)
+    for i, (n, s0) in enumerate(zip(lens, starts)):
+        for p in range(s0 + n):
+            used[md["block_tables"][i, p // bs], p % bs] = True
+    tiles = md["tile_seq"] >= 5
+    md["tile_seq"], md["tile_qoff"] = md["tile_seq"][tiles], md["tile_qoff"][tiles]
+    want = mref.sink_attention(q[:, 8:8 + H * d].unflatten(1, (H, d)), k, v.repeat_interleave(share, 1), md["block_tables"],
+                               md["seq_kvlen"], md["seq_qstart"], d ** -0.5, True, sink, window, gate, keep)
+    k.permute(0, 2, 1, 3)[~used] = float("nan")
+    v.permute(0, 3, 1, 2)[~used] = float("nan")
+    g, qg = cuda(md), q.cuda()[:, 8:8 + H * d].unflatten(1, (H, d))
+
+    def run(by, **kw):
+        at = [torch.empty(t.numel() + by, device="cuda")[by:].view(t.shape).copy_(t) for t in (k, v)]
+        return mx.sink_attention(qg, *at, g["block_tables"], g["seq_kvlen"], g["seq_qstart"], g["tile_seq"], g["tile_qoff"],
+                                 d ** -0.5, num_decode=5, max_decode_kv=640, window=window, keep_first=keep, **kw).cpu()
+
+    # scores are sums of d products and results of up to 670, 2^-24 each, in another order than the reference's
+    got = run(0, sink=True, sink_values=sink.cuda(), gate=gate.cuda())
+    assert torch.allclose(got, want, **tol(torch.float32))
+    assert torch.allclose(run(1, sink=True, sink_values=sink.cuda(), gate=gate.cuda()), want, **tol(torch.float32))
+    assert torch.allclose(run(0, sink=False), run(1, sink=False), **tol(torch.float32))
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
