@@ -28,10 +28,12 @@
 // * matrix-core decode kernel (bf16, dim % 8 == 0, dim <= 256, vdim % 16 == 0, H <= 64): one
 //   workgroup per (sequence, 64-key partition), columns = the query heads of a KV head; the mix
 //   runs on the VALU in fp32; the partition's sums go to `part`, a combine kernel adds them.
+// * 32 bits (widths in multiples of 16 up to 128, H <= 32, aligned), prompts and decode: sigmoid_float.hip.
 // * rows kernel (any dtype and widths): fp32 FMA, all heads of up to 8 query rows per workgroup;
 //   also the decode form of the shapes the matrix-core decode kernel does not take.
 #include "mix_common.h"
 #include "mixers.h"
+#include "sigmoid_attention.h"
 
 namespace mixk {
 
@@ -40,10 +42,8 @@ typedef __attribute__((ext_vector_type(4))) __bf16 sg_bf16x4;
 typedef __attribute__((ext_vector_type(4))) float sg_f32x4;
 typedef __attribute__((ext_vector_type(4))) unsigned int sg_u32x4;
 
-constexpr int kSgTile = 64;     // query tokens per entry of the host's tile list
 constexpr int kSgTok = 16;      // query tokens per workgroup (matrix-core prefill)
 constexpr int kSgKeys = 32;     // keys per tile
-constexpr int kSgPart = 64;     // keys per decode partition
 constexpr int kSgRow = kSgTok * 32;   // LDS row of a slot: 16 tokens x 32 keys
 // head slots per wave (a run of 2 or 4, so 16 or 32 slots: the K of the mixing product)
 __host__ __device__ constexpr int sg_slots(int HW) { return HW <= 2 ? 2 : 4; }
@@ -52,22 +52,6 @@ constexpr int kSgAcc = 64;      // accumulators per thread of the rows kernel
 // all of a CU's 160 KB)
 __host__ __device__ constexpr int sg_q_lds(int HW, int ND) { return HW == 4 && ND == 4 ? 2 : 0; }
 constexpr float kLog2e = 1.44269504088896341f;
-
-struct SigArgs {
-  const int* block_tables;
-  const int* seq_kvlen;
-  const int* seq_qstart;
-  const int* tile_seq;
-  const int* tile_qoff;
-  float* part;          // decode partials [S, H, max_parts, vdim]
-  const float* bias;    // [H]
-  const float* talk;    // [H, H]
-  int bt_width, H, G, dim, vdim, block_size, bs_shift, max_parts, rows;
-  float scale, cap;
-  float* split_out;     // prefill split over the keys: fp32 partial rows [split, T, H, vdim]
-  int split, total_rows;   // split: most shares
-  int room;                // query tiles that take as long together as one alone
-};
 
 // Key shares of a launch's query tiles.  The host knows how many tiles there are and not how many keys they have; where
 // the shares do not all run at once, the better number is a question of these: at 24 heads a second share takes 3300 rows
@@ -908,6 +892,8 @@ extern "C" int mixk_sigmoid_attention(void* out, const void* q, const void* k_ca
     if (rc) return rc;
     rows_decode = 0;
   }
+  if (use_mfma && dtype == 2 && launch_sigmoid_float(out, q, k_cache, v_cache, a, num_tiles, num_decode, parts, st))
+    rows_tiles = rows_decode = 0;   // (sigmoid_float.hip has the rule and both sides' times)
   if (rows_tiles > 0 || rows_decode > 0) {
     MIXK_DISPATCH(dtype, rc = sg_launch_rows<T>(out, q, k_cache, v_cache, a, rows_tiles,
                                                 rows_decode, parts, st));

@@ -1443,6 +1443,47 @@ def test_attention_in_32_bits_edges(H, G, share, d, dv, window, keep, bs):
     assert torch.allclose(run(0, sink=False), run(1, sink=False), **tol(torch.float32))
 
 
+@pytest.mark.parametrize("H,G,dim,vdim", [(1, 1, 16, 16), (8, 2, 128, 128), (5, 5, 48, 64), (12, 4, 64, 32), (24, 8, 128, 96),
+                                          (26, 2, 64, 64), (32, 8, 112, 128)])
+@pytest.mark.parametrize("bs,cap", [(16, 7.0), (48, 0.0)])
+def test_sigmoid_attention_in_32_bits_edges(H, G, dim, vdim, bs, cap):
+    """Matrix cores in 32 bits: portions around the blocks (16 tokens, 16 keys), rows around the partitions (64 keys), heads
+    that do not fill the waves; page slots that no key is in hold NaN.  Caches between 16-byte borders take the general
+    kernel.  An infinite value reaches only the tokens that see its key."""
+    torch.manual_seed(H)
+    lens, starts = [1, 1, 1, 1, 15, 16, 17, 33, 130, 2], [0, 63, 64, 200, 0, 0, 63, 310, 62, 15]
+    md = ragged(lens, starts, list(range(len(lens))), bs=bs, width=32)
+    q, (k, v) = torch.randn(int(md["seq_qstart"][-1]), H, dim), ragged_pages(md, G, dim, vdim, bs, torch.float32)
+    bias, talk, scale = torch.randn(H) - 3.0, torch.eye(H) + 0.3 * torch.randn(H, H), 1.7 * dim ** -0.5
+    used = torch.zeros(md["num_pages"], bs, dtype=torch.bool)
+    for i, (n, s0) in enumerate(zip(lens, starts)):
+        for p in range(s0 + n):
+            used[md["block_tables"][i, p // bs], p % bs] = True
+    tiles = md["tile_seq"] >= 4
+    md["tile_seq"], md["tile_qoff"] = md["tile_seq"][tiles], md["tile_qoff"][tiles]
+    want = mref.sigmoid_attention(q, k, v, md["block_tables"], md["seq_kvlen"], md["seq_qstart"], scale, cap, bias, talk)
+    k.permute(0, 2, 1, 3)[~used] = float("nan")
+    v.permute(0, 3, 1, 2)[~used] = float("nan")
+    g = cuda(md)
+
+    def run(v, by=0):
+        at = [torch.empty(t.numel() + by, device="cuda")[by:].view(t.shape).copy_(t) for t in (k, v)]
+        return mx.sigmoid_attention(q.cuda(), *at, g["block_tables"], g["seq_kvlen"], g["seq_qstart"], g["tile_seq"],
+                                    g["tile_qoff"], scale, cap, bias.cuda(), talk.cuda(), 4, 201).cpu()
+
+    got = run(v)
+    for x in (got, run(v, 1)):
+        # sums of up to 350 x H weights with errors of a few 2^-24 each, in another order than the reference's
+        assert float(((x - want).abs() / (want.abs() + want.pow(2).mean().sqrt())).max()) < 2e-5
+    last, at = int(md["seq_qstart"][9]), 62 + 121          # token 121 of the portion of 130
+    inf = v.clone()
+    inf[md["block_tables"][8, at // bs], :, :, at % bs] = float("inf")
+    got_inf = run(inf)
+    # (its block of 16 tokens is summed key by key: another order)
+    assert torch.allclose(got_inf[:last - 9], got[:last - 9], **tol(torch.float32)) and torch.equal(got_inf[last:], got[last:])
+    assert not torch.isfinite(got_inf[last - 9:last]).any()
+
+
 CHUNK_LENS = [1, 4, 5, 15, 16, 17, 33, 70, 3, 128]
 CHUNK_STARTS = [9, 0, 0, 4, 0, 31, 0, 100, 0, 0]
 
