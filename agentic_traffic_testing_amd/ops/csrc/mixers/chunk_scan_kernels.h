@@ -934,7 +934,10 @@ scan_scores_kernel(ChunkArgs a, int step_blocks, int step_cols, int v4) {
     if ((w & 1) == 0) {   // A and the scales
       f32x4 x = both(s0.sq[m], s1.sq[m]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = (4 * gr + i == m ? qk : x[i]) * qi * kj[i];
+      for (int i = 0; i < 4; ++i) {   // (zeros above the diagonal: a later token's scale may be NaN)
+        const int j = 4 * gr + i;
+        x[i] = j <= m ? (j == m ? qk : x[i]) * qi * kj[i] : 0.f;
+      }
       *reinterpret_cast<f32x4*>(rec + m * 16 + 4 * gr) = x;
       if (lane < 16) {
         rec[kRecQ + lane] = qi;

@@ -1631,16 +1631,16 @@ def test_chunked_scans_keep_earlier_tokens(bad):
 
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
-def test_chunked_scans_pass_non_finite_inputs(dt, bad):
+def test_chunked_scans_pass_non_finite_inputs(dt, bad, d=64):
     """One non-finite entry in any input of a recurrence: finite results and states exactly where the token-by-token
     reference has them, rows before it and other sequences untouched."""
     torch.manual_seed(1)
-    H, d, dv, hit, col = 2, 64, 64, 41, 5       # token 41: third chunk of the first portion
+    H, dv, hit, col = 2, 64, 41, 5              # token 41: third chunk of the first portion
     md = ragged([170, 140], [0, 0], [0, 1], width=64)
     T, g, z, zz = 310, cuda(md), torch.zeros(H), torch.zeros(H * d)
     at = (md["positions"], md["seq_qstart"], md["seq_slot"])
     at_g = (g["positions"], g["seq_qstart"], g["seq_slot"])
-    q, k, v, wide = (torch.randn(T, H * d).to(dt) for _ in range(4))
+    q, k, v, wide = (torch.randn(T, H * n).to(dt) for n in (d, d, dv, d))
     one, two = torch.randn(T, H).to(dt), torch.randn(T, H).to(dt)
     tab, pw = torch.zeros(T, 0), mx.retention_powers([0.9, 0.99], "cpu")
     for name, inputs, rest, last in (
@@ -1664,6 +1664,15 @@ def test_chunked_scans_pass_non_finite_inputs(dt, bad):
                 assert torch.equal(got[0][:hit], fine[:hit]) and torch.equal(got[0][170:], fine[170:]), (name, i, c)
                 for a, b in zip(got, want):
                     assert torch.equal(torch.isfinite(a), torch.isfinite(b)), (name, i, c)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("d", [100, 128])
+def test_chunked_scans_of_wide_keys_pass_non_finite_inputs(dt, bad, d):
+    """The same for keys that the kernels of up to 128 channels take: scores of 16-bit inputs with a decay per channel by two
+    waves, half of the channels each."""
+    test_chunked_scans_pass_non_finite_inputs(dt, bad, d)
 
 
 def portions_and_rows(call, n, S):
