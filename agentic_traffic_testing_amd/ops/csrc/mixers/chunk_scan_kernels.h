@@ -1611,11 +1611,19 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         }
       }
     };
-    // Full chunks of full columns and ordinary numbers are walked in loops of their own.  A wave issues in order, and left to
+    // A wave without columns only keeps the barriers: the first, a chunk's, and the last of an odd number of them.
+    if (col0 >= a.dv) {
+      for (int c = 0; c <= nc + (nc & 1); ++c) lds_barrier();
+      return;
+    }
+    // Full chunks of ordinary numbers are walked in loops of their own.  A wave issues in order, and left to
     // itself the compiler puts every load, part and product right in front of what waits for it; here all have been on their
     // way for a few products.  A chunk that is not ordinary is left, untouched, to the loop behind (two ways in one loop cost
-    // a move per number of the state and chunk).
-    const int full = col0 + 16 * CT <= a.dv ? n / kScanChunk : 0;
+    // a move per number of the state and chunk).  Columns past the last one go along, on copies of the last one's values, and
+    // are not stored: the loop behind takes a wave's two tiles one after the other, and everybody waits for it at the barrier
+    // (us, such waves in the loop behind / here, 32 heads, 16 x 512, 96 columns: forget gate 267 / 233, state space 190 / 150;
+    // 96 heads of 40, one prompt of 1023 in 32 bits 97 / 86).
+    const int full = !DELTA || col0 + 16 <= a.dv ? n / kScanChunk : 0;
     int c = 0;
     lds_barrier();
     if constexpr (DELTA) {
@@ -1975,8 +1983,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             if (MODE == kModeStateSpace) O += skip * U[ct];
             float* oc = op + static_cast<int64_t>(c) * kScanChunk * o_stride;
             const unsigned at = (4 * gr * o_stride + col0 + 16 * ct + m) * sizeof(float);
+            if (col0 + 16 * ct + m < a.dv)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = O[i];
+              for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = O[i];
           }
         } else {
           keys(0);

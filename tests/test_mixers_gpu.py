@@ -2610,6 +2610,76 @@ def test_two_heads_in_segments(dt, H, G, dv, lens):
         assert float((a - b).abs().max()) <= 2e-5 * float(b.abs().max())
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,G,d,dv,lens", [
+    (16, 8, 128, 128, [47] * 17 + [100]), (16, 16, 64, 72, [47] * 17 + [100]), (32, 8, 128, 48, [47] * 17 + [100]),   # whole
+    (40, 40, 128, 96, [40, 2100]), (96, 24, 128, 40, [33, 950, 1])])                                                # in segments
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_non_finite_values_in_wide_workgroups(dt, H, G, d, dv, lens, bad):
+    """Two tiles of 16 columns per wave, of a head's 128 columns or of two heads with the same keys, widths that leave waves
+    with some of their columns or none: one non-finite entry in a middle chunk of the longest portion, in either tile of a
+    wave and in the last column.  It is in every result of its column (keys and queries: of its head) from its token on,
+    and nothing else changes a bit."""
+    torch.manual_seed(H + dv)
+    S, T = len(lens), sum(lens)
+    long = lens.index(max(lens))
+    md = ragged(lens, [5 * (i % 2) for i in range(S)], list(range(S))[::-1], width=160)
+    g, first = cuda(md), int(md["seq_qstart"][long])
+    at = (g["positions"], g["seq_qstart"], g["seq_slot"])
+    hit, end, slot = first + max(lens) // 32 * 16 + 5, first + max(lens), S - 1 - long
+    rand = lambda n: torch.randn(T, n).to(dt).cuda()  # noqa: E731
+    z, tab, bias = torch.zeros(H).cuda(), torch.zeros(T, 0).cuda(), torch.randn(H * d).cuda()
+    lower, start = 0.9 + 0.1 * torch.rand(H * d).cuda(), torch.randn(S, H, d, dv).cuda()
+    pw = mx.retention_powers([1 - 2.0 ** (-5 - h % 6) for h in range(H)], "cuda")
+    for name, groups in (("forget_gate_scan", H), ("state_space_scan", G), ("retention", H)):
+        p = scan_plan(name, lens, H, groups, d, dv)
+        if dv > 64:
+            assert (p["waves"], p["cols"]) == (8, 128)
+        elif name != "state_space_scan":
+            continue
+        else:
+            assert (p["waves"], p["heads"]) == (8, 2)
+        assert (p["states"] > 0 and segments_of(-(-max(lens) // 16), p["chunks"])[0] > 1) == (max(lens) > 100)
+        x = {"q": rand(groups * d), "k": rand(groups * d), "v": rand(H * dv)}
+        dts = rand(H)
+
+        def run(x, st):
+            args, last = {
+                "forget_gate_scan": ((x["q"], x["k"], x["v"], bias, lower), (H, d, dv)),
+                "state_space_scan": ((x["v"], x["k"], x["q"], dts, z - 4, z, z), (H, groups, d, dv)),
+                "retention": ((x["q"], x["k"], x["v"], pw, tab), (H, d, dv))}[name]
+            return getattr(mx, name)(*args, st, *at, *last), st
+
+        fine = run(x, start.clone())
+        assert all(bool(torch.isfinite(t).all()) for t in fine)
+        head = H - 2
+        for which, col in (("v", 3), ("v", 20), ("v", dv - 1), ("state", 20), ("state", dv - 1), ("k", 7), ("q", 7)):
+            broken, st = dict(x), start.clone()
+            out, state = torch.zeros(T, H, dv, dtype=torch.bool), torch.zeros(S, H, d, dv, dtype=torch.bool)
+            heads = slice(head, head + 1) if groups == H else slice(head // (H // G) * (H // G), (head // (H // G) + 1) * (H // G))
+            if which == "state":
+                st[slot, head, 3, col] = bad
+                out[first:end, head, col] = state[slot, head, 3, col] = True
+            else:
+                broken[which] = x[which].clone()
+                at_col = head * dv + col if which == "v" else heads.start // (H // groups) * d + col
+                broken[which][hit, at_col] = bad
+                if which == "v":
+                    out[hit:end, head, col] = state[slot, head, :, col] = True
+                elif which == "q":
+                    out[hit, heads] = True
+                elif name == "forget_gate_scan":       # (a gate: 1 in place of infinity, as the channel's decay)
+                    if bad == bad:
+                        continue
+                    out[hit:end, heads], state[slot, heads, col] = True, True
+                else:
+                    out[hit:end, heads], state[slot, heads, col] = True, True
+            got = run(broken, st)
+            for a, b, odd in zip(got, fine, (out, state)):
+                assert torch.equal(a.cpu()[~odd], b.cpu()[~odd]), (name, which, col)
+                assert not torch.isfinite(a.cpu()[odd]).any(), (name, which, col)
+
+
 def test_forget_gate_results_in_bf16():
     """16-bit inputs, portions of 60 tokens: a chunk's own part of the results is summed in the tokens' order, which leaves
     rows of early tokens fewer roundings.  Relative error of 2^18 results from 64 bits 7.26e-8, over every fourth token at a
