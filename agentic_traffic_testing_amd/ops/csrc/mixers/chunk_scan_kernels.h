@@ -1142,9 +1142,10 @@ struct WalkBuf {
   static constexpr bool DELTA = MODE >= kModeDelta, CH = per_channel<MODE>();
   static constexpr int COLS = DELTA ? kWalkCols : 2 * kWalkCols, HEADS = MODE == kModeStateSpace ? 2 : 1;
   // rows in three parts, per four tokens and channel as the lane that prepares them holds them; the reads transpose
-  typedef u32x2 Rows[ONE ? 1 : 3][4][DK + 16];
+  static constexpr int ROW = DK + (DK == 64 ? 8 : 16);
+  typedef u32x2 Rows[ONE ? 1 : 3][4][ROW];
   Rows qe;                              // P_i q_i; one number as the decay: q_i
-  u32x2 ke[DELTA && !ONE ? 3 : 1][DELTA ? 4 : 1][DK + 16];   // P_i k_i; k_i
+  u32x2 ke[DELTA && !ONE ? 3 : 1][DELTA ? 4 : 1][DELTA ? ROW : 1];   // P_i k_i; k_i
   // D_end,j k_j; not EXACT and one number as the decay: k_j.  Per four tokens and channel two parts of each
   // parts 0 and 1; EXACT: 0; ONE: the number, which a delta rule has in ke
   std::conditional_t<EXACT || ONE, u32x2, u32x4> kt01[DELTA && ONE ? 1 : 4][DK];
@@ -1164,6 +1165,12 @@ struct WalkLds {
     float start[DELTA ? 1 : DK][2 * kWalkCols + 4];   // the state at a segment's start
   };
 };
+// Waves per SIMD that the walk's registers are for: 12 in a workgroup, or eight with two tiles each and twice the registers.
+// Keys of up to 64 channels, 16 columns per wave: two workgroups of eight waves fit on a CU, their buffers too (below; us, one
+// / two of them, 32 portions of 20 in 32 bits, 32 heads of 64: state space 46 / 36, delta rule 35 / 30).
+template <int MODE, int DK, int CT>
+constexpr int walk_simd_waves() { return DK == 64 && CT == 1 && MODE != kModeRetention ? 4 : 4 - CT; }
+constexpr size_t kLdsBytes = 160 * 1024;
 
 // VEC 2: aligned rows of q, k and v; 1: but for v (an odd width or row, which only the loads of two columns at once mind: with
 // the rows of q and k element by element as well, a retention of 16 x 512 tokens, 32 heads of 64 with rows of v one element
@@ -1186,6 +1193,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
   constexpr int RP = ONE ? 1 : 3;   // parts of the rows
   using Buf = WalkBuf<MODE, DK, EXACT, ONE>;
   constexpr int BUFS = WalkLds<MODE, DK, EXACT, ONE>::BUFS, OW = operand_waves(MODE, DK);
+  static_assert(DK != 64 || 2 * sizeof(lds) <= kLdsBytes, "two workgroups per CU (walk_simd_waves)");
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const Identity id(lane);
@@ -1342,7 +1350,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
     // The rows of the 16 tokens, 32 channels in the order that a product over 32 rows of S takes them (of two tiles of S the
     // rows 4 gr + i).  The read transposes pieces of four tokens in groups of 16 lanes, four channels of all tokens; a lane's
     // own piece is at (token group m % 4, channel m / 4).
-    auto row = [&](const u32x2 (&x)[4][DK + 16], int s) {
+    auto row = [&](const u32x2 (&x)[4][Buf::ROW], int s) {
       typedef __attribute__((ext_vector_type(4))) short s16x4;
       auto get = [&](int t) {
         const u32x2* at = &x[m & 3][32 * s + 16 * t + 4 * gr + (m >> 2)];
@@ -2334,7 +2342,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    auto put = [&](u32x2 (&rows)[RP][4][DK + 16], int g) {
+    auto put = [&](u32x2 (&rows)[RP][4][Buf::ROW], int g) {
 #pragma unroll
       for (int e = 0; e < RP; ++e) {
         if constexpr (CPW == 2)
@@ -2377,7 +2385,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 }
 
 template <typename T, int MODE, int DK, int VEC, int CT>
-__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
+__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, (walk_simd_waves<MODE, DK, CT>()))
 scan_walk_kernel(ChunkArgs a, int portion0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg{find_portion(a, portion0 + static_cast<int>(blockIdx.y)), 0, 1, 0, 0};
@@ -2386,7 +2394,7 @@ scan_walk_kernel(ChunkArgs a, int portion0) {
 
 // segment0 + blockIdx.y = segment of the batch.  First kernel: pass 1, and the portions that are not cut.
 template <typename T, int MODE, int DK, int VEC, int CT>
-__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
+__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, (walk_simd_waves<MODE, DK, CT>()))
 scan_segments_kernel(ChunkArgs a, int segment0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg = find_segment<false>(a, segment0 + blockIdx.y);
@@ -2397,7 +2405,7 @@ scan_segments_kernel(ChunkArgs a, int segment0) {
     walk<T, MODE, DK, VEC, 1, CT>(a, sg, lds);
 }
 template <typename T, int MODE, int DK, int VEC, int CT>
-__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, 4 - CT)
+__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, (walk_simd_waves<MODE, DK, CT>()))
 scan_segments_end_kernel(ChunkArgs a, int segment0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg = find_segment<true>(a, segment0 + blockIdx.y);
