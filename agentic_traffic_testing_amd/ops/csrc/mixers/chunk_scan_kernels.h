@@ -2263,7 +2263,10 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         sum += fabsf(k[i][j]);
         if (CH && MODE != kModeForget) sum += d[i][j];   // (the forget gate's key holds it)
       }
-    const bool odd = !ONE && __any(!(sum <= 0.5f * kSplitMax));
+    // (Keys of up to 64 channels: a lane has one, and would wait for the products.  On the vector units, a layer's call, us, 32
+    // heads of 64, bf16, products / here: retention 16 x 512 124 / 121, 64 x 12 69 / 65, 16 x 100 49 / 46.)
+    constexpr bool VECTOR = DK == 64 && !ONE;
+    const bool odd = VECTOR || (!ONE && __any(!(sum <= 0.5f * kSplitMax)));
     float f[CPW], behind[CPW];   // products of the decays of the lane groups before / behind this one
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
