@@ -1169,7 +1169,7 @@ struct WalkLds {
 // Keys of up to 64 channels, 16 columns per wave: two workgroups of eight waves fit on a CU, their buffers too (below; us, one
 // / two of them, 32 portions of 20 in 32 bits, 32 heads of 64: state space 46 / 36, delta rule 35 / 30).
 template <int MODE, int DK, int CT>
-constexpr int walk_simd_waves() { return DK == 64 && CT == 1 && MODE != kModeRetention ? 4 : 4 - CT; }
+constexpr int walk_simd_waves() { return DK == 64 && CT == 1 ? 4 : 4 - CT; }
 constexpr size_t kLdsBytes = 160 * 1024;
 
 // VEC 2: aligned rows of q, k and v; 1: but for v (an odd width or row, which only the loads of two columns at once mind: with
@@ -2114,8 +2114,9 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
   };
   // Retention's rows come with their partners and tables: two chunks of them ahead are 172 bytes of spilled registers per
   // lane in 32 bits (us with two / one, 32 heads of 128: 16 x 512 463 / 279, 1023 109 / 77, 300 61 / 45; bf16, where few
-  // are spilled, 245 / 242, 69.5 / 69.5, 42 / 41).
-  constexpr int AHEAD = MODE == kModeRetention && DK == 128 ? 1 : 2;
+  // are spilled, 245 / 242, 69.5 / 69.5, 42 / 41; 32 heads of 64, bf16, where two workgroups fit on a CU with one, 121 / 113,
+  // values at odd addresses 194 / 125).
+  constexpr int AHEAD = MODE == kModeRetention ? 1 : 2;
   In raw[AHEAD];
   // A lane's offsets into the chunk's rows; only the last chunk's differ.  Channels that are not there: the last ones.
   constexpr bool KEYS = MODE != kModeForget, DEC = MODE == kModeDeltaChannel, SCALED = DEC || (EXACT && !CH), TURN = MODE == kModeRetention;
