@@ -371,15 +371,15 @@ c10::optional<at::Tensor> scan_records(const at::Tensor& like, int64_t T, int64_
   return at::empty({mixk::scan_scratch_floats(T, S, H, G, dk, dv, mode)}, like.options().dtype(at::kFloat));
 }
 
-// What a batch of a recurrence (ScanMode) runs as: the route (ScanRoute); in chunks the walk's product waves, heads and
-// columns per workgroup, the chunks per segment that it aims at, the scratch's segment states (0: not cut), floats of scratch.
+// What a batch of a recurrence (ScanMode) runs as: the route (ScanRoute); in chunks the walk's tiles of 16 columns, heads
+// and columns per workgroup, the chunks per segment that it aims at, the scratch's segment states (0: not cut), floats of scratch.
 std::vector<int64_t> scan_plan(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dk, int64_t dv, int64_t mode) {
   TORCH_CHECK(T >= 0 && S > 0 && H > 0 && G > 0 && dk > 0 && dk <= 256 && dv > 0 && mode >= 0 && mode <= mixk::kModeDeltaChannel,
               "scan_plan: sizes");
   const int m = static_cast<int>(mode);
   const mixk::WalkShape w = mixk::walk_shape(T, S, H, G, dv, m);
   const mixk::ScanSegments g = mixk::scan_segments(T, S, H, G, dk, dv, m);
-  return {mixk::scan_route(T, S, H, dk, dv, m), w.waves, w.heads, w.cols, g.chunks, g.states,
+  return {mixk::scan_route(T, S, H, dk, dv, m), w.tiles, w.heads, w.cols, g.chunks, g.states,
           mixk::scan_scratch_floats(T, S, H, G, dk, dv, m)};
 }
 

@@ -9,10 +9,9 @@ constexpr int kScanChunk = 16;         // tokens per chunk
 constexpr int kPowers = 65;            // retention: powers 0 ... 64 of a head's decay
 enum ScanMode { kModeRetention = 0, kModeForget = 1, kModeStateSpace = 2, kModeDelta = 3,
                 kModeDeltaChannel = 4 };
-constexpr int kWalkCols = 64;          // value columns of four of the walk's waves
+constexpr int kWalkCols = 64;          // value columns of the walk's four waves with one tile of 16 each
 // the walk's waves that prepare operands for keys of up to dk channels
 constexpr int operand_waves(int mode, int dk) { return mode >= kModeDelta ? dk / 16 : 4; }
-constexpr int kWalkThreads = 64 * 12;
 
 struct ChunkArgs {
   float* out;             // [T, H, dv]
@@ -60,22 +59,22 @@ constexpr int scan_record_floats(int mode, int dk) {
 // (a segment's start is put together from all segments before it; us with at least 10 / 7, 8 heads: 350 rows forget gate
 // 55 / 46, state space 42 / 35, retention 49 / 40, 600 rows 53 / 48, 40 / 36, 46 / 41).  A batch of less than 20 chunks is
 // not cut.
-// A workgroup of the walk: eight waves of 16 columns of S beside four that prepare the operands, once for 128 columns or
-// for two heads of 64 whose keys are the same (the operands' vector work is half of the walk's at 64 columns), or four waves
-// and 64 columns; so the delta rule, whose portions are not cut, with eight waves for its operands.  256 workgroups run at
-// once.  In `units` of a head's 64 columns, S portions make S x units of them:
-// - From 512 on eight waves, if there are 6 chunks per CU: few rows in many portions are decode rows and one prompt, which is
-//   done sooner in more workgroups (state space, 32 heads, us with four / eight waves: 63 rows + 128 64 / 69, 127 + 256
+// A workgroup of the walk: four waves beside four that prepare the operands, with two tiles of 16 columns of S each (wide:
+// the operands serve 128 columns, or two heads of 64 whose keys are the same) or with one, 64 columns; so the delta rule,
+// whose portions are not cut, with up to eight waves for its operands.  256 workgroups run at once.  In `units` of a head's
+// 64 columns, S portions make S x units of them (the figures are of wide workgroups of eight waves with one tile each):
+// - From 512 on wide, if there are 6 chunks per CU: few rows in many portions are decode rows and one prompt, which is
+//   done sooner in more workgroups (state space, 32 heads, us, narrow / wide: 63 rows + 128 64 / 69, 127 + 256
 //   123 / 132, 31 + 300 74 / 80, but 64 x 12 132 / 93, 127 + 600 192 / 170, 8 x 512 127 / 91 and, on the wrong side of the
 //   line, 20 + 8 x 40 50 / 40); from 257 on if there are as many as for long portions.
-// - 192 - 256 fill the chip with four waves, and uncut: a portion in half the workgroups would have to be cut to fill it
-//   (32 heads, four waves uncut / eight cut: retention 4 x 350 55 / 72, 4 x 1000 135 / 159, 4 x 2000 283 / 297, forget gate
+// - 192 - 256 fill the chip with narrow ones, and uncut: a portion in half the workgroups would have to be cut to fill it
+//   (32 heads, narrow uncut / wide cut: retention 4 x 350 55 / 72, 4 x 1000 135 / 159, 4 x 2000 283 / 297, forget gate
 //   4 x 700 126 / 135, state space 4 x 1000 121 / 130, 8 heads 16 x 512 68 / 86).
-// - Fewer: long portions are cut, with eight waves where a 16th of the batch per segment is enough to fill the chip (32
-//   heads, one prompt of 2048, four / eight waves: retention 120 / 98, state space 102 / 84; 8 heads, 4 x 2000: retention
+// - Fewer: long portions are cut, and wide where a 16th of the batch per segment is enough to fill the chip (32
+//   heads, one prompt of 2048, narrow / wide: retention 120 / 98, state space 102 / 84; 8 heads, 4 x 2000: retention
 //   120 / 143, one of 8192 138 / 156).
 struct WalkShape {
-  int waves, heads, cols;   // waves with products; heads per workgroup; columns per workgroup and head
+  int tiles, heads, cols;   // of 16 columns, one or two per wave; heads per workgroup; columns per workgroup and head
 };
 inline int64_t walk_units(int64_t H, int64_t dv) { return H * ((dv + kWalkCols - 1) / kWalkCols); }
 inline WalkShape walk_shape(int64_t T, int64_t S, int64_t H, int64_t G, int64_t dv, int mode) {
@@ -103,7 +102,7 @@ inline ScanSegments scan_segments(int64_t T, int64_t S, int64_t H, int64_t G, in
   // gate 240 / 264, state space 157 / 180 us) or fit on a CU twice (the forget gate's with keys of up to 64: 64 heads of
   // 64, one prompt of 2048 86 / 95, 2 x 1000 84 / 93; retention, that do not, 107 / 95).
   const int64_t busy = S * units;
-  const bool wide = walk_shape(T, S, H, G, dv, mode).waves == 8;
+  const bool wide = walk_shape(T, S, H, G, dv, mode).tiles == 8;
   const bool fits = 512 / units * 10 > 256 / units * 24 || (mode == kModeForget && dk <= 64);
   const int64_t all = wide || (fits && n * units >= 5120 && (busy < 192 || busy > 256)) ? 512 : 256;
   int64_t chunks = (n * units + all - 1) / all;

@@ -17,7 +17,7 @@
 // * scores kernel: a wave or two (score_pairs) per (chunk, head) prepare what does not need the state - A, T and the
 //   per-token scales - into a record in scratch.  All chunks at once, off the serial chain.
 // * walk kernel: a workgroup walks the chunks of one (sequence, head), or of two heads with the same keys, for 64 or 128
-//   value columns (walk_shape).  Four waves hold 16 or 32 columns of S each (eight 16, by rows at any address), in accumulators: the accumulator tiles of
+//   value columns (walk_shape).  Four waves hold 16 or 32 columns of S each, in accumulators: the accumulator tiles of
 //   16 x 16 are, split, at once the operands of the products with S, so S, W and U never leave registers, and a wave does
 //   not wait for another one's products.  The others prepare the chunks' operands in LDS, one step ahead (one barrier per
 //   chunk), with their loads one or two steps ahead of that.
@@ -1165,11 +1165,15 @@ struct WalkLds {
     float start[DELTA ? 1 : DK][2 * kWalkCols + 4];   // the state at a segment's start
   };
 };
-// Waves per SIMD that the walk's registers are for: 12 in a workgroup, or eight with two tiles each and twice the registers.
-// Keys of up to 64 channels, 16 columns per wave: two workgroups of eight waves fit on a CU, their buffers too (below; us, one
-// / two of them, 32 portions of 20 in 32 bits, 32 heads of 64: state space 46 / 36, delta rule 35 / 30).
+// The walk's workgroup: four waves with products, and those with operands.
+constexpr int kWalkWaves = 4;
+template <int MODE, int DK>
+constexpr int walk_threads() { return kWave * (kWalkWaves + operand_waves(MODE, DK)); }
+// Waves per SIMD that its registers are for: one workgroup's; with keys of up to 64 channels and one tile of columns per wave
+// those of two workgroups of eight waves, whose buffers fit on a CU too (us, one / two of them, 32 portions of 20 in 32 bits,
+// 32 heads of 64: state space 46 / 36, delta rule 35 / 30).
 template <int MODE, int DK, int CT>
-constexpr int walk_simd_waves() { return DK == 64 && CT == 1 ? 4 : 4 - CT; }
+constexpr int walk_simd_waves() { return walk_threads<MODE, DK>() > 512 ? 3 : CT == 1 && DK == 64 ? 4 : 2; }
 constexpr size_t kLdsBytes = 160 * 1024;
 
 // VEC 2: aligned rows of q, k and v; 1: but for v (an odd width or row, which only the loads of two columns at once mind: with
@@ -1197,7 +1201,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const Identity id(lane);
-  const int waves = (blockDim.x >> 6) - OW, tiles = CT * waves;   // of the products; columns in 16s
+  constexpr int waves = kWalkWaves, tiles = CT * waves;   // of the products; columns in 16s
   const int hb = a.H / a.walk_heads, cb = blockIdx.x / hb, h0 = blockIdx.x % hb * a.walk_heads;
   // wave w: 16 CT columns of a head
   const bool two = a.walk_heads == 2;
@@ -1223,7 +1227,8 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
            (static_cast<int64_t>(sg.state + j) * a.H + h) * a.dk * a.dv;
   };
   if constexpr (PASS == 2 && !DELTA) {
-    if (sg.j > 0) {   // by 512 threads, 64 columns four at a time, up to four segments' loads ahead
+    if (sg.j > 0) {   // by all 512 threads, 64 columns four at a time, up to four segments' loads ahead
+      static_assert(PASS != 2 || DELTA || walk_threads<MODE, DK>() == 512);
       auto put_together = [&](auto blocks) {
         constexpr int B = decltype(blocks)::value, U = DK * (kWalkCols / 4) / 512, AHEAD = 4 / B;
         f32x4 acc[B][U];
@@ -1272,10 +1277,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             *reinterpret_cast<f32x4*>(&lds.start[f >> 4][kWalkCols * b + 4 * (f & 15)]) = acc[b][u];
           }
       };
-      if (tid < 512) {
-        if (tiles == 8) put_together(std::integral_constant<int, 2>{});
-        else put_together(std::integral_constant<int, 1>{});
-      }
+      put_together(std::integral_constant<int, CT>{});
       lds_barrier();
     }
   }
@@ -2007,9 +2009,6 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           if (__builtin_expect(__any(!(sum <= 0.5f * kSplitMax)), 0)) break;
         }
         const float end = end_of(b, c);
-        // The waves of a SIMD end their steps in different places: while one waits for the read-out's products, the other
-        // one has those with kt, whose vector work and operands take longer.
-        if (CT == 1 && w >= 4) lds_barrier();
         f32x4 D[2][2][CT];
         auto small = [&](int t) {
 #pragma unroll
@@ -2038,12 +2037,12 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
           if (t + 2 < NT) small(t + 2);
           order();
         }
-        if (CT == 2 || w < 4) lds_barrier();
+        lds_barrier();
       }
       for (; c < nc; ++c) {
         const Buf& b = lds.buf[c % BUFS];
         const float end = end_of(b, c);
-        auto chunk = [&](f32x4 (&S)[NT], int ct, bool sync) __attribute__((always_inline)) {
+        auto chunk = [&](f32x4 (&S)[NT], int ct) __attribute__((always_inline)) {
           const f32x4 U = b.v[gr][16 * (CT * w + ct) + m], Us = CH || EXACT ? U : U * scale(b, kRecKt);
           f32x4 R = zero, AV = zero;
           if (PASS != 1) {
@@ -2058,23 +2057,20 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             R = total(Rs);
           }
           if constexpr (PASS == 1) {
-            if (sync) lds_barrier();
             advance(b, U, end, [&] { return !ordinary(b, Us, zero); }, S);
           } else if (__builtin_expect(ordinary(b, Us, EXACT ? abs(R) + abs(AV) : R), 1)) {
             write(b, U, R, scale(b, kRecQ), U, c, std::false_type{}, AV, col0 + 16 * ct);
-            if (sync) lds_barrier();
             advance(b, U, end, [] { return false; }, S);
           } else {
             f32x4 sq = scale(b, kRecQ);
             replace(R, sq, sum_fp32(b, b.qe, kRecQ, S));
             write(b, U, R, sq, U, c, std::true_type{}, AV, col0 + 16 * ct);
-            if (sync) lds_barrier();
             advance(b, U, end, [] { return true; }, S);
           }
         };
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) chunk(S[ct], ct, CT == 1 && w >= 4);
-        if (CT == 2 || w < 4) lds_barrier();
+        for (int ct = 0; ct < CT; ++ct) chunk(S[ct], ct);
+        lds_barrier();
       }
       if (nc & 1) lds_barrier();
       if (PASS == 1) {
@@ -2389,7 +2385,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
 }
 
 template <typename T, int MODE, int DK, int VEC, int CT>
-__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, (walk_simd_waves<MODE, DK, CT>()))
+__global__ void __launch_bounds__((walk_threads<MODE, DK>()), (walk_simd_waves<MODE, DK, CT>()))
 scan_walk_kernel(ChunkArgs a, int portion0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg{find_portion(a, portion0 + static_cast<int>(blockIdx.y)), 0, 1, 0, 0};
@@ -2398,7 +2394,7 @@ scan_walk_kernel(ChunkArgs a, int portion0) {
 
 // segment0 + blockIdx.y = segment of the batch.  First kernel: pass 1, and the portions that are not cut.
 template <typename T, int MODE, int DK, int VEC, int CT>
-__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, (walk_simd_waves<MODE, DK, CT>()))
+__global__ void __launch_bounds__((walk_threads<MODE, DK>()), (walk_simd_waves<MODE, DK, CT>()))
 scan_segments_kernel(ChunkArgs a, int segment0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg = find_segment<false>(a, segment0 + blockIdx.y);
@@ -2409,7 +2405,7 @@ scan_segments_kernel(ChunkArgs a, int segment0) {
     walk<T, MODE, DK, VEC, 1, CT>(a, sg, lds);
 }
 template <typename T, int MODE, int DK, int VEC, int CT>
-__global__ void __launch_bounds__(kWalkThreads / CT + (CT - 1) * 128, (walk_simd_waves<MODE, DK, CT>()))
+__global__ void __launch_bounds__((walk_threads<MODE, DK>()), (walk_simd_waves<MODE, DK, CT>()))
 scan_segments_end_kernel(ChunkArgs a, int segment0) {
   __shared__ __attribute__((aligned(16))) WalkLds<MODE, DK, exact_values<T, MODE>(), exact_rows<T, MODE>()> lds;
   const Segment sg = find_segment<true>(a, segment0 + blockIdx.y);
@@ -2438,7 +2434,7 @@ int launch(const ChunkArgs& a, hipStream_t st) {
   const unsigned gx = a.H / shape.heads * ((a.dv + shape.cols - 1) / shape.cols);
   auto walk = [&](auto tiles) {
     constexpr int CT = decltype(tiles)::value;
-    const dim3 block(kWave * (shape.waves / CT + operand_waves(MODE, DK)));
+    const dim3 block(walk_threads<MODE, DK>());
     if constexpr (MODE < kModeDelta) {
       if (a.seg_states > 0) {
         // at most a segment per portion, and those of the cut ones
@@ -2455,8 +2451,8 @@ int launch(const ChunkArgs& a, hipStream_t st) {
       hipLaunchKernelGGL((scan_walk_kernel<T, MODE, DK, VEC, CT>), grid, block, 0, st, b, first);
     });
   };
-  constexpr bool WIDE = MODE < kModeDelta && VEC == 2;
-  if (WIDE && shape.waves == 8) walk(std::integral_constant<int, WIDE ? 2 : 1>{});
+  constexpr bool WIDE = MODE < kModeDelta;
+  if (WIDE && shape.tiles == 8) walk(std::integral_constant<int, WIDE ? 2 : 1>{});
   else walk(std::integral_constant<int, 1>{});
   return static_cast<int>(hipGetLastError());
 }
