@@ -29,7 +29,7 @@
 // errors below fp32 products' (they add eight terms between roundings, those four), and a sum over 128 rows takes 24
 // instructions of 16 cycles instead of 32 of 32 cycles.  What a part leaves of its number is a matrix product too (Identity):
 // the parts of 128 rows take 48 vector instructions in place of 176.
-// The products' waves go through full chunks in an order of their own (`full` below), 32 columns per wave where the operands
+// The products' waves go through chunks in an order of their own (`ours` below), 32 columns per wave where the operands
 // serve 128, so that every operand read from LDS is used twice.  Walk, us, before / with parts by products / in order:
 // delta rule per channel, 4 x 1.9k tokens 257 / 241 / 222, forget gate, 16 x 460 158 / 148 / 129; without the operands'
 // waves' work 207 / 196 and 125 / 119, without the products' 165 / 135 and 114 / 104.
@@ -1626,14 +1626,15 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       for (int c = 0; c <= nc + (nc & 1); ++c) lds_barrier();
       return;
     }
-    // Full chunks of ordinary numbers are walked in loops of their own.  A wave issues in order, and left to
-    // itself the compiler puts every load, part and product right in front of what waits for it; here all have been on their
-    // way for a few products.  A chunk that is not ordinary is left, untouched, to the loop behind (two ways in one loop cost
-    // a move per number of the state and chunk).  Columns past the last one go along, on copies of the last one's values, and
-    // are not stored: the loop behind takes a wave's two tiles one after the other, and everybody waits for it at the barrier
-    // (us, such waves in the loop behind / here, 32 heads, 16 x 512, 96 columns: forget gate 267 / 233, state space 190 / 150;
-    // 96 heads of 40, one prompt of 1023 in 32 bits 97 / 86).
-    const int full = !DELTA || col0 + 16 <= a.dv ? n / kScanChunk : 0;
+    // Chunks of ordinary numbers (delta rule: full ones of full columns) are walked in loops of their own.  A wave issues in
+    // order, and left to itself the compiler puts every load, part and product right in front of what waits for it; here all
+    // have been on their way for a few products.  A chunk that is not ordinary is left, untouched, to the loop behind (two ways
+    // in one loop cost a move per number of the state and chunk), which takes a wave's two tiles one after the other, and
+    // everybody waits for it at the barrier.  Columns past the last one go along, on copies of the last one's values, and tokens
+    // past it, on zeros; neither is stored.  us, such waves and chunks in the loop behind / here: 32 heads, 16 x 512, 96 columns,
+    // forget gate 267 / 233, state space 190 / 150; 96 heads of 40, one prompt of 1023 in 32 bits 97 / 86; state space, 32 heads,
+    // 64 x 12 tokens 90 / 85, keys of 66 channels in 32 bits 100 / 96.
+    const int ours = !DELTA ? nc : col0 + 16 <= a.dv ? n / kScanChunk : 0;
     int c = 0;
     lds_barrier();
     if constexpr (DELTA) {
@@ -1645,7 +1646,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
       if constexpr (NT == 8) {
         u32x4 p[3][3];   // of S's rows 0 - 31 and 96 - 127, 32 - 63, 64 - 95
         state_parts(p[0], 0, S[0]);
-        for (; c < full; ++c) {
+        for (; c < ours; ++c) {
           const Buf& b = lds.buf[c % BUFS];
           const auto& key_rows = *reinterpret_cast<const typename Buf::Rows*>(&b.ke);
           Sum Ws = {zero, {zero, zero}}, Rs = Ws;
@@ -1894,7 +1895,7 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
         return end;
       };
       auto worst = [&](const Buf& b) { return CH ? 0.f : b.scale[head][kRecNoParts - kRecQ]; };
-      for (; c < full; ++c) {
+      for (; c < ours; ++c) {
         const Buf& b = lds.buf[c % BUFS];
         f32x4 U[CT], f[2][2];
         Kt hm[2][2];
@@ -1993,9 +1994,16 @@ __device__ __forceinline__ void walk(const ChunkArgs& a, const Segment sg, WalkL
             if (MODE == kModeStateSpace) O += skip * U[ct];
             float* oc = op + static_cast<int64_t>(c) * kScanChunk * o_stride;
             const unsigned at = (4 * gr * o_stride + col0 + 16 * ct + m) * sizeof(float);
-            if (col0 + 16 * ct + m < a.dv)
+            if (n - c * kScanChunk >= kScanChunk) {   // (uniform)
+              if (col0 + 16 * ct + m < a.dv)
 #pragma unroll
-              for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = O[i];
+                for (int i = 0; i < 4; ++i) at_bytes<float>(oc + i * o_stride, at) = O[i];
+            } else {
+              const int rows = col0 + 16 * ct + m < a.dv ? n - c * kScanChunk - 4 * gr : 0;
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (i < rows) at_bytes<float>(oc + i * o_stride, at) = O[i];
+            }
           }
         } else {
           keys(0);
