@@ -1,8 +1,12 @@
 """The in-tree native libraries build for gfx950 and load on a CPU-only host (catches
 undefined symbols / missing registrations before a GPU box ever sees them)."""
 import re
+import struct
+import subprocess
 import types
+from pathlib import Path
 
+import pytest
 import torch
 
 from agentic_traffic_testing_amd.ops import build
@@ -151,3 +155,41 @@ def test_flash_kernels_share_their_assembly():
     assert len(llama) >= 3
     # (4-byte transfers are the mixers' alone)
     assert mixers - llama == {t for t in mixers if "global_load_lds_dword %1" in t} and llama <= mixers
+
+
+def kernel_resources(so, tmp_path):
+    """{kernel: its metadata's numbers} of a library built here."""
+    readelf, data, found = Path(build.ROCM) / "llvm/bin/llvm-readelf", Path(so).read_bytes(), {}
+    if not readelf.exists():
+        pytest.skip("no llvm-readelf")
+    for start in (m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)):
+        at = start + 32
+        for _ in range(struct.unpack_from("<Q", data, start + 24)[0]):
+            offset, size, n = struct.unpack_from("<3Q", data, at)
+            if b"gfx950" in data[at + 24:at + 24 + n]:
+                (tmp_path / "object").write_bytes(data[start + offset:start + offset + size])
+                text = subprocess.run([readelf, "--notes", tmp_path / "object"], capture_output=True, text=True, check=True).stdout
+                for kernel in text.split("- .agpr_count:")[1:]:
+                    values = dict(re.findall(r"\.(\w+): +(\S+)", kernel))
+                    found[values["name"]] = {k: int(v) for k, v in values.items() if v.isdigit()}
+            at += 24 + n
+    return found
+
+
+def test_walk_of_the_recurrences_keeps_to_its_registers(tmp_path):
+    """Without a delta rule nothing of the walk's is in scratch where a workgroup has a CU to itself, keys of 65 - 128 channels;
+    narrower ones, one tile of columns per wave: two workgroups of eight waves fit on a CU, by registers and LDS."""
+    wide = narrow = 0
+    for name, r in kernel_resources(build.build_mixers(), tmp_path).items():
+        m = re.search(r"scan_(?:walk|segments|segments_end)_kernelI(?:f|DF16b)Li(\d)ELi(\d+)ELi\dELi(\d)E", name)
+        if m is None:
+            continue
+        mode, keys, tiles = map(int, m.groups())
+        if mode < 3 and keys == 128:
+            wide += 1
+            assert r["private_segment_fixed_size"] == 0, (name, r)
+        if keys == 64 and tiles == 1:
+            narrow += 1
+            assert r["vgpr_count"] <= 512 // 4 and 2 * r["group_segment_fixed_size"] <= 160 * 1024, (name, r)
+    # (forms, types, alignments, tiles, kernels)
+    assert wide >= 3 * 2 * 3 * 2 * 3 and narrow >= 3 * 2 * 2 * 3 + 2 * 2
