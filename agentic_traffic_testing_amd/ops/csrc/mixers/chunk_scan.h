@@ -62,17 +62,17 @@ constexpr int scan_record_floats(int mode, int dk) {
 // A workgroup of the walk: four waves beside four that prepare the operands, with two tiles of 16 columns of S each (wide:
 // the operands serve 128 columns, or two heads of 64 whose keys are the same) or with one, 64 columns; so the delta rule,
 // whose portions are not cut, with up to eight waves for its operands.  256 workgroups run at once.  In `units` of a head's
-// 64 columns, S portions make S x units of them (the figures are of wide workgroups of eight waves with one tile each):
+// 64 columns, S portions make S x units of them:
 // - From 512 on wide, if there are 6 chunks per CU: few rows in many portions are decode rows and one prompt, which is
 //   done sooner in more workgroups (state space, 32 heads, us, narrow / wide: 63 rows + 128 64 / 69, 127 + 256
-//   123 / 132, 31 + 300 74 / 80, but 64 x 12 132 / 93, 127 + 600 192 / 170, 8 x 512 127 / 91 and, on the wrong side of the
-//   line, 20 + 8 x 40 50 / 40); from 257 on if there are as many as for long portions.
+//   125 / 128, 31 + 300 68 / 75, but 64 x 12 92 / 86, 127 + 600 184 / 162, 8 x 512 103 / 88 and, on the wrong side of the
+//   line, 20 + 8 x 40 47 / 42); from 257 on if there are as many as for long portions.
 // - 192 - 256 fill the chip with narrow ones, and uncut: a portion in half the workgroups would have to be cut to fill it
-//   (32 heads, narrow uncut / wide cut: retention 4 x 350 55 / 72, 4 x 1000 135 / 159, 4 x 2000 283 / 297, forget gate
-//   4 x 700 126 / 135, state space 4 x 1000 121 / 130, 8 heads 16 x 512 68 / 86).
+//   (32 heads, narrow uncut / wide cut: retention 4 x 350 60 / 68, 4 x 1000 134 / 138, 4 x 2000 260 / 269, forget gate
+//   4 x 700 107 / 112, state space 4 x 1000 98 / 114, 8 heads 16 x 512 59 / 77).
 // - Fewer: long portions are cut, and wide where a 16th of the batch per segment is enough to fill the chip (32
-//   heads, one prompt of 2048, narrow / wide: retention 120 / 98, state space 102 / 84; 8 heads, 4 x 2000: retention
-//   120 / 143, one of 8192 138 / 156).
+//   heads, one prompt of 2048, narrow / wide: retention 112 / 89, state space 82 / 76; 8 heads, 4 x 2000: retention
+//   114 / 127, one of 8192 121 / 141).
 struct WalkShape {
   int tiles, heads, cols;   // of 16 columns, one or two per wave; heads per workgroup; columns per workgroup and head
 };

@@ -23,7 +23,9 @@
 //   chunk), with their loads one or two steps ahead of that.
 //
 // Bound of the walk: the chain of a chunk's products, parts and LDS reads in a wave that has a SIMD's matrix unit to itself,
-// and the operands' vector work beside it.  fp32 matrix products run on the vector units (the walk with 16x16x4 products:
+// and the operands' vector work beside it (vector and matrix units busy, of the kernel's time: delta rule per channel 50 and
+// 42 %, forget gate 55 and 33, second pass of state space in 32 bits 32 and 28, of retention 39 and 21; scores of the first
+// two vector 79 and 67, matrix 14 and 8).  fp32 matrix products run on the vector units (the walk with 16x16x4 products:
 // matrix busy 36 - 42 %, vector busy 50 %, and twelve waves per CU bring no more than eight), bf16 ones beside them.
 // So the products with the state are made of bf16 parts: three parts hold the 24 bits of a number, six products of parts leave
 // errors below fp32 products' (they add eight terms between roundings, those four), and a sum over 128 rows takes 24
@@ -39,10 +41,10 @@
 // Measured: the token-by-token kernels, fp32 products with 64 columns per workgroup, bf16 parts, and with the scores' halves of
 // channels, pairs inside four tokens and values in one part where they are exact (us, scores + walk; 32 heads of 128, bf16
 // unless noted):
-//   delta rule, per-channel decay, 4 x ~1850 tokens: 1798, 130 + 343, 132 + 262, 99 + 256, today 83 + 224
-//   forget gate, 16 x ~460 tokens:                    777, 111 + 308, 98 + 168, 83 + 158, today 71 + 129
-//   state space, 96 heads of 128 x 64, 1023 tokens, fp32: 250, 21 + 94, 22 + 64, 19 + 63 in five segments of head pairs
-//   retention, one portion of 1500 tokens (+ 11 rows): 260, 21 + 88, 22 + 69, 21 + 65 in eight segments, the rows inside the
+//   delta rule, per-channel decay, 4 x ~1850 tokens: 1798, 130 + 343, 132 + 262, 99 + 256, today 84 + 232
+//   forget gate, 16 x ~460 tokens:                    777, 111 + 308, 98 + 168, 83 + 158, today 70 + 136 + 5 (both passes)
+//   state space, 96 heads of 128 x 64, 1023 tokens, fp32: 250, 21 + 94, 22 + 64, 18 + 64 in five segments of head pairs
+//   retention, one portion of 1500 tokens (+ 11 rows): 260, 21 + 88, 22 + 69, 21 + 61 in eight segments, the rows inside the
 //   scores launch
 // What did not work: 16x16x4 products with a second wave per SIMD for the read-out (delta rule: no gain, see above);
 // waves of a SIMD half a step apart without that; a higher priority for the operands' waves (delta rule + 15 %); four tiles
@@ -104,7 +106,9 @@ __device__ __forceinline__ float abs_sum(const f32x4 x) { return (fabsf(x[0]) + 
 // The same for four numbers per lane, what a part leaves by the matrix cores: minus the identity times the part, added to
 // the numbers.  Their layout as 16 x 16 numbers is that of the part as an operand of 16 rows, and one product (16 cycles
 // beside the vector units) takes the place of four instructions that unpack the part and four that subtract it; the
-// difference has at most 24 bits, and it is exact.  A number without parts leaves NaN in the lane's and the column's
+// difference has at most 24 bits, and it is exact.  Between a product of 16 terms, as this one is, and one of 32 that adds to
+// its result a vector instruction has to use that result (the compiler leaves too few cycles: first_parts()); what is left of
+// a number is packed into the next part, so it always does.  A number without parts leaves NaN in the lane's and the column's
 // other three lanes' parts 1 and 2, so it is for numbers whose products are looked at by column, or that have parts.
 struct Identity {
   u32x2 minus;   // row m, columns 4 gr ... + 3

@@ -160,8 +160,9 @@ __global__ __launch_bounds__(256) void rope_cache_tile_kernel(
 // throughout, so all of its rows, its V and its 16 numbers of the table are loaded before any is used (above, every task's
 // loads wait for its token's position), and the pages' addresses are worked out once per token.
 // Workgroups of a tile's KV heads are neighbours, so that a token's row is read at one time.
-// Bound: memory traffic.  Llama layer of 7580 tokens, 32 + 8 + 8 heads (186 MB here; a copy of as many bytes takes 28 us):
-// tiles 169.9 us, here 165.7, KV heads side by side 164.2.
+// Bound: memory traffic.  Llama layer of 7580 tokens, 32 + 8 + 8 heads (186 MB in 33 us; a copy of as many bytes takes 26 us
+// between buffers that stay in the 256 MB cache, 36 from and to memory): tiles 169.9 us, here 165.7, KV heads side by side
+// 164.2.
 template <typename T, int G>
 __global__ __launch_bounds__(256) void rope_cache_group_kernel(
     uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,

@@ -157,22 +157,33 @@ def test_flash_kernels_share_their_assembly():
     assert mixers - llama == {t for t in mixers if "global_load_lds_dword %1" in t} and llama <= mixers
 
 
-def kernel_resources(so, tmp_path):
-    """{kernel: its metadata's numbers} of a library built here."""
-    readelf, data, found = Path(build.ROCM) / "llvm/bin/llvm-readelf", Path(so).read_bytes(), {}
-    if not readelf.exists():
-        pytest.skip("no llvm-readelf")
+def code_objects(so):
+    """The gfx950 code objects of a library built here."""
+    data = Path(so).read_bytes()
     for start in (m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)):
         at = start + 32
         for _ in range(struct.unpack_from("<Q", data, start + 24)[0]):
             offset, size, n = struct.unpack_from("<3Q", data, at)
             if b"gfx950" in data[at + 24:at + 24 + n]:
-                (tmp_path / "object").write_bytes(data[start + offset:start + offset + size])
-                text = subprocess.run([readelf, "--notes", tmp_path / "object"], capture_output=True, text=True, check=True).stdout
-                for kernel in text.split("- .agpr_count:")[1:]:
-                    values = dict(re.findall(r"\.(\w+): +(\S+)", kernel))
-                    found[values["name"]] = {k: int(v) for k, v in values.items() if v.isdigit()}
+                yield data[start + offset:start + offset + size]
             at += 24 + n
+
+
+def llvm(tool, *args):
+    path = Path(build.ROCM) / "llvm/bin" / tool
+    if not path.exists():
+        pytest.skip(f"no {tool}")
+    return subprocess.run([path, *args], capture_output=True, text=True, check=True).stdout
+
+
+def kernel_resources(so, tmp_path):
+    """{kernel: its metadata's numbers} of a library built here."""
+    found = {}
+    for code in code_objects(so):
+        (tmp_path / "object").write_bytes(code)
+        for kernel in llvm("llvm-readelf", "--notes", tmp_path / "object").split("- .agpr_count:")[1:]:
+            values = dict(re.findall(r"\.(\w+): +(\S+)", kernel))
+            found[values["name"]] = {k: int(v) for k, v in values.items() if v.isdigit()}
     return found
 
 
@@ -193,3 +204,46 @@ def test_walk_of_the_recurrences_keeps_to_its_registers(tmp_path):
             assert r["vgpr_count"] <= 512 // 4 and 2 * r["group_segment_fixed_size"] <= 160 * 1024, (name, r)
     # (forms, types, alignments, tiles, kernels)
     assert wide >= 3 * 2 * 3 * 2 * 3 and narrow >= 3 * 2 * 2 * 3 + 2 * 2
+
+
+def products_added_at_once(lines):
+    """Matrix products of 32 terms that add to the result of one of 16 which no vector instruction has used in between."""
+    def registers(x):
+        m = re.match(r"v\[(\d+):(\d+)\]$", x) or re.match(r"v((\d+))$", x)
+        return range(int(m[1]), int(m[2]) + 1) if m else ()
+
+    fresh = set()
+    for line in lines:
+        op, _, args = line.split("//")[0].strip().partition(" ")
+        if not op.startswith("v_"):
+            if line.endswith(">:"):
+                fresh.clear()
+            continue
+        if not fresh and not op.startswith("v_mfma_f32_16x16x16"):
+            continue
+        args = [x.strip() for x in args.split(",")]
+        if op.startswith("v_mfma_f32_16x16x16"):
+            fresh.update(registers(args[0]))
+        elif op.startswith("v_mfma"):
+            if "16x16x32" in op and fresh.intersection(registers(args[3])):
+                yield line
+            fresh.difference_update(registers(args[0]))
+        else:
+            for x in args:
+                fresh.difference_update(registers(x))
+
+
+def test_products_of_32_terms_wait_for_those_of_16(tmp_path):
+    """The compiler leaves too few cycles between the two where nothing else reads the sum: the recurrences' kernels keep a
+    vector instruction in between."""
+    first, then = "v_mfma_f32_16x16x16_bf16 v[0:3], v[8:9], v[10:11], 0", "v_mfma_f32_16x16x32_bf16 v[4:7], v[12:15], v[16:19], v[0:3]"
+    assert list(products_added_at_once([first, "s_nop 1", then])) == [then]
+    assert not list(products_added_at_once([first, "v_fma_f32 v0, v0, v20, v21", "v_add_f32_e32 v30, v1, v2", "v_mov_b32_e32 v3, v3", then]))
+    lines = pairs = 0
+    for code in code_objects(build.build_mixers()):
+        if b"scan_walk_kernel" in code:
+            (tmp_path / "object").write_bytes(code)
+            text = llvm("llvm-objdump", "-d", "--mcpu=gfx950", "--no-show-raw-insn", tmp_path / "object")
+            lines += text.count("v_mfma_f32_16x16x16")
+            pairs += len(list(products_added_at_once(text.split("\n"))))
+    assert lines > 1000 and pairs == 0
